@@ -275,6 +275,10 @@ void build_ghosts(mapp_dmd* ctx) {
     HIP_OK(hipStreamSynchronize(ctx->stream));
 }
 
+// columns of the per-site alpha / c arrays: nt for DMD, one (the type) for EAM
+inline bool is_md(const mapp_dmd* ctx) { return ctx->variant >= MAPP_DMD_VARIANT_EAM; }
+inline int acols(const mapp_dmd* ctx) { return is_md(ctx) ? 1 : ctx->nt; }
+
 template <int NT>
 void finish_lists(mapp_dmd* ctx);
 void finish_meam(mapp_dmd* ctx);
@@ -370,6 +374,12 @@ void finish_lists(mapp_dmd* ctx) {
     ctx->d_pair_i.reserve(ctx->npairs + 1);
     hipLaunchKernelGGL(k_pair_owner, dim3(nblk(natms)), dim3(kBlock), 0, st, ctx->d_off.p, natms, ctx->d_pair_i.p);
     launch_check("k_pair_owner");
+    if (!is_md(ctx) && nrev > 0) {
+        ctx->d_rowner.reserve(nrev);
+        hipLaunchKernelGGL(k_rev_owner, dim3(nblk(nrev)), dim3(kBlock), 0, st, ctx->d_rev.p, ctx->d_pair_i.p, nrev,
+                           ctx->d_rowner.p);
+        launch_check("k_rev_owner");
+    }
     ctx->nrev = nrev;
     // element read by the reference's dE[jatm + jtype] quirk: jatm + jtype (one cell)
     ctx->d_qidx.reserve((size_t)ntot * NT);
@@ -387,12 +397,17 @@ void finish_lists(mapp_dmd* ctx) {
     ctx->d_f.reserve((size_t)natms * (3 + NT));
     ctx->d_fown.reserve((size_t)natms * (3 + NT));
     ctx->d_pairE.reserve((size_t)(nrev + 1) * NT);
-    ctx->d_deriv.reserve((size_t)(ctx->npairs + 1) * DerivRec<NT>::kLen);
-    ctx->d_pairF.reserve((size_t)(nrev + 1) * (3 + NT));
-    // every pair starts outside the quadrature cut with zero partner shares; pass 1
-    // writes the shares of the pairs inside and clears those of a pair that leaves
-    HIP_OK(hipMemsetAsync(ctx->d_pairE.p, 0, sizeof(double) * (size_t)(nrev + 1) * NT, st));
-    HIP_OK(hipMemsetAsync(ctx->d_pairF.p, 0, sizeof(double) * (size_t)(nrev + 1) * (3 + NT), st));
+    if (is_md(ctx)) {
+        ctx->d_pairF.reserve((size_t)(nrev + 1) * 3);
+    } else {
+        // pass 1's records in either quadrature type
+        using R = PairRec<NT, double>;
+        ctx->d_pairF.reserve((size_t)(nrev + 1) * ForceShare<NT>::kLen);
+        // every pair starts outside the quadrature cut with a zero density share
+        HIP_OK(hipMemsetAsync(ctx->d_pairE.p, 0, sizeof(double) * (size_t)(nrev + 1) * NT, st));
+        ctx->d_deriv.reserve(R::groups(ctx->npairs, natms) * R::kG * R::kComps);
+        ctx->d_info.reserve(natms + 1);
+    }
     ctx->d_crd.reserve(ntot);
     ctx->d_x0.reserve(natms);
     HIP_OK(hipMemcpyAsync(ctx->d_x0.p, ctx->d_pos.p, sizeof(double4) * natms, hipMemcpyDeviceToDevice, st));
@@ -400,10 +415,6 @@ void finish_lists(mapp_dmd* ctx) {
     ctx->have_list2 = false;
     ctx->cache_valid = false;
 }
-
-// columns of the per-site alpha / c arrays: nt for DMD, one (the type) for EAM
-inline bool is_md(const mapp_dmd* ctx) { return ctx->variant >= MAPP_DMD_VARIANT_EAM; }
-inline int acols(const mapp_dmd* ctx) { return is_md(ctx) ? 1 : ctx->nt; }
 
 // f(std::integral_constant<int, NT>) for the number of DMD types nt = 1..kMaxTypes
 template <typename F>
@@ -638,38 +649,29 @@ void pack_atoms(mapp_dmd* ctx) {
     launch_check("k_pack_atoms");
 }
 
-// blocks of a force-pass launch: one wave per site unless the shape caps the waves
-inline int shape_blocks(const mapp_dmd::Shape& sh, int natms) {
-    const long w = sh.waves > 0 ? std::min<long>(sh.waves, natms) : natms;
+// blocks of a force-pass launch: one wave per per_wave sites unless the shape caps the waves
+inline int shape_blocks(const mapp_dmd::Shape& sh, int natms, int per_wave = 1) {
+    const long all = (natms + per_wave - 1) / per_wave;
+    const long w = sh.waves > 0 ? std::min<long>(sh.waves, all) : all;
     return (int)std::max<long>(1, (w + sh.wpb - 1) / sh.wpb);
-}
-
-// the DMD force shares inside d_pairF: nrev + 1 slots of 4 doubles, then nrev + 1 of nt - 1
-template <int NT>
-ForceShares force_shares(mapp_dmd* ctx) {
-    return ForceShares{ctx->d_pairF.p, ctx->d_pairF.p + (size_t)(ctx->nrev + 1) * 4};
 }
 
 // pass 1 with the schedule's lanes per (pair, type pair)
 template <int NT, typename Q, int NQ, bool ENERGY_ONLY, bool FULL>
-void launch_pass1(mapp_dmd* ctx, dim3 grid, const Q* quad, const FFParams<Q>& PQ, const PairBufs& L, Q* deriv,
-                  double* part) {
+void launch_pass1(mapp_dmd* ctx, dim3 grid, const Q* quad, const FFParams<Q>& PQ, const PairBufs& L,
+                  typename Vec2<Q>::T* deriv, double* part) {
     const dim3 blk(64 * ctx->sh1.wpb);
     const size_t lds = (size_t)ctx->sh1.wpb * Pass1Stage<NT>::kBytes;  // one stage per wavefront
     hipStream_t st = ctx->stream;
-    const CutState C{ctx->d_nlrp.p, force_shares<NT>(ctx)};
-    if (ctx->sh1.parts == 1)
-        hipLaunchKernelGGL((k_pass1<NT, Q, NQ, ENERGY_ONLY, FULL, 1>), grid, blk, lds, st, ctx->P, PQ, ctx->d_pos.p,
-                           ctx->d_arec.p, L, ctx->d_nlrp.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_Eown.p,
-                           ctx->d_pairE.p, deriv, part, C);
-    else if (ctx->sh1.parts == 2)
-        hipLaunchKernelGGL((k_pass1<NT, Q, NQ, ENERGY_ONLY, FULL, 2>), grid, blk, lds, st, ctx->P, PQ, ctx->d_pos.p,
-                           ctx->d_arec.p, L, ctx->d_nlrp.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_Eown.p,
-                           ctx->d_pairE.p, deriv, part, C);
-    else
-        hipLaunchKernelGGL((k_pass1<NT, Q, NQ, ENERGY_ONLY, FULL, 4>), grid, blk, lds, st, ctx->P, PQ, ctx->d_pos.p,
-                           ctx->d_arec.p, L, ctx->d_nlrp.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_Eown.p,
-                           ctx->d_pairE.p, deriv, part, C);
+    const CutState C{ctx->d_nlrp.p, ctx->d_rowner.p};
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, blk, lds, st, ctx->P, PQ, ctx->d_pos.p, ctx->d_arec.p, L.off, ctx->d_nlrp.p,
+                           quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_Eown.p, ctx->d_pairE.p, deriv, ctx->d_info.p,
+                           part, C, ctx->sh1.wpb);
+    };
+    if (ctx->sh1.parts == 1) launch(k_pass1<NT, Q, NQ, ENERGY_ONLY, FULL, 1>);
+    else if (ctx->sh1.parts == 2) launch(k_pass1<NT, Q, NQ, ENERGY_ONLY, FULL, 2>);
+    else launch(k_pass1<NT, Q, NQ, ENERGY_ONLY, FULL, 4>);
     launch_check("k_pass1");
 }
 
@@ -679,7 +681,7 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
     const int natms = ctx->natms;
     const int nb = nblk((long)natms * kGatherG);             // force gather
     const int nbe = nblk((long)natms * kEmbedG);             // embedding
-    const int nbw = shape_blocks(ctx->sh2, natms);           // pass 2
+    const int nbw = shape_blocks(ctx->sh2, natms, 64 / kPass2Lanes);  // pass 2
     // the surrogate's pass 1: one block of kSurWaves wavefronts per CU, persistent
     const int nb1 = sur ? std::min(natms, kSurBlocks) : shape_blocks(ctx->sh1, natms);
     PairBufs L{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p};
@@ -692,7 +694,7 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
     double* part1 = ctx->d_part.p;
     double* part2 = part1 + (size_t)np1 * 2;
     double* part3 = part2 + (size_t)np2;
-    Q* deriv = reinterpret_cast<Q*>(ctx->d_deriv.p);
+    auto* deriv = reinterpret_cast<typename Vec2<Q>::T*>(ctx->d_deriv.p);
     if (ctx->timing) HIP_OK(hipEventRecord(ctx->ev[0], st));
     pack_atoms<NT>(ctx);
     if constexpr (NT == 2 && std::is_same<Q, double>::value) {
@@ -706,8 +708,8 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
                 HIP_OK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSurLds));
                 hipLaunchKernelGGL(kern, dim3(nb1), dim3(kSurBlock), kSurLds, st, ctx->P, ctx->Pf, S, ctx->d_pos.p,
                                    ctx->d_arec.p, L, ctx->d_nlrp.p, ctx->d_quad32.p, ctx->d_rho7.p, ctx->d_phi7.p,
-                                   ctx->d_Eown.p, ctx->d_pairE.p, (double*)deriv, part1, ctx->d_nfall.p,
-                                   CutState{ctx->d_nlrp.p, force_shares<NT>(ctx)});
+                                   ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_deriv.p, ctx->d_info.p, part1, ctx->d_nfall.p,
+                                   CutState{ctx->d_nlrp.p, ctx->d_rowner.p});
             };
             if (q == 5) launch(k_pass1_sur<5>);
             else if (q == 3) launch(k_pass1_sur<3>);
@@ -721,7 +723,7 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
     }
     if (ctx->timing) HIP_OK(hipEventRecord(ctx->ev[1], st));
     hipLaunchKernelGGL((k_embed<NT, false>), dim3(nbe), dim3(kBlock), 0, st, ctx->P, ctx->d_alpha.p,
-                       ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_F9.p, ctx->d_E.p, ctx->d_dE.p,
+                       ctx->d_conc.p, ctx->d_roff.p, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_F9.p, ctx->d_E.p, ctx->d_dE.p,
                        ctx->d_fa.p, ctx->d_arec.p, part2);
     launch_check("k_embed");
     ghost_copy(ctx, ctx->d_dE.p, NT);
@@ -731,12 +733,12 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
         launch_check("k_ghost_copy arec");
     }
     if (ctx->timing) HIP_OK(hipEventRecord(ctx->ev[2], st));
-    hipLaunchKernelGGL((k_pass2<NT, Q>), dim3(nbw), dim3(64 * ctx->sh2.wpb), 0, st, ctx->P, ctx->d_pos.p,
-                       ctx->d_arec.p, L, ctx->d_nlrp.p, deriv, ctx->d_fown.p, force_shares<NT>(ctx), part3);
+    hipLaunchKernelGGL((k_pass2<NT, Q>), dim3(nbw), dim3(64 * ctx->sh2.wpb), 0, st, natms, ctx->d_pos.p,
+                       ctx->d_arec.p, ctx->d_info.p, deriv, ctx->d_fown.p, ctx->d_pairF.p, part3, ctx->sh2.wpb);
     launch_check("k_pass2");
     if (ctx->timing) HIP_OK(hipEventRecord(ctx->ev[3], st));
-    hipLaunchKernelGGL((k_fgather<NT>), dim3(nb), dim3(kBlock), 0, st, natms, L, ctx->d_fown.p, force_shares<NT>(ctx),
-                       ctx->d_fa.p, ctx->d_f.p);
+    hipLaunchKernelGGL((k_fgather<NT>), dim3(nb), dim3(kBlock), 0, st, natms, ctx->d_pos.p, ctx->d_roff.p,
+                       ctx->d_rowner.p, ctx->d_fown.p, ctx->d_pairF.p, ctx->d_fa.p, ctx->d_f.p);
     launch_check("k_fgather");
     double* out = ctx->d_out.p;
     {
@@ -776,12 +778,12 @@ double run_energy(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
     double* part1 = ctx->d_part.p;
     double* part2 = part1 + (size_t)np1 * 2;
     pack_atoms<NT>(ctx);
-    if (ctx->energy_full) launch_pass1<NT, Q, NQ, true, true>(ctx, dim3(nbw), quad, PQ, L, (Q*)nullptr, part1);
-    else launch_pass1<NT, Q, NQ, true, false>(ctx, dim3(nbw), quad, PQ, L, (Q*)nullptr, part1);
+    if (ctx->energy_full) launch_pass1<NT, Q, NQ, true, true>(ctx, dim3(nbw), quad, PQ, L, (typename Vec2<Q>::T*)nullptr, part1);
+    else launch_pass1<NT, Q, NQ, true, false>(ctx, dim3(nbw), quad, PQ, L, (typename Vec2<Q>::T*)nullptr, part1);
     launch_check("k_pass1 energy");
     hipLaunchKernelGGL((k_embed<NT, true>), dim3(nb), dim3(kBlock), 0, st, ctx->P, ctx->d_alpha.p, ctx->d_conc.p,
-                       L, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_F9.p, ctx->d_E.p, ctx->d_dE.p, ctx->d_fa.p,
-                       ctx->d_arec.p, part2);
+                       ctx->d_roff.p, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_F9.p, ctx->d_E.p, ctx->d_dE.p,
+                       ctx->d_fa.p, ctx->d_arec.p, part2);
     launch_check("k_embed energy");
     double* out = ctx->d_out.p;
     {
@@ -848,6 +850,9 @@ void upload_tables(mapp_dmd* ctx) {
                     d[(size_t)m * quad_stride(nt) + 4 + k] = ps[(size_t)m * 7 + k];
                 }
         }
+    // row nr - 1 of the quadrature tables is zero: pass 1 reads it for the points beyond
+    // the cutoff (no evaluation inside it uses a row past nr - 2)
+    std::fill(q64.end() - quad_stride(nt), q64.end(), 0.0);
     for (size_t k = 0; k < q64.size(); ++k) q32[k] = (float)q64[k];
     ctx->d_quad64.reserve(q64.size());
     ctx->d_quad32.reserve(q32.size());
@@ -881,6 +886,8 @@ void fill_float_params(mapp_dmd* ctx) {
     F.alpha_max = (float)P.alpha_max;
     F.inv_amin = (float)P.inv_amin;
     F.inv_amax = (float)P.inv_amax;
+    F.ia_quad_lo = (float)P.ia_quad_lo;
+    F.ia_quad_hi = (float)P.ia_quad_hi;
     F.kbT = (float)P.kbT;
     F.beta = (float)P.beta;
     F.xw = (float)P.xw;
@@ -1662,16 +1669,20 @@ void sur_scales(mapp_dmd* ctx, const SurNorm& Nm, const std::vector<double>& pro
     if (ctx->npairs > 0)
         HIP_OK(hipMemcpy(nl.data(), ctx->d_nl.p, (size_t)ctx->npairs * sizeof(int), hipMemcpyDeviceToHost));
     std::vector<double> pairE((size_t)std::max(roff[natms], 1) * nt);
-    if (roff[natms] > 0)
+    std::vector<int> rowner((size_t)std::max(roff[natms], 1));
+    if (roff[natms] > 0) {
         HIP_OK(hipMemcpy(pairE.data(), ctx->d_pairE.p, (size_t)roff[natms] * nt * sizeof(double),
                          hipMemcpyDeviceToHost));
+        HIP_OK(hipMemcpy(rowner.data(), ctx->d_rowner.p, (size_t)roff[natms] * sizeof(int), hipMemcpyDeviceToHost));
+    }
     double fmax = 0.0, dfmax = 0.0, rho_lo = 1e300, rho_hi = -1e300;
     for (double v : f) fmax = std::max(fmax, std::fabs(v));
     for (double v : dE) dfmax = std::max(dfmax, std::fabs(v));
     for (int i = 0; i < natms; ++i)
         for (int t = 0; t < nt; ++t) {
             double rho = Eown[(size_t)i * nt + t];
-            for (int q = roff[i]; q < roff[i + 1]; ++q) rho += pairE[(size_t)q * nt + t];
+            for (int q = roff[i]; q < roff[i + 1]; ++q)
+                if (rowner[q] < 0) rho += pairE[(size_t)q * nt + t];  // inside the cut
             rho_lo = std::min(rho_lo, rho);
             rho_hi = std::max(rho_hi, rho);
         }
@@ -2109,6 +2120,10 @@ int mapp_dmd_coef(mapp_dmd_t* ctx, double r_crd, int no_i, double alpha_min, dou
         P.alpha_max = alpha_max;
         P.inv_amin = 1.0 / alpha_min;
         P.inv_amax = 1.0 / alpha_max;
+        // 1/alpha strictly between these: the quadrature regime, beyond the rounding that
+        // alpha_branch looks into
+        P.ia_quad_lo = P.inv_amax * (1.0 + 4e-12);
+        P.ia_quad_hi = P.inv_amin * (1.0 - 4e-12);
         const double kb = 8.617332478e-5, hbar = 6.5821192815e-16;
         for (int t = 0; t < kMaxTypes; ++t) P.c0[t] = 0.0;
         for (int t = 0; t < ctx->nt; ++t) {

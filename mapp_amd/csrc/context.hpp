@@ -54,8 +54,9 @@ struct mapp_dmd {
     mappdmd::DevBuf<int> d_off2, d_nl2, d_roff2, d_rev2, d_crd;
     mappdmd::DevBuf<int> d_sort_tmp;  // out-of-place segment sort
     mappdmd::DevBuf<int> d_pair_i, d_pair_i2, d_rpos;
-    mappdmd::DevBuf<double> d_inva, d_deriv;
-    mappdmd::DevBuf<double4> d_arec;  // [ntot][nt] {alpha, c, 1/alpha, dE}  // deriv: [npairs][DerivRec<nt>::kLen] of the quadrature type
+    mappdmd::DevBuf<double2> d_deriv;  // pass 1's records (PairRec) of the quadrature type
+    mappdmd::DevBuf<int2> d_info;      // [natms] {list offset, pairs inside the cut at the last force pass 1}
+    mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}
     long nrev = 0;
     std::vector<mappdmd::DevBuf<int>*> scan_levels;
     long npairs = 0, npairs2 = 0;
@@ -63,10 +64,13 @@ struct mapp_dmd {
     // per-atom vectors ([ntot][nt] unless noted) and pair buffers
     mappdmd::DevBuf<double> d_E, d_dE, d_ddE, d_n, d_s, d_t, d_v, d_cd, d_fa, d_Eown, d_a, d_g;
     mappdmd::DevBuf<double> d_f, d_fown;        // [natms][3+nt]
-    mappdmd::DevBuf<double> d_pairE, d_pairF;   // [npairs][nt], [npairs][3+nt]
-    // per half-list entry {partner, reverse position}; the partner's top bit: inside the
-    // quadrature cut at the last pass 1 (the shares of entries outside it stay zero)
+    // partner shares in reverse-list order: densities [nrev][nt]; forces, DMD
+    // [nrev][ForceShare<nt>::kLen], MD potentials [nrev][3]
+    mappdmd::DevBuf<double> d_pairE, d_pairF;
+    // DMD: per half-list entry {partner, reverse position} and per reverse-list entry the
+    // pair's owner; the top bit of the first: inside the quadrature cut at the last pass 1
     mappdmd::DevBuf<int2> d_nlrp;
+    mappdmd::DevBuf<int> d_rowner;
     mappdmd::DevBuf<double> d_rhoc, d_phic;     // pair values for c_d_calc / calc_g, per half-list pair
     mappdmd::DevBuf<int> d_toff, d_tidx;        // site table: both ends of every contributing pair
     mappdmd::DevBuf<double> d_trho, d_tphi;

@@ -20,6 +20,7 @@ template <typename T>
 struct FFParams {
     int natms, ntot, nr, nrho, no_i;
     T dr_inv, drho_inv, rho_max, rc, cut_sq, cut_sq_mod, alpha_min, alpha_max, inv_amin, inv_amax;
+    T ia_quad_lo, ia_quad_hi;  // 1/alpha between these: surely the quadrature regime
     T kbT, beta;
     T xw;  // energy weight of cross-type pair terms: 1 (reference) or 2 (consistent energy)
     T xi[kMaxPoints], w0[kMaxPoints], w1[kMaxPoints], w2[kMaxPoints];

@@ -10,13 +10,13 @@
 //            averaged density and pair terms, the site's own density sums
 //            stay in registers, the partner's density share (nt doubles)
 //            goes to its share slot, and the r- and alpha-derivatives go to
-//            the pair's derivative record (DerivRec);
+//            the pair's derivative record (PairRec);
 //   embed    a lane group per site adds the density shares of the sites that
 //            list it (reverse CSR, ascending pair index), then F(rho_bar), F',
 //            the per-site energy terms and the alpha entropic force;
-//   pass 2   lanes (pair, type pair) combine the derivative records with F'
-//            of both ends into the site's force row and the partner's force
-//            share (3 + nt doubles);
+//   pass 2   half a wavefront per site, one lane per pair: the lane combines the
+//            pair's derivative record with F' of both ends into the site's force
+//            row and the partner's force share (3 + nt doubles);
 //   gather   a lane group per site adds its force shares (reverse CSR).
 // No floating-point atomics: every sum has a fixed order, so results are
 // bitwise reproducible run to run.  Energy and virial partials are written per
@@ -210,52 +210,48 @@ struct PairBufs {
     const int* rev;
 };
 
-// Partner force shares of the DMD passes, one slot per reverse-list entry, in
-// two arrays: sh4[slot] = {fx, fy, fz, alpha force of type 0} (32 bytes, so a
-// pair's share is written with 16-byte stores) and shx[slot] = the alpha
-// forces of types 1..nt-1.
-struct ForceShares {
-    double* sh4;
-    double* shx;
-};
-
-// Which half-list entries lay inside the quadrature cut at the last pass 1:
-// the top bit of the partner index in the packed list {partner, reverse
-// position}, read with the entry at no extra cost.  The partner shares (pairE
-// of pass 1, the force shares of pass 2) of an entry outside the cut must read
-// zero in the embedding and the force gather: they are cleared when the list
-// is built and again only when an entry leaves the cut, instead of being
-// rewritten with zeros at every evaluation.
+// Which half-list entries lay inside the quadrature cut at the last pass 1: the
+// top bit of the partner index in the packed list {partner, reverse position},
+// read with the entry at no extra cost, and the top bit of the owner's index in
+// the partner's reverse list, by which the force gather knows the shares that
+// count.  Both are written only when an entry enters or leaves the cut.  The
+// density share of an entry outside reads zero in the embedding: it is cleared
+// when the list is built and again only when the entry leaves (the embedding
+// reading the owners too took 0.29 ms in place of 0.21 at 1,048,576 sites).
 constexpr int kInsideBit = (int)0x80000000u;
 __device__ __forceinline__ int list_partner(int2 e) { return e.x & 0x7fffffff; }
 struct CutState {
     int2* nlrp;
-    ForceShares F;
-    // entry pc (as read: e, partner jc) is inside the cut now: record a change; on
-    // leaving, clear both shares of an owned partner
+    int* rowner;
+    // entry pc of owner i (as read: e, partner jc) is inside the cut now or not: record a
+    // change; on leaving, clear the density share of an owned partner
     template <int NT>
-    __device__ __forceinline__ void update(int pc, int2 e, bool in, int jc, int natms, double* pairE) const {
+    __device__ __forceinline__ void update(int pc, int2 e, bool in, int i, int jc, int natms, double* pairE) const {
         const bool was = (e.x & kInsideBit) != 0;
         if (was != in) {
             nlrp[pc].x = in ? (jc | kInsideBit) : jc;
-            if (!in && jc < natms) {
-                const int rp = e.y;
+            if (jc < natms) {
+                rowner[e.y] = in ? (i | kInsideBit) : i;
+                if (!in) {
 #pragma unroll
-                for (int t = 0; t < NT; ++t) pairE[(size_t)rp * NT + t] = 0.0;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) F.sh4[(size_t)rp * 4 + c] = 0.0;
-#pragma unroll
-                for (int c = 0; c < NT - 1; ++c) F.shx[(size_t)rp * (NT - 1) + c] = 0.0;
+                    for (int t = 0; t < NT; ++t) pairE[(size_t)e.y * NT + t] = 0.0;
+                }
             }
         }
     }
 };
 
-// ---------------------------------------------------------------- lane mapping
-// NT*NT lanes per site, lane q = it*NT + jt owns the ordered type pair
-// (it, jt) of every pair of the site's list.  For NT = 2 the four lanes of a
-// site form a DPP quad: the transposed pair (jt, it) is quad_perm [0,2,1,3],
-// sums over jt are xor 1, sums over it are xor 2.
+// Force share of a pair, kLen doubles at the pair's position in the partner's reverse
+// list: {S, alpha forces of the partner's types}, the force on the owner being
+// S (x_owner - x_partner); padded to whole 16-byte pieces (two types: one 32-byte
+// sector, where the three components and two alpha forces took two writes of 32 and
+// 8 bytes).
+template <int NT>
+struct ForceShare {
+    static constexpr int kLen = (1 + NT + 1) / 2 * 2;
+};
+
+// ---------------------------------------------------------------- lane exchanges
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
     int lo = __double2loint(v), hi = __double2hiint(v);
@@ -263,15 +259,11 @@ __device__ __forceinline__ double dpp_f64(double v) {
     hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, false);
     return __hiloint2double(hi, lo);
 }
-constexpr int kDppTranspose = 0xD8;  // quad_perm [0,2,1,3]
 constexpr int kDppXor1 = 0xB1;       // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;       // quad_perm [2,3,0,1]
 constexpr int kDppRowRor8 = 0x128;   // row_ror:8 (rotate by 8 lanes within a row of 16)
 constexpr int kDppRowRor4 = 0x124;   // row_ror:4
 constexpr int kDppRowRor12 = 0x12C;  // row_ror:12: lane l reads lane (l + 4) mod 16 of its row
-constexpr int kDppQuad0022 = 0xA0;   // quad_perm [0,0,2,2]: lane q = 1 reads lane q = 0
-constexpr int kDppQuad0000 = 0x00;   // quad_perm [0,0,0,0]: every lane of a quad reads q = 0
-constexpr int kDppQuad0033 = 0xF0;   // quad_perm [0,0,3,3]: lane 1 reads lane 0, lane 2 reads lane 3
 
 // v summed with the same lane of the paired row (rows 0+1, 2+3: permlane16
 // swap) or of the other half of the wavefront (permlane32 swap); both lanes of
@@ -284,61 +276,6 @@ __device__ __forceinline__ double row_pair_sum(double v) {
     const auto b = HALVES ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
                           : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
     return __hiloint2double(b[0], a[0]) + __hiloint2double(b[1], a[1]);
-}
-
-// Sums over the 16 quads of a wavefront, per position q in the quad, of two
-// registers at once: afterwards lane q of the wavefront holds, in A and B, the
-// totals of A and B over the lanes 4k + q (fixed tree: two rotations within each
-// row of 16, then the rows in pairs and the halves; the result is read from lane q).
-__device__ __forceinline__ void quad_slot_sums(double& A, double& B) {
-    A += dpp_f64<kDppRowRor4>(A);
-    B += dpp_f64<kDppRowRor4>(B);
-    A += dpp_f64<kDppRowRor8>(A);
-    B += dpp_f64<kDppRowRor8>(B);
-    A = row_pair_sum<false>(A);
-    B = row_pair_sum<false>(B);
-    A = row_pair_sum<true>(A);
-    B = row_pair_sum<true>(B);
-}
-
-template <int NT>
-__device__ __forceinline__ double transpose_tp(double v) {
-    if constexpr (NT == 2) {
-        return dpp_f64<kDppTranspose>(v);
-    } else if constexpr (NT == 1) {
-        return v;
-    } else {  // lane (it, jt) of the pair's NT*NT lanes reads lane (jt, it)
-        const int lane = threadIdx.x & 63, q = lane % (NT * NT);
-        return __shfl(v, lane - q + (q % NT) * NT + q / NT, 64);
-    }
-}
-template <int NT>
-__device__ __forceinline__ double sum_over_jt(double v) {
-    if constexpr (NT == 2) {
-        return v + dpp_f64<kDppXor1>(v);
-    } else if constexpr (NT == 1) {
-        return v;
-    } else {  // the NT lanes (it, 0..NT-1) in a fixed order
-        const int lane = threadIdx.x & 63, q = lane % (NT * NT), row = lane - q + (q / NT) * NT;
-        double s = 0.0;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) s += __shfl(v, row + t, 64);
-        return s;
-    }
-}
-template <int NT>
-__device__ __forceinline__ double sum_over_it(double v) {
-    if constexpr (NT == 2) {
-        return v + dpp_f64<kDppXor2>(v);
-    } else if constexpr (NT == 1) {
-        return v;
-    } else {  // the NT lanes (0..NT-1, jt) in a fixed order
-        const int lane = threadIdx.x & 63, q = lane % (NT * NT), col = lane - q + q % NT;
-        double s = 0.0;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) s += __shfl(v, col + t * NT, 64);
-        return s;
-    }
 }
 
 // which branch of the reference applies to the pair width alpha = 1/ia:
@@ -414,50 +351,6 @@ __device__ __forceinline__ bool gh_avg(const FFParams<Q>& P, Q r, Q r_inv, Q asq
     return rule;
 }
 
-// 1/alpha per (site, type), ghosts included
-__global__ void k_inv_alpha(const double* __restrict__ alpha, long n, double* __restrict__ inva) {
-    long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) inva[k] = 1.0 / alpha[k];
-}
-
-// pair values (and r-, alpha-derivatives when DERIV) of the lane's type pair
-template <int NT, typename Q, int NQ, bool DERIV>
-__device__ __forceinline__ void lane_pair(const FFParams<double>& P, const FFParams<Q>& PQ, int it, int jt,
-                                          double rsq, double r, double r_inv, double ai, double aj, double ia,
-                                          double asq, const Q* __restrict__ quad, const double* __restrict__ rho7,
-                                          const double* __restrict__ phi7, double* g, double* f) {
-    const int br = alpha_branch(P, ia, ai, aj);
-    if (br == 1) {
-        Q gq[3], fq[3];
-        const Q* tab = quad + (size_t)(it * NT + jt) * kQuadRow;
-        if (gh_avg<Q, NQ, DERIV>(PQ, (Q)r, (Q)r_inv, (Q)asq, (Q)ia, tab, quad_stride(NT), gq, fq)) {
-            g[0] = (double)gq[0];
-            f[0] = (double)fq[0];
-            if (DERIV) {
-                g[1] = (double)gq[1];
-                g[2] = (double)gq[2];
-                f[1] = (double)fq[1];
-                f[2] = (double)fq[2];
-            }
-        }
-    } else if (br == 2 && rsq < P.cut_sq) {
-        classical_pair(P, rsq, r_inv, rho7 + (size_t)type2rho(NT, it, jt) * P.nr * 7,
-                       phi7 + (size_t)type2phi(it, jt) * P.nr * 7, true, g, f);
-    }
-}
-
-// ---------------------------------------------------------------- wave per site
-// One wavefront per site i: lane l = k*LPP + q works on pair k of the current
-// chunk of i's half list (PPW = 64/LPP pairs per chunk) and on ordered type
-// pair q = it*NT + jt.  Streams indexed by the pair (list, rpos, derivative
-// records) are then contiguous across the wave, the site's own data is
-// wave-uniform, and each neighbour's attributes are one 32-byte record per type.
-template <int NT>
-struct WaveMap {
-    static constexpr int LPP = NT * NT;
-    static constexpr int PPW = 64 / LPP;
-};
-
 // per (site, type) record {alpha, c, 1/alpha, dE}, ghosts included
 __global__ void k_pack_atoms(const double* __restrict__ alpha, const double* __restrict__ conc, long n,
                              double4* __restrict__ rec) {
@@ -474,6 +367,13 @@ __global__ void k_pack_nlrp(const int* __restrict__ nl, const int* __restrict__ 
                             int2* __restrict__ nlrp) {
     const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) nlrp[k] = make_int2(nl[k], rpos[k]);
+}
+
+// per reverse-list entry the owner of the pair (every entry starts outside the cut)
+__global__ void k_rev_owner(const int* __restrict__ rev, const int* __restrict__ pair_i, long n,
+                            int* __restrict__ rowner) {
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) rowner[k] = pair_i[rev[k]];
 }
 
 // sum over the wavefront, the same value in every lane: a DPP rotation tree
@@ -524,28 +424,30 @@ __device__ __forceinline__ void wave_store(const double* v, double* __restrict__
     }
 }
 
-// Sites of one wavefront.  Dispatch places block b on XCD b % 8; the sites are
-// split into 8 contiguous ranges, one per XCD, so spatial neighbours share an
-// L2, and the waves of an XCD stride through its range.  With one wave per
-// site (the default grid) each wave takes one site; a smaller grid makes the
-// launch persistent.  Every wave of a block runs the same number of
-// iterations or fewer; kernels that synchronise a block inside the loop must
-// not use it.
+// Sites of one group of LANES consecutive lanes (a wavefront, or half of one).
+// Dispatch places block b on XCD b % 8; the sites are split into 8 contiguous
+// ranges, one per XCD, so spatial neighbours share an L2, and the groups of an
+// XCD stride through its range.  With one group per site (the default grid)
+// each group takes one site; a smaller grid makes the launch persistent.
+// Every group of a block runs the same number of iterations or fewer; kernels
+// that synchronise a block inside the loop must not use it.
+template <int LANES = 64>
 struct SiteLoop {
     int first, end, stride;
-    __device__ __forceinline__ explicit SiteLoop(int n) {
-        const int wpb = blockDim.x >> 6, w = threadIdx.x >> 6;
+    // wpb: wavefronts per block (an argument, because reading blockDim is a load)
+    __device__ __forceinline__ SiteLoop(int n, int wpb) {
+        const int gpb = wpb * (64 / LANES), g = threadIdx.x / LANES;
         const int nb = gridDim.x, b = blockIdx.x;
         if (nb >= 8) {
             const int x = b & 7, lb = b >> 3;
             const int nbx = (nb - x + 7) >> 3;
-            first = (int)((long long)n * x / 8) + lb * wpb + w;
+            first = (int)((long long)n * x / 8) + lb * gpb + g;
             end = (int)((long long)n * (x + 1) / 8);
-            stride = nbx * wpb;
+            stride = nbx * gpb;
         } else {
-            first = b * wpb + w;
+            first = b * gpb + g;
             end = n;
-            stride = nb * wpb;
+            stride = nb * gpb;
         }
     }
 };
@@ -602,29 +504,80 @@ __device__ __forceinline__ int pack_in_range(int p, bool in, int* out) {
 // only for itype == jtype; src/ff_dmd_I.cpp:508).  The partner's density share
 // goes to pairE in reverse-CSR order (rpos), so the embedding reads it
 // contiguously.  Unless ENERGY_ONLY, the rho lane stores {drho/dr, drho/dalpha}
-// and the phi lane {dphi/dr, dphi/dalpha} in the record (DerivRec) of the k-th
-// pair of site i inside the quadrature cut, at off[i] + k (the reference's
-// per-pair caches, src/ff_dmd_I.cpp:227-242, restricted to what the back-pass
-// reads): a site's records are contiguous, and pass 2 ranks its inside pairs
-// the same way.  The phi lanes of the type pairs it < jt neither evaluate nor
-// store: the back-pass takes their phi from the transposed pair.
+// and the phi lane {dphi/dr, dphi/dalpha} in the pair's record (PairRec; the
+// reference's per-pair caches, src/ff_dmd_I.cpp:227-242, restricted to what the
+// back-pass reads), for the site's pairs inside the quadrature cut, whose number
+// goes to info with the site's list offset.  The phi lanes of the type pairs it < jt do not evaluate: the
+// back-pass takes their phi from the transposed pair.
+// Lanes of pass 1.  In general lane l works on pair slot k = l / kLPP and, within it,
+// on part prt of type pair q: lane k*kLPP + q*PARTS + prt.
+// Three types with two lanes per type pair have their own map: of the 18 lanes of
+// a pair 3 would do nothing (the phi of it < jt), and 3 pairs fill 54 lanes.  With
+// the 6 type pairs it >= jt as (rho, phi) lanes, then the 3 densities it < jt, a pair
+// takes 15 lanes, 4 pairs fill 60, and the last 4 lanes write the 4 partners: pass 1
+// at 114,840 sites 0.77 -> 0.64 ms.
 template <int NT, int PARTS = 4>
 struct Pass1Map {
-    static constexpr int LPP = NT * NT * PARTS;
-    static constexpr int PPW = 64 / LPP;
+    static constexpr bool kCompact = NT == 3 && PARTS == 2;
+    static constexpr int kLPP = kCompact ? 15 : NT * NT * PARTS;
+    static constexpr int kPPW = 64 / kLPP;
+    int k, it, jt, prt;
+    bool on;  // the lane evaluates
+    __device__ __forceinline__ explicit Pass1Map(int lane) {
+        k = lane / kLPP;
+        on = k < kPPW;
+        const int l = lane % kLPP;
+        if constexpr (kCompact) {
+            if (!on) k = lane - kLPP * kPPW;  // the lane that writes slot k's partner
+            const int c = l < 12 ? l / 2 : 0;
+            prt = l < 12 ? l % 2 : 0;
+            it = c >= 3 ? 2 : (c >= 1 ? 1 : 0);
+            jt = c - it * (it + 1) / 2;
+            if (l >= 12) {
+                it = l == 14 ? 1 : 0;
+                jt = l == 12 ? 1 : 2;
+            }
+        } else {
+            const int q = l / PARTS;
+            prt = l % PARTS;
+            it = q / NT;
+            jt = q % NT;
+        }
+    }
+    // lane of the density of type pair (a, b) within a pair's lanes
+    __device__ static int rho_at(int a, int b) {
+        if constexpr (kCompact) return a >= b ? a * (a + 1) + 2 * b : (a == 0 ? 11 + b : 14);
+        else return (a * NT + b) * PARTS;
+    }
 };
 
-// The derivative record of one pair inside the cut, kLen values of the
-// quadrature type: {drho/dr, drho/dalpha} of every ordered type pair
-// q = it*NT + jt, then {dphi/dr, dphi/dalpha} of the type pairs it >= jt only.
-// The back-pass uses the phi of (it, jt) for it >= jt on both (it, jt) and
-// (jt, it), as ForceField_DMD_I::force_calc reads one phi cache slot for both
-// orders (src/ff_dmd_I.cpp:244-248, :376), so the other half is never read.
-template <int NT>
-struct DerivRec {
-    static constexpr int kLen = 2 * NT * NT + NT * (NT + 1);
-    __host__ __device__ static constexpr int rho(int q) { return 2 * q; }
-    __host__ __device__ static constexpr int phi(int it, int jt) { return 2 * NT * NT + it * (it + 1) + 2 * jt; }
+// The records of the pairs of a site inside the cut, what pass 1 leaves for
+// pass 2.  A record has kComps components of two values of the quadrature type:
+// {drho/dr, drho/dalpha} of every ordered type pair q = it*NT + jt, then
+// {dphi/dr, dphi/dalpha} of the type pairs it >= jt only (the back-pass uses the
+// phi of (it, jt) for it >= jt on both (it, jt) and (jt, it), as
+// ForceField_DMD_I::force_calc reads one phi cache slot for both orders,
+// src/ff_dmd_I.cpp:244-248, :376), then {partner, reverse position or -1 for a
+// ghost partner} as two ints.  The k-th inside pair of site i is pair k % kG of
+// the site's group k / kG; a group holds its kG pairs component by component, so
+// a component of a group is one 64-byte run: pass 1's lanes (pair, type pair)
+// write whole cache lines, and pass 2's lanes (one pair each) read 16-byte
+// quarters of the same 64-byte runs instead of 16-byte pieces 112 bytes apart.
+// Site i's groups start at off[i] / kG + i, which leaves room for every listed
+// pair in whole groups.
+template <int NT, typename Q>
+struct PairRec {
+    static constexpr int kG = 64 / (2 * (int)sizeof(Q));
+    static constexpr int kComps = NT * NT + NT * (NT + 1) / 2 + 1;
+    __host__ __device__ static constexpr int rho(int q) { return q; }
+    __host__ __device__ static constexpr int phi(int it, int jt) { return NT * NT + type2phi(it, jt); }
+    static constexpr int kIdx = kComps - 1;
+    // groups to hold npairs listed pairs of natms sites
+    __host__ __device__ static size_t groups(long npairs, long natms) { return (size_t)(npairs / kG + natms + 1); }
+    // first element ({value, value}) of site i's records
+    __device__ static size_t first(int off_i, int i) { return ((size_t)(off_i / kG) + (size_t)i) * (kG * kComps); }
+    // element of component c of the site's pair k, relative to first()
+    __device__ static int elem(int k, int c) { return (k / kG) * (kG * kComps) + c * kG + k % kG; }
 };
 
 template <typename Q>
@@ -632,11 +585,22 @@ struct Vec2;
 template <>
 struct Vec2<double> {
     using T = double2;
+    // two ints in the bits of one component
+    static __device__ __forceinline__ double2 ints(int a, int b) { return make_double2(__hiloint2double(b, a), 0.0); }
+    static __device__ __forceinline__ int2 ints(double2 v) { return make_int2(__double2loint(v.x), __double2hiint(v.x)); }
 };
 template <>
 struct Vec2<float> {
     using T = float2;
+    static __device__ __forceinline__ float2 ints(int a, int b) { return make_float2(__int_as_float(a), __int_as_float(b)); }
+    static __device__ __forceinline__ int2 ints(float2 v) { return make_int2(__float_as_int(v.x), __float_as_int(v.y)); }
 };
+// streaming store of one component (whole lines, read back only after the pass)
+template <typename Q2>
+__device__ __forceinline__ void store_comp(Q2* p, Q2 v) {
+    __builtin_nontemporal_store(v.x, &p->x);
+    __builtin_nontemporal_store(v.y, &p->y);
+}
 
 template <typename Q>
 __device__ __forceinline__ Q dpp_xor1_q(Q v);
@@ -650,19 +614,21 @@ __device__ __forceinline__ float dpp_xor1_q<float>(float v) {
 }
 
 
-// Per-wavefront LDS stage of pass 1 (dynamic shared memory, kPass1StageBytes per
-// wavefront): for the inside entries of the current chunk, in rank order,
-// {list entry, partner, reverse position} and per type {alpha, 1/alpha, c, r^2}.
+// Per-wavefront LDS stage of pass 1 (dynamic shared memory, kBytes per wavefront):
+// for the inside entries of the current chunk, in rank order, {r^2, 1/r},
+// {1/alpha, c} of the partner per type, and {partner, reverse position or -1}.
 template <int NT>
 struct Pass1Stage {
-    static constexpr int kBytes = 64 * (16 + 32 * NT);
-    int4* idx;
-    double4* rec;
+    static constexpr int kBytes = 64 * (16 + 16 * NT + 8);
+    double2* geo;
+    double2* typ;
+    int2* idx;
     __device__ __forceinline__ explicit Pass1Stage(int wave) {
         extern __shared__ __attribute__((aligned(32))) unsigned char pass1_lds[];
         unsigned char* base = pass1_lds + (size_t)wave * kBytes;
-        rec = reinterpret_cast<double4*>(base);
-        idx = reinterpret_cast<int4*>(base + 64 * 32 * NT);
+        geo = reinterpret_cast<double2*>(base);
+        typ = geo + 64;
+        idx = reinterpret_cast<int2*>(typ + 64 * NT);
     }
 };
 
@@ -690,56 +656,162 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p, int nb
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, nbytes, 0x00020000);
 }
 
+// 1/x by the hardware estimate and two Newton steps (x normal and positive here)
+__device__ __forceinline__ double rcp_nr(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = y * (2.0 - x * y);
+    return y * (2.0 - x * y);
+}
+// 1/sqrt(x) by the hardware estimate and one third-order step: the arithmetic of
+// rsqrt() without its test for zero and infinity
+__device__ __forceinline__ double rsqrt_nr(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = 1.0 - (x * y) * y;
+    return y + (y * e) * (0.5 + 0.375 * e);
+}
+
+// What the lane's cubic is multiplied by at u = r - xi/sqrt(alpha): u for the
+// density (rho lane: keep = ~0, unit = 0), the sign of u for the pair term
+// (keep = the sign bit, unit = the bits of 1) -- the odd extensions u rho(|u|)
+// and sgn(u) r*phi(|u|), without a comparison or a select.
+template <typename Q>
+struct OddFactor;
+template <>
+struct OddFactor<double> {
+    int lo, hi, unit;
+    __device__ __forceinline__ explicit OddFactor(bool rho)
+        : lo(rho ? -1 : 0), hi(rho ? -1 : kInsideBit), unit(rho ? 0 : 0x3FF00000) {}
+    __device__ __forceinline__ double operator()(double u) const {
+        return __hiloint2double((__double2hiint(u) & hi) | unit, __double2loint(u) & lo);
+    }
+};
+template <>
+struct OddFactor<float> {
+    int hi, unit;
+    __device__ __forceinline__ explicit OddFactor(bool rho) : hi(rho ? -1 : kInsideBit), unit(rho ? 0 : 0x3F800000) {}
+    __device__ __forceinline__ float operator()(float u) const { return __int_as_float((__float_as_int(u) & hi) | unit); }
+};
+
+// The weighted sums of a Gauss-Hermite rule over x[k] = g(r - xi[k]/sqrt(alpha)):
+// s0 = sum w0 x, s1 = sum w1 x, s2 = sum w2 x with w1 = w0 xi, w2 = w0 xi^2.
+// The nodes come in pairs -xi, xi of equal weight (exactly, in the tables in
+// use) around a middle node 0, so a pair costs two additions and three
+// multiply-adds instead of six.
+template <typename Q, int NQ, bool DERIV>
+__device__ __forceinline__ void gh_sums(const FFParams<Q>& P, int nq, const Q* x, Q* s0, Q* s1, Q* s2) {
+    Q a0 = 0, a1 = 0, a2 = 0;
+    if constexpr (NQ > 0) {
+        if constexpr (NQ % 2) a0 = P.w0[NQ / 2] * x[NQ / 2];
+#pragma unroll
+        for (int k = NQ / 2 + NQ % 2; k < NQ; ++k) {
+            const Q e = x[k] + x[NQ - 1 - k];
+            a0 += P.w0[k] * e;
+            if (DERIV) {
+                a1 += P.w1[k] * (x[k] - x[NQ - 1 - k]);
+                a2 += P.w2[k] * e;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kMaxPoints; ++k) {
+            if (k >= nq) break;
+            a0 += P.w0[k] * x[k];
+            if (DERIV) {
+                a1 += P.w1[k] * x[k];
+                a2 += P.w2[k] * x[k];
+            }
+        }
+    }
+    *s0 = a0;
+    *s1 = a1;
+    *s2 = a2;
+}
+
 // ENERGY_ONLY: the loop of ForceField_DMD_I::energy_calc (src/ff_dmd_I.cpp:454-668),
 // type pairs jt >= it only (:508) unless FULL, which sums every ordered pair so the
 // energy equals force_calc's.
+//
+// What bounds it: about 1,000 cycles of a CU's vector ALUs, of its address unit
+// (the 64-byte spline rows) and of its L1-to-L2 path per site, and the latency of
+// the rows between them.  So the loop over the pairs is straight-line code: every
+// lane evaluates (a lane past the last pair repeats it with zero weight), a point
+// beyond the cutoff reads the table's zero row nr - 1 (u < rc exactly when
+// u/dr < nr - 1, so this is the reference's window test, src/ff_dmd_I.cpp:196-204),
+// 1/r is formed once per list entry when it is staged, and the pair widths
+// outside the quadrature regime, if a chunk has any, are put right behind one
+// uniform branch: 2.90 -> 2.68 ms at 1,048,576 sites of two types, 3-point rule,
+// FP64, with 14% more bytes of records.  Of the 2.68 ms, 0.5 go with the record
+// stores, 0.24 with the scattered density shares and 0.2 with the rows' L1 misses.
+// Loads of the next round ahead of a round's stores (128 registers) took 2.73 ms,
+// rows read by four lanes as whole 64-byte segments (a quarter fewer cache accesses,
+// a fifth more vector instructions) 2.80, ordinary stores of the records 3.16.
 template <int NT, typename Q, int NQ, bool ENERGY_ONLY, bool FULL = false, int PARTS = 4>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_pass1(FFParams<double> P, FFParams<Q> PQ,
-                                                  const double4* __restrict__ pos,
-                                                  const double4* __restrict__ arec, PairBufs L,
-                                                  const int2* nlrp, const Q* __restrict__ quad,
-                                                  const double* __restrict__ rho7, const double* __restrict__ phi7,
-                                                  double* __restrict__ Eown, double* __restrict__ pairE,
-                                                  Q* __restrict__ deriv, double* __restrict__ part,
-                                                  CutState C) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_pass1(
+    FFParams<double> P, FFParams<Q> PQ, const double4* __restrict__ pos, const double4* __restrict__ arec,
+    const int* __restrict__ off, const int2* nlrp, const Q* __restrict__ quad, const double* __restrict__ rho7,
+    const double* __restrict__ phi7, double* __restrict__ Eown, double* __restrict__ pairE,
+    typename Vec2<Q>::T* __restrict__ deriv, int2* __restrict__ info, double* __restrict__ part, CutState C, int wpb) {
     static_assert(PARTS == 1 || PARTS == 2 || PARTS == 4, "one, two or four lanes per (pair, type pair)");
     using Q2 = typename Vec2<Q>::T;
-    constexpr int LPP = Pass1Map<NT, PARTS>::LPP, PPW = Pass1Map<NT, PARTS>::PPW;
+    using R = PairRec<NT, Q>;
+    using Map = Pass1Map<NT, PARTS>;
+    constexpr int LPP = Map::kLPP, PPW = Map::kPPW;
     const int lane = threadIdx.x & 63;
-    const int k = lane / LPP, q = (lane % LPP) / PARTS, prt = lane % PARTS;
-    const int it = q / NT, jt = q % NT;
-    const bool active = !ENERGY_ONLY || FULL || jt >= it;
-    const bool want_phi = it >= jt;
+    const Map map(lane);
+    const int k = map.k, prt = map.prt, it = map.it, jt = map.jt, q = it * NT + jt;
+    const bool on = map.on && (!ENERGY_ONLY || FULL || jt >= it);
     // four parts: quarters of the row, rho in parts 0/1 and phi in 2/3 (results in 0 and 2);
     // two parts: part 0 the rho cubic, part 1 the phi cubic; one part: both
     const bool rho_lane = prt == 0, phi_lane = prt == PARTS / 2;
+    const bool want_phi = it >= jt;
+    const bool live = on && (PARTS == 1 || prt < PARTS / 2 || want_phi);
+    // a phi lane whose phi is not kept reads its type pair's rho row instead (the same cache line)
+    const int half = PARTS == 1 ? 0 : (prt >= PARTS / 2 && !want_phi ? prt - PARTS / 2 : prt) * (8 / PARTS);
+    const int tab_off = (q * kQuadRow + half) * (int)sizeof(Q);
+    const __amdgpu_buffer_rsrc_t qrs = raw_rsrc(quad, P.nr * quad_stride(NT) * (int)sizeof(Q));
+    const OddFactor<Q> odd(prt < (PARTS + 1) / 2);
+    // the lane's record component; the partner goes out on a lane whose phi is not kept
+    // (type pair (0, NT-1)), on a spare lane, or with one type on the phi lane too
+    const bool ix = Map::kCompact ? !map.on : NT > 1 && phi_lane && PARTS > 1 && q == NT - 1;
+    const int comp = (ix ? R::kIdx : (rho_lane ? R::rho(q) : R::phi(it, jt))) * R::kG;
+    const bool keeps = ix || (map.on && (rho_lane || (phi_lane && want_phi)));
     double en = 0.0, npair = 0.0;  // energy, pairs inside the quadrature cut (this lane's share)
     const Pass1Stage<NT> st(threadIdx.x >> 6);
-    const SiteLoop sl(P.natms);
+    const SiteLoop<> sl(P.natms, wpb);
     for (int i0 = sl.first; i0 < sl.end; i0 += sl.stride) {
         const int i = __builtin_amdgcn_readfirstlane(i0);
+        const int p0 = off[i], p1 = off[i + 1];
         const double4 xi = pos[i];
-        double ci[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) ci[t] = arec[(size_t)i * NT + t].y;
         const double4 ra = arec[(size_t)i * NT + it];
-        const double ai = ra.x, iai = ra.z;
-        const __amdgpu_buffer_rsrc_t qrs = raw_rsrc(quad, P.nr * quad_stride(NT) * (int)sizeof(Q));
-        const int tab_off = (q * kQuadRow + (PARTS == 1 ? 0 : prt * (8 / PARTS))) * (int)sizeof(Q);
-        double Ei = 0.0;
-        const int p0 = L.off[i], p1 = L.off[i + 1];
-        int done = 0;  // inside entries of the earlier chunks: records go to off[i] + rank
+        const double ai = ra.x, iai = ra.z, ci = ra.y, ci_jt = arec[(size_t)i * NT + jt].y;
+        double ia_min = arec[(size_t)i * NT].z, ia_max = ia_min;
+#pragma unroll
+        for (int t = 1; t < NT; ++t) {
+            const double v = arec[(size_t)i * NT + t].z;
+            ia_min = v < ia_min ? v : ia_min;
+            ia_max = v > ia_max ? v : ia_max;
+        }
+        // weights of the lane's value: the partner's c for a rho lane, the pair energy's
+        // c c + c c for a phi lane (src/ff_dmd_I.cpp:244-255)
+        const double xw = it != jt ? P.xw : 1.0;
+        const double wr = on && rho_lane ? 1.0 : 0.0;
+        const double wa = on && phi_lane && want_phi ? xw * ci : 0.0;
+        const double wb = on && phi_lane && want_phi ? xw * ci_jt : 0.0;
+        Q2* const rec = deriv + R::first(p0, i);
+        double Ei = 0.0, ep = 0.0;  // sums of the rho and of the phi lanes (one register unless PARTS == 1)
+        int done = 0;  // inside entries of the earlier chunks: the pair's rank among the site's
         for (int chunk = p0; chunk < p1; chunk += 64) {
             // one list entry per lane: the cut state of each entry is kept current
             // (CutState); each entry inside the cut is staged in LDS at its rank
-            // among the inside entries, with its partner's width, inverse width
-            // and concentration of every type, read from HBM once per entry
+            // among the inside entries, with its partner's inverse width and
+            // concentration of every type, read from HBM once per entry
             int cnt;
+            bool regular = true;  // every pair width surely in the quadrature regime
             {
                 const int pc = chunk + lane;
                 bool in = false;
                 int jc = 0, rp = 0;
-                double r2 = 0.0;
+                double r2 = 1.0;
                 if (pc < p1) {
                     const int2 e = nlrp[pc];
                     jc = list_partner(e);
@@ -751,78 +823,58 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                         r2 = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;
                     }
                     in = r2 < P.cut_sq_mod;
-                    C.update<NT>(pc, e, in, jc, P.natms, pairE);
+                    C.update<NT>(pc, e, in, i, jc, P.natms, pairE);
                 }
                 const int dest = pack_dest(in, &cnt);
                 if (in) {
-                    st.idx[dest] = make_int4(pc, jc, rp, 0);
-                    // the partner's {alpha, c} of every type in one 16-byte load each; the
-                    // division gives the same bits as the stored 1/alpha (both correctly rounded)
+                    double2 ac[NT];
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        ac[t] = *reinterpret_cast<const double2*>(arec + (size_t)jc * NT + t);
+                    st.geo[dest] = make_double2(r2, rsqrt_nr(r2));
+                    st.idx[dest] = make_int2(jc, jc < P.natms ? rp : -1);
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
-                        const double2 ac = *reinterpret_cast<const double2*>(arec + (size_t)jc * NT + t);
-                        st.rec[dest * NT + t] = make_double4(ac.x, 1.0 / ac.x, ac.y, r2);
+                        const double iaj = rcp_nr(ac[t].x);
+                        regular = regular && iaj + ia_min > P.ia_quad_lo && iaj + ia_max < P.ia_quad_hi;
+                        st.typ[dest * NT + t] = make_double2(iaj, ac[t].y);
                     }
                 }
+                regular = __builtin_amdgcn_ballot_w64(!regular) == 0;
                 __builtin_amdgcn_wave_barrier();
             }
-        for (int base = 0; base < cnt; base += PPW) {
-            const int slot = base + k;
-            const bool valid = slot < cnt && (64 % LPP == 0 || k < PPW);  // lanes past PPW pairs idle
-            int p = 0, j = 0, rp = 0;
-            double rsq = 1.0, aj = 1.0, iaj = 1.0;
-            double cj[NT];
-#pragma unroll
-            for (int t = 0; t < NT; ++t) cj[t] = 0.0;
-            if (valid) {
-                const int4 e = st.idx[slot];
-                p = e.x;
-                j = e.y;
-                rp = e.z;
-                const double4 rj = st.rec[slot * NT + jt];
-                aj = rj.x;
-                iaj = rj.y;
-                rsq = rj.w;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) cj[t] = t == jt ? rj.z : st.rec[slot * NT + t].z;
-            }
-            const bool inr = valid;  // inside the cut by construction
-            double ej = 0.0;
-            if (inr) {
-                const double r_inv = rsqrt(rsq), r = rsq * r_inv;
-                const double ia = iai + iaj, asq = rsqrt(ia);
-                // the phi lanes of it < jt are idle (DerivRec)
-                const bool live = PARTS == 1 || prt < PARTS / 2 || want_phi;
-                const int br = active && live ? alpha_branch(P, ia, ai, aj) : 0;
+            // whole groups of records are written (whole cache lines), also past the last pair
+            const int kept = chunk + 64 < p1 ? cnt : (done + cnt + R::kG - 1) / R::kG * R::kG - done;
+            for (int base = 0; base < cnt; base += PPW) {
+                const int slot = base + k, s = slot < cnt ? slot : cnt - 1;
+                const bool valid = slot < cnt && map.on;
+                const int2 e = st.idx[s];
+                const double2 geo = st.geo[s];
+                const double2 tj = st.typ[s * NT + jt];
+                const double cj = tj.y, cj_it = st.typ[s * NT + it].y;
+                const double r_inv = geo.y, r = geo.x * r_inv;
+                const double ia = iai + tj.x, asq = rsqrt_nr(ia);
                 // v1: the lane's function (rho on the rho lane, phi on the phi lane) or,
                 // with one lane per pair, rho; v2: phi with one lane per pair.
                 // Each holds value, d/dr, d/dalpha.
-                double v1[3] = {0.0, 0.0, 0.0};
-                double v2[3] = {0.0, 0.0, 0.0};
-                if (br == 1) {
-                    const Q rq = (Q)r, iq = (Q)ia, aq = (Q)asq;
-                    const Q inv = iq * aq;
-                    const Q upper = (rq + PQ.rc) * aq, lower = (rq - PQ.rc) * aq;
+                double v1[3], v2[3];
+                {
+                    const Q rq = (Q)r, iq = (Q)ia, aq = (Q)asq, inv = iq * aq;
                     const int nq = NQ > 0 ? NQ : PQ.no_i;
-                    const bool rule = lower < PQ.xi[nq - 1];
-                    Q s0 = 0, s1 = 0, s2 = 0;  // rho sums (PARTS 1) or this lane's function
-                    Q u0 = 0, u1 = 0, u2 = 0;  // phi sums (PARTS 1)
                     // all rows of the rule are requested before any is used, so their
-                    // latencies overlap (a point outside the window reads a clamped row)
+                    // latencies overlap
                     constexpr int KP = NQ > 0 ? NQ : kMaxPoints;
                     constexpr int NV = PARTS == 4 ? 1 : (PARTS == 2 ? 2 : 4);
                     Q2 rowv[KP][NV];
-                    Q ppv[KP];
+                    Q ppv[KP], uv[KP];
 #pragma unroll
                     for (int kp = 0; kp < KP; ++kp) {
                         if (NQ == 0 && kp >= nq) break;
-                        const Q t = rq - PQ.xi[kp] * inv;
-                        Q pp = fabs(t) * PQ.dr_inv;
-                        int m = (int)pp;
-                        m = m < P.nr - 2 ? m : P.nr - 2;
-                        m = m > 0 ? m : 0;
-                        pp -= (Q)m;
-                        ppv[kp] = pp < Q(1) ? pp : Q(1);
+                        const Q u = rq - PQ.xi[kp] * inv;
+                        int m = (int)(fabs(u) * PQ.dr_inv);
+                        m = m < P.nr - 1 ? m : P.nr - 1;  // the zero row beyond the cutoff
+                        uv[kp] = u;
+                        ppv[kp] = fabs(u) * PQ.dr_inv - (Q)m;
                         const int row = tab_off + m * (quad_stride(NT) * (int)sizeof(Q));
 #pragma unroll
                         for (int v = 0; v < NV; ++v)  // one lane per pair: the phi half only where it >= jt
@@ -833,154 +885,120 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     // keep the requests ahead of the arithmetic where the rows fit the
                     // register budget of four waves per SIMD (at most 24 registers)
                     if constexpr (KP * NV * sizeof(Q2) <= 96) __builtin_amdgcn_sched_barrier(0);
+                    Q x[KP], y[KP];
 #pragma unroll
                     for (int kp = 0; kp < KP; ++kp) {
                         if (NQ == 0 && kp >= nq) break;
-                        const Q xk = PQ.xi[kp];
-                        const bool inside = rule && xk > lower && xk < upper;
-                        const Q t = rq - xk * inv, pp = ppv[kp];
-                        const Q p2 = pp * pp;
+                        const Q pp = ppv[kp], p2 = pp * pp;
                         if constexpr (PARTS == 4) {
                             const Q2 c = rowv[kp][0];
                             const Q h = c.x + c.y * pp;
-                            const Q hb = dpp_xor1_q<Q>(h);
-                            const Q val = h + p2 * hb;
-                            Q x = prt == 0 ? val * t : (t < Q(0) ? -val : val);
-                            x = inside ? x : Q(0);
-                            s0 += PQ.w0[kp] * x;
-                            if (!ENERGY_ONLY) {
-                                s1 += PQ.w1[kp] * x;
-                                s2 += PQ.w2[kp] * x;
-                            }
-                        } else if constexpr (PARTS == 2) {
-                            const Q2 lo = rowv[kp][0];
-                            const Q2 hi = rowv[kp][1];
-                            const Q val = (lo.x + lo.y * pp) + p2 * (hi.x + hi.y * pp);
-                            Q x = prt == 0 ? val * t : (t < Q(0) ? -val : val);
-                            x = inside ? x : Q(0);
-                            s0 += PQ.w0[kp] * x;
-                            if (!ENERGY_ONLY) {
-                                s1 += PQ.w1[kp] * x;
-                                s2 += PQ.w2[kp] * x;
-                            }
+                            x[kp] = (h + p2 * dpp_xor1_q<Q>(h)) * odd(uv[kp]);
                         } else {
-                            const Q2 a0 = rowv[kp][0];
-                            const Q2 a1 = rowv[kp][1];
-                            const Q2 b0 = rowv[kp][2];
-                            const Q2 b1 = rowv[kp][3];
-                            const Q vrho = (a0.x + a0.y * pp) + p2 * (a1.x + a1.y * pp);
-                            const Q vphi = (b0.x + b0.y * pp) + p2 * (b1.x + b1.y * pp);
-                            const Q xr = inside ? vrho * t : Q(0);
-                            const Q xp = inside ? (t < Q(0) ? -vphi : vphi) : Q(0);
-                            s0 += PQ.w0[kp] * xr;
-                            u0 += PQ.w0[kp] * xp;
-                            if (!ENERGY_ONLY) {
-                                s1 += PQ.w1[kp] * xr;
-                                s2 += PQ.w2[kp] * xr;
-                                u1 += PQ.w1[kp] * xp;
-                                u2 += PQ.w2[kp] * xp;
+                            const Q2 a0 = rowv[kp][0], a1 = rowv[kp][1];
+                            x[kp] = ((a0.x + a0.y * pp) + p2 * (a1.x + a1.y * pp)) * odd(uv[kp]);
+                            if constexpr (PARTS == 1) {
+                                const Q2 b0 = rowv[kp][2], b1 = rowv[kp][3];
+                                y[kp] = ((b0.x + b0.y * pp) + p2 * (b1.x + b1.y * pp)) * OddFactor<Q>(false)(uv[kp]);
                             }
                         }
                     }
-                    if (rule) {
-                        const Q sc = Q(kPiInSq) * (Q)r_inv;
-                        auto fin = [&](Q a0, Q a1, Q a2, double* v) {
-                            const Q v0 = a0 * sc;
-                            v[0] = (double)v0;
-                            if (!ENERGY_ONLY) {
-                                v[1] = (double)(-v0 * (Q)r_inv - Q(2) * aq * (a1 * sc));
-                                v[2] = (double)((Q(0.5) * v0 - a2 * sc) * iq);
-                            }
-                        };
-                        fin(s0, s1, s2, v1);
-                        if constexpr (PARTS == 1) fin(u0, u1, u2, v2);
-                    }
-                } else if (br == 2 && rsq < P.cut_sq) {
-                    double g[3], f[3];
-                    classical_pair(P, rsq, r_inv, rho7 + (size_t)type2rho(NT, it, jt) * P.nr * 7,
-                                   phi7 + (size_t)type2phi(it, jt) * P.nr * 7, true, g, f);
-                    for (int c = 0; c < 3; ++c) {
-                        if constexpr (PARTS == 1) {
-                            v1[c] = g[c];
-                            v2[c] = f[c];
-                        } else {
-                            v1[c] = rho_lane ? g[c] : f[c];
+                    const Q sc = Q(kPiInSq) * (Q)r_inv;
+                    auto close = [&](const Q* z, double* v) {
+                        Q s0, s1, s2;
+                        gh_sums<Q, NQ, !ENERGY_ONLY>(PQ, nq, z, &s0, &s1, &s2);
+                        const Q v0 = s0 * sc;
+                        v[0] = (double)v0;
+                        if (!ENERGY_ONLY) {
+                            v[1] = (double)(-v0 * (Q)r_inv - Q(2) * aq * (s1 * sc));
+                            v[2] = (double)((Q(0.5) * v0 - s2 * sc) * iq);
                         }
-                    }
+                    };
+                    close(x, v1);
+                    if constexpr (PARTS == 1) close(y, v2);
                 }
-                if constexpr (PARTS == 1) {
-                    Ei += v1[0] * cj[jt];
-                    ej = v1[0] * ci[it];
-                    if (want_phi && active) {
-                        const double half = (j < P.natms ? 0.5 : 0.25) * (it != jt ? P.xw : 1.0);
-                        en += half * (cj[jt] * ci[it] + cj[it] * ci[jt]) * v2[0];
-                    }
-                    if (!ENERGY_ONLY) {
-                        Q* d = deriv + (size_t)(p0 + done + slot) * DerivRec<NT>::kLen;
-                        __builtin_nontemporal_store((Q)v1[1], d + DerivRec<NT>::rho(q));
-                        __builtin_nontemporal_store((Q)v1[2], d + DerivRec<NT>::rho(q) + 1);
-                        if (want_phi) {
-                            __builtin_nontemporal_store((Q)v2[1], d + DerivRec<NT>::phi(it, jt));
-                            __builtin_nontemporal_store((Q)v2[2], d + DerivRec<NT>::phi(it, jt) + 1);
-                        }
-                    }
-                } else {
-                    if (rho_lane) {
-                        Ei += v1[0] * cj[jt];
-                        ej = v1[0] * ci[it];
-                    }
-                    if (phi_lane && want_phi && active) {
-                        const double half = (j < P.natms ? 0.5 : 0.25) * (it != jt ? P.xw : 1.0);
-                        en += half * (cj[jt] * ci[it] + cj[it] * ci[jt]) * v1[0];
-                    }
-                    if (!ENERGY_ONLY && (rho_lane || (phi_lane && want_phi))) {
-                        Q* d = deriv + (size_t)(p0 + done + slot) * DerivRec<NT>::kLen +
-                               (rho_lane ? DerivRec<NT>::rho(q) : DerivRec<NT>::phi(it, jt));
-                        __builtin_nontemporal_store((Q)v1[1], d);
-                        __builtin_nontemporal_store((Q)v1[2], d + 1);
-                    }
-                }
-            }
-            // sum over it: the (0, jt) and (1, jt) lanes of a pair are NT * PARTS apart
-            if constexpr (NT == 2 && PARTS == 4) ej += dpp_f64<kDppRowRor8>(ej);
-            if constexpr (NT == 2 && PARTS == 2) ej += dpp_f64<kDppRowRor12>(ej);  // lane l + 4 for l % 8 < 4
-            if constexpr (NT == 2 && PARTS == 1) ej += __shfl_xor(ej, 2, 64);
-            if constexpr (NT > 2) {  // the rho lanes (0..NT-1, jt) of the pair, in a fixed order
-                const int col = lane - lane % LPP + jt * PARTS;
-                double s = 0.0;
+                // pair widths outside the quadrature regime, or within rounding of its bounds
+                if (!regular) {
+                    const int br = live ? alpha_branch(P, ia, ai, arec[(size_t)e.x * NT + jt].x) : 1;
+                    if (br != 1) {
+                        double g[3] = {0.0, 0.0, 0.0}, f[3] = {0.0, 0.0, 0.0};
+                        if (br == 2 && geo.x < P.cut_sq)
+                            classical_pair(P, geo.x, r_inv, rho7 + (size_t)type2rho(NT, it, jt) * P.nr * 7,
+                                           phi7 + (size_t)type2phi(it, jt) * P.nr * 7, true, g, f);
 #pragma unroll
-                for (int t = 0; t < NT; ++t) s += __shfl(ej, col + t * NT * PARTS, 64);
-                ej = s;
+                        for (int c = 0; c < 3; ++c) {
+                            v1[c] = PARTS == 1 || rho_lane ? g[c] : f[c];
+                            v2[c] = f[c];
+                        }
+                    }
+                }
+                // the site's density (rho lanes) and the pair energy (phi lanes)
+                const double hw = valid ? (e.y >= 0 ? 0.5 : 0.25) : 0.0;
+                const double we = (cj * wa + cj_it * wb) * hw;
+                const double wE = valid ? cj * wr : 0.0;
+                if constexpr (PARTS == 1) {
+                    Ei += v1[0] * wE;
+                    if (want_phi) ep += v2[0] * we;
+                } else {
+                    if (live) Ei += v1[0] * (rho_lane ? wE : we);
+                }
+                double ej = on && rho_lane ? v1[0] * ci : 0.0;
+                if (!ENERGY_ONLY && slot < kept) {
+                    Q2* d = rec + R::elem(done + slot, 0);
+                    if constexpr (PARTS == 1) {
+                        if (keeps) {
+                            store_comp(d + comp, Q2{(Q)v1[1], (Q)v1[2]});
+                            if (want_phi) store_comp(d + R::phi(it, jt) * R::kG, Q2{(Q)v2[1], (Q)v2[2]});
+                            if (NT == 1 || q == NT - 1) store_comp(d + R::kIdx * R::kG, Vec2<Q>::ints(e.x, e.y));
+                        }
+                    } else {
+                        const Q2 v = ix ? Vec2<Q>::ints(e.x, e.y) : Q2{(Q)v1[1], (Q)v1[2]};
+                        if (keeps) store_comp(d + comp, v);
+                        if (NT == 1 && phi_lane) store_comp(d + R::kIdx * R::kG, Vec2<Q>::ints(e.x, e.y));
+                    }
+                }
+                // sum over it: the (0, jt) and (1, jt) lanes of a pair are NT * PARTS apart
+                if constexpr (NT == 2 && PARTS == 4) ej += dpp_f64<kDppRowRor8>(ej);
+                if constexpr (NT == 2 && PARTS == 2) ej += dpp_f64<kDppRowRor12>(ej);  // lane l + 4 for l % 8 < 4
+                if constexpr (NT == 2 && PARTS == 1) ej += __shfl_xor(ej, 2, 64);
+                if constexpr (NT > 2) {  // the rho lanes (0..NT-1, jt) of the pair, in a fixed order
+                    double sum = 0.0;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) sum += __shfl(ej, k * LPP + Map::rho_at(t, jt), 64);
+                    ej = sum;
+                }
+                // an ordinary store: the 16-byte shares land scattered, and L2 merges them into lines
+                if (valid && rho_lane && it == 0 && e.y >= 0) pairE[(size_t)e.y * NT + jt] = ej;
             }
-            // an ordinary store: the 16-byte shares land scattered, and L2 merges them into lines
-            if (valid && rho_lane && it == 0 && j < P.natms) pairE[(size_t)rp * NT + jt] = ej;
+            done += cnt;
         }
-        done += cnt;
+        if (lane == 0) {
+            npair += (double)done;  // the site's pairs inside the cut
+            if (!ENERGY_ONLY) info[i] = make_int2(p0, done);
         }
-        if (lane == 0) npair += (double)done;  // the site's pairs inside the cut
         if constexpr (NT == 2 && PARTS == 2) {
-            // Ei[it] lives on the rho lanes 8k + 2q (q = 2 it + jt): join the jt lanes
-            // (then lanes 8k + 4 it hold slot k's share), add the two slots of each row
-            // and the four rows
-            double e = rho_lane ? Ei : 0.0;
-            e += dpp_f64<kDppXor2>(e);
+            // the pair slots of a wavefront are 8 lanes apart; then the jt lanes are
+            // joined: lanes 0 and 4 hold the densities of type 0 and 1, lanes 1 and 5
+            // the energies of (0, *) and (1, *)
+            double e = Ei;
             e += dpp_f64<kDppRowRor8>(e);
             e = row_pair_sum<false>(e);
             e = row_pair_sum<true>(e);
-            const double e0 = read_lane(e, 0), e1 = read_lane(e, 4);
-            if (lane == 0) {
-                Eown[(size_t)i * NT] = e0;
-                Eown[(size_t)i * NT + 1] = e1;
-            }
+            e += dpp_f64<kDppXor2>(e);
+            if ((lane & ~4) == 0) Eown[(size_t)i * NT + (lane >> 2)] = e;
+            if ((lane & ~4) == 1) en += e;
         } else {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const double s = wave_sum(rho_lane && it == t ? Ei : 0.0);
-                if (lane == 0) Eown[(size_t)i * NT + t] = s;
+                const double sum = wave_sum(rho_lane && it == t ? Ei : 0.0);
+                if (lane == 0) Eown[(size_t)i * NT + t] = sum;
             }
+            en += PARTS == 1 ? ep : (phi_lane ? Ei : 0.0);
         }
     }
-    double acc[2] = {wave_sum(en), npair};  // npair: lane 0 only
+    double acc[2] = {0.0, npair};  // npair: lane 0 only
+    if constexpr (NT == 2 && PARTS == 2) acc[0] = read_lane(en, 1) + read_lane(en, 5);
+    else acc[0] = wave_sum(en);
     wave_store<2>(acc, part);
 }
 
@@ -1028,7 +1046,7 @@ constexpr int kEmbedG = 4;    // lanes per site of the embedding (its per-site a
 // contiguous reverse range); F, F', energy terms, alpha entropic force
 template <int NT, bool ENERGY_ONLY>
 __global__ __launch_bounds__(kBlock) void k_embed(FFParams<double> P, const double* __restrict__ alpha,
-                                                  const double* __restrict__ conc, PairBufs L,
+                                                  const double* __restrict__ conc, const int* __restrict__ roff,
                                                   const double* __restrict__ Eown,
                                                   const double* __restrict__ pairE,
                                                   const double* __restrict__ F9, double* __restrict__ E,
@@ -1041,8 +1059,8 @@ __global__ __launch_bounds__(kBlock) void k_embed(FFParams<double> P, const doub
         double e[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) e[t] = 0.0;
-        const int q1 = L.roff[i + 1];
-        for (int q = L.roff[i] + g.l; q < q1; q += kEmbedG) {
+        const int q1 = roff[i + 1];
+        for (int q = roff[i] + g.l; q < q1; q += kEmbedG) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) e[t] += pairE[(size_t)q * NT + t];
         }
@@ -1072,224 +1090,173 @@ __global__ __launch_bounds__(kBlock) void k_embed(FFParams<double> P, const doub
 }
 
 // ---------------------------------------------------------------- pass 2
-// src/ff_dmd_I.cpp:357-436: fpair/apair of each ordered type pair from the
-// derivative records of pass 1 (slot type2rho[jt][it], i.e. the transposed
-// lane's record, pairs with dE_i; phi for it < jt is the phi record of
-// (jt, it), as in the reference's shared COMP slot).  No table lookups.
-template <int NT, typename Q>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_pass2(FFParams<double> P, const double4* __restrict__ pos,
-                                                  const double4* __restrict__ arec, PairBufs L,
-                                                  const int2* __restrict__ nlrp, const Q* __restrict__ deriv,
-                                                  double* __restrict__ fown, ForceShares F,
-                                                  double* __restrict__ part) {
-    constexpr int LPP = WaveMap<NT>::LPP, PPW = WaveMap<NT>::PPW;
-    constexpr int XD = 3 + NT;
-    const int lane = threadIdx.x & 63;
-    const int k = lane / LPP, q = lane % LPP, it = q / NT, jt = q % NT;
-    const int qT = jt * NT + it;
-    const bool want_phi = it >= jt;
-    double vir[6] = {0, 0, 0, 0, 0, 0};
-    const SiteLoop sl(P.natms);
-    for (int i0 = sl.first; i0 < sl.end; i0 += sl.stride) {
-        const int i = __builtin_amdgcn_readfirstlane(i0);
-        const double4 xi = pos[i];
-        const double4 ra = arec[(size_t)i * NT + it];
-        const double ai = ra.x, ci = ra.y, iai = ra.z, dEi = ra.w;
-        double fx = 0.0, fy = 0.0, fz = 0.0, fa = 0.0;
-        const int p0 = L.off[i], p1 = L.off[i + 1];
-        int done = 0;  // inside entries of the earlier chunks (records at off[i] + rank)
-        for (int chunk = p0; chunk < p1; chunk += 64) {
-            // partner and separation of the inside pairs, packed
-            int pk_j, pk_rp, cnt;
-            double pk_d0, pk_d1, pk_d2, pk_r2;
-            {
-                const int pc = chunk + lane;
-                bool in = false;
-                int jc = 0, rp = 0;
-                double e0 = 0.0, e1 = 0.0, e2 = 0.0, r2 = 0.0;
-                if (pc < p1) {
-                    // pass 1 of this evaluation left each entry's cut state in its
-                    // partner's top bit (same positions): only the entries inside
-                    // need a position; the shares of the others stay zero (CutState)
-                    const int2 e = nlrp[pc];
-                    in = (e.x & kInsideBit) != 0;
-                    if (in) {
-                        jc = list_partner(e);
-                        rp = e.y;  // meaningful for owned partners only
-                        const double4 xj = pos[jc];
-                        e0 = xi.x - xj.x;
-                        e1 = xi.y - xj.y;
-                        e2 = xi.z - xj.z;
-                        {
-#pragma clang fp contract(off)
-                            r2 = e0 * e0 + e1 * e1 + e2 * e2;
-                        }
-                    }
-                }
-                const int dest = pack_dest(in, &cnt);
-                pk_j = packed(dest, jc);
-                pk_rp = packed(dest, rp);
-                pk_d0 = packed(dest, e0);
-                pk_d1 = packed(dest, e1);
-                pk_d2 = packed(dest, e2);
-                pk_r2 = packed(dest, r2);
-            }
-        for (int base = 0; base < cnt; base += PPW) {
-            const int slot = base + k;
-            const bool valid = slot < cnt && (64 % LPP == 0 || k < PPW);  // lanes past PPW pairs idle
-            const int src = valid ? slot : 0;
-            const int j = __shfl(pk_j, src, 64);
-            const int rp = __shfl(pk_rp, src, 64);
-            const double dx0 = __shfl(pk_d0, src, 64), dx1 = __shfl(pk_d1, src, 64), dx2 = __shfl(pk_d2, src, 64);
-            const double rsq = __shfl(pk_r2, src, 64);
-            const bool inr = valid;  // inside the cut by construction
-            const bool owned = j < P.natms;
-            double S = 0.0, aJ = 0.0;
-            if (inr) {
-                double aj, iaj, cj, dEj;
-                if constexpr (NT == 2) {
-                    // lanes (0, jt) and (1, jt) share the partner's record of type jt:
-                    // each loads one half ({alpha, c} or {1/alpha, F'}) and the quad
-                    // exchange (xor 2) brings the other
-                    const double2 h = reinterpret_cast<const double2*>(arec + (size_t)j * NT + jt)[it];
-                    const double o0 = dpp_f64<kDppXor2>(h.x), o1 = dpp_f64<kDppXor2>(h.y);
-                    aj = it == 0 ? h.x : o0;
-                    cj = it == 0 ? h.y : o1;
-                    iaj = it == 0 ? o0 : h.x;
-                    dEj = it == 0 ? o1 : h.y;
-                } else {
-                    const double4 rj = arec[(size_t)j * NT + jt];
-                    aj = rj.x;
-                    cj = rj.y;
-                    iaj = rj.z;
-                    dEj = rj.w;
-                }
-                const double r_inv = rsqrt(rsq);
-                // the lane's own density record; the transposed type pair's comes from
-                // its lane (transpose_tp)
-                const Q* rec = deriv + (size_t)(p0 + done + slot) * DerivRec<NT>::kLen;
-                const typename Vec2<Q>::T rg =
-                    *reinterpret_cast<const typename Vec2<Q>::T*>(rec + DerivRec<NT>::rho(q));
-                // one phi slot serves (it, jt) and (jt, it)
-                const typename Vec2<Q>::T rf = *reinterpret_cast<const typename Vec2<Q>::T*>(
-                    rec + DerivRec<NT>::phi(want_phi ? it : jt, want_phi ? jt : it));
-                const double g_dr = (double)rg.x, g_da = (double)rg.y;
-                const double f_dr = (double)rf.x, f_da = (double)rf.y;
-                const double gT_dr = transpose_tp<NT>(g_dr), gT_da = transpose_tp<NT>(g_da);
-                const double fr_dr = f_dr, fr_da = f_da;
-                const double cc = ci * cj;
-                // 1/(alpha_i + alpha_j) = (1/alpha_i)(1/alpha_j) / (1/alpha_i + 1/alpha_j)
-                const double ia = iai + iaj;
-                double ria = __builtin_amdgcn_rcp(ia);
-                ria = ria * (2.0 - ia * ria);
-                ria = ria * (2.0 - ia * ria);
-                const double is = iai * iaj * ria;
-                const double fpair = -(gT_dr * dEi + g_dr * dEj + fr_dr) * cc * r_inv;
-                const double apair = -(gT_da * dEi + g_da * dEj + fr_da) * cc * (is * is);
-                fa += apair * aj * aj;
-                aJ = apair * ai * ai;
-                S = fpair;
-            }
-            S = sum_over_it<NT>(sum_over_jt<NT>(S));
-            aJ = sum_over_it<NT>(aJ);
-            if (inr && q == 0) {
-                fx += dx0 * S;
-                fy += dx1 * S;
-                fz += dx2 * S;
-                const double wf = owned ? S : 0.5 * S;
-                vir[0] -= wf * dx0 * dx0;
-                vir[1] -= wf * dx1 * dx1;
-                vir[2] -= wf * dx2 * dx2;
-                vir[3] -= wf * dx1 * dx2;
-                vir[4] -= wf * dx2 * dx0;
-                vir[5] -= wf * dx0 * dx1;
-            }
-            if constexpr (NT == 2) {
-                // lanes 0 and 1 of the pair store {fx, fy} and {fz, alpha force 0} (32
-                // contiguous bytes), lane 2 the alpha force of type 1: aJ of type jt
-                // lives on the lanes it = 0, 1 of that jt, moved to lanes 1 and 2
-                const double aJx = dpp_f64<kDppQuad0033>(aJ);
-                if (valid && owned) {
-                    if (q < 2) {
-                        const double2 v = q == 0 ? make_double2(-dx0 * S, -dx1 * S) : make_double2(-dx2 * S, aJx);
-                        reinterpret_cast<double2*>(F.sh4 + (size_t)rp * 4)[q] = v;
-                    } else if (q == 2) {
-                        F.shx[rp] = aJx;
-                    }
-                }
-            } else {
-                if (valid && owned) {
-                    double* dst = F.sh4 + (size_t)rp * 4;
-                    if (q == 0) {
-                        dst[0] = -dx0 * S;
-                        dst[1] = -dx1 * S;
-                        dst[2] = -dx2 * S;
-                    }
-                    if (it == 0) {
-                        if (jt == 0) dst[3] = aJ;
-                        else F.shx[(size_t)rp * (NT - 1) + jt - 1] = aJ;
-                    }
-                }
-            }
-        }
-        done += cnt;
-        }
-        double sx, sy, sz, sa[NT];
-        if constexpr (NT == 2) {
-            // fx, fy, fz live on the lanes q = 0 and fa[it] on q = 2 it + jt: join the
-            // jt lanes (q = 0 and 2 then hold fa[0], fa[1]), pack the five sums into two
-            // registers -- q = 0: (fx, fy), q = 1: (fz, fa[0]), q = 2: (fa[1], 0) -- and
-            // sum both over the 16 pair slots at once
-            const double fa2 = fa + dpp_f64<kDppXor1>(fa);
-            const double fz1 = dpp_f64<kDppQuad0022>(fz), fa1 = dpp_f64<kDppQuad0022>(fa2);
-            double A = q == 0 ? fx : (q == 1 ? fz1 : (q == 2 ? fa2 : 0.0));
-            double B = q == 0 ? fy : (q == 1 ? fa1 : 0.0);
-            quad_slot_sums(A, B);
-            sx = read_lane(A, 0);
-            sy = read_lane(B, 0);
-            sz = read_lane(A, 1);
-            sa[0] = read_lane(B, 1);
-            sa[1] = read_lane(A, 2);
-        } else {
-            sx = wave_sum(fx);
-            sy = wave_sum(fy);
-            sz = wave_sum(fz);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) sa[t] = wave_sum(it == t ? fa : 0.0);
-        }
-        if (lane == 0) {
-            fown[(size_t)i * XD + 0] = sx;
-            fown[(size_t)i * XD + 1] = sy;
-            fown[(size_t)i * XD + 2] = sz;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) fown[(size_t)i * XD + 3 + t] = sa[t];
-        }
-    }
-    if constexpr (NT == 2) {
-        // the virial lives on the lanes q = 0: q = 0 packs (v0, v1), q = 1 (v2, v3), q = 2 (v4, v5)
-        double w[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) w[c] = dpp_f64<kDppQuad0000>(vir[2 + c]);
-        double A = q == 0 ? vir[0] : (q == 1 ? w[0] : (q == 2 ? w[2] : 0.0));
-        double B = q == 0 ? vir[1] : (q == 1 ? w[1] : (q == 2 ? w[3] : 0.0));
-        quad_slot_sums(A, B);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            vir[2 * c] = read_lane(A, c);
-            vir[2 * c + 1] = read_lane(B, c);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) vir[c] = wave_sum(vir[c]);
-    }
-    wave_store<6>(vir, part);
+// Two values summed over pairs of lanes: even lanes get the pair's sum of a, odd
+// lanes the pair's sum of b (XOR1), or lanes with bit 1 clear / set (XOR2).
+template <int CTRL>
+__device__ __forceinline__ double fold2(double a, double b) {
+    const bool hi = threadIdx.x & (CTRL == kDppXor1 ? 1 : 2);
+    return (hi ? b : a) + dpp_f64<CTRL>(hi ? a : b);
+}
+// Sums over 32 lanes (half a wavefront), the value of lane l % 4 in each lane
+// (fixed tree: lane pairs, quads, the four quads of a row, the two rows).
+__device__ __forceinline__ double half_sums(double quad) {
+    quad += dpp_f64<kDppRowRor4>(quad);
+    quad += dpp_f64<kDppRowRor8>(quad);
+    return row_pair_sum<false>(quad);
+}
+__device__ __forceinline__ double quad4(double a, double b, double c, double d) {
+    return fold2<kDppXor2>(fold2<kDppXor1>(a, b), fold2<kDppXor1>(c, d));
 }
 
+constexpr int kPass2Lanes = 32;  // lanes per site
+
+// src/ff_dmd_I.cpp:357-436: fpair/apair of each ordered type pair from the
+// records of pass 1 (slot type2rho[jt][it], i.e. the transposed type pair's
+// values, pairs with dE_i; phi for it < jt is the phi of (jt, it), as in the
+// reference's shared COMP slot).  No table lookups.
+//
+// One lane per pair: it reads the pair's whole record (16-byte pieces of 64-byte
+// runs, PairRec), the partner's position and {alpha, c, F'} of every type, and
+// sums over the type pairs in registers, so nothing is exchanged between lanes
+// but the site's sums at the end; the record names the partner, so no list entry
+// is read and nothing is packed.  Half a wavefront per site, since a site of a
+// close-packed crystal has about 27 pairs inside the cut.  With a lane per (pair,
+// type pair) and the pairs packed through ds_permute this pass took 1.69 ms at
+// 1,048,576 sites of two types (572 vector instructions per site, 15 memory
+// instructions per site) and now takes 1.36 ms (FP32 records 1.57 -> 1.07).  Its
+// bound is the bytes: without the records it takes 1.10 ms, without the shares'
+// scattered writes 0.99 ms.  Shares at the pair's own list position, written in
+// whole lines and read scattered by the gather, took 1.25 ms here and 0.51 ms
+// there in place of 0.37.
+template <int NT, typename Q>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 4 : (NT == 3 ? 3 : 2)))) void k_pass2(
+    int natms, const double4* __restrict__ pos, const double4* __restrict__ arec, const int2* __restrict__ info,
+    const typename Vec2<Q>::T* __restrict__ deriv, double* __restrict__ fown, double* __restrict__ share,
+    double* __restrict__ part, int wpb) {
+    using R = PairRec<NT, Q>;
+    using Q2 = typename Vec2<Q>::T;
+    constexpr int XD = 3 + NT, NPHI = NT * (NT + 1) / 2;
+    const int l = threadIdx.x % kPass2Lanes;
+    const bool odd = l & 1;
+    double vir[6] = {0, 0, 0, 0, 0, 0};
+    const SiteLoop<kPass2Lanes> sl(natms, wpb);
+    for (int i = sl.first; i < sl.end; i += sl.stride) {
+        const int2 in = info[i];  // list offset, pairs inside the cut
+        const double4 xi = pos[i];
+        double ai[NT], ci[NT], dEi[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const double4 ra = arec[(size_t)i * NT + t];
+            ai[t] = ra.x;
+            ci[t] = ra.y;
+            dEi[t] = ra.w;
+        }
+        const int cnt = in.y;
+        const Q2* const rec = deriv + R::first(in.x, i);
+        double f[3] = {0.0, 0.0, 0.0}, fa[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) fa[t] = 0.0;
+        for (int base = 0; base < cnt; base += kPass2Lanes) {
+            // lanes past the last pair repeat it with zero weight and store nothing
+            const bool valid = base + l < cnt;
+            const Q2* const d = rec + R::elem(valid ? base + l : cnt - 1, 0);
+            const int2 e = Vec2<Q>::ints(d[R::kIdx * R::kG]);
+            const int j = e.x, rp = valid ? e.y : -1;
+            Q2 g[NT * NT], ph[NPHI];
+#pragma unroll
+            for (int q = 0; q < NT * NT; ++q) g[q] = d[R::rho(q) * R::kG];
+#pragma unroll
+            for (int q = 0; q < NPHI; ++q) ph[q] = d[(NT * NT + q) * R::kG];
+            const double4 xj = pos[j];
+            double aj[NT], cj[NT], dEj[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const double4 rj = arec[(size_t)j * NT + t];
+                aj[t] = rj.x;
+                cj[t] = valid ? rj.y : 0.0;
+                dEj[t] = rj.w;
+            }
+            const double dx0 = xi.x - xj.x, dx1 = xi.y - xj.y, dx2 = xi.z - xj.z;
+            double rsq;
+            {
+#pragma clang fp contract(off)
+                rsq = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;
+            }
+            double S = 0.0, aJ[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) aJ[t] = 0.0;
+#pragma unroll
+            for (int it = 0; it < NT; ++it)
+#pragma unroll
+                for (int jt = 0; jt < NT; ++jt) {
+                    const Q2 gq = g[it * NT + jt], gT = g[jt * NT + it], pq = ph[type2phi(it, jt)];
+                    const double cc = ci[it] * cj[jt];
+                    // 1/(alpha_i + alpha_j)
+                    const double as = ai[it] + aj[jt];
+                    double is = __builtin_amdgcn_rcp(as);
+                    is = is * (2.0 - as * is);
+                    is = is * (2.0 - as * is);
+                    S += ((double)gT.x * dEi[it] + (double)gq.x * dEj[jt] + (double)pq.x) * cc;
+                    const double ap = ((double)gT.y * dEi[it] + (double)gq.y * dEj[jt] + (double)pq.y) * cc * (is * is);
+                    fa[it] -= ap * (aj[jt] * aj[jt]);
+                    aJ[jt] -= ap * (ai[it] * ai[it]);
+                }
+            S *= -rsqrt(rsq);
+            const double h0 = dx0 * S, h1 = dx1 * S, h2 = dx2 * S;
+            f[0] += h0;
+            f[1] += h1;
+            f[2] += h2;
+            const double wf = rp >= 0 ? 1.0 : 0.5;  // an owned partner, or half of a pair seen from both ends
+            vir[0] -= wf * (h0 * dx0);
+            vir[1] -= wf * (h1 * dx1);
+            vir[2] -= wf * (h2 * dx2);
+            vir[3] -= wf * (h1 * dx2);
+            vir[4] -= wf * (h2 * dx0);
+            vir[5] -= wf * (h0 * dx1);
+            // partner shares: the two lanes of a pair of lanes write the 16-byte halves
+            // {fx, fy}, {fz, alpha force 0} of one share together, first the even lane's
+            // pair, then the odd lane's (32 contiguous bytes each)
+            double out[ForceShare<NT>::kLen] = {S};
+#pragma unroll
+            for (int t = 0; t < NT; ++t) out[1 + t] = aJ[t];
+            if constexpr (ForceShare<NT>::kLen == 4) {
+                // the two lanes of a pair of lanes write the 16-byte halves of one share
+                // together, first the even lane's pair, then the odd lane's: one 32-byte write
+                const double r0 = dpp_f64<kDppXor1>(odd ? out[0] : out[2]), r1 = dpp_f64<kDppXor1>(odd ? out[1] : out[3]);
+                const int rpx = __builtin_amdgcn_update_dpp(0, rp, kDppXor1, 0xF, 0xF, false);
+                const int rpe = odd ? rpx : rp, rpo = odd ? rp : rpx;
+                if (rpe >= 0)
+                    reinterpret_cast<double2*>(share + (size_t)rpe * 4)[odd] = make_double2(odd ? r0 : out[0], odd ? r1 : out[1]);
+                if (rpo >= 0)
+                    reinterpret_cast<double2*>(share + (size_t)rpo * 4)[odd] = make_double2(odd ? out[2] : r0, odd ? out[3] : r1);
+            } else if (rp >= 0) {
+                double2* const d2 = reinterpret_cast<double2*>(share + (size_t)rp * ForceShare<NT>::kLen);
+#pragma unroll
+                for (int t = 0; t < ForceShare<NT>::kLen / 2; ++t) d2[t] = make_double2(out[2 * t], out[2 * t + 1]);
+            }
+        }
+        double* const fo = fown + (size_t)i * XD;
+        const double s = half_sums(quad4(f[0], f[1], f[2], fa[0]));
+        if (l < 4) fo[l] = s;
+        if constexpr (NT > 1) {
+            const double sx = half_sums(quad4(fa[1], NT > 2 ? fa[NT > 2 ? 2 : 0] : 0.0, NT > 3 ? fa[NT > 3 ? 3 : 0] : 0.0, 0.0));
+            if (l < NT - 1) fo[4 + l] = sx;
+        }
+    }
+    const double v03 = row_pair_sum<true>(half_sums(quad4(vir[0], vir[1], vir[2], vir[3])));
+    const double v45 = row_pair_sum<true>(half_sums(quad4(vir[4], vir[5], 0.0, 0.0)));
+    const int lane = threadIdx.x & 63;
+    const size_t w = (size_t)blockIdx.x * wpb + (threadIdx.x >> 6);
+    if (lane < 4) part[w * 6 + lane] = v03;
+    if (lane < 2) part[w * 6 + 4 + lane] = v45;
+}
 
 // ---------------------------------------------------------------- force gather
 template <int NT>
-__global__ __launch_bounds__(kBlock) void k_fgather(int natms, PairBufs L, const double* __restrict__ fown,
-                                                    ForceShares F,
+__global__ __launch_bounds__(kBlock) void k_fgather(int natms, const double4* __restrict__ pos,
+                                                    const int* __restrict__ roff, const int* __restrict__ rowner,
+                                                    const double* __restrict__ fown,
+                                                    const double* __restrict__ share,
                                                     const double* __restrict__ fa, double* __restrict__ f) {
     constexpr int XD = 3 + NT;
     const SiteGroup<kGatherG> g;
@@ -1298,12 +1265,26 @@ __global__ __launch_bounds__(kBlock) void k_fgather(int natms, PairBufs L, const
     double acc[XD];
 #pragma unroll
     for (int k = 0; k < XD; ++k) acc[k] = 0.0;
-    const int q1 = L.roff[i + 1];
-    for (int q = L.roff[i] + g.l; q < q1; q += kGatherG) {
+    const double4 xi = pos[i];
+    const int q1 = roff[i + 1];
+    for (int q = roff[i] + g.l; q < q1; q += kGatherG) {
+        const int o = rowner[q];
+        if (o < 0) {  // inside the cut
+            const double2* const d2 = reinterpret_cast<const double2*>(share + (size_t)q * ForceShare<NT>::kLen);
+            double v[ForceShare<NT>::kLen];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] += F.sh4[(size_t)q * 4 + k];
+            for (int t = 0; t < ForceShare<NT>::kLen / 2; ++t) {
+                const double2 w = d2[t];
+                v[2 * t] = w.x;
+                v[2 * t + 1] = w.y;
+            }
+            const double4 xo = pos[o & ~kInsideBit];
+            acc[0] -= (xo.x - xi.x) * v[0];
+            acc[1] -= (xo.y - xi.y) * v[0];
+            acc[2] -= (xo.z - xi.z) * v[0];
 #pragma unroll
-        for (int k = 4; k < XD; ++k) acc[k] += F.shx[(size_t)q * (NT - 1) + k - 4];
+            for (int t = 0; t < NT; ++t) acc[3 + t] += v[1 + t];
+        }
     }
 #pragma unroll
     for (int k = 0; k < XD; ++k) acc[k] = group_sum<kGatherG>(acc[k]);

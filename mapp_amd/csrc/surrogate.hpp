@@ -540,8 +540,9 @@ __global__ __launch_bounds__(kSurBlock) void k_pass1_sur(FFParams<double> P, FFP
                                                          const int2* nlrp, const float* __restrict__ quad,
                                                          const double* __restrict__ rho7,
                                                          const double* __restrict__ phi7, double* __restrict__ Eown,
-                                                         double* __restrict__ pairE, double* __restrict__ deriv,
-                                                         double* __restrict__ part, int* __restrict__ nfall,
+                                                         double* __restrict__ pairE, double2* __restrict__ deriv,
+                                                         int2* __restrict__ info, double* __restrict__ part,
+                                                         int* __restrict__ nfall,
                                                          CutState C) {
     constexpr int NT = 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char sur_lds_raw[];
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(kSurBlock) void k_pass1_sur(FFParams<double> P, FFP
     const bool want_phi = it >= jt;
     const float* tab = quad + (size_t)tp * kQuadRow;
     double en = 0.0, npair = 0.0;
-    const SiteLoop sl(P.natms);
+    const SiteLoop<> sl(P.natms, kSurWaves);
     for (int i0 = sl.first; i0 < sl.end; i0 += sl.stride) {
         const int i = __builtin_amdgcn_readfirstlane(i0);
         int fallbacks = 0;
@@ -564,7 +565,9 @@ __global__ __launch_bounds__(kSurBlock) void k_pass1_sur(FFParams<double> P, FFP
         const double ai = ra.x, iai = ra.z;
         double Ei = 0.0;
         const int p0 = L.off[i], p1 = L.off[i + 1];
-        int done = 0;  // inside entries of the earlier chunks (records at off[i] + rank)
+        using R = PairRec<NT, double>;
+        double2* const rec = deriv + R::first(p0, i);
+        int done = 0;  // inside entries of the earlier chunks: the pair's rank among the site's
         for (int chunk = p0; chunk < p1; chunk += 64) {
             int packed;
             int cnt;
@@ -582,7 +585,7 @@ __global__ __launch_bounds__(kSurBlock) void k_pass1_sur(FFParams<double> P, FFP
                         r2 = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;
                     }
                     in = r2 < P.cut_sq_mod;
-                    C.update<NT>(pc, e, in, jc, P.natms, pairE);
+                    C.update<NT>(pc, e, in, i, jc, P.natms, pairE);
                 }
                 cnt = pack_in_range(pc, in, &packed);
             }
@@ -661,13 +664,10 @@ __global__ __launch_bounds__(kSurBlock) void k_pass1_sur(FFParams<double> P, FFP
                     const double half = (j < P.natms ? 0.5 : 0.25) * (it != jt ? P.xw : 1.0);
                     en += half * (cj[jt] * ci[it] + cj[it] * ci[jt]) * fv[0];
                 }
-                double* d = deriv + (size_t)(p0 + done + slot) * DerivRec<NT>::kLen;
-                __builtin_nontemporal_store(gv[1], d + DerivRec<NT>::rho(tp));
-                __builtin_nontemporal_store(gv[2], d + DerivRec<NT>::rho(tp) + 1);
-                if (want_phi) {
-                    __builtin_nontemporal_store(fv[1], d + DerivRec<NT>::phi(it, jt));
-                    __builtin_nontemporal_store(fv[2], d + DerivRec<NT>::phi(it, jt) + 1);
-                }
+                double2* d = rec + R::elem(done + slot, 0);
+                store_comp(d + R::rho(tp) * R::kG, make_double2(gv[1], gv[2]));
+                if (want_phi) store_comp(d + R::phi(it, jt) * R::kG, make_double2(fv[1], fv[2]));
+                else store_comp(d + R::kIdx * R::kG, Vec2<double>::ints(j, j < P.natms ? nlrp[p].y : -1));
             }
             ej += __shfl_xor(ej, 32, 64);  // sum over it: type pairs (0,jt) and (1,jt) are 32 lanes apart
             if (valid && it == 0 && j < P.natms) pairE[(size_t)nlrp[p].y * NT + jt] = ej;  // scattered: L2 merges lines
@@ -680,7 +680,10 @@ __global__ __launch_bounds__(kSurBlock) void k_pass1_sur(FFParams<double> P, FFP
             if (lane == 0) Eown[(size_t)i * NT + t] = s;
         }
         const double sf = wave_sum((double)fallbacks);
-        if (lane == 0) nfall[i] = (int)sf;
+        if (lane == 0) {
+            nfall[i] = (int)sf;
+            info[i] = make_int2(p0, done);
+        }
     }
     double acc[2] = {wave_sum(en), wave_sum(npair)};
     block_store_waves<2, kSurWaves>(acc, part);

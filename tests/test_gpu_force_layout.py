@@ -1,0 +1,59 @@
+"""The force passes where their layout can go wrong: every rule size (the paired
+sums of 3 and 5 points, the general loop of the others), every lanes-per-pair
+schedule, one to four types, tables that do not vanish at the cutoff (the points
+beyond it read the tables' zero row instead of being tested), and sites with
+fewer pairs inside the cut than a round or a half wavefront, and with more.
+Against the FP64 oracle: forces and densities to 1e-12 (a few hundred double
+roundings), 1e-5 with FP32 quadrature sums."""
+import numpy as np
+import pytest
+
+from tests.conftest import rel_inf
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ff, orc, bound):
+    en, eo = ff.force_calc(1), orc.force_calc(1)
+    assert abs(en[0] - eo[0]) <= bound * abs(eo[0])
+    assert rel_inf(en[1:], eo[1:]) <= bound
+    for name in ("f", "E", "dE"):
+        assert rel_inf(ff.get(name), orc.get(name)) <= bound, name
+
+
+@pytest.mark.parametrize("no_i", [1, 2, 3, 4, 5, 7])
+@pytest.mark.parametrize("nt,parts", [(1, 2), (2, 1), (2, 2), (2, 4), (3, 1), (3, 2), (4, 2)])
+def test_rules_and_schedules(nt, parts, no_i):
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    tables = W.johnson_tables(elements=("Ni", "Cu", "Pd", "Ag")[:nt], nr=2001, nrho=2001)
+    end = 1e-3 * (1.0 + np.arange(nt * nt).reshape(nt, nt))
+    tables.rho = tables.rho + end[:, :, None]  # not zero at the cutoff
+    tables.rphi = tables.rphi + 1e-3
+    lat = W.fcc_alloy(6, nt=nt, seed=40 + no_i)
+    for precision, bound in (("fp64", 1e-12), ("mixed", 1e-5)):
+        ff = setup(lat, tables, no_i=no_i, precision=precision)
+        ff.set_schedule([parts, 4, 0, 2, 0])
+        _check(ff, O.make(lat, tables, no_i=no_i), bound)
+        ff.close()
+
+
+@pytest.mark.parametrize("keep", [1, 2, 5, 33, 200])
+def test_few_and_many_pairs(tables, keep):
+    """a cluster in a large box: from no pair at all to a whole half wavefront and more"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    lat = W.fcc_alloy(6, seed=9)
+    order = np.argsort(np.linalg.norm(lat.cart - lat.cart.mean(axis=0), axis=1), kind="stable")[:keep]
+    L = 60.0
+    x = lat.x[order].copy()
+    x[:, :3] = (lat.cart[order] - lat.cart.mean(axis=0) + 0.5 * L) / L
+    # closer than the lattice: up to about 60 pairs inside the cut for one site
+    x[:, :3] = 0.5 + (x[:, :3] - 0.5) * 0.85
+    box = W.Lattice(H=np.diag([L] * 3), x=np.ascontiguousarray(x), c=np.ascontiguousarray(lat.c[order]),
+                    cart=x[:, :3] * L)
+    ff = setup(box, tables, no_i=3)
+    _check(ff, O.make(box, tables, no_i=3), 1e-12)
+    ff.close()
