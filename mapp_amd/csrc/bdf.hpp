@@ -35,11 +35,11 @@ __global__ void k_bdf_interp(long n, int q, BdfInterp C, BdfHist Y, const double
     ak -= yk;
     a[k] = ak;
     y0[k] = yk;
-    if (yk < 0.0 || yk > 1.0) atomicOr(flag, 1);
+    if (yk < 0.0 || yk > 1.0) *flag = 1;  // host memory, zero at the start
 }
 
 // largest fraction of the step base + scale*dir that stays inside [0,1]
-// (src/clock_bdf.cpp:704-712 predictor, :740-752 CG step): per-block minima
+// (src/clock_bdf.cpp:704-712 predictor, :740-752 CG step): per-block {minimum, 0}
 __global__ __launch_bounds__(kBlock) void k_bdf_bound(long n, const double* __restrict__ base,
                                                       const double* __restrict__ dir, double scale,
                                                       double* __restrict__ part) {
@@ -58,7 +58,10 @@ __global__ __launch_bounds__(kBlock) void k_bdf_bound(long n, const double* __re
         if (threadIdx.x < w) sm[threadIdx.x] = fmin(sm[threadIdx.x], sm[threadIdx.x + w]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sm[0];
+    if (threadIdx.x == 0) {
+        part[blockIdx.x * 2] = sm[0];
+        part[blockIdx.x * 2 + 1] = 0.0;
+    }
 }
 
 // c = y0 + dy * del_t * ratio  (src/clock_bdf.cpp:714-715)

@@ -29,7 +29,7 @@
 using namespace mappdmd;
 
 mapp_dmd::~mapp_dmd() {
-    for (auto* b : scan_levels) delete b;
+    if (h_box) (void)hipHostFree(h_box);
     for (auto& e : ev)
         if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
@@ -100,72 +100,50 @@ void sort_segments(mapp_dmd* ctx, const int* start, const int* key, int* v, long
     HIP_OK(hipMemcpyAsync(v, ctx->d_sort_tmp.p, sizeof(int) * n, hipMemcpyDeviceToDevice, ctx->stream));
 }
 
-// exclusive scan of n ints; returns the total (synchronizes the stream)
-long exclusive_scan(mapp_dmd* ctx, const int* in, int* out, long n, int depth = 0) {
-    if (n <= 0) return 0;
-    const int nb = (int)((n + kScanTile - 1) / kScanTile);
-    while ((int)ctx->scan_levels.size() < 2 * (depth + 1)) ctx->scan_levels.push_back(new DevBuf<int>());
-    DevBuf<int>& sums = *ctx->scan_levels[2 * depth];
-    DevBuf<int>& sums_x = *ctx->scan_levels[2 * depth + 1];
-    sums.reserve(nb);
-    sums_x.reserve(nb);
-    hipLaunchKernelGGL(k_scan_tile, dim3(nb), dim3(kScanThreads), 0, ctx->stream, in, out, sums.p, n);
-    launch_check("k_scan_tile");
-    if (nb > 1) {
-        exclusive_scan(ctx, sums.p, sums_x.p, nb, depth + 1);
-        hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kScanThreads), 0, ctx->stream, out, sums_x.p, n);
-        launch_check("k_scan_add");
+// The context's mailbox: pinned host memory that the last kernel of a call writes its
+// scalars to, so that no copy follows it (a copy of a few bytes costs the stream about
+// as much as a small kernel).  Valid after the stream is synchronised.
+void wait_box(mapp_dmd* ctx) { HIP_OK(hipStreamSynchronize(ctx->stream)); }
+
+// exclusive scan of n ints; returns the total (synchronizes the stream); out[n] = the
+// total too when end is set (out then has n + 1 elements).  Refused when the total
+// does not fit an int.
+long exclusive_scan(mapp_dmd* ctx, const int* in, int* out, long n, bool end = false) {
+    if (n <= 0) {
+        if (end) HIP_OK(hipMemsetAsync(out, 0, sizeof(int), ctx->stream));
+        return 0;
     }
-    int last[2];
-    HIP_OK(hipMemcpyAsync(&last[0], out + n - 1, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_OK(hipMemcpyAsync(&last[1], in + n - 1, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_OK(hipStreamSynchronize(ctx->stream));
-    return (long)last[0] + last[1];
+    const int nb = (int)((n + kScanTile - 1) / kScanTile);
+    ctx->d_scan.reserve((size_t)nb + 1);
+    unsigned long long* sums = ctx->d_scan.p;
+    unsigned long long* box = reinterpret_cast<unsigned long long*>(ctx->h_box);
+    hipLaunchKernelGGL(k_scan_tile, dim3(nb), dim3(kScanThreads), 0, ctx->stream, in, out, sums, n);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanSumThreads), 0, ctx->stream, sums, nb, sums + nb);
+    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kScanThreads), 0, ctx->stream, out, sums, n, sums + nb,
+                       end ? out + n : (int*)nullptr, box);
+    launch_check("k_scan");
+    wait_box(ctx);
+    const unsigned long long total = *box;
+    if (total >= (1ull << 31))
+        throw ApiError(MAPP_DMD_E_RANGE, "a list or table needs " + std::to_string(total) +
+                                             " entries; its int offsets hold fewer than 2^31");
+    return (long)total;
 }
 
 // CSR offsets (n+1) from counts (n); the offsets are int, so a total of 2^31
 // entries or more is refused before any caller sizes its entry array by it
 long counts_to_offsets(mapp_dmd* ctx, const int* cnt, DevBuf<int>& off, long n) {
     off.reserve(n + 1);
-    unsigned long long total = 0;
-    if (n > 0) {
-        ctx->d_total.reserve(1);
-        HIP_OK(hipMemsetAsync(ctx->d_total.p, 0, sizeof(unsigned long long), ctx->stream));
-        hipLaunchKernelGGL(k_count_total, dim3((int)std::min<long>(nblk(n, kCountThreads), 1024)), dim3(kCountThreads),
-                           0, ctx->stream,
-                           cnt, n, ctx->d_total.p);
-        launch_check("k_count_total");
-        HIP_OK(hipMemcpyAsync(&total, ctx->d_total.p, sizeof(total), hipMemcpyDeviceToHost, ctx->stream));
-    }
-    long tot = exclusive_scan(ctx, cnt, off.p, n);  // synchronizes the stream: total is in
-    if (total >= (1ull << 31))
-        throw ApiError(MAPP_DMD_E_RANGE, "a list or table needs " + std::to_string(total) +
-                                             " entries; its int offsets hold fewer than 2^31");
-    int t = (int)tot;
-    HIP_OK(hipMemcpyAsync(off.p + n, &t, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-    HIP_OK(hipStreamSynchronize(ctx->stream));
-    return tot;
+    return exclusive_scan(ctx, cnt, off.p, n, true);
 }
 
-// partials per first-stage block of reduce_partials
-constexpr long kReduceChunk = 4096;
-// doubles of stage memory reduce_partials needs for nparts partials
+// doubles of stage memory a reduction needs for nparts partials
 inline long reduce_stage_doubles(long nparts) { return ((nparts + kReduceChunk - 1) / kReduceChunk + 1) * 8; }
 
-// out[0..nv) = sum over nparts partials (stride doubles each, starting at offset),
-// in two fixed-shape stages through stage[reduce_stage_doubles(nparts)]
-void reduce_partials_in(mapp_dmd* ctx, const double* part, long nparts, int nv, int stride, int offset, double* stage,
-                        double* out) {
-    const long nb1 = (nparts + kReduceChunk - 1) / kReduceChunk;
-    hipLaunchKernelGGL(k_reduce_stage, dim3((int)nb1), dim3(kBlock), 0, ctx->stream, part, nparts, nv, stride, offset,
-                       kReduceChunk, stage, 8);
-    hipLaunchKernelGGL(k_reduce_stage, dim3(1), dim3(kBlock), 0, ctx->stream, stage, nb1, nv, 8, 0, nb1, out, 1);
-    launch_check("k_reduce_stage");
-}
-
-// several reduce_partials (parts[s], nparts[s], nv[s] <= 8 values, stride[s] -> out[out_off[s]..]) in two launches
-void reduce_partials_segs(mapp_dmd* ctx, int nseg, const double* const* parts, const long* nparts, const int* nv,
-                          const int* stride, const int* out_off, double* out) {
+// out[out_off[s]..) = the sums of parts[s] (nparts[s] partials of nv[s] <= 8 values, stride[s]
+// doubles apart) in two launches, through stage memory
+void reduce_segs_in(mapp_dmd* ctx, int nseg, const double* const* parts, const long* nparts, const int* nv,
+                    const int* stride, const int* out_off, double* stage, double* out) {
     ReduceSegs R{};
     R.nseg = nseg;
     int tot = 0;
@@ -179,17 +157,21 @@ void reduce_partials_segs(mapp_dmd* ctx, int nseg, const double* const* parts, c
         R.nb[k] = (int)((nparts[k] + kReduceChunk - 1) / kReduceChunk);
         tot += R.nb[k];
     }
-    ctx->d_stage.reserve((size_t)(tot + 1) * 8);
-    if (tot > 0)
-        hipLaunchKernelGGL(k_reduce_segs1, dim3(tot), dim3(kBlock), 0, ctx->stream, R, kReduceChunk, ctx->d_stage.p);
-    hipLaunchKernelGGL(k_reduce_segs2, dim3(nseg), dim3(kBlock), 0, ctx->stream, R, ctx->d_stage.p, out);
+    if (tot > 0) hipLaunchKernelGGL(k_reduce_segs1, dim3(tot), dim3(kBlock), 0, ctx->stream, R, stage);
+    hipLaunchKernelGGL(k_reduce_segs2, dim3(nseg), dim3(kBlock), 0, ctx->stream, R, stage, out);
     launch_check("k_reduce_segs");
 }
-
-// the same with the context's stage buffer
-void reduce_partials(mapp_dmd* ctx, const double* part, long nparts, int nv, int stride, int offset, double* out) {
-    ctx->d_stage.reserve((size_t)reduce_stage_doubles(nparts));
-    reduce_partials_in(ctx, part, nparts, nv, stride, offset, ctx->d_stage.p, out);
+void reduce_partials_segs(mapp_dmd* ctx, int nseg, const double* const* parts, const long* nparts, const int* nv,
+                          const int* stride, const int* out_off, double* out) {
+    long need = 0;
+    for (int k = 0; k < nseg; ++k) need += reduce_stage_doubles(nparts[k]);
+    ctx->d_stage.reserve((size_t)need);
+    reduce_segs_in(ctx, nseg, parts, nparts, nv, stride, out_off, ctx->d_stage.p, out);
+}
+// one array of partials, nv values each
+void reduce_partials(mapp_dmd* ctx, const double* part, long nparts, int nv, double* out) {
+    const int zero = 0;
+    reduce_partials_segs(ctx, 1, &part, &nparts, &nv, &nv, &zero, out);
 }
 
 void require(bool cond, int code, const char* msg) {
@@ -520,8 +502,6 @@ void md_passes(mapp_dmd* ctx, bool energy_only, int nb, const PairBufs& L, const
             hipLaunchKernelGGL((k_eam_embed<MODEL, false>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md,
                                ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_E.p, ctx->d_dE.p, part2);
         launch_check("k_eam_embed");
-    } else {
-        HIP_OK(hipMemsetAsync(part2, 0, sizeof(double) * nb, st));  // no embedding term
     }
 }
 
@@ -534,7 +514,6 @@ double run_eam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     PairBufs L{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p};
     EamBufs T{ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_F7.p, ctx->nt};
     ctx->d_part.reserve((size_t)nb * 14 + 16);
-    ctx->d_out.reserve(16);
     ctx->d_drho.reserve(2 * ((size_t)ctx->npairs + 1));  // one double2 per pair
     ctx->d_pairF2.reserve((size_t)(ctx->nrev + 1) * 3);
     double* part1 = ctx->d_part.p;
@@ -546,26 +525,27 @@ double run_eam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     else if (lj) md_passes<kModelLj>(ctx, energy_only, nb, L, T, drho, part1, part2);
     else if (ctx->variant == MAPP_DMD_VARIANT_FS) md_passes<kModelFs>(ctx, energy_only, nb, L, T, drho, part1, part2);
     else md_passes<kModelFsm>(ctx, energy_only, nb, L, T, drho, part1, part2);
-    double* out = ctx->d_out.p;
-    reduce_partials(ctx, part1, nb, 7, 7, 0, out);
-    reduce_partials(ctx, part2, nb, 1, 1, 0, out + 7);
     if (!energy_only) {
         if (!lj) {
             ghost_copy(ctx, ctx->d_dE.p, 1);
             hipLaunchKernelGGL(k_eam_pass2, dim3(nb), dim3(kBlock), 0, st, ctx->P, ctx->d_pos.p, L, ctx->d_rpos.p,
                                drho, ctx->d_dE.p, ctx->d_fown.p, ctx->d_pairF2.p, part3);
             launch_check("k_eam_pass2");
-        } else {
-            HIP_OK(hipMemsetAsync(part3, 0, sizeof(double) * nb * 6, st));
         }
         hipLaunchKernelGGL(k_eam_gather, dim3(nb), dim3(kBlock), 0, st, natms, L, ctx->d_fown.p, ctx->d_pairF.p,
                            lj ? (const double*)nullptr : ctx->d_pairF2.p, ctx->d_f.p);
         launch_check("k_eam_gather");
-        reduce_partials(ctx, part3, nb, 6, 6, 0, out + 8);
     }
-    double h[14];
-    HIP_OK(hipMemcpyAsync(h, out, sizeof(double) * (energy_only ? 8 : 14), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
+    // pass 1's energy and virial, the embedding energy, pass 2's virial (LJ has only the first)
+    double* h = ctx->h_box;
+    for (int k = 0; k < 14; ++k) h[k] = 0.0;
+    {
+        const double* parts[3] = {part1, part2, part3};
+        const long nparts[3] = {nb, nb, nb};
+        const int nv[3] = {7, 1, 6}, off[3] = {0, 7, 8};
+        reduce_partials_segs(ctx, lj ? 1 : (energy_only ? 2 : 3), parts, nparts, nv, nv, off, h);
+    }
+    wait_box(ctx);
     const double energy = h[0] + h[7];
     if (en_st) {
         en_st[0] = energy;
@@ -602,11 +582,9 @@ double run_meam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     const int nb = (natms + kMeamWaves - 1) / kMeamWaves;
     const MeamDev M = ctx->meam.device(ctx->meam_fix);
     ctx->d_part.reserve((size_t)nb * 14 + 16);
-    ctx->d_out.reserve(16);
     double* part1 = ctx->d_part.p;
     double* part2 = part1 + nb;
     double* part3 = part2 + (size_t)nb * 7;
-    double* out = ctx->d_out.p;
     if (energy_only)
         hipLaunchKernelGGL((k_meam_density<true>), dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p,
                            ctx->d_off.p, ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p, ctx->d_mrec.p, part1);
@@ -614,7 +592,6 @@ double run_meam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
         hipLaunchKernelGGL((k_meam_density<false>), dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p,
                            ctx->d_off.p, ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p, ctx->d_mrec.p, part1);
     launch_check("k_meam_density");
-    reduce_partials(ctx, part1, nb, 1, 1, 0, out);
     if (!energy_only) {
         ghost_copy(ctx, ctx->d_mrec.p, kMeamRec);
         hipLaunchKernelGGL(k_meam_force, dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p,
@@ -624,12 +601,15 @@ double run_meam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
         hipLaunchKernelGGL(k_meam_kforce, dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p,
                            ctx->d_nl.p, natms, ctx->d_mpairs.p, ctx->d_mactive.p, ctx->d_mact.p, ctx->d_f.p, part3);
         launch_check("k_meam_kforce");
-        reduce_partials(ctx, part2, nb, 7, 7, 0, out + 1);
-        reduce_partials(ctx, part3, nb, 6, 6, 0, out + 8);
     }
-    double h[14];
-    HIP_OK(hipMemcpyAsync(h, out, sizeof(double) * (energy_only ? 1 : 14), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
+    const double* h = ctx->h_box;
+    {
+        const double* parts[3] = {part1, part2, part3};
+        const long nparts[3] = {nb, nb, nb};
+        const int nv[3] = {1, 7, 6}, off[3] = {0, 1, 8};
+        reduce_partials_segs(ctx, energy_only ? 1 : 3, parts, nparts, nv, nv, off, ctx->h_box);
+    }
+    wait_box(ctx);
     const double energy = energy_only ? h[0] : h[0] + h[1];
     if (en_st) {
         en_st[0] = energy;
@@ -690,7 +670,6 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
     const long np1 = sur ? (long)nb1 : (long)nb1 * ctx->sh1.wpb;
     const long np2 = (long)nbe * (kBlock / 64), np3 = (long)nbw * ctx->sh2.wpb;
     ctx->d_part.reserve((size_t)np1 * 2 + (size_t)np3 * 6 + (size_t)np2 + 16);
-    ctx->d_out.reserve(16);
     double* part1 = ctx->d_part.p;
     double* part2 = part1 + (size_t)np1 * 2;
     double* part3 = part2 + (size_t)np2;
@@ -740,17 +719,15 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
     hipLaunchKernelGGL((k_fgather<NT>), dim3(nb), dim3(kBlock), 0, st, natms, ctx->d_pos.p, ctx->d_roff.p,
                        ctx->d_rowner.p, ctx->d_fown.p, ctx->d_pairF.p, ctx->d_fa.p, ctx->d_f.p);
     launch_check("k_fgather");
-    double* out = ctx->d_out.p;
     {
         const double* parts[3] = {part1, part2, part3};
         const long nparts[3] = {np1, np2, np3};
         const int nv[3] = {2, 1, 6}, stride[3] = {2, 1, 6}, off[3] = {0, 2, 3};
-        reduce_partials_segs(ctx, 3, parts, nparts, nv, stride, off, out);
+        reduce_partials_segs(ctx, 3, parts, nparts, nv, stride, off, ctx->h_box);
     }
     if (ctx->timing) HIP_OK(hipEventRecord(ctx->ev[4], st));
-    double h[9];
-    HIP_OK(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
+    wait_box(ctx);
+    const double* h = ctx->h_box;
     ctx->n_inrange = (long)h[1];
     en_st[0] = h[0] + h[2];
     if (st_clc)
@@ -774,7 +751,6 @@ double run_energy(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
     PairBufs L{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p};
     const long np1 = (long)nbw * ctx->sh1.wpb, np2 = (long)nb * (kBlock / 64);  // one partial per wavefront
     ctx->d_part.reserve((size_t)np1 * 2 + (size_t)np2 + 16);
-    ctx->d_out.reserve(16);
     double* part1 = ctx->d_part.p;
     double* part2 = part1 + (size_t)np1 * 2;
     pack_atoms<NT>(ctx);
@@ -785,17 +761,14 @@ double run_energy(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
                        ctx->d_roff.p, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_F9.p, ctx->d_E.p, ctx->d_dE.p,
                        ctx->d_fa.p, ctx->d_arec.p, part2);
     launch_check("k_embed energy");
-    double* out = ctx->d_out.p;
     {
         const double* parts[2] = {part1, part2};
         const long nparts[2] = {np1, np2};
         const int nv[2] = {1, 1}, stride[2] = {2, 1}, off[2] = {0, 1};
-        reduce_partials_segs(ctx, 2, parts, nparts, nv, stride, off, out);
+        reduce_partials_segs(ctx, 2, parts, nparts, nv, stride, off, ctx->h_box);
     }
-    double h[2];
-    HIP_OK(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
-    return h[0] + h[1];
+    wait_box(ctx);
+    return ctx->h_box[0] + ctx->h_box[1];
 }
 
 template <int NT>
@@ -1043,11 +1016,10 @@ void run_c_d(mapp_dmd* ctx) {
 }
 
 // device memory calc_g needs beyond the per-atom vectors: the per-block partials
-// of the cost, the reduction's stage and the reduced cost
+// of the cost and the reduction's stage
 struct GScratch {
     double* part;
     double* stage;
-    double* out;
 };
 
 // blocks of the 2nd-list sweeps of calc_g (one partial each)
@@ -1076,16 +1048,18 @@ double run_calc_g(mapp_dmd* ctx, int chk, double alpha_t, const double* a, doubl
         S = *fixed;
     } else {
         ctx->d_part.reserve((size_t)nb2 + 16);
-        ctx->d_out.reserve(16);
         ctx->d_stage.reserve((size_t)reduce_stage_doubles(nb2));
-        S = GScratch{ctx->d_part.p, ctx->d_stage.p, ctx->d_out.p};
+        S = GScratch{ctx->d_part.p, ctx->d_stage.p};
     }
     hipLaunchKernelGGL((k_calc_g_s<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, alpha_t, ctx->d_conc.p, a,
                        ctx->d_foff2.p, ctx->d_fidx2.p, ctx->d_n.p, ctx->d_s.p, ctx->d_cd.p, S.part);
     launch_check("k_calc_g_s");
-    reduce_partials_in(ctx, S.part, nb2, 1, 1, 0, S.stage, S.out);
-    double inner = 0.0;
-    HIP_OK(hipMemcpyAsync(&inner, S.out, sizeof(double), hipMemcpyDeviceToHost, st));
+    {
+        const double* parts[1] = {S.part};
+        const long nparts[1] = {nb2};
+        const int one = 1, zero = 0;
+        reduce_segs_in(ctx, 1, parts, nparts, &one, &one, &zero, S.stage, ctx->h_box);
+    }
     if (!chk) {
         ghost_copy(ctx, ctx->d_s.p, NT);
         hipLaunchKernelGGL((k_calc_g_t<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, alpha_t, ctx->d_conc.p,
@@ -1101,8 +1075,8 @@ double run_calc_g(mapp_dmd* ctx, int chk, double alpha_t, const double* a, doubl
                            ctx->d_ddE.p, ctx->d_v.p, g);
         launch_check("k_calc_g_w");
     }
-    HIP_OK(hipStreamSynchronize(st));
-    return inner * 0.25;
+    wait_box(ctx);
+    return ctx->h_box[0] * 0.25;
 }
 
 template <int NT>
@@ -1174,13 +1148,13 @@ int update_x_device(mapp_dmd* ctx) {
     const int nt = acols(ctx), natms = ctx->natms;
     if (is_md(ctx)) scatter_x<1, 0>(ctx, ctx->d_xaos.p);
     else with_nt(nt, [&](auto c) { scatter_x<decltype(c)::value>(ctx, ctx->d_xaos.p); });
-    HIP_OK(hipMemsetAsync(ctx->d_iflag.p, 0, sizeof(int), ctx->stream));
+    int* const box = reinterpret_cast<int*>(ctx->h_box);
+    *box = 0;
     hipLaunchKernelGGL(k_skin_check, dim3(nblk(natms)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p, ctx->d_x0.p, natms,
-                       ctx->skin * ctx->skin, ctx->d_iflag.p);
+                       ctx->skin * ctx->skin, box);
     launch_check("k_skin_check");
-    int flag = 0;
-    HIP_OK(hipMemcpyAsync(&flag, ctx->d_iflag.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_OK(hipStreamSynchronize(ctx->stream));
+    wait_box(ctx);
+    const int flag = *box;
     if (flag) {
         hipLaunchKernelGGL(k_x2s, dim3(nblk(natms)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p, natms, ctx->bp);
         launch_check("k_x2s");
@@ -1204,17 +1178,18 @@ double energy_any(mapp_dmd* ctx) {
     return with_nt(ctx->nt, [&](auto c) { return dispatch_energy<decltype(c)::value>(ctx); });
 }
 
-constexpr int kVecBlocks = 1024;  // grid of the grid-stride vector kernels (fixed: deterministic sums)
+// grid of the grid-stride vector kernels over n entries (a function of n alone: deterministic sums)
+inline int vec_blocks(long n) { return (int)std::min<long>(1024, std::max<long>(1, (n + 4 * kBlock - 1) / (4 * kBlock))); }
 
 template <int ND>
 void dots(mapp_dmd* ctx, long n, const DotArgs& D, double* res) {
-    ctx->d_part.reserve((size_t)kVecBlocks * 8 + 16);
-    ctx->d_out.reserve(16);
-    hipLaunchKernelGGL((k_dots<ND>), dim3(kVecBlocks), dim3(kBlock), 0, ctx->stream, D, n, ctx->d_part.p);
+    const int nb = vec_blocks(n);
+    ctx->d_part.reserve((size_t)nb * 8 + 16);
+    hipLaunchKernelGGL((k_dots<ND>), dim3(nb), dim3(kBlock), 0, ctx->stream, D, n, ctx->d_part.p);
     launch_check("k_dots");
-    reduce_partials(ctx, ctx->d_part.p, kVecBlocks, ND, ND, 0, ctx->d_out.p);
-    HIP_OK(hipMemcpyAsync(res, ctx->d_out.p, sizeof(double) * ND, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_OK(hipStreamSynchronize(ctx->stream));
+    reduce_partials(ctx, ctx->d_part.p, nb, ND, ctx->h_box);
+    wait_box(ctx);
+    for (int k = 0; k < ND; ++k) res[k] = ctx->h_box[k];
 }
 double dot1(mapp_dmd* ctx, long n, const double* a, const double* b) {
     DotArgs D{{a, nullptr, nullptr, nullptr}, {b, nullptr, nullptr, nullptr}};
@@ -1237,17 +1212,13 @@ int line_min(mapp_dmd* ctx, long n, double* nrgy, double* alph, long* n_energy) 
     hipLaunchKernelGGL(k_axpby, dim3(nblk(n)), dim3(kBlock), 0, st, n, 0.0, h, hh, h);
     launch_check("k_axpby");
     const double inner = dot1(ctx, n, ctx->d_f.p, h);
-    ctx->d_part.reserve((size_t)kVecBlocks * 8 + 16);
-    hipLaunchKernelGGL(k_extrema, dim3(kVecBlocks), dim3(kBlock), 0, st, n, xd, h, x0, ctx->d_part.p);
+    const int nb = vec_blocks(n);
+    ctx->d_part.reserve((size_t)nb * 8 + 16);
+    hipLaunchKernelGGL(k_extrema, dim3(nb), dim3(kBlock), 0, st, n, xd, h, x0, ctx->d_part.p);
+    hipLaunchKernelGGL(k_fold_minmax, dim3(1), dim3(kBlock), 0, st, ctx->d_part.p, nb, ctx->h_box);
     launch_check("k_extrema");
-    std::vector<double> ex((size_t)kVecBlocks * 2);
-    HIP_OK(hipMemcpyAsync(ex.data(), ctx->d_part.p, ex.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
-    double max_h = 0.0, min_a = INFINITY;
-    for (int b = 0; b < kVecBlocks; ++b) {
-        max_h = std::max(max_h, ex[b * 2]);
-        min_a = std::min(min_a, ex[b * 2 + 1]);
-    }
+    wait_box(ctx);
+    const double min_a = ctx->h_box[0], max_h = std::max(0.0, ctx->h_box[1]);
     if (!is_md(ctx)) a_min = std::min(a_min, 0.99 * min_a);
     *alph = 0.0;
     if (inner <= 0) return 1;
@@ -1298,20 +1269,14 @@ struct BdfState {
             HIP_OK(hipMemcpyAsync(ctx->d_conc.p, src, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
         ghost_copy(ctx, ctx->d_conc.p, nt);
     }
-    double min_blocks(const double* part, int nb, double init) {
-        std::vector<double> h_(nb);
-        HIP_OK(hipMemcpyAsync(h_.data(), part, nb * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_OK(hipStreamSynchronize(ctx->stream));
-        double r = init;
-        for (double v : h_) r = v < r ? v : r;
-        return r;
-    }
     double bound(const double* base, const double* dir, double scale, double init) {
-        ctx->d_part.reserve((size_t)kVecBlocks * 8 + 16);
-        hipLaunchKernelGGL(k_bdf_bound, dim3(kVecBlocks), dim3(kBlock), 0, ctx->stream, n, base, dir, scale,
-                           ctx->d_part.p);
+        const int nb = vec_blocks(n);
+        ctx->d_part.reserve((size_t)nb * 8 + 16);
+        hipLaunchKernelGGL(k_bdf_bound, dim3(nb), dim3(kBlock), 0, ctx->stream, n, base, dir, scale, ctx->d_part.p);
+        hipLaunchKernelGGL(k_fold_minmax, dim3(1), dim3(kBlock), 0, ctx->stream, ctx->d_part.p, nb, ctx->h_box);
         launch_check("k_bdf_bound");
-        return min_blocks(ctx->d_part.p, kVecBlocks, init);
+        wait_box(ctx);
+        return ctx->h_box[0] < init ? ctx->h_box[0] : init;
     }
     double dot(const double* u, const double* v) { return dot1(ctx, n, u, v); }
 
@@ -1350,14 +1315,12 @@ struct BdfState {
             C.ay[j] = alpha_y[j];
             Y.y[j] = y[j];
         }
-        HIP_OK(hipMemsetAsync(ctx->d_iflag.p, 0, sizeof(int), ctx->stream));
-        hipLaunchKernelGGL(k_bdf_interp, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, n, q, C, Y, dy, a, y0,
-                           ctx->d_iflag.p);
+        int* const box = reinterpret_cast<int*>(ctx->h_box);
+        *box = 0;
+        hipLaunchKernelGGL(k_bdf_interp, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, n, q, C, Y, dy, a, y0, box);
         launch_check("k_bdf_interp");
-        int flag = 0;
-        HIP_OK(hipMemcpyAsync(&flag, ctx->d_iflag.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_OK(hipStreamSynchronize(ctx->stream));
-        return flag ? -1 : 1;
+        wait_box(ctx);
+        return *box ? -1 : 1;
     }
 
     // Clock_BDF::solve (src/clock_bdf.cpp:677-883), curr_t = t[0] + del_t; -1 if c left [0,1]
@@ -1418,20 +1381,17 @@ struct BdfState {
             if (i != 0) a_1 *= (curr_t - t[i]) / (t[0] - t[i]);
         }
         const double err_pre_fac = -1.0 / (l1_q * (1.0 + a_1));
-        ctx->d_part.reserve((size_t)kVecBlocks * 8 + 16);
-        hipLaunchKernelGGL(k_bdf_err, dim3(kVecBlocks), dim3(kBlock), 0, st, n, y0, c, ctx->d_cd.p, ctx->d_part.p);
+        const int nb = vec_blocks(n);
+        ctx->d_part.reserve((size_t)nb * 8 + 16);
+        hipLaunchKernelGGL(k_bdf_err, dim3(nb), dim3(kBlock), 0, st, n, y0, c, ctx->d_cd.p, ctx->d_part.p);
         launch_check("k_bdf_err");
-        reduce_partials(ctx, ctx->d_part.p, kVecBlocks, 2, 2, 0, ctx->d_out.p);
-        double e2[2];
-        HIP_OK(hipMemcpyAsync(e2, ctx->d_out.p, sizeof(e2), hipMemcpyDeviceToHost, st));
-        hipLaunchKernelGGL(k_minmax, dim3(kVecBlocks), dim3(kBlock), 0, st, n, c, ctx->d_part.p);
+        reduce_partials(ctx, ctx->d_part.p, nb, 2, ctx->h_box);
+        hipLaunchKernelGGL(k_minmax, dim3(nb), dim3(kBlock), 0, st, n, c, ctx->d_part.p);
+        hipLaunchKernelGGL(k_fold_minmax, dim3(1), dim3(kBlock), 0, st, ctx->d_part.p, nb, ctx->h_box + 8);
         launch_check("k_minmax");
-        std::vector<double> mm((size_t)kVecBlocks * 2);
-        HIP_OK(hipMemcpyAsync(mm.data(), ctx->d_part.p, mm.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipStreamSynchronize(st));
-        *err = std::sqrt(e2[0] / ((double)n * a_tol)) * std::fabs(err_pre_fac);
-        for (int b = 0; b < kVecBlocks; ++b)
-            if (mm[b * 2] < 0.0 || mm[b * 2 + 1] > 1.0) return -1.0;
+        wait_box(ctx);
+        *err = std::sqrt(ctx->h_box[0] / ((double)n * a_tol)) * std::fabs(err_pre_fac);
+        if (ctx->h_box[8] < 0.0 || ctx->h_box[9] > 1.0) return -1.0;
         return curr_cost / (m_tol * (double)n);
     }
 
@@ -1480,16 +1440,15 @@ struct BdfState {
             H.la_y = -c0_ * c1 * lo_pre;
             H.c1c0 = c1 / c0_;
         }
-        ctx->d_part.reserve((size_t)kVecBlocks * 8 + 16);
-        hipLaunchKernelGGL(k_bdf_hilo, dim3(kVecBlocks), dim3(kBlock), 0, ctx->stream, n, H, Y, ctx->d_conc.p,
-                           ctx->d_cd.p, y0, e_n, ctx->d_part.p);
+        const int nb = vec_blocks(n);
+        ctx->d_part.reserve((size_t)nb * 8 + 16);
+        hipLaunchKernelGGL(k_bdf_hilo, dim3(nb), dim3(kBlock), 0, ctx->stream, n, H, Y, ctx->d_conc.p, ctx->d_cd.p, y0,
+                           e_n, ctx->d_part.p);
         launch_check("k_bdf_hilo");
-        reduce_partials(ctx, ctx->d_part.p, kVecBlocks, 2, 2, 0, ctx->d_out.p);
-        double r[2];
-        HIP_OK(hipMemcpyAsync(r, ctx->d_out.p, sizeof(r), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_OK(hipStreamSynchronize(ctx->stream));
-        *lo_err = std::sqrt(r[0] / ((double)n * a_tol));
-        *hi_err = std::sqrt(r[1] / ((double)n * a_tol));
+        reduce_partials(ctx, ctx->d_part.p, nb, 2, ctx->h_box);
+        wait_box(ctx);
+        *lo_err = std::sqrt(ctx->h_box[0] / ((double)n * a_tol));
+        *hi_err = std::sqrt(ctx->h_box[1] / ((double)n * a_tol));
     }
 };
 
@@ -1605,7 +1564,7 @@ void init_batch(mapp_dmd* ctx, double skin) {
 }
 // ---------------------------------------------------------- no-alloc calc_g
 // Scratch of mapp_dmd_calc_g_noalloc: calc_g's per-block partials of the cost
-// sweep over the 2nd list, the two-stage reduction's stage and its output, for
+// sweep over the 2nd list and the two-stage reduction's stage, for
 // systems of up to kNoAllocMaxSites owned sites (about 2.1 MB; each GPU the
 // library runs on holds its own copy until the process ends).  Every call on a
 // GPU shares that GPU's array: calls that overlap on one GPU race.  Each call
@@ -1844,6 +1803,7 @@ int mapp_dmd_create(mapp_dmd_t** out, int no_types, int variant, int device) {
         scratch_setup(device);
         HIP_OK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
         for (auto& e : ctx->ev) HIP_OK(hipEventCreate(&e));
+        HIP_OK(hipHostMalloc((void**)&ctx->h_box, 64 * sizeof(double), hipHostMallocDefault));
         ctx->d_iflag.reserve(4);
         return 0;
     });
@@ -2675,7 +2635,7 @@ int mapp_dmd_calc_g_noalloc(mapp_dmd_t* ctx, int chk, double alpha, const double
             throw ApiError(MAPP_DMD_E_HIP, std::string("no device address of the scratch array on this device: ") +
                                                hipGetErrorString(g_scratch_err[ctx->device]));
         const long nb2 = calc_g_blocks(ctx);
-        const GScratch S{base, base + nb2, base + nb2 + reduce_stage_doubles(nb2)};
+        const GScratch S{base, base + nb2};
         *cost = with_nt(ctx->nt,
                         [&](auto c) { return calc_g_variant<decltype(c)::value>(ctx, chk, alpha, a_dev, g_dev, &S); });
         return 0;

@@ -58,7 +58,6 @@ struct mapp_dmd {
     mappdmd::DevBuf<int2> d_info;      // [natms] {list offset, pairs inside the cut at the last force pass 1}
     mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}
     long nrev = 0;
-    std::vector<mappdmd::DevBuf<int>*> scan_levels;
     long npairs = 0, npairs2 = 0;
     bool have_list2 = false;
     // per-atom vectors ([ntot][nt] unless noted) and pair buffers
@@ -77,9 +76,10 @@ struct mapp_dmd {
     long ntable = 0;
     mappdmd::DevBuf<int> d_foff2, d_fidx2;      // 2nd list of both ends (~owner for the partner end)
     bool cache_valid = false;
-    mappdmd::DevBuf<double> d_part, d_out, d_xaos, d_stage;
+    mappdmd::DevBuf<double> d_part, d_xaos, d_stage;
+    double* h_box = nullptr;  // pinned host memory for the scalars a call's last kernel writes (64 doubles)
     mappdmd::DevBuf<int> d_iflag;
-    mappdmd::DevBuf<unsigned long long> d_total;  // 64-bit count total of counts_to_offsets
+    mappdmd::DevBuf<unsigned long long> d_scan;  // tile sums of exclusive_scan
     long n_inrange = 0;
 
     // learned surrogate

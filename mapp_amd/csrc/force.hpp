@@ -170,27 +170,6 @@ __device__ __forceinline__ void embed_F(const FFParams<double>& P, const double*
     if (ddF) *ddF = (3.0 * c[8] * p2 + c[7] * p + c[6]) * P.drho_inv;
 }
 
-// deterministic block sum of NV doubles (fixed tree), thread 0 writes out[blockIdx.x*NV + k]
-template <int NV>
-__device__ __forceinline__ void block_sum_store(double* v, double* __restrict__ out) {
-    __shared__ double sh[NV][kBlock];
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) sh[k][tid] = v[k];
-    __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (tid < s) {
-#pragma unroll
-            for (int k = 0; k < NV; ++k) sh[k][tid] += sh[k][tid + s];
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-#pragma unroll
-        for (int k = 0; k < NV; ++k) out[(size_t)blockIdx.x * NV + k] = sh[k][0];
-    }
-}
-
 // XCD-aware block order: consecutive atoms (spatial neighbours) land on the
 // same XCD, whose L2 then holds their shared neighbour rows.  Dispatch places
 // block b on XCD b % 8.
@@ -408,6 +387,26 @@ __device__ __forceinline__ void block_store_waves(const double* v, double* __res
             for (int q = 0; q < nw; ++q) s += sh[q][k];
             out[(size_t)blockIdx.x * NV + k] = s;
         }
+    }
+}
+
+// deterministic sum of NV doubles over a block of kBlock threads: a fixed tree in each
+// wavefront, then the wavefronts in order; thread k writes out[blockIdx.x*NV + k]
+template <int NV>
+__device__ __forceinline__ void block_sum_store(const double* v, double* __restrict__ out) {
+    __shared__ double sh[kBlock / 64][NV];
+    const int w = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const double t = wave_sum(v[k]);
+        if ((threadIdx.x & 63) == 0) sh[w][k] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < kBlock / 64; ++q) t += sh[q][threadIdx.x];
+        out[(size_t)blockIdx.x * NV + threadIdx.x] = t;
     }
 }
 
@@ -1296,58 +1295,39 @@ __global__ __launch_bounds__(kBlock) void k_fgather(int natms, const double4* __
     }
 }
 
-// Two-stage deterministic sum of per-block partials: stage 1 block b sums the
-// contiguous range [b*chunk, (b+1)*chunk) of partials in a fixed tree; stage 2
-// (one block) sums the stage-1 results the same way.
-__global__ __launch_bounds__(kBlock) void k_reduce_stage(const double* __restrict__ part, long nparts, int nv,
-                                                         int stride, int offset, long chunk,
-                                                         double* __restrict__ out, int out_stride) {
-    __shared__ double sh[kBlock];
-    const long lo = (long)blockIdx.x * chunk;
-    long hi = lo + chunk;
-    hi = hi < nparts ? hi : nparts;
-    for (int k = 0; k < nv; ++k) {
-        double s = 0.0;
-        for (long b = lo + threadIdx.x; b < hi; b += kBlock) s += part[(size_t)b * stride + offset + k];
-        sh[threadIdx.x] = s;
-        __syncthreads();
-        for (int w = kBlock / 2; w > 0; w >>= 1) {
-            if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) out[(size_t)blockIdx.x * out_stride + k] = sh[0];
-        __syncthreads();
-    }
-}
-
-// The same two-stage sums for up to kMaxSegs arrays of partials (at most 8
-// values each) in one pair of launches: segment s takes stage-1 blocks
-// [first[s], first[s] + nb[s]) and stage-2 block s; each sum keeps the fixed
-// shape of k_reduce_stage.
+// Two-stage deterministic sums of up to kMaxSegs arrays of partials (at most 8
+// values each) in one pair of launches.  Stage 1: segment s takes the blocks
+// [first[s], first[s] + nb[s]), each of which sums a contiguous range of kReduceChunk
+// partials; stage 2: block s sums the segment's stage-1 results.  Both in fixed trees.
+// A chunk is two partials per thread: with 4,096 (sixteen loads in a row) stage 1 took
+// 16 us on the 8,000 partials of a 4,000-site system, with a barrier per tree level and
+// value; at 1,048,576 sites (1.8 million partials) 25 us.
 constexpr int kMaxSegs = 4;
+constexpr long kReduceChunk = 2 * kBlock;
 struct ReduceSegs {
     const double* part[kMaxSegs];
     long nparts[kMaxSegs];
     int nv[kMaxSegs], stride[kMaxSegs], out_off[kMaxSegs], first[kMaxSegs], nb[kMaxSegs];
     int nseg;
 };
-__device__ __forceinline__ double block_tree_sum(double s, double* sh) {
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
+// sums of 8 values over the block, in thread 0..7 (fixed tree)
+__device__ __forceinline__ double block_sum8(const double* s, int nv) {
+    __shared__ double sh[kBlock / 64][8];
+    for (int k = 0; k < nv; ++k) {
+        const double t = wave_sum(s[k]);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][k] = t;
     }
-    const double r = sh[0];
     __syncthreads();
-    return r;
+    double t = 0.0;
+    if ((int)threadIdx.x < nv)
+        for (int q = 0; q < kBlock / 64; ++q) t += sh[q][threadIdx.x];
+    return t;
 }
-__global__ __launch_bounds__(kBlock) void k_reduce_segs1(ReduceSegs R, long chunk, double* __restrict__ stage) {
-    __shared__ double sh[kBlock];
+__global__ __launch_bounds__(kBlock) void k_reduce_segs1(ReduceSegs R, double* __restrict__ stage) {
     int sg = 0;
     while (sg + 1 < R.nseg && (int)blockIdx.x >= R.first[sg + 1]) ++sg;
-    const long lo = (long)(blockIdx.x - R.first[sg]) * chunk;
-    long hi = lo + chunk;
+    const long lo = (long)(blockIdx.x - R.first[sg]) * kReduceChunk;
+    long hi = lo + kReduceChunk;
     hi = hi < R.nparts[sg] ? hi : R.nparts[sg];
     const double* part = R.part[sg];
     const int nv = R.nv[sg], stride = R.stride[sg];
@@ -1359,20 +1339,45 @@ __global__ __launch_bounds__(kBlock) void k_reduce_segs1(ReduceSegs R, long chun
         for (int k = 0; k < 8; ++k)
             if (k < nv) s[k] += pb[k];
     }
-    for (int k = 0; k < nv; ++k) {
-        const double t = block_tree_sum(s[k], sh);
-        if (threadIdx.x == 0) stage[(size_t)blockIdx.x * 8 + k] = t;
-    }
+    const double t = block_sum8(s, nv);
+    if ((int)threadIdx.x < nv) stage[(size_t)blockIdx.x * 8 + threadIdx.x] = t;
 }
 __global__ __launch_bounds__(kBlock) void k_reduce_segs2(ReduceSegs R, const double* __restrict__ stage,
                                                          double* __restrict__ out) {
-    __shared__ double sh[kBlock];
-    const int sg = blockIdx.x;
-    for (int k = 0; k < R.nv[sg]; ++k) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < R.nb[sg]; b += kBlock) s += stage[(size_t)(R.first[sg] + b) * 8 + k];
-        s = block_tree_sum(s, sh);
-        if (threadIdx.x == 0) out[R.out_off[sg] + k] = s;
+    const int sg = blockIdx.x, nv = R.nv[sg];
+    double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < R.nb[sg]; b += kBlock) {
+        const double* pb = stage + (size_t)(R.first[sg] + b) * 8;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (k < nv) s[k] += pb[k];
+    }
+    const double t = block_sum8(s, nv);
+    if ((int)threadIdx.x < nv) out[R.out_off[sg] + threadIdx.x] = t;
+}
+
+// smallest and largest of n pairs {smallest, largest} (one block)
+__global__ __launch_bounds__(kBlock) void k_fold_minmax(const double* __restrict__ part, int n,
+                                                        double* __restrict__ out) {
+    __shared__ double mn[kBlock], mx[kBlock];
+    double lo = INFINITY, hi = -INFINITY;
+    for (int b = threadIdx.x; b < n; b += kBlock) {
+        lo = fmin(lo, part[2 * b]);
+        hi = fmax(hi, part[2 * b + 1]);
+    }
+    mn[threadIdx.x] = lo;
+    mx[threadIdx.x] = hi;
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            mn[threadIdx.x] = fmin(mn[threadIdx.x], mn[threadIdx.x + w]);
+            mx[threadIdx.x] = fmax(mx[threadIdx.x], mx[threadIdx.x + w]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        out[0] = mn[0];
+        out[1] = mx[0];
     }
 }
 

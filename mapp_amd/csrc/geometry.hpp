@@ -24,57 +24,91 @@ __device__ __forceinline__ double comp3c(const double4& p, int d) {
     return d == 0 ? p.x : (d == 1 ? p.y : p.z);
 }
 
-// ---- total of n non-negative int counts in 64 bits (the int scan below wraps
-// past 2^31; integer sums do not depend on the order of the additions) ----
-constexpr int kCountThreads = 256;
-__global__ __launch_bounds__(kCountThreads) void k_count_total(const int* __restrict__ in, long n,
-                                                        unsigned long long* __restrict__ total) {
-    unsigned long long s = 0;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        s += (unsigned)in[i];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
-    if ((threadIdx.x & 63) == 0) atomicAdd(total, s);
-}
-
-// ---- exclusive scan over int (tile scan + recursive scan of tile sums) ----
+// ---- exclusive scan over non-negative ints: tiles, the tile sums in one block,
+// the sums added.  The total is kept in 64 bits (offsets are int: a total of 2^31 or
+// more is refused by the caller) and written to host memory with the last launch. ----
 __global__ __launch_bounds__(kScanThreads) void k_scan_tile(const int* __restrict__ in, int* __restrict__ out,
-                                                            int* __restrict__ sums, long n) {
-    __shared__ int sh[kScanThreads];
-    const int tid = threadIdx.x;
+                                                            unsigned long long* __restrict__ sums, long n) {
+    __shared__ unsigned long long sh[kScanThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const long base = (long)blockIdx.x * kScanTile + (long)tid * kScanItems;
     int v[kScanItems];
-    int tsum = 0;
+    unsigned long long tsum = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         long idx = base + k;
         v[k] = idx < n ? in[idx] : 0;
-        tsum += v[k];
+        tsum += (unsigned)v[k];
     }
-    sh[tid] = tsum;
+    unsigned long long incl = tsum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned long long t = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += t;
+    }
+    if (lane == 63) sh[w] = incl;
     __syncthreads();
-    for (int off = 1; off < kScanThreads; off <<= 1) {
-        int t = tid >= off ? sh[tid - off] : 0;
-        __syncthreads();
-        sh[tid] += t;
-        __syncthreads();
+    unsigned long long before = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < kScanThreads / 64; ++q) {
+        if (q < w) before += sh[q];
+        all += sh[q];
     }
-    int excl = sh[tid] - tsum;
+    int excl = (int)(before + incl - tsum);
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         long idx = base + k;
         if (idx < n) out[idx] = excl;
         excl += v[k];
     }
-    if (tid == kScanThreads - 1) sums[blockIdx.x] = sh[tid];
+    if (tid == 0) sums[blockIdx.x] = all;
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ out, const int* __restrict__ add, long n) {
+constexpr int kScanSumThreads = 1024;
+// exclusive scan of the nb tile sums in place by one block; the total to *total
+__global__ __launch_bounds__(kScanSumThreads) void k_scan_sums(unsigned long long* __restrict__ sums, int nb,
+                                                               unsigned long long* __restrict__ total) {
+    __shared__ unsigned long long sh[kScanSumThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    unsigned long long carry = 0;
+    for (int base = 0; base < nb; base += kScanSumThreads) {
+        const unsigned long long v = base + tid < nb ? sums[base + tid] : 0;
+        unsigned long long incl = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned long long t = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += t;
+        }
+        if (lane == 63) sh[w] = incl;
+        __syncthreads();
+        unsigned long long before = 0, all = 0;
+#pragma unroll
+        for (int q = 0; q < kScanSumThreads / 64; ++q) {
+            if (q < w) before += sh[q];
+            all += sh[q];
+        }
+        if (base + tid < nb) sums[base + tid] = carry + before + incl - v;
+        carry += all;
+        __syncthreads();
+    }
+    if (tid == 0) *total = carry;
+}
+
+// adds the tile sums; with the last tile, *end (optional) = the total
+__global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ out,
+                                                           const unsigned long long* __restrict__ add, long n,
+                                                           const unsigned long long* __restrict__ total,
+                                                           int* __restrict__ end, unsigned long long* host_total) {
     const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
-    const int a = add[blockIdx.x];
+    const int a = (int)add[blockIdx.x];
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         long idx = base + k;
         if (idx < n) out[idx] += a;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (end) *end = (int)*total;
+        *host_total = *total;
     }
 }
 
@@ -387,7 +421,9 @@ __global__ void k_skin_check(const double4* __restrict__ pos, const double4* __r
     sq += d0 * d0;
     sq += d1 * d1;
     sq += d2 * d2;
-    if (sq > sq_skin) atomicOr(flag, 1);
+    // flag lies in host memory and starts at zero; one store per wavefront with a moved site
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(sq > sq_skin);
+    if (m && (int)(threadIdx.x & 63) == __ffsll((long long)m) - 1) *flag = 1;
 }
 
 }  // namespace mappdmd

@@ -50,7 +50,7 @@ __global__ void k_sy(long n, double a, const double* __restrict__ h, const doubl
     }
 }
 
-// per-block max |h| and min alpha (alpha columns 3..xd-1 of the owned rows of x)
+// per-block {min alpha, max |h|} (alpha columns 3..xd-1 of the owned rows of x)
 __global__ __launch_bounds__(kBlock) void k_extrema(long n, int xd, const double* __restrict__ h,
                                                     const double* __restrict__ x, double* __restrict__ part) {
     __shared__ double smax[kBlock], smin[kBlock];
@@ -71,8 +71,8 @@ __global__ __launch_bounds__(kBlock) void k_extrema(long n, int xd, const double
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        part[blockIdx.x * 2] = smax[0];
-        part[blockIdx.x * 2 + 1] = smin[0];
+        part[blockIdx.x * 2] = smin[0];
+        part[blockIdx.x * 2 + 1] = smax[0];
     }
 }
 
