@@ -883,29 +883,28 @@ void sync_sizes(mapp_dmd* ctx) {
 
 void ensure_pair_cache(mapp_dmd* ctx);
 
+// the site table's values, both ends (k_table_values)
 template <int NT, typename Q, int NQ>
-void run_pair_values(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
-    const size_t np = (size_t)ctx->npairs + 1;
-    ctx->d_rhoc.reserve(np * NT * NT);
-    ctx->d_phic.reserve(np * NT * (NT + 1) / 2);
-    hipLaunchKernelGGL((k_pair_values<NT, Q, NQ>), dim3(nblk(ctx->npairs)), dim3(kBlock), 0, ctx->stream, ctx->P, PQ,
-                       ctx->d_pos.p, ctx->d_alpha.p, ctx->d_nl.p, ctx->d_pair_i.p, (long)ctx->npairs, quad,
-                       ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_rhoc.p, ctx->d_phic.p);
-    launch_check("k_pair_values");
+void run_table_values(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
+    hipLaunchKernelGGL((k_table_values<NT, Q, NQ>), dim3(nblk((long)ctx->natms * 64)), dim3(kBlock),
+                       (kBlock / 64) * TableStage<NT>::kBytes, ctx->stream, ctx->P, PQ, ctx->d_pos.p, ctx->d_alpha.p,
+                       ctx->d_off.p, ctx->d_nl.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_toff.p, ctx->d_town.p,
+                       ctx->d_trank.p, ctx->d_tidx.p, ctx->d_trho.p, ctx->d_tphi.p);
+    launch_check("k_table_values");
 }
 
 template <int NT>
-void pair_values_dispatch(mapp_dmd* ctx) {
+void table_values_dispatch(mapp_dmd* ctx) {
     const int q = ctx->P.no_i;
     // the surrogate's c_d_calc / calc_g pair values come from its fallback, the FP32 quadrature
     if (ctx->prec == MAPP_DMD_PREC_MIXED || ctx->prec == MAPP_DMD_PREC_SURROGATE) {
-        if (q == 3) run_pair_values<NT, float, 3>(ctx, ctx->d_quad32.p, ctx->Pf);
-        else if (q == 5) run_pair_values<NT, float, 5>(ctx, ctx->d_quad32.p, ctx->Pf);
-        else run_pair_values<NT, float, 0>(ctx, ctx->d_quad32.p, ctx->Pf);
+        if (q == 3) run_table_values<NT, float, 3>(ctx, ctx->d_quad32.p, ctx->Pf);
+        else if (q == 5) run_table_values<NT, float, 5>(ctx, ctx->d_quad32.p, ctx->Pf);
+        else run_table_values<NT, float, 0>(ctx, ctx->d_quad32.p, ctx->Pf);
     } else {
-        if (q == 3) run_pair_values<NT, double, 3>(ctx, ctx->d_quad64.p, ctx->P);
-        else if (q == 5) run_pair_values<NT, double, 5>(ctx, ctx->d_quad64.p, ctx->P);
-        else run_pair_values<NT, double, 0>(ctx, ctx->d_quad64.p, ctx->P);
+        if (q == 3) run_table_values<NT, double, 3>(ctx, ctx->d_quad64.p, ctx->P);
+        else if (q == 5) run_table_values<NT, double, 5>(ctx, ctx->d_quad64.p, ctx->P);
+        else run_table_values<NT, double, 0>(ctx, ctx->d_quad64.p, ctx->P);
     }
 }
 
@@ -914,23 +913,24 @@ RevBufs rev_second(mapp_dmd* ctx) {
     return RevBufs{ctx->d_off2.p, ctx->d_nl2.p, ctx->d_roff2.p, ctx->d_rev2.p, ctx->d_pair_i2.p};
 }
 
-// site table of the pair values (both ends of every contributing pair)
+// site table of the pair values (both ends of every pair inside the quadrature cut)
 template <int NT>
 void build_site_table(mapp_dmd* ctx) {
     hipStream_t st = ctx->stream;
     const int natms = ctx->natms;
     const RevBufs L = rev_half(ctx);
+    const dim3 grid(nblk((long)natms * kTableG));
     ctx->d_cnt.reserve(natms + 1);
-    hipLaunchKernelGGL((k_table_count<NT>), dim3(nblk((long)natms * kTableG)), dim3(kBlock), 0, st, L, natms, ctx->d_rhoc.p,
-                       ctx->d_phic.p, ctx->d_cnt.p);
+    ctx->d_town.reserve(natms + 1);
+    ctx->d_trank.reserve(ctx->npairs + 1);
+    hipLaunchKernelGGL(k_table_count, grid, dim3(kBlock), 0, st, L, ctx->d_rowner.p, natms, ctx->d_pos.p,
+                       ctx->P.cut_sq_mod, ctx->d_town.p, ctx->d_cnt.p, ctx->d_trank.p);
     launch_check("k_table_count");
     const long ne = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_toff, natms);
     ctx->d_tidx.reserve(ne + 1);
     ctx->d_trho.reserve((size_t)(ne + 1) * NT * NT);
     ctx->d_tphi.reserve((size_t)(ne + 1) * NT * (NT + 1) / 2);
-    hipLaunchKernelGGL((k_table_fill<NT>), dim3(nblk((long)natms * kTableG)), dim3(kBlock), 0, st, L, natms, ctx->d_rhoc.p,
-                       ctx->d_phic.p, ctx->d_toff.p, ctx->d_tidx.p, ctx->d_trho.p, ctx->d_tphi.p);
-    launch_check("k_table_fill");
+    table_values_dispatch<NT>(ctx);
     ctx->ntable = ne;
 }
 
@@ -938,10 +938,7 @@ SiteTable site_table(mapp_dmd* ctx) { return SiteTable{ctx->d_toff.p, ctx->d_tid
 
 void ensure_pair_cache(mapp_dmd* ctx) {
     if (ctx->cache_valid) return;
-    with_nt(ctx->nt, [&](auto c) {
-        pair_values_dispatch<decltype(c)::value>(ctx);
-        build_site_table<decltype(c)::value>(ctx);
-    });
+    with_nt(ctx->nt, [&](auto c) { build_site_table<decltype(c)::value>(ctx); });
     ctx->cache_valid = true;
 }
 

@@ -70,8 +70,8 @@ struct mapp_dmd {
     // pair's owner; the top bit of the first: inside the quadrature cut at the last pass 1
     mappdmd::DevBuf<int2> d_nlrp;
     mappdmd::DevBuf<int> d_rowner;
-    mappdmd::DevBuf<double> d_rhoc, d_phic;     // pair values for c_d_calc / calc_g, per half-list pair
-    mappdmd::DevBuf<int> d_toff, d_tidx;        // site table: both ends of every contributing pair
+    mappdmd::DevBuf<int> d_toff, d_tidx;        // site table: both ends of every pair inside the quadrature cut
+    mappdmd::DevBuf<int> d_town, d_trank;       // own entries per site; a pair's rank in its partner's reverse entries
     mappdmd::DevBuf<double> d_trho, d_tphi;
     long ntable = 0;
     mappdmd::DevBuf<int> d_foff2, d_fidx2;      // 2nd list of both ends (~owner for the partner end)

@@ -55,71 +55,6 @@ __device__ __forceinline__ T horner3(const T* c, T p) {
     return fma(fma(fma(c[3], p, c[2]), p, c[1]), p, c[0]);
 }
 
-// Gauss-Hermite average of rho (odd extension u*rho(|u|)) and r*phi (odd
-// extension sgn(u) r*phi(|u|)) of one ordered type pair; src/ff_dmd_I.cpp:180-242.
-// g, f receive {value, d/dr, d/dalpha} (derivatives when DERIV).
-// Returns false when the whole rule lies beyond the cutoff (lower >= xi_max).
-template <typename Q, int NQ, bool DERIV, bool PHI>
-__device__ __forceinline__ bool gh_average(const FFParams<Q>& P, Q r, Q r_inv, Q alpha,
-                                           const Q* __restrict__ tab, int stride, Q* g, Q* f) {
-    const int nq = NQ > 0 ? NQ : P.no_i;
-    const Q asq = sqrt(alpha);
-    const Q inv = Q(1) / asq;
-    const Q upper = (r + P.rc) * asq;
-    const Q lower = (r - P.rc) * asq;
-    if (!(lower < P.xi[nq - 1])) return false;
-    Q g0 = 0, g1 = 0, g2 = 0, f0 = 0, f1 = 0, f2 = 0;
-#pragma unroll
-    for (int k = 0; k < (NQ > 0 ? NQ : kMaxPoints); ++k) {
-        if (NQ == 0 && k >= nq) break;
-        const Q xk = P.xi[k];
-        if (xk > lower && xk < upper) {
-            const Q t = fma(-xk, inv, r);
-            Q p = fabs(t) * P.dr_inv;
-            int m = (int)p;
-            m = m < P.nr - 2 ? m : P.nr - 2;
-            p -= (Q)m;
-            p = p < Q(1) ? p : Q(1);
-            const Q* row = tab + (size_t)m * stride;
-            const Q rv = horner3(row, p) * t;
-            g0 = fma(P.w0[k], rv, g0);
-            if (DERIV) {
-                g1 = fma(P.w1[k], rv, g1);
-                g2 = fma(P.w2[k], rv, g2);
-            }
-            if (PHI) {
-                Q pv = horner3(row + 4, p);
-                pv = t < Q(0) ? -pv : pv;
-                f0 = fma(P.w0[k], pv, f0);
-                if (DERIV) {
-                    f1 = fma(P.w1[k], pv, f1);
-                    f2 = fma(P.w2[k], pv, f2);
-                }
-            }
-        }
-    }
-    const Q sc = Q(kPiInSq) * r_inv;
-    g0 *= sc;
-    g[0] = g0;
-    if (DERIV) {
-        g1 *= sc;
-        g2 *= sc;
-        g[1] = -g0 * r_inv - Q(2) * asq * g1;
-        g[2] = (Q(0.5) * g0 - g2) / alpha;
-    }
-    if (PHI) {
-        f0 *= sc;
-        f[0] = f0;
-        if (DERIV) {
-            f1 *= sc;
-            f2 *= sc;
-            f[1] = -f0 * r_inv - Q(2) * asq * f1;
-            f[2] = (Q(0.5) * f0 - f2) / alpha;
-        }
-    }
-    return true;
-}
-
 // classical EAM values for alpha >= alpha_max (src/ff_dmd_I.cpp:261-310), FP64
 __device__ __forceinline__ void classical_pair(const FFParams<double>& P, double rsq, double r_inv,
                                                const double* __restrict__ rho7, const double* __restrict__ phi7,

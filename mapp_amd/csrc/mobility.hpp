@@ -9,13 +9,12 @@
 //
 // Pair values.  rho_bar (every ordered type pair) and phi_bar depend on
 // positions and widths only; the reference caches them in force_calc.  Here
-// k_pair_values evaluates them per half-list pair with the same quadrature as
-// force_calc, and k_table_fill turns them into the site table: for each
-// owned site, the entries of its own half-list row, then the entries of the
-// lower-index sites that list it (ascending owner), each holding the partner
-// index and the pair's nt^2 + nt(nt+1)/2 values in the owner's orientation.
-// Pairs whose values are all zero (outside the cut, or the width pair out of
-// range) add nothing to any sum and are left out.  Seen from site i with
+// k_table_values evaluates them with the same quadrature as force_calc into the
+// site table: for each owned site, the entries of its own half-list row inside
+// the quadrature cut, then the entries of the lower-index sites that list it
+// (ascending owner), each holding the partner index and the pair's
+// nt^2 + nt(nt+1)/2 values in the owner's orientation.  Pairs outside the cut add
+// nothing to any sum and are left out.  Seen from site i with
 // type m and a partner k of type b, each sweep's term is the same expression
 // whichever end owns the pair (slot(b, m) for the density, slot(m, b) for the
 // chemical potential and the last g sweep), so one loop covers both.
@@ -49,66 +48,6 @@ __global__ void k_pair_owner(const int* __restrict__ off, int natms, int* __rest
     for (int p = off[i]; p < off[i + 1]; ++p) pair_i[p] = i;
 }
 
-// rho_bar for every ordered type pair and phi_bar for it >= jt, per half-list
-// pair (one thread per pair, owner from pair_i); zeros where the reference
-// computes nothing (outside the cut, alpha out of range, or the rule beyond rc)
-template <int NT, typename Q, int NQ>
-__global__ __launch_bounds__(kBlock) void k_pair_values(FFParams<double> P, FFParams<Q> PQ,
-                                                        const double4* __restrict__ pos,
-                                                        const double* __restrict__ alpha, const int* __restrict__ nl,
-                                                        const int* __restrict__ pair_i, long npairs,
-                                                        const Q* __restrict__ quad, const double* __restrict__ rho7,
-                                                        const double* __restrict__ phi7, double* __restrict__ rhoc,
-                                                        double* __restrict__ phic) {
-    constexpr int NPHI = NT * (NT + 1) / 2;
-    const long p = (long)blockIdx.x * kBlock + threadIdx.x;
-    if (p >= npairs) return;
-    const int i = pair_i[p], j = nl[p];
-    const double4 xi = pos[i], xj = pos[j];
-    const double dx0 = xi.x - xj.x, dx1 = xi.y - xj.y, dx2 = xi.z - xj.z;
-    double rsq;
-    {
-#pragma clang fp contract(off)
-        rsq = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;  // as force_calc
-    }
-    double rv[NT * NT], pv[NPHI];
-#pragma unroll
-    for (int k = 0; k < NT * NT; ++k) rv[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < NPHI; ++k) pv[k] = 0.0;
-    if (rsq < P.cut_sq_mod) {
-        const double r = sqrt(rsq), r_inv = 1.0 / r;
-#pragma unroll
-        for (int it = 0; it < NT; ++it)
-#pragma unroll
-            for (int jt = 0; jt < NT; ++jt) {
-                const bool want_phi = it >= jt;
-                const double ai = alpha[(size_t)i * NT + it], aj = alpha[(size_t)j * NT + jt];
-                const double a = (ai * aj) / (ai + aj);
-                if (P.alpha_min < a && a < P.alpha_max) {
-                    Q g[3], f[3];
-                    const Q* tab = quad + (size_t)(it * NT + jt) * kQuadRow;
-                    bool hit = want_phi ? gh_average<Q, NQ, false, true>(PQ, (Q)r, (Q)r_inv, (Q)a, tab, quad_stride(NT), g, f)
-                                        : gh_average<Q, NQ, false, false>(PQ, (Q)r, (Q)r_inv, (Q)a, tab, quad_stride(NT), g, f);
-                    if (hit) {
-                        rv[type2rho(NT, it, jt)] = (double)g[0];
-                        if (want_phi) pv[type2phi(it, jt)] = (double)f[0];
-                    }
-                } else if (P.alpha_max <= a && rsq < P.cut_sq) {
-                    double g[3], f[3];
-                    classical_pair(P, rsq, r_inv, rho7 + (size_t)type2rho(NT, it, jt) * P.nr * 7,
-                                   phi7 + (size_t)type2phi(it, jt) * P.nr * 7, want_phi, g, f);
-                    rv[type2rho(NT, it, jt)] = g[0];
-                    if (want_phi) pv[type2phi(it, jt)] = f[0];
-                }
-            }
-    }
-#pragma unroll
-    for (int k = 0; k < NT * NT; ++k) rhoc[(size_t)p * NT * NT + k] = rv[k];
-#pragma unroll
-    for (int k = 0; k < NPHI; ++k) phic[(size_t)p * NPHI + k] = pv[k];
-}
-
 // ---------------------------------------------------------------- site table
 constexpr int kTableG = 16;  // lanes per site over the pair table
 constexpr int kList2G = 4;   // lanes per site over the 2nd list
@@ -120,31 +59,15 @@ struct SiteTable {
     const double* phi;  // [entry][nt(nt+1)/2] phi_bar
 };
 
-template <int NT>
-__device__ __forceinline__ bool pair_contributes(const double* __restrict__ rhoc, const double* __restrict__ phic,
-                                                 long p) {
-    constexpr int NPHI = NT * (NT + 1) / 2;
-    bool nz = false;
-#pragma unroll
-    for (int k = 0; k < NT * NT; ++k) nz |= rhoc[p * NT * NT + k] != 0.0;
-#pragma unroll
-    for (int k = 0; k < NPHI; ++k) nz |= phic[p * NPHI + k] != 0.0;
-    return nz;
-}
-
-// entries per site: contributing pairs of the own row and of the reverse CSR
-// (16 lanes per site, strided over both ranges)
-template <int NT>
-__global__ __launch_bounds__(kBlock) void k_table_count(RevBufs L, int natms, const double* __restrict__ rhoc,
-                                                        const double* __restrict__ phic, int* __restrict__ cnt) {
-    const SiteGroup<kTableG> g;
-    const int i = g.site;
-    if (i >= natms) return;
-    int c = 0;
-    for (int p = L.off[i] + g.l; p < L.off[i + 1]; p += kTableG) c += pair_contributes<NT>(rhoc, phic, p) ? 1 : 0;
-    for (int q = L.roff[i] + g.l; q < L.roff[i + 1]; q += kTableG) c += pair_contributes<NT>(rhoc, phic, L.rev[q]) ? 1 : 0;
-    const double s = group_sum<kTableG>((double)c);
-    if (g.l == 0) cnt[i] = (int)s;
+// |x_i - x_j|^2 as force_calc forms it (the same bits from either end)
+__device__ __forceinline__ double pair_rsq(double4 xi, double4 xj) {
+    const double dx0 = xi.x - xj.x, dx1 = xi.y - xj.y, dx2 = xi.z - xj.z;
+    double rsq;
+    {
+#pragma clang fp contract(off)
+        rsq = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;
+    }
+    return rsq;
 }
 
 // rank of this lane's flag among the set flags of lower lanes of its 16-lane group,
@@ -157,43 +80,181 @@ __device__ __forceinline__ int group_rank16(bool flag, int l, int* total) {
     return __popc(bits & ((1u << l) - 1u));
 }
 
-// the entries, in list order, own row first; 16 lanes per site, each stride of
-// 16 entries placed by ballot rank
-template <int NT>
-__global__ __launch_bounds__(kBlock) void k_table_fill(RevBufs L, int natms, const double* __restrict__ rhoc,
-                                                       const double* __restrict__ phic, const int* __restrict__ toff,
-                                                       int* __restrict__ tidx, double* __restrict__ trho,
-                                                       double* __restrict__ tphi) {
-    constexpr int NPHI = NT * (NT + 1) / 2;
+// Entries per site: the pairs inside the quadrature cut of the own row (own[i]) and of
+// the reverse list, and for each pair its rank among the partner's reverse entries
+// inside the cut (16 lanes per site, strided over both ranges).
+__global__ __launch_bounds__(kBlock) void k_table_count(RevBufs L, const int* __restrict__ rowner, int natms,
+                                                        const double4* __restrict__ pos, double cut_sq,
+                                                        int* __restrict__ own, int* __restrict__ cnt,
+                                                        int* __restrict__ rrank) {
     const SiteGroup<kTableG> g;
     const int i = g.site;
     if (i >= natms) return;
-    long e = toff[i];
-    auto put = [&](long dst, long p, int partner) {
-        tidx[dst] = partner;
-#pragma unroll
-        for (int k = 0; k < NT * NT; ++k) trho[dst * NT * NT + k] = rhoc[p * NT * NT + k];
-#pragma unroll
-        for (int k = 0; k < NPHI; ++k) tphi[dst * NPHI + k] = phic[p * NPHI + k];
-    };
-    const int o0 = L.off[i], o1 = L.off[i + 1];
-    for (int b = o0; b < o1; b += kTableG) {
-        const int p = b + g.l;
-        const bool in = p < o1 && pair_contributes<NT>(rhoc, phic, p);
-        int tot;
-        const int rk = group_rank16(in, g.l, &tot);
-        if (in) put(e + rk, p, L.nl[p]);
-        e += tot;
-    }
-    const int q0 = L.roff[i], q1 = L.roff[i + 1];
-    for (int b = q0; b < q1; b += kTableG) {
+    const double4 xi = pos[i];
+    int c = 0, r = 0;
+    for (int p = L.off[i] + g.l; p < L.off[i + 1]; p += kTableG) c += pair_rsq(xi, pos[L.nl[p]]) < cut_sq ? 1 : 0;
+    const int q1 = L.roff[i + 1];
+    for (int b = L.roff[i]; b < q1; b += kTableG) {
         const int q = b + g.l;
-        const int p = q < q1 ? L.rev[q] : 0;
-        const bool in = q < q1 && pair_contributes<NT>(rhoc, phic, p);
+        const bool in = q < q1 && pair_rsq(xi, pos[rowner[q < q1 ? q : b] & ~kInsideBit]) < cut_sq;
         int tot;
         const int rk = group_rank16(in, g.l, &tot);
-        if (in) put(e + rk, p, L.pair_i[p]);
-        e += tot;
+        if (in) rrank[L.rev[q]] = r + rk;
+        r += tot;
+    }
+    const double sc = group_sum<kTableG>((double)c);
+    if (g.l == 0) {
+        own[i] = (int)sc;
+        cnt[i] = (int)sc + r;
+    }
+}
+
+// The table: rho_bar of every ordered type pair and phi_bar for it >= jt of the pairs
+// inside the quadrature cut, written from the pair's owner to both ends' rows; zeros
+// where the reference computes nothing (alpha out of range, or the whole rule beyond
+// rc).  A site's row holds its own pairs in list order, then those of its reverse list
+// in that order (rrank, k_table_count).  One wavefront per site and two lanes per
+// (pair, type pair), the lanes and the arithmetic of pass 1 (k_pass1) without the
+// derivatives.  Bound by the stores: the partner's entries are 8-byte words of rows
+// that 50 other waves fill.  At 442,368 sites of two types 1.26 ms, with 0.18 for the
+// count; one thread per listed pair, values kept in list order, counted and copied to
+// both rows took 1.04 + 0.47 + 1.33 ms, and own rows here with the partner's rows
+// copied by a second kernel 0.84 + 0.12 + 0.61.
+template <int NT>
+struct TableStage {
+    static constexpr int kBytes = 64 * (16 + 8 * NT + 8);
+    double2* geo;  // {r^2, 1/r}
+    double* typ;   // 1/alpha of the partner per type
+    int2* idx;     // {partner, the pair's entry in the partner's row or -1 for a ghost}
+    __device__ __forceinline__ explicit TableStage(int wave) {
+        extern __shared__ __attribute__((aligned(32))) unsigned char table_lds[];
+        unsigned char* base = table_lds + (size_t)wave * kBytes;
+        geo = reinterpret_cast<double2*>(base);
+        typ = reinterpret_cast<double*>(geo + 64);
+        idx = reinterpret_cast<int2*>(typ + 64 * NT);
+    }
+};
+template <int NT, typename Q, int NQ>
+__global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFParams<Q> PQ,
+                                                         const double4* __restrict__ pos,
+                                                         const double* __restrict__ alpha,
+                                                         const int* __restrict__ off, const int* __restrict__ nl,
+                                                         const Q* __restrict__ quad, const double* __restrict__ rho7,
+                                                         const double* __restrict__ phi7,
+                                                         const int* __restrict__ toff, const int* __restrict__ own,
+                                                         const int* __restrict__ rrank, int* __restrict__ tidx,
+                                                         double* __restrict__ trho,
+                                                         double* __restrict__ tphi) {
+    using Q2 = typename Vec2<Q>::T;
+    using Map = Pass1Map<NT, 2>;
+    constexpr int NPHI = NT * (NT + 1) / 2;
+    constexpr int KP = NQ > 0 ? NQ : kMaxPoints;
+    const int lane = threadIdx.x & 63;
+    const Map map(lane);
+    const int k = map.k, prt = map.prt, it = map.it, jt = map.jt;
+    const bool rho_lane = prt == 0, keeps = map.on && (rho_lane || it >= jt);
+    const int tab_off = ((it * NT + jt) * kQuadRow + (rho_lane || it < jt ? 0 : 4)) * (int)sizeof(Q);
+    const __amdgpu_buffer_rsrc_t qrs = raw_rsrc(quad, P.nr * quad_stride(NT) * (int)sizeof(Q));
+    const OddFactor<Q> odd(rho_lane);
+    const TableStage<NT> st(threadIdx.x >> 6);
+    const SiteLoop<> sl(P.natms, kBlock / 64);
+    for (int i0 = sl.first; i0 < sl.end; i0 += sl.stride) {
+        const int i = __builtin_amdgcn_readfirstlane(i0);
+        const int p0 = off[i], p1 = off[i + 1];
+        const double4 xi = pos[i];
+        const double ai = alpha[(size_t)i * NT + it], iai = rcp_nr(ai);
+        double ia_min = rcp_nr(alpha[(size_t)i * NT]), ia_max = ia_min;
+#pragma unroll
+        for (int t = 1; t < NT; ++t) {
+            const double v = rcp_nr(alpha[(size_t)i * NT + t]);
+            ia_min = v < ia_min ? v : ia_min;
+            ia_max = v > ia_max ? v : ia_max;
+        }
+        size_t at = (size_t)toff[i];
+        for (int chunk = p0; chunk < p1; chunk += 64) {
+            int cnt;
+            bool regular = true;  // every pair width surely in the quadrature regime
+            {
+                const int pc = chunk + lane;
+                bool in = false;
+                int jc = 0;
+                double r2 = 1.0;
+                if (pc < p1) {
+                    jc = nl[pc];
+                    r2 = pair_rsq(xi, pos[jc]);
+                    in = r2 < P.cut_sq_mod;
+                }
+                const int dest = pack_dest(in, &cnt);
+                if (in) {
+                    double a[NT];
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) a[t] = alpha[(size_t)jc * NT + t];
+                    const int there = jc < P.natms ? toff[jc] + own[jc] + rrank[pc] : -1;
+                    tidx[at + dest] = jc;
+                    if (there >= 0) tidx[there] = i;
+                    st.geo[dest] = make_double2(r2, rsqrt_nr(r2));
+                    st.idx[dest] = make_int2(jc, there);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        const double iaj = rcp_nr(a[t]);
+                        regular = regular && iaj + ia_min > P.ia_quad_lo && iaj + ia_max < P.ia_quad_hi;
+                        st.typ[dest * NT + t] = iaj;
+                    }
+                }
+                regular = __builtin_amdgcn_ballot_w64(!regular) == 0;
+                __builtin_amdgcn_wave_barrier();
+            }
+            for (int base = 0; base < cnt; base += Map::kPPW) {
+                const int slot = base + k, s = slot < cnt ? slot : cnt - 1;
+                const double2 geo = st.geo[s];
+                const double r_inv = geo.y, r = geo.x * r_inv;
+                const double ia = iai + st.typ[s * NT + jt], asq = rsqrt_nr(ia);
+                const Q rq = (Q)r, inv = (Q)ia * (Q)asq;
+                const int nq = NQ > 0 ? NQ : PQ.no_i;
+                Q2 lo[KP], hi[KP];
+                Q ppv[KP];
+#pragma unroll
+                for (int kp = 0; kp < KP; ++kp) {
+                    if (NQ == 0 && kp >= nq) break;
+                    const Q u = rq - PQ.xi[kp] * inv;
+                    int m = (int)(fabs(u) * PQ.dr_inv);
+                    m = m < P.nr - 1 ? m : P.nr - 1;  // the zero row beyond the cutoff
+                    ppv[kp] = fabs(u) * PQ.dr_inv - (Q)m;
+                    const int row = tab_off + m * (quad_stride(NT) * (int)sizeof(Q));
+                    lo[kp] = RowLoad<Q2>::get(qrs, row);
+                    hi[kp] = RowLoad<Q2>::get(qrs, row + (int)sizeof(Q2));
+                }
+                if constexpr (KP * 2 * sizeof(Q2) <= 96) __builtin_amdgcn_sched_barrier(0);
+                Q x[KP], s0, s1, s2;
+#pragma unroll
+                for (int kp = 0; kp < KP; ++kp) {
+                    if (NQ == 0 && kp >= nq) break;
+                    const Q u = rq - PQ.xi[kp] * inv, pp = ppv[kp], p2 = pp * pp;
+                    x[kp] = ((lo[kp].x + lo[kp].y * pp) + p2 * (hi[kp].x + hi[kp].y * pp)) * odd(u);
+                }
+                gh_sums<Q, NQ, false>(PQ, nq, x, &s0, &s1, &s2);
+                double v = (double)(s0 * (Q(kPiInSq) * (Q)r_inv));
+                if (!regular && keeps) {
+                    const int br = alpha_branch(P, ia, ai, alpha[(size_t)st.idx[s].x * NT + jt]);
+                    if (br != 1) {
+                        double gv[3] = {0.0, 0.0, 0.0}, fv[3] = {0.0, 0.0, 0.0};
+                        if (br == 2 && geo.x < P.cut_sq)
+                            classical_pair(P, geo.x, r_inv, rho7 + (size_t)type2rho(NT, it, jt) * P.nr * 7,
+                                           phi7 + (size_t)type2phi(it, jt) * P.nr * 7, true, gv, fv);
+                        v = rho_lane ? gv[0] : fv[0];
+                    }
+                }
+                if (keeps && slot < cnt) {
+                    const int there = st.idx[s].y;
+                    double* const row = rho_lane ? trho + type2rho(NT, it, jt) : tphi + type2phi(it, jt);
+                    const int len = rho_lane ? NT * NT : NPHI;
+                    row[(at + slot) * len] = v;
+                    if (there >= 0) row[(size_t)there * len] = v;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            at += cnt;
+        }
     }
 }
 

@@ -2,7 +2,8 @@
 sums of 3 and 5 points, the general loop of the others), every lanes-per-pair
 schedule, one to four types, tables that do not vanish at the cutoff (the points
 beyond it read the tables' zero row instead of being tested), and sites with
-fewer pairs inside the cut than a round or a half wavefront, and with more.
+fewer pairs inside the cut than a round or a half wavefront, and with more; and
+the site table of the mobility sweeps, which has the same lanes and edges.
 Against the FP64 oracle: forces and densities to 1e-12 (a few hundred double
 roundings), 1e-5 with FP32 quadrature sums."""
 import numpy as np
@@ -21,6 +22,15 @@ def _check(ff, orc, bound):
         assert rel_inf(ff.get(name), orc.get(name)) <= bound, name
 
 
+def _check_rates(ff, orc, bound, names=("E", "dE", "n", "c_d")):
+    """the site table through the sweeps that read it; bound: a few hundred double roundings"""
+    for m in (ff, orc):
+        m.create_2nd_neigh_lst()
+        m.c_d_calc()
+    for name in names:
+        assert rel_inf(ff.get(name), orc.get(name)) <= bound, name
+
+
 @pytest.mark.parametrize("no_i", [1, 2, 3, 4, 5, 7])
 @pytest.mark.parametrize("nt,parts", [(1, 2), (2, 1), (2, 2), (2, 4), (3, 1), (3, 2), (4, 2)])
 def test_rules_and_schedules(nt, parts, no_i):
@@ -35,7 +45,10 @@ def test_rules_and_schedules(nt, parts, no_i):
     for precision, bound in (("fp64", 1e-12), ("mixed", 1e-5)):
         ff = setup(lat, tables, no_i=no_i, precision=precision)
         ff.set_schedule([parts, 4, 0, 2, 0])
-        _check(ff, O.make(lat, tables, no_i=no_i), bound)
+        orc = O.make(lat, tables, no_i=no_i)
+        _check(ff, orc, bound)
+        if parts == 2:
+            _check_rates(ff, orc, bound, ("E", "dE", "n", "c_d") if precision == "fp64" else ("E", "dE"))
         ff.close()
 
 
@@ -55,5 +68,7 @@ def test_few_and_many_pairs(tables, keep):
     box = W.Lattice(H=np.diag([L] * 3), x=np.ascontiguousarray(x), c=np.ascontiguousarray(lat.c[order]),
                     cart=x[:, :3] * L)
     ff = setup(box, tables, no_i=3)
-    _check(ff, O.make(box, tables, no_i=3), 1e-12)
+    orc = O.make(box, tables, no_i=3)
+    _check(ff, orc, 1e-12)
+    _check_rates(ff, orc, 1e-12)
     ff.close()
