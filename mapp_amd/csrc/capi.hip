@@ -88,53 +88,51 @@ void launch_check(const char* what) {
     if (e != hipSuccess) throw HipError(e, what, 0);
 }
 
-// ascending order inside every segment of v[0..n) (segments start[0..nseg]),
-// key[value] = the segment that holds the value; pos_of (optional) receives the
-// final position of every value
-void sort_segments(mapp_dmd* ctx, const int* start, const int* key, int* v, long n, int* pos_of = nullptr) {
-    if (n <= 0) return;
-    ctx->d_sort_tmp.reserve(n);
-    hipLaunchKernelGGL(k_rank_place, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, v, n, key, start,
-                       ctx->d_sort_tmp.p, pos_of);
-    launch_check("k_rank_place");
-    HIP_OK(hipMemcpyAsync(v, ctx->d_sort_tmp.p, sizeof(int) * n, hipMemcpyDeviceToDevice, ctx->stream));
-}
-
 // The context's mailbox: pinned host memory that the last kernel of a call writes its
 // scalars to, so that no copy follows it (a copy of a few bytes costs the stream about
 // as much as a small kernel).  Valid after the stream is synchronised.
 void wait_box(mapp_dmd* ctx) { HIP_OK(hipStreamSynchronize(ctx->stream)); }
 
-// exclusive scan of n ints; returns the total (synchronizes the stream); out[n] = the
-// total too when end is set (out then has n + 1 elements).  Refused when the total
-// does not fit an int.
-long exclusive_scan(mapp_dmd* ctx, const int* in, int* out, long n, bool end = false) {
+// exclusive scan of n ints; out[n] = the total too when end is set (out then has n + 1
+// elements).  Once the stream is synchronised, scan_total(slot) is the total and
+// scan_mid(slot) = out[mid] if mid >= 0.
+enum ScanSlot { kScanA = 0, kScanB = 1, kScanFree = 2 };  // kScanFree: the total is not read
+unsigned long long* scan_box(mapp_dmd* ctx, ScanSlot slot) {
+    return reinterpret_cast<unsigned long long*>(ctx->h_box) + 2 * slot;
+}
+void scan(mapp_dmd* ctx, ScanSlot slot, const int* in, int* out, long n, bool end, long mid = -1) {
+    unsigned long long* box = scan_box(ctx, slot);
     if (n <= 0) {
         if (end) HIP_OK(hipMemsetAsync(out, 0, sizeof(int), ctx->stream));
-        return 0;
+        box[0] = box[1] = 0;
+        return;
     }
     const int nb = (int)((n + kScanTile - 1) / kScanTile);
     ctx->d_scan.reserve((size_t)nb + 1);
     unsigned long long* sums = ctx->d_scan.p;
-    unsigned long long* box = reinterpret_cast<unsigned long long*>(ctx->h_box);
     hipLaunchKernelGGL(k_scan_tile, dim3(nb), dim3(kScanThreads), 0, ctx->stream, in, out, sums, n);
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanSumThreads), 0, ctx->stream, sums, nb, sums + nb);
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kScanThreads), 0, ctx->stream, out, sums, n, sums + nb,
-                       end ? out + n : (int*)nullptr, box);
+                       end ? out + n : (int*)nullptr, mid, box);
     launch_check("k_scan");
-    wait_box(ctx);
-    const unsigned long long total = *box;
+}
+// Refused when the total does not fit the int offsets.
+long scan_total(mapp_dmd* ctx, ScanSlot slot) {
+    const unsigned long long total = scan_box(ctx, slot)[0];
     if (total >= (1ull << 31))
         throw ApiError(MAPP_DMD_E_RANGE, "a list or table needs " + std::to_string(total) +
                                              " entries; its int offsets hold fewer than 2^31");
     return (long)total;
 }
+long scan_mid(mapp_dmd* ctx, ScanSlot slot) { return (long)scan_box(ctx, slot)[1]; }
 
 // CSR offsets (n+1) from counts (n); the offsets are int, so a total of 2^31
 // entries or more is refused before any caller sizes its entry array by it
 long counts_to_offsets(mapp_dmd* ctx, const int* cnt, DevBuf<int>& off, long n) {
     off.reserve(n + 1);
-    return exclusive_scan(ctx, cnt, off.p, n, true);
+    scan(ctx, kScanA, cnt, off.p, n, true);
+    wait_box(ctx);
+    return scan_total(ctx, kScanA);
 }
 
 // doubles of stage memory a reduction needs for nparts partials
@@ -213,48 +211,38 @@ void build_ghosts(mapp_dmd* ctx) {
     ctx->swap_off.assign(1, 0);
     ctx->swap_dim.clear();
     ctx->swap_dir.clear();
-    int lo_dim = 0, hi_dim = natms;
+    // One swap per face (init refuses a box that needs more), dimension by dimension over
+    // the sites and the ghosts so far.  The flags of both faces are counted by one scan,
+    // the low face first, which numbers the ghosts as one swap after the other does.
     for (int idim = 0; idim < 3; ++idim) {
-        const int comm_need = (int)(bp.cut_ph_s[idim] / (1.0 - 0.0)) + 1;
-        for (int dir = 0; dir < 2; ++dir) {
-            int lo = lo_dim, hi = hi_dim;
-            for (int k = 0; k < comm_need; ++k) {
-                const int tmp_r = natms + ctx->nghost;
-                const int n = hi - lo;
-                int cnt = 0;
-                if (n > 0) {
-                    ctx->d_flag.reserve(n);
-                    ctx->d_offs.reserve(n);
-                    double thr = dir == 0 ? bp.s_ph_lo[idim] : bp.s_ph_hi[idim];
-                    hipLaunchKernelGGL(k_ghost_flag, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p, lo,
-                                       hi, idim, dir, thr, ctx->d_flag.p);
-                    launch_check("k_ghost_flag");
-                    cnt = (int)exclusive_scan(ctx, ctx->d_flag.p, ctx->d_offs.p, n);
-                }
-                const int need = natms + ctx->nghost + cnt;
-                ctx->d_pos.reserve(need, true, ctx->stream);
-                ctx->d_alpha.reserve((size_t)need * NT, true, ctx->stream);
-                ctx->d_conc.reserve((size_t)need * NT, true, ctx->stream);
-                ctx->d_ghost_src.reserve(ctx->nghost + cnt + 1, true, ctx->stream);
-                ctx->d_ghost_owner.reserve(ctx->nghost + cnt + 1, true, ctx->stream);
-                if (cnt > 0)
-                    hipLaunchKernelGGL((k_ghost_emit<NT>), dim3(nblk(n)), dim3(kBlock), 0, ctx->stream,
-                                       ctx->d_pos.p, ctx->d_alpha.p, ctx->d_conc.p, lo, hi, idim, dir,
-                                       ctx->d_flag.p, ctx->d_offs.p, natms + ctx->nghost, natms,
-                                       ctx->d_ghost_src.p, ctx->d_ghost_owner.p);
-                launch_check("k_ghost_emit");
-                ctx->nghost += cnt;
-                ctx->swap_dim.push_back(idim);
-                ctx->swap_dir.push_back(dir);
-                ctx->swap_off.push_back(ctx->nghost);
-                hi = natms + ctx->nghost;
-                lo = tmp_r;
-            }
+        const int n = natms + ctx->nghost;
+        ctx->d_flag.reserve(2 * (size_t)n);
+        ctx->d_offs.reserve(2 * (size_t)n);
+        hipLaunchKernelGGL(k_ghost_flag, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p, n, idim,
+                           bp.s_ph_lo[idim], bp.s_ph_hi[idim], ctx->d_flag.p);
+        launch_check("k_ghost_flag");
+        scan(ctx, kScanA, ctx->d_flag.p, ctx->d_offs.p, 2 * (long)n, false, n);
+        wait_box(ctx);
+        const int cnt = (int)scan_total(ctx, kScanA), cnt_lo = (int)scan_mid(ctx, kScanA);
+        const int need = n + cnt;
+        ctx->d_pos.reserve(need, true, ctx->stream);
+        ctx->d_alpha.reserve((size_t)need * NT, true, ctx->stream);
+        ctx->d_conc.reserve((size_t)need * NT, true, ctx->stream);
+        ctx->d_ghost_src.reserve(ctx->nghost + cnt + 1, true, ctx->stream);
+        ctx->d_ghost_owner.reserve(ctx->nghost + cnt + 1, true, ctx->stream);
+        if (cnt > 0) {
+            hipLaunchKernelGGL((k_ghost_emit<NT>), dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p,
+                               ctx->d_alpha.p, ctx->d_conc.p, n, idim, ctx->d_flag.p, ctx->d_offs.p, natms,
+                               ctx->d_ghost_src.p, ctx->d_ghost_owner.p);
+            launch_check("k_ghost_emit");
         }
-        lo_dim = 0;
-        hi_dim = natms + ctx->nghost;
+        for (int dir = 0; dir < 2; ++dir) {
+            ctx->nghost += dir == 0 ? cnt_lo : cnt - cnt_lo;
+            ctx->swap_dim.push_back(idim);
+            ctx->swap_dir.push_back(dir);
+            ctx->swap_off.push_back(ctx->nghost);
+        }
     }
-    HIP_OK(hipStreamSynchronize(ctx->stream));
 }
 
 // columns of the per-site alpha / c arrays: nt for DMD, one (the type) for EAM
@@ -284,7 +272,7 @@ __global__ void k_quirk_cell(int n, int g, int own_base, int gh_dst, int nt, int
     }
 }
 
-// ghosts + bins + s->x + half list + reverse CSR; positions hold s on entry
+// ghosts + bins + s->x + half list + reverse list; positions hold s on entry
 template <int NT>
 void rebuild(mapp_dmd* ctx) {
     BoxParams& bp = ctx->bp;
@@ -294,75 +282,68 @@ void rebuild(mapp_dmd* ctx) {
     hipStream_t st = ctx->stream;
     // bins
     ctx->d_bin_of.reserve(ntot);
+    ctx->d_bin_slot.reserve(ntot);
     ctx->d_bin_cnt.reserve(bp.tot_bin + 1);
+    ctx->d_bin_start.reserve((size_t)bp.tot_bin + 1);
+    ctx->d_arrived.reserve(ntot);
     ctx->d_bin_atoms.reserve(ntot);
+    ctx->d_bin_pos.reserve(ntot);
     HIP_OK(hipMemsetAsync(ctx->d_bin_cnt.p, 0, sizeof(int) * (bp.tot_bin + 1), st));
     hipLaunchKernelGGL(k_s2bin, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_pos.p, ntot, bp, ctx->d_bin_of.p,
-                       ctx->d_bin_cnt.p);
+                       ctx->d_bin_cnt.p, ctx->d_bin_slot.p);
     launch_check("k_s2bin");
-    counts_to_offsets(ctx, ctx->d_bin_cnt.p, ctx->d_bin_start, bp.tot_bin);
-    HIP_OK(hipMemsetAsync(ctx->d_bin_cnt.p, 0, sizeof(int) * (bp.tot_bin + 1), st));
+    scan(ctx, kScanFree, ctx->d_bin_cnt.p, ctx->d_bin_start.p, bp.tot_bin, true);  // the total is ntot
     hipLaunchKernelGGL(k_bin_fill, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_bin_of.p, ntot,
-                       ctx->d_bin_start.p, ctx->d_bin_cnt.p, ctx->d_bin_atoms.p);
+                       ctx->d_bin_start.p, ctx->d_bin_slot.p, ctx->d_arrived.p);
     launch_check("k_bin_fill");
-    sort_segments(ctx, ctx->d_bin_start.p, ctx->d_bin_of.p, ctx->d_bin_atoms.p, ntot);
-    // Neighbor::bin_atoms_s ends with s2x of every atom
-    hipLaunchKernelGGL(k_s2x, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_pos.p, ntot, bp);
-    launch_check("k_s2x");
-    // half list
+    hipLaunchKernelGGL(k_bin_place, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_arrived.p, ntot, ctx->d_bin_of.p,
+                       ctx->d_bin_start.p, bp, ctx->d_conc.p, ctx->d_pos.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p);
+    launch_check("k_bin_place");
+    // half list and reverse list
     ctx->d_cnt.reserve(natms + 1);
-    hipLaunchKernelGGL((k_half_list<false>), dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, ctx->d_pos.p, natms,
-                       ctx->d_bin_of.p, ctx->d_bin_start.p, ctx->d_bin_atoms.p, bp, ctx->d_conc.p, ctx->d_cnt.p,
-                       (int*)nullptr);
+    ctx->d_rcnt.reserve(natms + 1);
+    ctx->d_off.reserve(natms + 1);
+    ctx->d_roff.reserve(natms + 1);
+    ctx->d_list_mask.reserve((size_t)natms * kMaskWords);
+    HalfLists L{ctx->d_list_mask.p, ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p, ctx->d_roff.p, nullptr, nullptr};
+    const dim3 grid(bp.tot_bin), blk(64 * kBinWaves);
+    hipLaunchKernelGGL((bp.pairwise ? k_half_list<false, true> : k_half_list<false, false>), grid, blk, 0, st, natms,
+                       ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
     launch_check("k_half_list count");
-    ctx->npairs = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_off, natms);
+    scan(ctx, kScanA, ctx->d_cnt.p, ctx->d_off.p, natms, true);
+    scan(ctx, kScanB, ctx->d_rcnt.p, ctx->d_roff.p, natms, true);
+    wait_box(ctx);
+    ctx->npairs = scan_total(ctx, kScanA);
+    ctx->nrev = scan_total(ctx, kScanB);
     ctx->d_nl.reserve(ctx->npairs + 1);
-    hipLaunchKernelGGL((k_half_list<true>), dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, ctx->d_pos.p, natms,
-                       ctx->d_bin_of.p, ctx->d_bin_start.p, ctx->d_bin_atoms.p, bp, ctx->d_conc.p, ctx->d_off.p,
-                       ctx->d_nl.p);
+    ctx->d_rowner.reserve(ctx->nrev + 1);
+    ctx->d_rtmp.reserve(ctx->nrev + 1);
+    L.nl = ctx->d_nl.p;
+    L.rlist = ctx->d_rtmp.p;
+    hipLaunchKernelGGL((bp.pairwise ? k_half_list<true, true> : k_half_list<true, false>), grid, blk, 0, st, natms,
+                       ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
     launch_check("k_half_list fill");
+    if (ctx->nrev > 0) {
+        hipLaunchKernelGGL(k_sort_owners, dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, natms, ctx->d_roff.p,
+                           ctx->d_rtmp.p, ctx->d_rowner.p);
+        launch_check("k_sort_owners");
+    }
     if (ctx->variant == MAPP_DMD_VARIANT_MEAM) finish_meam(ctx);
     else finish_lists<NT>(ctx);
 }
 
-// reverse CSR, pair owners, reverse positions and per-site / per-pair buffers
-// for the half list in d_off / d_nl
+// pair links and per-site / per-pair buffers for the half list in d_off / d_nl and the
+// reverse list in d_roff / d_rowner
 template <int NT>
 void finish_lists(mapp_dmd* ctx) {
     const int natms = ctx->natms;
     const int ntot = natms + ctx->nghost;
+    const long nrev = ctx->nrev;
     hipStream_t st = ctx->stream;
-    ctx->d_cnt.reserve(natms + 1);
-    // reverse CSR (partner j owned)
-    HIP_OK(hipMemsetAsync(ctx->d_cnt.p, 0, sizeof(int) * (natms + 1), st));
-    hipLaunchKernelGGL(k_rev_count, dim3(nblk((long)natms * kRevG)), dim3(kBlock), 0, st, ctx->d_off.p, ctx->d_nl.p, natms,
-                       ctx->d_cnt.p);
-    launch_check("k_rev_count");
-    long nrev = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_roff, natms);
-    ctx->d_rev.reserve(nrev + 1);
-    HIP_OK(hipMemsetAsync(ctx->d_cnt.p, 0, sizeof(int) * (natms + 1), st));
-    hipLaunchKernelGGL(k_rev_fill, dim3(nblk((long)natms * kRevG)), dim3(kBlock), 0, st, ctx->d_off.p, ctx->d_nl.p, natms,
-                       ctx->d_roff.p, ctx->d_cnt.p, ctx->d_rev.p);
-    launch_check("k_rev_fill");
-    // reverse positions of the pairs with an owned partner (rpos) come with the ordering
-    ctx->d_rpos.reserve(ctx->npairs + 1);
-    sort_segments(ctx, ctx->d_roff.p, ctx->d_nl.p, ctx->d_rev.p, nrev, ctx->d_rpos.p);
     ctx->d_nlrp.reserve(ctx->npairs + 1);
-    if (ctx->npairs > 0) {
-        hipLaunchKernelGGL(k_pack_nlrp, dim3(nblk(ctx->npairs)), dim3(kBlock), 0, st, ctx->d_nl.p, ctx->d_rpos.p,
-                           ctx->npairs, ctx->d_nlrp.p);
-        launch_check("k_pack_nlrp");
-    }
-    ctx->d_pair_i.reserve(ctx->npairs + 1);
-    hipLaunchKernelGGL(k_pair_owner, dim3(nblk(natms)), dim3(kBlock), 0, st, ctx->d_off.p, natms, ctx->d_pair_i.p);
-    launch_check("k_pair_owner");
-    if (!is_md(ctx) && nrev > 0) {
-        ctx->d_rowner.reserve(nrev);
-        hipLaunchKernelGGL(k_rev_owner, dim3(nblk(nrev)), dim3(kBlock), 0, st, ctx->d_rev.p, ctx->d_pair_i.p, nrev,
-                           ctx->d_rowner.p);
-        launch_check("k_rev_owner");
-    }
-    ctx->nrev = nrev;
+    hipLaunchKernelGGL(k_pair_links, dim3(nblk((long)natms * kLinkG)), dim3(kBlock), 0, st, ctx->d_off.p, ctx->d_nl.p,
+                       natms, ctx->d_roff.p, ctx->d_rowner.p, ctx->d_nlrp.p);
+    launch_check("k_pair_links");
     // element read by the reference's dE[jatm + jtype] quirk: jatm + jtype (one cell)
     ctx->d_qidx.reserve((size_t)ntot * NT);
     hipLaunchKernelGGL(k_quirk_identity, dim3(nblk((long)ntot * NT)), dim3(kBlock), 0, st, ntot, NT, ctx->d_qidx.p);
@@ -480,6 +461,8 @@ void gather_x_any(mapp_dmd* ctx, double* dst, int n, const double4* pos, const d
     launch_check("k_gather_x");
 }
 
+PairBufs pair_bufs(mapp_dmd* ctx) { return PairBufs{ctx->d_off.p, ctx->d_nlrp.p, ctx->d_roff.p}; }
+
 // ------------------------------------------------------------------ MD-mode potentials
 template <int MODEL>
 void md_passes(mapp_dmd* ctx, bool energy_only, int nb, const PairBufs& L, const EamBufs& T, double2* drho,
@@ -487,11 +470,11 @@ void md_passes(mapp_dmd* ctx, bool energy_only, int nb, const PairBufs& L, const
     hipStream_t st = ctx->stream;
     if (energy_only)
         hipLaunchKernelGGL((k_eam_pass1<MODEL, true>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md, ctx->d_pos.p,
-                           ctx->d_conc.p, L, ctx->d_rpos.p, ctx->d_Eown.p, ctx->d_fown.p, ctx->d_pairE.p,
+                           ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_fown.p, ctx->d_pairE.p,
                            ctx->d_pairF.p, drho, part1);
     else
         hipLaunchKernelGGL((k_eam_pass1<MODEL, false>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md,
-                           ctx->d_pos.p, ctx->d_conc.p, L, ctx->d_rpos.p, ctx->d_Eown.p, ctx->d_fown.p,
+                           ctx->d_pos.p, ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_fown.p,
                            ctx->d_pairE.p, ctx->d_pairF.p, drho, part1);
     launch_check("k_eam_pass1");
     if constexpr (MODEL != kModelLj) {
@@ -511,7 +494,7 @@ double run_eam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     if (ctx->variant == MAPP_DMD_VARIANT_MEAM) return run_meam(ctx, energy_only, st_clc, en_st);
     hipStream_t st = ctx->stream;
     const int natms = ctx->natms, nb = nblk((long)natms * kEamG);  // 16-lane site groups
-    PairBufs L{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p};
+    const PairBufs L = pair_bufs(ctx);
     EamBufs T{ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_F7.p, ctx->nt};
     ctx->d_part.reserve((size_t)nb * 14 + 16);
     ctx->d_drho.reserve(2 * ((size_t)ctx->npairs + 1));  // one double2 per pair
@@ -528,7 +511,7 @@ double run_eam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     if (!energy_only) {
         if (!lj) {
             ghost_copy(ctx, ctx->d_dE.p, 1);
-            hipLaunchKernelGGL(k_eam_pass2, dim3(nb), dim3(kBlock), 0, st, ctx->P, ctx->d_pos.p, L, ctx->d_rpos.p,
+            hipLaunchKernelGGL(k_eam_pass2, dim3(nb), dim3(kBlock), 0, st, ctx->P, ctx->d_pos.p, L,
                                drho, ctx->d_dE.p, ctx->d_fown.p, ctx->d_pairF2.p, part3);
             launch_check("k_eam_pass2");
         }
@@ -664,7 +647,7 @@ void run_force(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ, int st_clc, 
     const int nbw = shape_blocks(ctx->sh2, natms, 64 / kPass2Lanes);  // pass 2
     // the surrogate's pass 1: one block of kSurWaves wavefronts per CU, persistent
     const int nb1 = sur ? std::min(natms, kSurBlocks) : shape_blocks(ctx->sh1, natms);
-    PairBufs L{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p};
+    const PairBufs L = pair_bufs(ctx);
     // partials: one per wavefront in pass 1, the embedding and pass 2 (one per block
     // in the surrogate's pass 1)
     const long np1 = sur ? (long)nb1 : (long)nb1 * ctx->sh1.wpb;
@@ -748,7 +731,7 @@ double run_energy(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
     hipStream_t st = ctx->stream;
     const int nb = nblk((long)ctx->natms * kEmbedG);
     const int nbw = shape_blocks(ctx->sh1, ctx->natms);
-    PairBufs L{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p};
+    const PairBufs L = pair_bufs(ctx);
     const long np1 = (long)nbw * ctx->sh1.wpb, np2 = (long)nb * (kBlock / 64);  // one partial per wavefront
     ctx->d_part.reserve((size_t)np1 * 2 + (size_t)np2 + 16);
     double* part1 = ctx->d_part.p;
@@ -888,7 +871,7 @@ template <int NT, typename Q, int NQ>
 void run_table_values(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
     hipLaunchKernelGGL((k_table_values<NT, Q, NQ>), dim3(nblk((long)ctx->natms * 64)), dim3(kBlock),
                        (kBlock / 64) * TableStage<NT>::kBytes, ctx->stream, ctx->P, PQ, ctx->d_pos.p, ctx->d_alpha.p,
-                       ctx->d_off.p, ctx->d_nl.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_toff.p, ctx->d_town.p,
+                       ctx->d_off.p, ctx->d_nlrp.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_toff.p, ctx->d_town.p,
                        ctx->d_trank.p, ctx->d_tidx.p, ctx->d_trho.p, ctx->d_tphi.p);
     launch_check("k_table_values");
 }
@@ -908,21 +891,16 @@ void table_values_dispatch(mapp_dmd* ctx) {
     }
 }
 
-RevBufs rev_half(mapp_dmd* ctx) { return RevBufs{ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rev.p, ctx->d_pair_i.p}; }
-RevBufs rev_second(mapp_dmd* ctx) {
-    return RevBufs{ctx->d_off2.p, ctx->d_nl2.p, ctx->d_roff2.p, ctx->d_rev2.p, ctx->d_pair_i2.p};
-}
-
 // site table of the pair values (both ends of every pair inside the quadrature cut)
 template <int NT>
 void build_site_table(mapp_dmd* ctx) {
     hipStream_t st = ctx->stream;
     const int natms = ctx->natms;
-    const RevBufs L = rev_half(ctx);
+    const PairBufs L = pair_bufs(ctx);
     const dim3 grid(nblk((long)natms * kTableG));
     ctx->d_cnt.reserve(natms + 1);
     ctx->d_town.reserve(natms + 1);
-    ctx->d_trank.reserve(ctx->npairs + 1);
+    ctx->d_trank.reserve(ctx->nrev + 1);
     hipLaunchKernelGGL(k_table_count, grid, dim3(kBlock), 0, st, L, ctx->d_rowner.p, natms, ctx->d_pos.p,
                        ctx->P.cut_sq_mod, ctx->d_town.p, ctx->d_cnt.p, ctx->d_trank.p);
     launch_check("k_table_count");
@@ -946,41 +924,27 @@ template <int NT>
 void build_list2(mapp_dmd* ctx) {
     hipStream_t st = ctx->stream;
     const int natms = ctx->natms;
+    const dim3 grid(nblk((long)natms * 64));
     ctx->d_cnt.reserve(natms + 1);
-    hipLaunchKernelGGL((k_list2<false>), dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, ctx->d_pos.p, natms, ctx->d_off.p,
-                       ctx->d_nl.p, ctx->rsq_crd, ctx->d_cnt.p, (int*)nullptr);
+    ctx->d_rcnt.reserve(natms + 1);
+    ctx->d_crd.reserve(natms + ctx->nghost);
+    hipLaunchKernelGGL((k_list2<false>), grid, dim3(kBlock), 0, st, ctx->d_pos.p, natms, ctx->d_off.p, ctx->d_nl.p,
+                       ctx->d_roff.p, ctx->d_rowner.p, ctx->rsq_crd, ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_crd.p,
+                       (int*)nullptr, (int*)nullptr);
     launch_check("k_list2 count");
-    ctx->npairs2 = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_off2, natms);
+    ctx->d_off2.reserve(natms + 1);
+    ctx->d_foff2.reserve(natms + 1);
+    scan(ctx, kScanA, ctx->d_cnt.p, ctx->d_off2.p, natms, true);
+    scan(ctx, kScanB, ctx->d_rcnt.p, ctx->d_foff2.p, natms, true);
+    wait_box(ctx);
+    ctx->npairs2 = scan_total(ctx, kScanA);
+    const long nf = scan_total(ctx, kScanB);
     ctx->d_nl2.reserve(ctx->npairs2 + 1);
-    hipLaunchKernelGGL((k_list2<true>), dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, ctx->d_pos.p, natms, ctx->d_off.p,
-                       ctx->d_nl.p, ctx->rsq_crd, ctx->d_off2.p, ctx->d_nl2.p);
-    launch_check("k_list2 fill");
-    HIP_OK(hipMemsetAsync(ctx->d_cnt.p, 0, sizeof(int) * (natms + 1), st));
-    hipLaunchKernelGGL(k_rev_count, dim3(nblk((long)natms * kRevG)), dim3(kBlock), 0, st, ctx->d_off2.p, ctx->d_nl2.p, natms,
-                       ctx->d_cnt.p);
-    launch_check("k_rev_count 2");
-    long nrev = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_roff2, natms);
-    ctx->d_rev2.reserve(nrev + 1);
-    HIP_OK(hipMemsetAsync(ctx->d_cnt.p, 0, sizeof(int) * (natms + 1), st));
-    hipLaunchKernelGGL(k_rev_fill, dim3(nblk((long)natms * kRevG)), dim3(kBlock), 0, st, ctx->d_off2.p, ctx->d_nl2.p, natms,
-                       ctx->d_roff2.p, ctx->d_cnt.p, ctx->d_rev2.p);
-    launch_check("k_rev_fill 2");
-    sort_segments(ctx, ctx->d_roff2.p, ctx->d_nl2.p, ctx->d_rev2.p, nrev);
-    ctx->d_pair_i2.reserve(ctx->npairs2 + 1);
-    hipLaunchKernelGGL(k_pair_owner, dim3(nblk(natms)), dim3(kBlock), 0, st, ctx->d_off2.p, natms, ctx->d_pair_i2.p);
-    launch_check("k_pair_owner 2");
-    // both ends of every 2nd-list pair per site
-    const RevBufs L2 = rev_second(ctx);
-    hipLaunchKernelGGL(k_list2_count, dim3(nblk(natms)), dim3(kBlock), 0, st, L2, natms, ctx->d_cnt.p);
-    launch_check("k_list2_count");
-    const long nf = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_foff2, natms);
     ctx->d_fidx2.reserve(nf + 1);
-    hipLaunchKernelGGL(k_list2_fill, dim3(nblk(natms)), dim3(kBlock), 0, st, L2, natms, ctx->d_foff2.p, ctx->d_fidx2.p);
-    launch_check("k_list2_fill");
-    const int ntot = natms + ctx->nghost;
-    ctx->d_crd.reserve(ntot);
-    hipLaunchKernelGGL(k_crd, dim3(nblk(natms)), dim3(kBlock), 0, st, ctx->d_off2.p, ctx->d_roff2.p, natms, ctx->d_crd.p);
-    launch_check("k_crd");
+    hipLaunchKernelGGL((k_list2<true>), grid, dim3(kBlock), 0, st, ctx->d_pos.p, natms, ctx->d_off.p, ctx->d_nl.p,
+                       ctx->d_roff.p, ctx->d_rowner.p, ctx->rsq_crd, ctx->d_off2.p, ctx->d_foff2.p, (int*)nullptr,
+                       ctx->d_nl2.p, ctx->d_fidx2.p);
+    launch_check("k_list2 fill");
     if (ctx->nghost > 0) {
         hipLaunchKernelGGL((k_ghost_copy<int>), dim3(nblk(ctx->nghost)), dim3(kBlock), 0, st, ctx->d_crd.p, 1, natms,
                            ctx->nghost, ctx->d_ghost_owner.p);
@@ -1472,11 +1436,15 @@ __global__ void k_merge_sites(int n_own, int n_gh, const double4* __restrict__ p
     if (s >= n_own) Owner[gh_index_base + (s - n_own)] = own_base + owner[s - n_own];
 }
 
-__global__ void k_merge_list(int n_own, const int* __restrict__ off, const int* __restrict__ nl, int own_base,
-                             int pair_base, int gh_dst, int* __restrict__ Off, int* __restrict__ Nl) {
+__global__ void k_merge_list(int n_own, const int* __restrict__ off, const int* __restrict__ nl,
+                             const int* __restrict__ roff, const int* __restrict__ rowner, int own_base, int pair_base,
+                             int rev_base, int gh_dst, int* __restrict__ Off, int* __restrict__ Nl,
+                             int* __restrict__ Roff, int* __restrict__ Rowner) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_own) return;
     Off[own_base + i] = pair_base + off[i];
+    Roff[own_base + i] = rev_base + roff[i];
+    for (int q = roff[i]; q < roff[i + 1]; ++q) Rowner[rev_base + q] = own_base + rowner[q];
     for (int p = off[i]; p < off[i + 1]; ++p) {
         const int j = nl[p];
         Nl[pair_base + p] = j < n_own ? own_base + j : gh_dst + (j - n_own);
@@ -1495,7 +1463,7 @@ void init_batch(mapp_dmd* ctx, double skin) {
         }
     } guard{sub};
     std::vector<int> own_base(ncell + 1, 0), gh_base(ncell + 1, 0);
-    std::vector<long> pair_base(ncell + 1, 0);
+    std::vector<long> pair_base(ncell + 1, 0), rev_base(ncell + 1, 0);
     const int xc = xcols(ctx);
     size_t xo = 0;
     for (int k = 0; k < ncell; ++k) {
@@ -1517,6 +1485,7 @@ void init_batch(mapp_dmd* ctx, double skin) {
         own_base[k + 1] = own_base[k] + sp->natms;
         gh_base[k + 1] = gh_base[k] + sp->nghost;
         pair_base[k + 1] = pair_base[k] + sp->npairs;
+        rev_base[k + 1] = rev_base[k] + sp->nrev;
     }
     const int natms = own_base[ncell], nghost = gh_base[ncell];
     require(pair_base[ncell] < (1L << 31), MAPP_DMD_E_RANGE, "batch exceeds 2^31 pairs");
@@ -1524,6 +1493,7 @@ void init_batch(mapp_dmd* ctx, double skin) {
     ctx->natms = natms;
     ctx->nghost = nghost;
     ctx->npairs = pair_base[ncell];
+    ctx->nrev = rev_base[ncell];  // no more than the pairs
     const int ntot = natms + nghost;
     ctx->d_pos.reserve(ntot);
     ctx->d_alpha.reserve((size_t)ntot * NT);
@@ -1531,6 +1501,8 @@ void init_batch(mapp_dmd* ctx, double skin) {
     ctx->d_ghost_owner.reserve(nghost + 1);
     ctx->d_off.reserve(natms + 1);
     ctx->d_nl.reserve(ctx->npairs + 1);
+    ctx->d_roff.reserve(natms + 1);
+    ctx->d_rowner.reserve(ctx->nrev + 1);
     for (int k = 0; k < ncell; ++k) {
         mapp_dmd* c = sub[k];
         const int n = c->natms, g = c->nghost;
@@ -1538,12 +1510,14 @@ void init_batch(mapp_dmd* ctx, double skin) {
                            c->d_alpha.p, c->d_conc.p, c->d_ghost_owner.p, own_base[k], natms + gh_base[k], gh_base[k],
                            ctx->d_pos.p, ctx->d_alpha.p, ctx->d_conc.p, ctx->d_ghost_owner.p);
         launch_check("k_merge_sites");
-        hipLaunchKernelGGL(k_merge_list, dim3(nblk(n)), dim3(kBlock), 0, st, n, c->d_off.p, c->d_nl.p, own_base[k],
-                           (int)pair_base[k], natms + gh_base[k], ctx->d_off.p, ctx->d_nl.p);
+        hipLaunchKernelGGL(k_merge_list, dim3(nblk(n)), dim3(kBlock), 0, st, n, c->d_off.p, c->d_nl.p, c->d_roff.p,
+                           c->d_rowner.p, own_base[k], (int)pair_base[k], (int)rev_base[k], natms + gh_base[k],
+                           ctx->d_off.p, ctx->d_nl.p, ctx->d_roff.p, ctx->d_rowner.p);
         launch_check("k_merge_list");
     }
-    const int last = (int)ctx->npairs;
+    const int last = (int)ctx->npairs, rlast = (int)ctx->nrev;
     HIP_OK(hipMemcpyAsync(ctx->d_off.p + natms, &last, sizeof(int), hipMemcpyHostToDevice, st));
+    HIP_OK(hipMemcpyAsync(ctx->d_roff.p + natms, &rlast, sizeof(int), hipMemcpyHostToDevice, st));
     HIP_OK(hipStreamSynchronize(st));
     ctx->swap_off.assign(1, 0);  // no box-wide ghost swaps: positions stay fixed in a batch
     ctx->swap_dim.clear();

@@ -49,11 +49,12 @@ struct mapp_dmd {
     mappdmd::DevBuf<double> d_alpha, d_conc;
     mappdmd::DevBuf<int> d_ghost_src, d_ghost_owner;
     // binning and lists
-    mappdmd::DevBuf<int> d_flag, d_offs, d_bin_of, d_bin_cnt, d_bin_start, d_bin_atoms;
-    mappdmd::DevBuf<int> d_cnt, d_off, d_nl, d_roff, d_rev;
-    mappdmd::DevBuf<int> d_off2, d_nl2, d_roff2, d_rev2, d_crd;
-    mappdmd::DevBuf<int> d_sort_tmp;  // out-of-place segment sort
-    mappdmd::DevBuf<int> d_pair_i, d_pair_i2, d_rpos;
+    mappdmd::DevBuf<int> d_flag, d_offs, d_bin_of, d_bin_cnt, d_bin_slot, d_bin_start, d_bin_atoms, d_arrived;
+    mappdmd::DevBuf<double4> d_bin_pos;               // positions in bin order
+    mappdmd::DevBuf<unsigned long long> d_list_mask;  // accept bits of the list build
+    mappdmd::DevBuf<int> d_cnt, d_rcnt, d_off, d_nl, d_roff;
+    mappdmd::DevBuf<int> d_off2, d_nl2, d_crd;
+    mappdmd::DevBuf<int> d_rtmp;  // owners of the reverse lists before they are sorted
     mappdmd::DevBuf<double2> d_deriv;  // pass 1's records (PairRec) of the quadrature type
     mappdmd::DevBuf<int2> d_info;      // [natms] {list offset, pairs inside the cut at the last force pass 1}
     mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}
@@ -71,7 +72,7 @@ struct mapp_dmd {
     mappdmd::DevBuf<int2> d_nlrp;
     mappdmd::DevBuf<int> d_rowner;
     mappdmd::DevBuf<int> d_toff, d_tidx;        // site table: both ends of every pair inside the quadrature cut
-    mappdmd::DevBuf<int> d_town, d_trank;       // own entries per site; a pair's rank in its partner's reverse entries
+    mappdmd::DevBuf<int> d_town, d_trank;       // own entries per site; a reverse entry's rank among those inside the cut
     mappdmd::DevBuf<double> d_trho, d_tphi;
     long ntable = 0;
     mappdmd::DevBuf<int> d_foff2, d_fidx2;      // 2nd list of both ends (~owner for the partner end)

@@ -122,7 +122,7 @@ template <int MODEL, bool ENERGY_ONLY>
 __global__ __launch_bounds__(kBlock) void k_eam_pass1(FFParams<double> P, EamBufs T, MdParams M,
                                                       const double4* __restrict__ pos,
                                                       const double* __restrict__ type, PairBufs L,
-                                                      const int* __restrict__ rpos, double* __restrict__ rho_own,
+                                                      double* __restrict__ rho_own,
                                                       double* __restrict__ fown, double* __restrict__ pairE,
                                                       double* __restrict__ pairF, double2* __restrict__ drho,
                                                       double* __restrict__ part) {
@@ -135,7 +135,8 @@ __global__ __launch_bounds__(kBlock) void k_eam_pass1(FFParams<double> P, EamBuf
         double rho = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
         const int p1 = L.off[i + 1];
         for (int p = L.off[i] + g.l; p < p1; p += kEamG) {
-            const int j = L.nl[p];
+            const int2 e = L.nlrp[p];
+            const int j = e.x;
             const double4 xj = pos[j];
             const double dx0 = xi.x - xj.x, dx1 = xi.y - xj.y, dx2 = xi.z - xj.z;
             double rsq;
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_pass1(FFParams<double> P, EamBuf
             }
             if (!ENERGY_ONLY && MODEL != kModelLj) drho[p] = dr;
             if (owned) {
-                const size_t q = (size_t)rpos[p];
+                const size_t q = (size_t)e.y;
                 if (MODEL != kModelLj) pairE[q] = rho_j;
                 if (!ENERGY_ONLY) {
                     pairF[q * 3 + 0] = -pf * dx0;
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_embed(FFParams<double> P, EamBuf
 
 // pass 2: embedding forces fpair = F'_i drho_i/dr + F'_j drho_j/dr
 __global__ __launch_bounds__(kBlock) void k_eam_pass2(FFParams<double> P, const double4* __restrict__ pos, PairBufs L,
-                                                      const int* __restrict__ rpos, const double2* __restrict__ drho,
+                                                      const double2* __restrict__ drho,
                                                       const double* __restrict__ dF, double* __restrict__ fown,
                                                       double* __restrict__ pairF2, double* __restrict__ part) {
     const SiteGroup<kEamG> g;
@@ -249,7 +250,8 @@ __global__ __launch_bounds__(kBlock) void k_eam_pass2(FFParams<double> P, const 
         double fx = 0.0, fy = 0.0, fz = 0.0;
         const int p1 = L.off[i + 1];
         for (int p = L.off[i] + g.l; p < p1; p += kEamG) {
-            const int j = L.nl[p];
+            const int2 e = L.nlrp[p];
+            const int j = e.x;
             const double2 dr = drho[p];
             const bool owned = j < P.natms;
             double fpair = 0.0, dx0 = 0.0, dx1 = 0.0, dx2 = 0.0;
@@ -271,7 +273,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_pass2(FFParams<double> P, const 
                 acc[5] -= w * fpair * dx0 * dx1;
             }
             if (owned) {
-                const size_t q = (size_t)rpos[p];
+                const size_t q = (size_t)e.y;
                 pairF2[q * 3 + 0] = -dx0 * fpair;
                 pairF2[q * 3 + 1] = -dx1 * fpair;
                 pairF2[q * 3 + 2] = -dx2 * fpair;

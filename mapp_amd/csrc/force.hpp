@@ -118,10 +118,9 @@ __device__ __forceinline__ int xcd_block(int nblocks) {
 }
 
 struct PairBufs {
-    const int* off;
-    const int* nl;
-    const int* roff;
-    const int* rev;
+    const int* off;    // half list
+    const int2* nlrp;  // {partner, its position in the partner's reverse list or -1}
+    const int* roff;   // reverse list: the owners of the pairs that list a site
 };
 
 // Which half-list entries lay inside the quadrature cut at the last pass 1: the
@@ -273,21 +272,6 @@ __global__ void k_pack_atoms(const double* __restrict__ alpha, const double* __r
         const double a = alpha[k];
         rec[k] = make_double4(a, conc[k], 1.0 / a, 0.0);
     }
-}
-
-// per half-list entry {partner, reverse position}: the force passes read both
-// with one load (every entry starts outside the quadrature cut)
-__global__ void k_pack_nlrp(const int* __restrict__ nl, const int* __restrict__ rpos, long n,
-                            int2* __restrict__ nlrp) {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) nlrp[k] = make_int2(nl[k], rpos[k]);
-}
-
-// per reverse-list entry the owner of the pair (every entry starts outside the cut)
-__global__ void k_rev_owner(const int* __restrict__ rev, const int* __restrict__ pair_i, long n,
-                            int* __restrict__ rowner) {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) rowner[k] = pair_i[rev[k]];
 }
 
 // sum over the wavefront, the same value in every lane: a DPP rotation tree

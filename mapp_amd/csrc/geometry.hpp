@@ -94,55 +94,65 @@ __global__ __launch_bounds__(kScanSumThreads) void k_scan_sums(unsigned long lon
     if (tid == 0) *total = carry;
 }
 
-// adds the tile sums; with the last tile, *end (optional) = the total
+// adds the tile sums; *end (optional) = the total; host[0] = the total and, with
+// mid >= 0, host[1] = out[mid]
 __global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ out,
                                                            const unsigned long long* __restrict__ add, long n,
                                                            const unsigned long long* __restrict__ total,
-                                                           int* __restrict__ end, unsigned long long* host_total) {
+                                                           int* __restrict__ end, long mid, unsigned long long* host) {
     const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
     const int a = (int)add[blockIdx.x];
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         long idx = base + k;
-        if (idx < n) out[idx] += a;
+        if (idx < n) {
+            const int v = out[idx] + a;
+            out[idx] = v;
+            if (idx == mid) host[1] = (unsigned long long)v;
+        }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (end) *end = (int)*total;
-        *host_total = *total;
+        host[0] = *total;
     }
 }
 
 // ---- ghosts ----------------------------------------------------------------
-// flag[i-lo] = 1 when atom i in [lo,hi) lies within the ghost shell of the
-// low (dir 0: s <= s_ph_lo) or high (dir 1: s_ph_hi <= s) face of dimension idim
-__global__ void k_ghost_flag(const double4* __restrict__ pos, int lo, int hi, int idim, int dir, double thr,
+// flag[i] = 1 when atom i lies within the ghost shell of the low face of dimension idim
+// (s <= thr_lo), flag[n + i] that of the high face (thr_hi <= s)
+__global__ void k_ghost_flag(const double4* __restrict__ pos, int n, int idim, double thr_lo, double thr_hi,
                              int* __restrict__ flag) {
-    int i = lo + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= hi) return;
-    double s = comp3c(pos[i], idim);
-    flag[i - lo] = dir == 0 ? (s <= thr ? 1 : 0) : (thr <= s ? 1 : 0);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double s = comp3c(pos[i], idim);
+    flag[i] = s <= thr_lo ? 1 : 0;
+    flag[(long)n + i] = thr_hi <= s ? 1 : 0;
 }
 
-// copies flagged atoms to ghost rows gbase + offs[i-lo], shifted by +-1 in s
+// copies flagged atoms to ghost rows n + offs[...], shifted by +1 (low face) or -1 in s
 template <int NT>
-__global__ void k_ghost_emit(double4* __restrict__ pos, double* __restrict__ alpha, double* __restrict__ conc,
-                             int lo, int hi, int idim, int dir, const int* __restrict__ flag,
-                             const int* __restrict__ offs, int gbase, int natms, int* __restrict__ ghost_src,
-                             int* __restrict__ ghost_owner) {
-    int i = lo + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= hi || !flag[i - lo]) return;
-    int g = gbase + offs[i - lo];
-    double4 p = pos[i];
-    if (dir == 0) comp3(p, idim) += 1.0;
-    else comp3(p, idim) -= 1.0;
-    pos[g] = p;
+__global__ void k_ghost_emit(double4* __restrict__ pos, double* __restrict__ alpha, double* __restrict__ conc, int n,
+                             int idim, const int* __restrict__ flag, const int* __restrict__ offs, int natms,
+                             int* __restrict__ ghost_src, int* __restrict__ ghost_owner) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        alpha[(long)g * NT + t] = alpha[(long)i * NT + t];
-        conc[(long)g * NT + t] = conc[(long)i * NT + t];
+    for (int dir = 0; dir < 2; ++dir) {
+        const long e = (long)dir * n + i;
+        if (!flag[e]) continue;
+        const int g = n + offs[e];
+        double4 p = pos[i];
+        if (dir == 0) comp3(p, idim) += 1.0;
+        else comp3(p, idim) -= 1.0;
+        pos[g] = p;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            alpha[(long)g * NT + t] = alpha[(long)i * NT + t];
+            conc[(long)g * NT + t] = conc[(long)i * NT + t];
+        }
+        ghost_src[g - natms] = i;
+        ghost_owner[g - natms] = i < natms ? i : ghost_owner[i - natms];
     }
-    ghost_src[g - natms] = i;
-    ghost_owner[g - natms] = i < natms ? i : ghost_owner[i - natms];
 }
 
 // Atoms::update of x between rebuilds: ghost = source +- H[idim][0..idim]
@@ -179,17 +189,14 @@ __global__ void k_ghost_copy(T* __restrict__ v, int d, int natms, int nghost, co
 
 // ---- box transforms --------------------------------------------------------
 // Atoms::s2x: x_j = s_j H_jj + sum_{k>j} H_kj s_k (lower-triangular H)
-__global__ void k_s2x(double4* __restrict__ pos, int n, BoxParams bp) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double4 s = pos[i];
+__device__ __forceinline__ double4 s2x(double4 s, const BoxParams& bp) {
     double x0 = s.x * bp.H[0][0];
     x0 += bp.H[1][0] * s.y;
     x0 += bp.H[2][0] * s.z;
     double x1 = s.y * bp.H[1][1];
     x1 += bp.H[2][1] * s.z;
-    double x2 = s.z * bp.H[2][2];
-    pos[i] = make_double4(x0, x1, x2, 0.0);
+    const double x2 = s.z * bp.H[2][2];
+    return make_double4(x0, x1, x2, 0.0);
 }
 
 // Atoms::x2s with the wrap into [0,1)
@@ -213,8 +220,9 @@ __global__ void k_x2s(double4* __restrict__ pos, int n, BoxParams bp) {
 }
 
 // ---- cell binning (reduced coordinates) -----------------------------------
+// slot[i] = the arrival number of atom i in its bin (arbitrary: atomics)
 __global__ void k_s2bin(const double4* __restrict__ pos, int n, BoxParams bp, int* __restrict__ bin_of,
-                        int* __restrict__ bin_cnt) {
+                        int* __restrict__ bin_cnt, int* __restrict__ slot) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     double4 s = pos[i];
@@ -226,62 +234,96 @@ __global__ void k_s2bin(const double4* __restrict__ pos, int n, BoxParams bp, in
         no += t * bp.denom[d];
     }
     bin_of[i] = no;
-    atomicAdd(&bin_cnt[no], 1);
+    slot[i] = atomicAdd(&bin_cnt[no], 1);
 }
 
 __global__ void k_bin_fill(const int* __restrict__ bin_of, int n, const int* __restrict__ bin_start,
-                           int* __restrict__ bin_cur, int* __restrict__ bin_atoms) {
+                           const int* __restrict__ slot, int* __restrict__ bin_atoms) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    int b = bin_of[i];
-    int k = atomicAdd(&bin_cur[b], 1);
-    bin_atoms[bin_start[b] + k] = i;
+    bin_atoms[bin_start[bin_of[i]] + slot[i]] = i;
 }
 
-// Ascending order inside every segment (atom indices inside each bin, as the
-// reference's linked bins built by pushing atoms from the highest index down,
-// src/neighbor.cpp:428-434; pair indices inside each reverse-list segment).
-// One thread per value: value x of segment s = key[x] goes to
-// out[start[s] + r], r = the number of the segment's values below x.  The
-// values of a segment are distinct, so the ranks are a permutation of the
-// segment and every write stays inside it; the segment is read through the
-// caches instead of being shifted entry by entry in memory.  With pos_of, also
-// pos_of[x] = the position x lands at (the reverse position of each pair).
-__global__ void k_rank_place(const int* __restrict__ v, long n, const int* __restrict__ key,
-                             const int* __restrict__ start, int* __restrict__ out, int* __restrict__ pos_of) {
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// Atom indices in ascending order inside every bin, as the reference's linked bins
+// built by pushing atoms from the highest index down (src/neighbor.cpp:428-434), and
+// the end of Neighbor::bin_atoms_s, s2x of every atom.  One thread per atom: atom x of
+// bin s goes to bin_start[s] + r, r = the number of the bin's atoms below x; its
+// position (w: its type, with a cutoff per type pair) is also kept in that order, where
+// the list kernel reads consecutive candidates from consecutive addresses.
+__global__ void k_bin_place(const int* __restrict__ v, int n, const int* __restrict__ bin_of,
+                            const int* __restrict__ bin_start, BoxParams bp, const double* __restrict__ type,
+                            double4* __restrict__ pos, int* __restrict__ bin_atoms, double4* __restrict__ bin_pos) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= n) return;
     const int x = v[q];
-    const int s = key[x];
-    const int lo = start[s], hi = start[s + 1];
+    const int s = bin_of[x];
+    const int lo = bin_start[s], hi = bin_start[s + 1];
     int r = 0;
     for (int t = lo; t < hi; ++t) r += v[t] < x ? 1 : 0;
-    out[lo + r] = x;
-    if (pos_of) pos_of[x] = lo + r;
+    double4 p = s2x(pos[x], bp);
+    pos[x] = p;
+    if (bp.pairwise) p.w = type[x];
+    bin_atoms[lo + r] = x;
+    bin_pos[lo + r] = p;
 }
 
 // ---- half neighbor list ----------------------------------------------------
 // stencil order of find_bin_no: offset of dimension 0 outermost, 2 innermost;
 // inside a bin ascending index; j > i (every j != i with bp.full, the full list
 // of src/neighbor.cpp:240-284); rsq = ((d0*d0) + d1*d1) + d2*d2 < cut.
-// One wavefront per site: lane s < 27 takes stencil bin s (s = 9(a+1) + 3(b+1)
-// + c+1 for offsets a, b, c), a prefix sum of the bin sizes concatenates the 27
-// bins in stencil order, and 64 consecutive candidates are tested per round;
-// ballot ranks write the accepted ones in candidate order, which is the list
-// order of a single thread walking the stencil.
-template <bool FILL>
-__global__ __launch_bounds__(256) void k_half_list(const double4* __restrict__ pos, int natms,
-                                                   const int* __restrict__ bin_of,
-                                                   const int* __restrict__ bin_start,
-                                                   const int* __restrict__ bin_atoms, BoxParams bp,
-                                                   const double* __restrict__ type,
-                                                   int* __restrict__ cnt_or_off, int* __restrict__ nl) {
-    const int lane = threadIdx.x & 63;
-    const long site = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (site >= natms) return;  // the whole wavefront
-    const int i = (int)site;
-    const int ti = bp.pairwise ? (int)type[i] : 0;
-    int tmp = bin_of[i];
+// One wavefront per group of kBinSites sites of one bin: lane s < 27 takes stencil bin s
+// (s = 9(a+1) + 3(b+1) + c+1 for offsets a, b, c), a prefix sum of the bin sizes
+// concatenates the 27 bins in stencil order, and 64 consecutive candidates, read once,
+// are tested per round against each site of the group; ballot ranks write the accepted
+// ones in candidate order, which is the list order of a single thread walking the
+// stencil.
+//
+// The same tests give a site's reverse list: the owners of pairs with site i are the
+// accepted j < i (the stencil and the distance are the same from either end).  The
+// count launch keeps each round's accept bits, kMaskWords rounds of them, and the fill
+// launch tests again only what lies beyond; the owners come out in stencil order and
+// are sorted by k_sort_owners.
+//
+// Bound by the vector instructions of the tests and, at the start of a wavefront, by
+// the chain of loads that finds the candidates.  At 293,000 sites (16 to a bin, 430
+// candidates each) the count takes 0.15 ms, the fill 0.17 and the sort 0.09; one
+// wavefront per site, both launches testing, took 0.33 + 0.36 for the half list alone,
+// and the reverse list made from it by atomics, a sort and four passes over the pairs
+// 0.74 where the sort and k_pair_links take 0.24.  Groups of 8 or 16 sites are slower
+// (0.20 and 0.50: fewer wavefronts, more registers).
+constexpr int kBinSites = 4;
+constexpr int kBinWaves = 4;  // wavefronts per bin: they take its groups in turn
+constexpr int kMaskWords = 16;
+// set bits of m below this lane
+__device__ __forceinline__ int lane_rank(unsigned long long m) {
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+__device__ __forceinline__ unsigned long long read_lane_u64(unsigned long long v, int l) {
+    const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)v, l);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(v >> 32), l);
+    return (unsigned long long)hi << 32 | lo;
+}
+struct HalfLists {
+    unsigned long long* mask;  // [natms][kMaskWords] accept bits
+    int *cnt, *rcnt;           // count: entries of the site's own and reverse lists
+    const int *off, *roff;     // fill: their offsets
+    int *nl, *rlist;           // fill: partners in list order; owners in stencil order
+};
+// PAIRWISE: a cutoff per type pair (bp.cut_sk_sq_tp), the type in bin_pos[].w
+template <bool FILL, bool PAIRWISE>
+__global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const int* __restrict__ bin_start,
+                                                              const int* __restrict__ bin_atoms,
+                                                              const double4* __restrict__ bin_pos, BoxParams bp,
+                                                              HalfLists L) {
+    __shared__ unsigned long long ends_lds[kBinWaves][64];
+    __shared__ int2 bin_lds[kBinWaves][32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int bin = blockIdx.x;
+    const int k1 = bin_start[bin + 1];
+    int k0 = bin_start[bin] + wave * kBinSites;
+    // owned sites come first in a bin
+    if (k0 >= k1 || bin_atoms[k0] >= natms) return;  // the whole wavefront
+    int tmp = bin;
     int loc[3];
     for (int d = 2; d > -1; --d) {
         loc[d] = tmp / bp.denom[d];
@@ -296,118 +338,215 @@ __global__ __launch_bounds__(256) void k_half_list(const double4* __restrict__ p
             bsize = bin_start[no + 1] - bstart;
         }
     }
-    int incl = bsize;  // inclusive prefix over the stencil bins
+    // the occupied bins packed into the low lanes, so that their last candidates are distinct
+    const unsigned long long occ = __ballot(bsize > 0);
+    const int nbin = __popcll(occ);
+    if (bsize > 0) bin_lds[wave][lane_rank(occ)] = make_int2(bstart, bsize);
+    __builtin_amdgcn_wave_barrier();
+    bstart = bsize = 0;
+    if (lane < nbin) {
+        const int2 e = bin_lds[wave][lane];
+        bstart = e.x;
+        bsize = e.y;
+    }
+    int incl = bsize;  // inclusive prefix over the bins
     for (int d = 1; d < 32; d <<= 1) {
         const int v = __shfl_up(incl, d, 64);
         if (lane >= d) incl += v;
     }
-    const int excl = incl - bsize;
-    const int total = __shfl(incl, 26, 64);
-    const double4 xi = pos[i];
-    int w = FILL ? cnt_or_off[i] : 0;
-    for (int base = 0; base < total; base += 64) {
-        const int q = base + lane;
-        // stencil bin of candidate q: the number of bins whose inclusive prefix is <= q
-        int s = 0;
+    const int to_bin = bstart - (incl - bsize);  // candidate number -> place in the bins
+    const int total = __builtin_amdgcn_readlane(incl, 31);
+    for (; k0 < k1; k0 += kBinWaves * kBinSites) {
+        int site[kBinSites], w[kBinSites], wr[kBinSites];
+        double4 xi[kBinSites];
+        unsigned long long keep[kBinSites];
 #pragma unroll
-        for (int step = 16; step >= 1; step >>= 1) {
-            const int probe = s + step - 1;
-            const int v = __shfl(incl, probe < 27 ? probe : 26, 64);
-            if (probe < 27 && v <= q) s += step;
-        }
-        s = s < 26 ? s : 26;
-        const int bs = __shfl(bstart, s, 64), ex = __shfl(excl, s, 64);
-        bool take = false;
-        int j = 0;
-        if (q < total) {
-            j = bin_atoms[bs + (q - ex)];
-            if (bp.full ? j != i : j > i) {
-                const double4 xj = pos[j];
-                double d0 = xi.x - xj.x, d1 = xi.y - xj.y, d2 = xi.z - xj.z;
-                double rsq = 0.0;
-                rsq += d0 * d0;
-                rsq += d1 * d1;
-                rsq += d2 * d2;
-                const double cut = bp.pairwise ? bp.cut_sk_sq_tp[md_comp(ti, (int)type[j])] : bp.cut_sk_sq;
-                take = rsq < cut;
+        for (int u = 0; u < kBinSites; ++u) {
+            const int k = k0 + u < k1 ? k0 + u : k1 - 1;
+            const int i = bin_atoms[k];
+            site[u] = k0 + u < k1 && i < natms ? i : -1;
+            xi[u] = bin_pos[k];
+            // in vector registers: as scalars the group does not fit, and each use pays a move
+            if (!FILL) asm("" : "+v"(xi[u].x), "+v"(xi[u].y), "+v"(xi[u].z));
+            w[u] = wr[u] = 0;
+            keep[u] = 0;
+            if (FILL && site[u] >= 0) {
+                w[u] = L.off[i];
+                wr[u] = L.roff[i];
+                if (lane < kMaskWords && lane * 64 < total) keep[u] = L.mask[(size_t)i * kMaskWords + lane];
             }
         }
-        const unsigned long long m = __ballot(take);
-        if (FILL && take)
-            nl[w + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = j;
-        w += __popcll(m);
-    }
-    if (!FILL && lane == 0) cnt_or_off[i] = w;
-}
-
-// ---- reverse CSR: for owned j, the list positions p whose partner is j ----
-// kRevG lanes per site over its list entries; the fill order inside a segment
-// is arbitrary (atomics) and is put in ascending pair order by k_rank_place
-constexpr int kRevG = 16;
-__global__ void k_rev_count(const int* __restrict__ off, const int* __restrict__ nl, int natms,
-                            int* __restrict__ rcnt) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = (int)(t / kRevG), l = (int)(t % kRevG);
-    if (i >= natms) return;
-    for (int p = off[i] + l; p < off[i + 1]; p += kRevG) {
-        const int j = nl[p];
-        if (j < natms) atomicAdd(&rcnt[j], 1);
-    }
-}
-
-__global__ void k_rev_fill(const int* __restrict__ off, const int* __restrict__ nl, int natms,
-                           const int* __restrict__ rstart, int* __restrict__ rcur, int* __restrict__ rev) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = (int)(t / kRevG), l = (int)(t % kRevG);
-    if (i >= natms) return;
-    for (int p = off[i] + l; p < off[i + 1]; p += kRevG) {
-        const int j = nl[p];
-        if (j < natms) {
-            const int k = atomicAdd(&rcur[j], 1);
-            rev[rstart[j] + k] = p;
+        if (site[0] < 0) break;
+        unsigned long long ends = 0;  // lane r: which candidates of the 64 rounds' round r are the last of their bin
+        int nb = 0;                   // bins that end before this round
+        for (int base = 0, round = 0; base < total; base += 64, ++round) {
+            if ((round & 63) == 0) {
+                __builtin_amdgcn_wave_barrier();
+                ends_lds[wave][lane] = 0;
+                __builtin_amdgcn_wave_barrier();
+                const int e = incl - 1 - base;
+                if (lane < nbin && e >= 0 && e < 4096)
+                    atomicOr(reinterpret_cast<unsigned*>(ends_lds[wave]) + (e >> 5), 1u << (e & 31));
+                __builtin_amdgcn_wave_barrier();
+                ends = ends_lds[wave][lane];
+            }
+            const unsigned long long last = read_lane_u64(ends, round & 63);
+            const int s = nb + lane_rank(last);  // bin of candidate base + lane
+            nb += __popcll(last);
+            const int q = base + lane;
+            const int k = __shfl(to_bin, s, 64) + q;
+            const bool kept = FILL && round < kMaskWords;
+            const unsigned long long valid = __builtin_amdgcn_ballot_w64(q < total);
+            int j = 0;
+            double4 xj{};
+            if (q < total) {
+                j = bin_atoms[k];
+                if (!kept) xj = bin_pos[k];
+            }
+#pragma unroll
+            for (int u = 0; u < kBinSites; ++u) {
+                const int i = site[u];
+                if (i < 0) continue;
+                unsigned long long near;
+                if (kept) {
+                    near = read_lane_u64(keep[u], round);
+                } else {
+                    double d0 = xi[u].x - xj.x, d1 = xi[u].y - xj.y, d2 = xi[u].z - xj.z;
+                    double rsq = 0.0;
+                    rsq += d0 * d0;
+                    rsq += d1 * d1;
+                    rsq += d2 * d2;
+                    const double cut =
+                        PAIRWISE ? bp.cut_sk_sq_tp[md_comp((int)xi[u].w, (int)xj.w)] : bp.cut_sk_sq;
+                    near = __builtin_amdgcn_ballot_w64(rsq < cut) & valid;
+                }
+                // j == i is neither
+                const unsigned long long above = __builtin_amdgcn_ballot_w64(j > i) & near;
+                const unsigned long long below = __builtin_amdgcn_ballot_w64(j < i) & near;
+                const unsigned long long own = bp.full ? above | below : above, rv = bp.full ? 0 : below;
+                if constexpr (FILL) {
+                    if (own >> lane & 1) L.nl[w[u] + lane_rank(own)] = j;
+                    if (rv >> lane & 1) L.rlist[wr[u] + lane_rank(rv)] = j;
+                } else if (lane == round) {
+                    keep[u] = own | rv;
+                }
+                w[u] += __popcll(own);
+                wr[u] += __popcll(rv);
+            }
+        }
+        if constexpr (!FILL) {
+#pragma unroll
+            for (int u = 0; u < kBinSites; ++u) {
+                const int i = site[u];
+                if (i < 0) continue;
+                if (lane < kMaskWords && lane * 64 < total) L.mask[(size_t)i * kMaskWords + lane] = keep[u];
+                if (lane == 0) {
+                    L.cnt[i] = w[u];
+                    L.rcnt[i] = wr[u];
+                }
+            }
         }
     }
 }
 
-// sub-list of the half list with rsq < rsq_crd (create_2nd_neigh_lst); one
-// wavefront per site, 64 list entries per round, ballot ranks keep the list order
+// the owners of a site's reverse list in ascending order: ranked 64 at a time against
+// each other (they are distinct), one wavefront per site
+__global__ __launch_bounds__(256) void k_sort_owners(int natms, const int* __restrict__ roff,
+                                                     const int* __restrict__ tmp, int* __restrict__ rowner) {
+    const int lane = threadIdx.x & 63;
+    const long site = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (site >= natms) return;  // the whole wavefront
+    const int i = __builtin_amdgcn_readfirstlane((int)site);
+    const int q0 = roff[i], q1 = roff[i + 1];
+    for (int a = q0; a < q1; a += 64) {
+        const int x = a + lane < q1 ? tmp[a + lane] : 0x7FFFFFFF;
+        int r = 0;
+        for (int b = q0; b < q1; b += 64) {
+            const int y = b == a ? x : (b + lane < q1 ? tmp[b + lane] : 0x7FFFFFFF);
+            const int ny = q1 - b < 64 ? q1 - b : 64;
+            for (int l = 0; l < ny; l += 8) {  // those beyond ny rank below nothing
+#pragma unroll
+                for (int d = 0; d < 8; ++d) r += __builtin_amdgcn_readlane(y, l + d) < x ? 1 : 0;
+            }
+        }
+        if (a + lane < q1) rowner[q0 + r] = x;
+    }
+}
+
+// per half-list entry {partner, its position in the partner's reverse list or -1 for a
+// ghost}: the owner's place among the partner's ascending owners, by bisection.  kLinkG
+// lanes per site.  Every entry starts outside the quadrature cut.
+constexpr int kLinkG = 32;
+__global__ void k_pair_links(const int* __restrict__ off, const int* __restrict__ nl, int natms,
+                             const int* __restrict__ roff, const int* __restrict__ rowner,
+                             int2* __restrict__ nlrp) {
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(t / kLinkG), l = (int)(t % kLinkG);
+    if (i >= natms) return;
+    for (int p = off[i] + l; p < off[i + 1]; p += kLinkG) {
+        const int j = nl[p];
+        int q = -1;
+        if (j < natms) {
+            int lo = roff[j], hi = roff[j + 1];
+            while (lo < hi) {
+                const int mid = lo + (hi - lo) / 2;
+                if (rowner[mid] < i) lo = mid + 1;
+                else hi = mid;
+            }
+            q = lo;
+        }
+        nlrp[p] = make_int2(j, q);
+    }
+}
+
+// Both ends of the 2nd list (create_2nd_neigh_lst: the half-list pairs with
+// rsq < rsq_crd) per site: own pairs in list order as the partner (also nl2, the list
+// itself), then the owners of the pairs that list the site, ascending, as ~owner.  One
+// wavefront per site, 64 entries per round, ballot ranks keep the order.  cnt / tot:
+// the own pairs and both ends, crd = both ends.
 template <bool FILL>
 __global__ __launch_bounds__(256) void k_list2(const double4* __restrict__ pos, int natms,
                                                const int* __restrict__ off, const int* __restrict__ nl,
+                                               const int* __restrict__ roff, const int* __restrict__ rowner,
                                                double rsq_crd, int* __restrict__ cnt_or_off,
-                                               int* __restrict__ nl2) {
+                                               int* __restrict__ tot_or_off, int* __restrict__ crd,
+                                               int* __restrict__ nl2, int* __restrict__ fidx) {
     const int lane = threadIdx.x & 63;
     const long site = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (site >= natms) return;  // the whole wavefront
     const int i = (int)site;
     const double4 xi = pos[i];
-    int w = FILL ? cnt_or_off[i] : 0;
-    const int p1 = off[i + 1];
-    for (int p0 = off[i]; p0 < p1; p0 += 64) {
-        const int p = p0 + lane;
-        bool take = false;
-        int j = 0;
-        if (p < p1) {
-            j = nl[p];
-            const double4 xj = pos[j];
-            double d0 = xi.x - xj.x, d1 = xi.y - xj.y, d2 = xi.z - xj.z;
-            double rsq = d0 * d0 + d1 * d1 + d2 * d2;
-            take = rsq < rsq_crd;
+    int w = FILL ? cnt_or_off[i] : 0, f = FILL ? tot_or_off[i] : 0;
+#pragma unroll
+    for (int end = 0; end < 2; ++end) {
+        const int* const list = end ? rowner : nl;
+        const int p1 = end ? roff[i + 1] : off[i + 1];
+        for (int p0 = end ? roff[i] : off[i]; p0 < p1; p0 += 64) {
+            const int p = p0 + lane;
+            bool take = false;
+            int j = 0;
+            if (p < p1) {
+                j = list[p] & 0x7FFFFFFF;  // owners carry a flag in the top bit
+                const double4 xj = pos[j];
+                double d0 = xi.x - xj.x, d1 = xi.y - xj.y, d2 = xi.z - xj.z;
+                double rsq = d0 * d0 + d1 * d1 + d2 * d2;
+                take = rsq < rsq_crd;
+            }
+            const unsigned long long m = __ballot(take);
+            if (FILL && take) {
+                const int r = lane_rank(m);
+                fidx[f + r] = end ? ~j : j;
+                if (!end) nl2[w + r] = j;
+            }
+            f += __popcll(m);
+            if (!end) w += __popcll(m);
         }
-        const unsigned long long m = __ballot(take);
-        if (FILL && take)
-            nl2[w + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = j;
-        w += __popcll(m);
     }
-    if (!FILL && lane == 0) cnt_or_off[i] = w;
-}
-
-// coordination: own 2nd-list size + number of lower-index owners listing i
-__global__ void k_crd(const int* __restrict__ off2, const int* __restrict__ roff2, int natms,
-                      int* __restrict__ crd) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= natms) return;
-    crd[i] = (off2[i + 1] - off2[i]) + (roff2[i + 1] - roff2[i]);
+    if (!FILL && lane == 0) {
+        cnt_or_off[i] = w;
+        tot_or_off[i] = f;
+        crd[i] = f;
+    }
 }
 
 // Atoms::update_0 skin test: any owned site moved more than skin since the build

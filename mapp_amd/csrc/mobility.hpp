@@ -33,21 +33,6 @@
 
 namespace mappdmd {
 
-struct RevBufs {
-    const int* off;    // half list (or 2nd list) CSR
-    const int* nl;
-    const int* roff;   // reverse CSR over owned partners
-    const int* rev;    // pair index
-    const int* pair_i; // owner row of each pair
-};
-
-// pair_i[p] = i for p in the row of i
-__global__ void k_pair_owner(const int* __restrict__ off, int natms, int* __restrict__ pair_i) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= natms) return;
-    for (int p = off[i]; p < off[i + 1]; ++p) pair_i[p] = i;
-}
-
 // ---------------------------------------------------------------- site table
 constexpr int kTableG = 16;  // lanes per site over the pair table
 constexpr int kList2G = 4;   // lanes per site over the 2nd list
@@ -81,9 +66,9 @@ __device__ __forceinline__ int group_rank16(bool flag, int l, int* total) {
 }
 
 // Entries per site: the pairs inside the quadrature cut of the own row (own[i]) and of
-// the reverse list, and for each pair its rank among the partner's reverse entries
-// inside the cut (16 lanes per site, strided over both ranges).
-__global__ __launch_bounds__(kBlock) void k_table_count(RevBufs L, const int* __restrict__ rowner, int natms,
+// the reverse list, and for each reverse entry its rank among those inside the cut
+// (16 lanes per site, strided over both ranges).
+__global__ __launch_bounds__(kBlock) void k_table_count(PairBufs L, const int* __restrict__ rowner, int natms,
                                                         const double4* __restrict__ pos, double cut_sq,
                                                         int* __restrict__ own, int* __restrict__ cnt,
                                                         int* __restrict__ rrank) {
@@ -92,14 +77,15 @@ __global__ __launch_bounds__(kBlock) void k_table_count(RevBufs L, const int* __
     if (i >= natms) return;
     const double4 xi = pos[i];
     int c = 0, r = 0;
-    for (int p = L.off[i] + g.l; p < L.off[i + 1]; p += kTableG) c += pair_rsq(xi, pos[L.nl[p]]) < cut_sq ? 1 : 0;
+    for (int p = L.off[i] + g.l; p < L.off[i + 1]; p += kTableG)
+        c += pair_rsq(xi, pos[list_partner(L.nlrp[p])]) < cut_sq ? 1 : 0;
     const int q1 = L.roff[i + 1];
     for (int b = L.roff[i]; b < q1; b += kTableG) {
         const int q = b + g.l;
         const bool in = q < q1 && pair_rsq(xi, pos[rowner[q < q1 ? q : b] & ~kInsideBit]) < cut_sq;
         int tot;
         const int rk = group_rank16(in, g.l, &tot);
-        if (in) rrank[L.rev[q]] = r + rk;
+        if (in) rrank[q] = r + rk;
         r += tot;
     }
     const double sc = group_sum<kTableG>((double)c);
@@ -138,7 +124,7 @@ template <int NT, typename Q, int NQ>
 __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFParams<Q> PQ,
                                                          const double4* __restrict__ pos,
                                                          const double* __restrict__ alpha,
-                                                         const int* __restrict__ off, const int* __restrict__ nl,
+                                                         const int* __restrict__ off, const int2* __restrict__ nlrp,
                                                          const Q* __restrict__ quad, const double* __restrict__ rho7,
                                                          const double* __restrict__ phi7,
                                                          const int* __restrict__ toff, const int* __restrict__ own,
@@ -177,10 +163,12 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
             {
                 const int pc = chunk + lane;
                 bool in = false;
-                int jc = 0;
+                int jc = 0, qc = -1;
                 double r2 = 1.0;
                 if (pc < p1) {
-                    jc = nl[pc];
+                    const int2 e = nlrp[pc];
+                    jc = e.x & ~kInsideBit;
+                    qc = e.y;
                     r2 = pair_rsq(xi, pos[jc]);
                     in = r2 < P.cut_sq_mod;
                 }
@@ -189,7 +177,7 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
                     double a[NT];
 #pragma unroll
                     for (int t = 0; t < NT; ++t) a[t] = alpha[(size_t)jc * NT + t];
-                    const int there = jc < P.natms ? toff[jc] + own[jc] + rrank[pc] : -1;
+                    const int there = qc >= 0 ? toff[jc] + own[jc] + rrank[qc] : -1;
                     tidx[at + dest] = jc;
                     if (there >= 0) tidx[there] = i;
                     st.geo[dest] = make_double2(r2, rsqrt_nr(r2));
@@ -257,21 +245,6 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
         }
     }
 }
-
-// 2nd list of both ends: own rows as partner j, reverse entries as ~owner
-__global__ void k_list2_count(RevBufs L2, int natms, int* __restrict__ cnt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= natms) return;
-    cnt[i] = (L2.off[i + 1] - L2.off[i]) + (L2.roff[i + 1] - L2.roff[i]);
-}
-__global__ void k_list2_fill(RevBufs L2, int natms, const int* __restrict__ foff, int* __restrict__ fidx) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= natms) return;
-    int e = foff[i];
-    for (int p = L2.off[i]; p < L2.off[i + 1]; ++p) fidx[e++] = L2.nl[p];
-    for (int q = L2.roff[i]; q < L2.roff[i + 1]; ++q) fidx[e++] = ~L2.pair_i[L2.rev[q]];
-}
-
 
 // E = sum c rho_bar; n = E = F(E), dE = F', ddE = F''
 // (first sweep of c_d_calc, src/ff_dmd_I.cpp:2269-2312, and calc_g, :2447-2493).
