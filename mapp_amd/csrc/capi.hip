@@ -361,7 +361,7 @@ void finish_lists(mapp_dmd* ctx) {
     ctx->d_fown.reserve((size_t)natms * (3 + NT));
     ctx->d_pairE.reserve((size_t)(nrev + 1) * NT);
     if (is_md(ctx)) {
-        ctx->d_pairF.reserve((size_t)(nrev + 1) * 3);
+        ctx->d_pairF.reserve(nrev + 1);
     } else {
         // pass 1's records in either quadrature type
         using R = PairRec<NT, double>;
@@ -465,25 +465,16 @@ PairBufs pair_bufs(mapp_dmd* ctx) { return PairBufs{ctx->d_off.p, ctx->d_nlrp.p,
 
 // ------------------------------------------------------------------ MD-mode potentials
 template <int MODEL>
-void md_passes(mapp_dmd* ctx, bool energy_only, int nb, const PairBufs& L, const EamBufs& T, double2* drho,
+void md_passes(mapp_dmd* ctx, bool energy_only, int nb, const PairBufs& L, const EamBufs& T, const EamPairs& O,
                double* part1, double* part2) {
     hipStream_t st = ctx->stream;
-    if (energy_only)
-        hipLaunchKernelGGL((k_eam_pass1<MODEL, true>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md, ctx->d_pos.p,
-                           ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_fown.p, ctx->d_pairE.p,
-                           ctx->d_pairF.p, drho, part1);
-    else
-        hipLaunchKernelGGL((k_eam_pass1<MODEL, false>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md,
-                           ctx->d_pos.p, ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_fown.p,
-                           ctx->d_pairE.p, ctx->d_pairF.p, drho, part1);
+    hipLaunchKernelGGL((energy_only ? k_eam_pass1<MODEL, true> : k_eam_pass1<MODEL, false>), dim3(nb), dim3(kBlock), 0,
+                       st, ctx->P, T, ctx->md, ctx->d_arec.p, L, O, ctx->d_Eown.p, ctx->d_fown.p, part1);
     launch_check("k_eam_pass1");
     if constexpr (MODEL != kModelLj) {
-        if (energy_only)
-            hipLaunchKernelGGL((k_eam_embed<MODEL, true>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md,
-                               ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_E.p, ctx->d_dE.p, part2);
-        else
-            hipLaunchKernelGGL((k_eam_embed<MODEL, false>), dim3(nb), dim3(kBlock), 0, st, ctx->P, T, ctx->md,
-                               ctx->d_conc.p, L, ctx->d_Eown.p, ctx->d_pairE.p, ctx->d_E.p, ctx->d_dE.p, part2);
+        hipLaunchKernelGGL((energy_only ? k_eam_embed<MODEL, true> : k_eam_embed<MODEL, false>), dim3(nb),
+                           dim3(kBlock), 0, st, ctx->P, T, ctx->md, ctx->d_conc.p, L, ctx->d_Eown.p, O.rho,
+                           ctx->d_E.p, ctx->d_dE.p, ctx->d_arec.p, part2);
         launch_check("k_eam_embed");
     }
 }
@@ -495,37 +486,47 @@ double run_eam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     hipStream_t st = ctx->stream;
     const int natms = ctx->natms, nb = nblk((long)natms * kEamG);  // 16-lane site groups
     const PairBufs L = pair_bufs(ctx);
-    EamBufs T{ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_F7.p, ctx->nt};
+    const bool lj = ctx->variant == MAPP_DMD_VARIANT_LJ;
+    const EamBufs T{ctx->d_eam_rows.p, ctx->d_F7.p, ctx->nt};
+    const size_t np = (size_t)ctx->npairs + 1;
     ctx->d_part.reserve((size_t)nb * 14 + 16);
-    ctx->d_drho.reserve(2 * ((size_t)ctx->npairs + 1));  // one double2 per pair
-    ctx->d_pairF2.reserve((size_t)(ctx->nrev + 1) * 3);
+    if (!lj && !energy_only) ctx->d_drho.reserve(3 * np);
+    const int ntot = natms + ctx->nghost;
+    ctx->d_arec.reserve(ntot);
+    double* const dr = ctx->d_drho.p;
+    const EamPairs O{dr, dr + np, dr + 2 * np, ctx->d_pairE.p, ctx->d_pairF.p};
     double* part1 = ctx->d_part.p;
     double* part2 = part1 + (size_t)nb * 7;
     double* part3 = part2 + (size_t)nb;
-    double2* drho = reinterpret_cast<double2*>(ctx->d_drho.p);
-    const bool lj = ctx->variant == MAPP_DMD_VARIANT_LJ;
-    if (ctx->variant == MAPP_DMD_VARIANT_EAM) md_passes<kModelEam>(ctx, energy_only, nb, L, T, drho, part1, part2);
-    else if (lj) md_passes<kModelLj>(ctx, energy_only, nb, L, T, drho, part1, part2);
-    else if (ctx->variant == MAPP_DMD_VARIANT_FS) md_passes<kModelFs>(ctx, energy_only, nb, L, T, drho, part1, part2);
-    else md_passes<kModelFsm>(ctx, energy_only, nb, L, T, drho, part1, part2);
+    hipLaunchKernelGGL(k_eam_pack, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_pos.p, ctx->d_conc.p, ntot,
+                       ctx->d_arec.p);
+    launch_check("k_eam_pack");
+    if (ctx->variant == MAPP_DMD_VARIANT_EAM) md_passes<kModelEam>(ctx, energy_only, nb, L, T, O, part1, part2);
+    else if (lj) md_passes<kModelLj>(ctx, energy_only, nb, L, T, O, part1, part2);
+    else if (ctx->variant == MAPP_DMD_VARIANT_FS) md_passes<kModelFs>(ctx, energy_only, nb, L, T, O, part1, part2);
+    else md_passes<kModelFsm>(ctx, energy_only, nb, L, T, O, part1, part2);
     if (!energy_only) {
         if (!lj) {
-            ghost_copy(ctx, ctx->d_dE.p, 1);
-            hipLaunchKernelGGL(k_eam_pass2, dim3(nb), dim3(kBlock), 0, st, ctx->P, ctx->d_pos.p, L,
-                               drho, ctx->d_dE.p, ctx->d_fown.p, ctx->d_pairF2.p, part3);
+            if (ctx->nghost > 0) {
+                hipLaunchKernelGGL(k_eam_ghost_dF, dim3(nblk(ctx->nghost)), dim3(kBlock), 0, st, ctx->d_arec.p, natms,
+                                   ctx->nghost, ctx->d_ghost_owner.p);
+                launch_check("k_eam_ghost_dF");
+            }
+            hipLaunchKernelGGL(k_eam_pass2, dim3(nb), dim3(kBlock), 0, st, ctx->P, ctx->d_arec.p, L, O, ctx->d_fown.p,
+                               part3);
             launch_check("k_eam_pass2");
         }
-        hipLaunchKernelGGL(k_eam_gather, dim3(nb), dim3(kBlock), 0, st, natms, L, ctx->d_fown.p, ctx->d_pairF.p,
-                           lj ? (const double*)nullptr : ctx->d_pairF2.p, ctx->d_f.p);
+        hipLaunchKernelGGL(k_eam_gather, dim3(nb), dim3(kBlock), 0, st, natms, L, ctx->d_rowner.p, ctx->d_arec.p, O.S,
+                           ctx->d_fown.p, ctx->d_f.p);
         launch_check("k_eam_gather");
     }
-    // pass 1's energy and virial, the embedding energy, pass 2's virial (LJ has only the first)
+    // pass 1's energy (LJ: and virial, the rest is zero), the embedding energy, pass 2's virial
     double* h = ctx->h_box;
     for (int k = 0; k < 14; ++k) h[k] = 0.0;
     {
         const double* parts[3] = {part1, part2, part3};
         const long nparts[3] = {nb, nb, nb};
-        const int nv[3] = {7, 1, 6}, off[3] = {0, 7, 8};
+        const int nv[3] = {lj && !energy_only ? 7 : 1, 1, 6}, off[3] = {0, 7, 8};
         reduce_partials_segs(ctx, lj ? 1 : (energy_only ? 2 : 3), parts, nparts, nv, nv, off, h);
     }
     wait_box(ctx);
@@ -820,6 +821,20 @@ void upload_tables(mapp_dmd* ctx) {
     HIP_OK(hipMemcpy(ctx->d_rho7.p, ctx->rho7.data(), ctx->rho7.size() * sizeof(double), hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(ctx->d_phi7.p, ctx->phi7.data(), ctx->phi7.size() * sizeof(double), hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(ctx->d_F9.p, ctx->F9.data(), ctx->F9.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (ctx->variant == MAPP_DMD_VARIANT_EAM) {
+        std::vector<double> rows((size_t)nr * nt * nt * kEamRow, 0.0);
+        for (int m = 0; m < nr; ++m)
+            for (int it = 0; it < nt; ++it)
+                for (int jt = 0; jt < nt; ++jt)
+                    for (int k = 0; k < 4; ++k) {
+                        double* d = rows.data() + ((size_t)m * nt * nt + it * nt + jt) * kEamRow + k;
+                        d[0] = ctx->rho7[((size_t)type2rho(nt, jt, it) * nr + m) * 7 + k];
+                        d[4] = ctx->rho7[((size_t)type2rho(nt, it, jt) * nr + m) * 7 + k];
+                        d[8] = ctx->phi7[((size_t)type2phi(it, jt) * nr + m) * 7 + k];
+                    }
+        ctx->d_eam_rows.reserve(rows.size());
+        HIP_OK(hipMemcpy(ctx->d_eam_rows.p, rows.data(), rows.size() * sizeof(double), hipMemcpyHostToDevice));
+    }
     ctx->d_F7.reserve(ctx->F7.size());
     HIP_OK(hipMemcpy(ctx->d_F7.p, ctx->F7.data(), ctx->F7.size() * sizeof(double), hipMemcpyHostToDevice));
 }

@@ -42,7 +42,7 @@ struct mapp_dmd {
     std::vector<int> swap_off, swap_dim, swap_dir;
 
     // device tables
-    mappdmd::DevBuf<double> d_quad64, d_rho7, d_phi7, d_F9, d_F7, d_drho, d_pairF2;
+    mappdmd::DevBuf<double> d_quad64, d_rho7, d_phi7, d_F9, d_F7, d_eam_rows, d_drho;
     mappdmd::DevBuf<float> d_quad32;
     // device atoms (owned rows first, ghosts after)
     mappdmd::DevBuf<double4> d_pos, d_x0;
@@ -57,7 +57,7 @@ struct mapp_dmd {
     mappdmd::DevBuf<int> d_rtmp;  // owners of the reverse lists before they are sorted
     mappdmd::DevBuf<double2> d_deriv;  // pass 1's records (PairRec) of the quadrature type
     mappdmd::DevBuf<int2> d_info;      // [natms] {list offset, pairs inside the cut at the last force pass 1}
-    mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}
+    mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}; MD potentials [ntot] {x, y, z, type, then F'}
     long nrev = 0;
     long npairs = 0, npairs2 = 0;
     bool have_list2 = false;
@@ -65,7 +65,7 @@ struct mapp_dmd {
     mappdmd::DevBuf<double> d_E, d_dE, d_ddE, d_n, d_s, d_t, d_v, d_cd, d_fa, d_Eown, d_a, d_g;
     mappdmd::DevBuf<double> d_f, d_fown;        // [natms][3+nt]
     // partner shares in reverse-list order: densities [nrev][nt]; forces, DMD
-    // [nrev][ForceShare<nt>::kLen], MD potentials [nrev][3]
+    // [nrev][ForceShare<nt>::kLen], MD potentials [nrev]
     mappdmd::DevBuf<double> d_pairE, d_pairF;
     // DMD: per half-list entry {partner, reverse position} and per reverse-list entry the
     // pair's owner; the top bit of the first: inside the quadrature cut at the last pass 1

@@ -19,11 +19,15 @@
 namespace mappdmd {
 
 struct EamBufs {
-    const double* rho7;  // [nt*nt][nr][7]
-    const double* phi7;  // [nphi][nr][7]
+    const double* rows;  // [nr][nt*nt][kEamRow]: per row and ordered type pair (i, j) the cubic
+                         // coefficients of j's density at i, i's density at j and r phi
     const double* F7;    // [nt][nrho+1][7]
     int nt;
 };
+// A pair reads 96 consecutive bytes of one 128-byte line; from the three tables of 7
+// coefficients it read 168 bytes of three or more (the derivative's coefficients are
+// those of the value times 1, 2, 3 and 1/dr).
+constexpr int kEamRow = 16;
 
 // FSM is FS with the cutoff tests on squares (rsq < cut^2, src/ff_fsm.cpp:424,
 // :463, :518); its one-sweep density force (:466-476) is the same sum as FS's
@@ -33,48 +37,74 @@ enum { kModelEam = 0, kModelLj = 1, kModelFs = 2, kModelFsm = 3 };
 // 16 lanes (one DPP row) per site in every pass: each lane takes every 16th
 // list entry, the group sums per-site values in a fixed tree
 constexpr int kEamG = 16;
+// rounds of a list whose loads are issued together, before the first of their stores
+// (a load waits for the stores issued before it)
+constexpr int kEamR = 3;
 
-__device__ __forceinline__ void eam_row(const FFParams<double>& P, double r, int* m_out, double* p_out) {
-    double p = r * P.dr_inv;
-    int m = (int)p;
-    m = m < P.nr - 2 ? m : P.nr - 2;
-    p -= m;
-    p = p < 1.0 ? p : 1.0;
-    *m_out = m;
-    *p_out = p;
+// {x, y, z, type} per site: a pair's partner comes with one 32-byte read
+__global__ void k_eam_pack(const double4* __restrict__ pos, const double* __restrict__ type, int n,
+                           double4* __restrict__ rec) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double4 p = pos[i];
+    p.w = type[i];
+    rec[i] = p;
+}
+// dF of the ghosts into rec[].w (pass 2 needs no types)
+__global__ void k_eam_ghost_dF(double4* __restrict__ rec, int natms, int nghost, const int* __restrict__ owner) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g < nghost) rec[natms + g].w = rec[owner[g]].w;
 }
 
-__device__ __forceinline__ double h3(const double* c, double p) { return ((c[3] * p + c[2]) * p + c[1]) * p + c[0]; }
-__device__ __forceinline__ double h2d(const double* c, double p) { return (c[6] * p + c[5]) * p + c[4]; }
+// the row of a pair at distance^2 rsq (any value: the last row beyond the table)
+struct EamLine {
+    double c[12], r_inv, p;
+    __device__ __forceinline__ void load(const FFParams<double>& P, const EamBufs& T, int it, int jt, double rsq) {
+        r_inv = rsqrt_nr(rsq);
+        p = rsq * r_inv * P.dr_inv;
+        int m = (int)p;
+        m = m < P.nr - 2 ? m : P.nr - 2;
+        m = m > 0 ? m : 0;
+        p -= m;
+        p = p < 1.0 ? p : 1.0;
+        const double2* row =
+            reinterpret_cast<const double2*>(T.rows + ((size_t)m * (T.nt * T.nt) + it * T.nt + jt) * kEamRow);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const double2 v = row[k];
+            c[2 * k] = v.x;
+            c[2 * k + 1] = v.y;
+        }
+    }
+    __device__ __forceinline__ double value(int f) const {
+        return ((c[4 * f + 3] * p + c[4 * f + 2]) * p + c[4 * f + 1]) * p + c[4 * f];
+    }
+    __device__ __forceinline__ double slope(int f, double dr_inv) const {
+        return ((3.0 * c[4 * f + 3] * p + 2.0 * c[4 * f + 2]) * p + c[4 * f + 1]) * dr_inv;
+    }
+};
 
 // one pair (i of type it, j of type jt at distance^2 rsq) of a model:
 // density shares rho_i (at i) and rho_j (at j), pair energy, pair force
 // coefficient fpair (force on i = fpair * dx) and the density records
 // {drho_i, drho_j} of pass 2; returns false when the pair contributes nothing
 template <int MODEL, bool ENERGY_ONLY>
-__device__ __forceinline__ bool md_pair(const FFParams<double>& P, const EamBufs& T, const MdParams& M, int it,
+__device__ __forceinline__ bool md_pair(const EamLine& row,
+                                        const FFParams<double>& P, const EamBufs& T, const MdParams& M, int it,
                                         int jt, double rsq, double* rho_i, double* rho_j, double* phi,
                                         double* fpair, double2* dr) {
     *rho_i = *rho_j = *phi = *fpair = 0.0;
     *dr = make_double2(0.0, 0.0);
     if constexpr (MODEL == kModelEam) {
         if (!(rsq < P.cut_sq)) return false;
-        const int nt = T.nt;
-        const double r = sqrt(rsq), r_inv = 1.0 / r;
-        int m;
-        double pp;
-        eam_row(P, r, &m, &pp);
-        const double* ci = T.rho7 + ((size_t)type2rho(nt, jt, it) * P.nr + m) * 7;
-        const double* cj = T.rho7 + ((size_t)type2rho(nt, it, jt) * P.nr + m) * 7;
-        const double* cp = T.phi7 + ((size_t)type2phi(it, jt) * P.nr + m) * 7;
-        *rho_i = h3(ci, pp);
-        *rho_j = h3(cj, pp);
-        const double z2 = h3(cp, pp), z2p = h2d(cp, pp);
-        *phi = ENERGY_ONLY ? z2 / r : z2 * r_inv;
+        const double r_inv = row.r_inv;
+        *rho_i = row.value(0);
+        *rho_j = row.value(1);
+        *phi = row.value(2) * r_inv;
         if (!ENERGY_ONLY) {
-            const double dphi_dr = z2p * r_inv - *phi * r_inv;
+            const double dphi_dr = row.slope(2, P.dr_inv) * r_inv - *phi * r_inv;
             *fpair = -dphi_dr * r_inv;
-            *dr = make_double2(-h2d(ci, pp) * r_inv, -h2d(cj, pp) * r_inv);
+            *dr = make_double2(-row.slope(0, P.dr_inv) * r_inv, -row.slope(1, P.dr_inv) * r_inv);
         }
         return true;
     } else if constexpr (MODEL == kModelLj) {
@@ -116,80 +146,125 @@ __device__ __forceinline__ bool md_pair(const FFParams<double>& P, const EamBufs
 }
 
 
-// pass 1: own density and pair forces; partner shares {rho_j, -fpair dx} to pair
-// buffers; per-pair density records for pass 2
+// Sums and records of a pair list go through three passes.  The force on i from a pair
+// is S (x_i - x_j), S = fpair + F'_i drho_i + F'_j drho_j: pass 1 keeps fpair, drho_i and
+// drho_j per pair (component by component, so that a round stores whole lines) and gives
+// the partner its density share; pass 2 forms S, the own force and the virial, and
+// leaves S at the pair's place in the partner's reverse list; the gather adds S
+// (x_owner - x_i) over that list.  The first version summed pair and embedding forces
+// separately, with a 24-byte share to the partner from each pass.  LJ has no densities:
+// pass 1 does the work of pass 2.
+struct EamPairs {
+    double *f, *di, *dj;  // per pair: fpair, drho_i, drho_j
+    double *rho, *S;      // per reverse-list entry: the partner's density share; S
+};
+
+// the pair's part of the force and the virial
+struct ForceSums {
+    double f[3] = {0.0, 0.0, 0.0}, v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    __device__ __forceinline__ void add(double S, double w, double dx0, double dx1, double dx2) {
+        const double s0 = S * dx0, s1 = S * dx1, s2 = S * dx2;
+        f[0] += s0;
+        f[1] += s1;
+        f[2] += s2;
+        v[0] -= w * s0 * dx0;
+        v[1] -= w * s1 * dx1;
+        v[2] -= w * s2 * dx2;
+        v[3] -= w * s1 * dx2;
+        v[4] -= w * s2 * dx0;
+        v[5] -= w * s0 * dx1;
+    }
+    // sums of the group, stored by its first lane
+    __device__ __forceinline__ void store(int l, double* fown) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double a = group_sum<kEamG>(f[k]);
+            if (l == 0) fown[k] = a;
+        }
+    }
+};
+
+// Pass 1 is bound by the gathers of positions and table rows (L2).  At 1,048,576 sites
+// of two EAM types (41 million list entries): 0.74 ms, pass 2 0.41 and the gather 0.18;
+// with rows of 7 coefficients, one entry at a time and both shares as vectors they took
+// 1.27, 0.65 and 0.28.  kEamR = 2 gives 0.76, 0.45, 0.21; 4 gives 0.77, 0.46, 0.20.
 template <int MODEL, bool ENERGY_ONLY>
 __global__ __launch_bounds__(kBlock) void k_eam_pass1(FFParams<double> P, EamBufs T, MdParams M,
-                                                      const double4* __restrict__ pos,
-                                                      const double* __restrict__ type, PairBufs L,
-                                                      double* __restrict__ rho_own,
-                                                      double* __restrict__ fown, double* __restrict__ pairE,
-                                                      double* __restrict__ pairF, double2* __restrict__ drho,
+                                                      const double4* __restrict__ rec, PairBufs L, EamPairs O,
+                                                      double* __restrict__ rho_own, double* __restrict__ fown,
                                                       double* __restrict__ part) {
+    constexpr bool kForce = MODEL == kModelLj && !ENERGY_ONLY;
     const SiteGroup<kEamG> g;
     const int i = g.site;
-    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+    double acc[kForce ? 7 : 1] = {};
     if (i < P.natms) {
-        const int it = (int)type[i];
-        const double4 xi = pos[i];
-        double rho = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+        const double4 xi = rec[i];
+        const int it = (int)xi.w;
+        double rho = 0.0;
+        ForceSums F;
         const int p1 = L.off[i + 1];
-        for (int p = L.off[i] + g.l; p < p1; p += kEamG) {
-            const int2 e = L.nlrp[p];
-            const int j = e.x;
-            const double4 xj = pos[j];
-            const double dx0 = xi.x - xj.x, dx1 = xi.y - xj.y, dx2 = xi.z - xj.z;
-            double rsq;
-            {
-#pragma clang fp contract(off)
-                rsq = dx0 * dx0 + dx1 * dx1 + dx2 * dx2;
+        for (int p0 = L.off[i] + g.l; p0 < p1; p0 += kEamG * kEamR) {
+            int2 e[kEamR];
+            double dx0[kEamR], dx1[kEamR], dx2[kEamR], rsq[kEamR], rho_j[kEamR], pf[kEamR];
+            double2 dr[kEamR];
+            int jt[kEamR];
+            EamLine row[kEamR];
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) {
+                const int p = p0 + r * kEamG;
+                e[r] = L.nlrp[p < p1 ? p : p1 - 1];
             }
-            const bool owned = j < P.natms;
-            double rho_i, rho_j, phi, pf;
-            double2 dr;
-            if (md_pair<MODEL, ENERGY_ONLY>(P, T, M, it, (int)type[j], rsq, &rho_i, &rho_j, &phi, &pf, &dr)) {
-                rho += rho_i;
-                acc[0] += owned ? phi : 0.5 * phi;
-                if (!ENERGY_ONLY) {
-                    fx += pf * dx0;
-                    fy += pf * dx1;
-                    fz += pf * dx2;
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) {
+                const double4 xj = rec[e[r].x];
+                dx0[r] = xi.x - xj.x;
+                dx1[r] = xi.y - xj.y;
+                dx2[r] = xi.z - xj.z;
+                jt[r] = (int)xj.w;
+                {
+#pragma clang fp contract(off)
+                    rsq[r] = dx0[r] * dx0[r] + dx1[r] * dx1[r] + dx2[r] * dx2[r];
+                }
+                if constexpr (MODEL == kModelEam) row[r].load(P, T, it, jt[r], rsq[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) {
+                const bool listed = p0 + r * kEamG < p1, owned = e[r].y >= 0;
+                double rho_i, phi;
+                rho_j[r] = pf[r] = 0.0;
+                dr[r] = make_double2(0.0, 0.0);
+                if (listed && md_pair<MODEL, ENERGY_ONLY>(row[r], P, T, M, it, jt[r], rsq[r], &rho_i, &rho_j[r], &phi,
+                                                          &pf[r], &dr[r])) {
                     const double w = owned ? 1.0 : 0.5;
-                    acc[1] -= w * pf * dx0 * dx0;
-                    acc[2] -= w * pf * dx1 * dx1;
-                    acc[3] -= w * pf * dx2 * dx2;
-                    acc[4] -= w * pf * dx1 * dx2;
-                    acc[5] -= w * pf * dx2 * dx0;
-                    acc[6] -= w * pf * dx0 * dx1;
+                    rho += rho_i;
+                    acc[0] += w * phi;
+                    if constexpr (kForce) F.add(pf[r], w, dx0[r], dx1[r], dx2[r]);
                 }
             }
-            if (!ENERGY_ONLY && MODEL != kModelLj) drho[p] = dr;
-            if (owned) {
-                const size_t q = (size_t)e.y;
-                if (MODEL != kModelLj) pairE[q] = rho_j;
-                if (!ENERGY_ONLY) {
-                    pairF[q * 3 + 0] = -pf * dx0;
-                    pairF[q * 3 + 1] = -pf * dx1;
-                    pairF[q * 3 + 2] = -pf * dx2;
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) {
+                const int p = p0 + r * kEamG;
+                if (p >= p1) continue;
+                if (!ENERGY_ONLY && MODEL != kModelLj) {
+                    O.f[p] = pf[r];
+                    O.di[p] = dr[r].x;
+                    O.dj[p] = dr[r].y;
+                }
+                if (e[r].y >= 0) {
+                    if (MODEL != kModelLj) O.rho[e[r].y] = rho_j[r];
+                    if (kForce) O.S[e[r].y] = pf[r];
                 }
             }
         }
         rho = group_sum<kEamG>(rho);
-        if (!ENERGY_ONLY) {
-            fx = group_sum<kEamG>(fx);
-            fy = group_sum<kEamG>(fy);
-            fz = group_sum<kEamG>(fz);
-        }
-        if (g.l == 0) {
-            rho_own[i] = rho;
-            if (!ENERGY_ONLY) {
-                fown[(size_t)i * 3 + 0] = fx;
-                fown[(size_t)i * 3 + 1] = fy;
-                fown[(size_t)i * 3 + 2] = fz;
-            }
+        if (g.l == 0) rho_own[i] = rho;
+        if constexpr (kForce) {
+            F.store(g.l, fown + (size_t)i * 3);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) acc[1 + k] = F.v[k];
         }
     }
-    block_sum_store<7>(acc, part);
+    block_sum_store<kForce ? 7 : 1>(acc, part);
 }
 
 // rho_i = own + partner shares; EAM: F(rho) (cubic rows, linear above
@@ -200,14 +275,21 @@ __global__ __launch_bounds__(kBlock) void k_eam_embed(FFParams<double> P, EamBuf
                                                       const double* __restrict__ type, PairBufs L,
                                                       const double* __restrict__ rho_own,
                                                       const double* __restrict__ pairE, double* __restrict__ rho,
-                                                      double* __restrict__ dF, double* __restrict__ part) {
+                                                      double* __restrict__ dF, double4* __restrict__ rec,
+                                                      double* __restrict__ part) {
     const SiteGroup<kEamG> g;
     const int i = g.site;
     double acc[1] = {0.0};
     if (i < P.natms) {
         double part_r = 0.0;
         const int q1 = L.roff[i + 1];
-        for (int q = L.roff[i] + g.l; q < q1; q += kEamG) part_r += pairE[q];
+        for (int q0 = L.roff[i] + g.l; q0 < q1; q0 += kEamG * kEamR) {
+            double v[kEamR];
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) v[r] = q0 + r * kEamG < q1 ? pairE[q0 + r * kEamG] : 0.0;
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) part_r += v[r];
+        }
         double r = rho_own[i] + group_sum<kEamG>(part_r);
         const int it = (int)type[i];
         if (g.l != 0) {
@@ -216,7 +298,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_embed(FFParams<double> P, EamBuf
             const double sq = sqrt(r);
             acc[0] = -(M.A[it] * sq);
             rho[i] = r;
-            if (!ENERGY_ONLY) dF[i] = -M.A[it] / sq;
+            if (!ENERGY_ONLY) dF[i] = rec[i].w = -M.A[it] / sq;
         } else {
             double pp = r * P.drho_inv;
             int m = (int)pp;
@@ -225,98 +307,92 @@ __global__ __launch_bounds__(kBlock) void k_eam_embed(FFParams<double> P, EamBuf
             pp -= m;
             pp = pp < 1.0 ? pp : 1.0;
             const double* c = T.F7 + ((size_t)it * (P.nrho + 1) + m) * 7;
-            const double d = h2d(c, pp);
-            double Fv = h3(c, pp);
+            const double d = (c[6] * pp + c[5]) * pp + c[4];
+            double Fv = ((c[3] * pp + c[2]) * pp + c[1]) * pp + c[0];
             if (r > P.rho_max) Fv += d * (r - P.rho_max);
             acc[0] = Fv;
             rho[i] = r;
-            if (!ENERGY_ONLY) dF[i] = d;
+            if (!ENERGY_ONLY) dF[i] = rec[i].w = d;
         }
     }
     block_sum_store<1>(acc, part);
 }
 
-// pass 2: embedding forces fpair = F'_i drho_i/dr + F'_j drho_j/dr
-__global__ __launch_bounds__(kBlock) void k_eam_pass2(FFParams<double> P, const double4* __restrict__ pos, PairBufs L,
-                                                      const double2* __restrict__ drho,
-                                                      const double* __restrict__ dF, double* __restrict__ fown,
-                                                      double* __restrict__ pairF2, double* __restrict__ part) {
+// rec = {x, y, z, F'}
+__global__ __launch_bounds__(kBlock) void k_eam_pass2(FFParams<double> P, const double4* __restrict__ rec, PairBufs L,
+                                                      EamPairs O, double* __restrict__ fown,
+                                                      double* __restrict__ part) {
     const SiteGroup<kEamG> g;
     const int i = g.site;
-    double acc[6] = {0, 0, 0, 0, 0, 0};
+    ForceSums F;
     if (i < P.natms) {
-        const double4 xi = pos[i];
-        const double dFi = dF[i];
-        double fx = 0.0, fy = 0.0, fz = 0.0;
+        const double4 xi = rec[i];
         const int p1 = L.off[i + 1];
-        for (int p = L.off[i] + g.l; p < p1; p += kEamG) {
-            const int2 e = L.nlrp[p];
-            const int j = e.x;
-            const double2 dr = drho[p];
-            const bool owned = j < P.natms;
-            double fpair = 0.0, dx0 = 0.0, dx1 = 0.0, dx2 = 0.0;
-            if (dr.x != 0.0 || dr.y != 0.0) {
-                const double4 xj = pos[j];
-                dx0 = xi.x - xj.x;
-                dx1 = xi.y - xj.y;
-                dx2 = xi.z - xj.z;
-                fpair = dFi * dr.x + dF[j] * dr.y;
-                fx += dx0 * fpair;
-                fy += dx1 * fpair;
-                fz += dx2 * fpair;
-                const double w = owned ? 1.0 : 0.5;
-                acc[0] -= w * fpair * dx0 * dx0;
-                acc[1] -= w * fpair * dx1 * dx1;
-                acc[2] -= w * fpair * dx2 * dx2;
-                acc[3] -= w * fpair * dx1 * dx2;
-                acc[4] -= w * fpair * dx2 * dx0;
-                acc[5] -= w * fpair * dx0 * dx1;
+        for (int p0 = L.off[i] + g.l; p0 < p1; p0 += kEamG * kEamR) {
+            int2 e[kEamR];
+            double S[kEamR], di[kEamR], dj[kEamR];
+            double4 xj[kEamR];
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) {
+                const int p = p0 + r * kEamG < p1 ? p0 + r * kEamG : p1 - 1;
+                e[r] = L.nlrp[p];
+                S[r] = O.f[p];
+                di[r] = O.di[p];
+                dj[r] = O.dj[p];
             }
-            if (owned) {
-                const size_t q = (size_t)e.y;
-                pairF2[q * 3 + 0] = -dx0 * fpair;
-                pairF2[q * 3 + 1] = -dx1 * fpair;
-                pairF2[q * 3 + 2] = -dx2 * fpair;
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) xj[r] = rec[e[r].x];
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r) {
+                // pairs outside the cutoff have zero records; F' of a site without density
+                // may be infinite (FS), and counts only where there is a slope
+                if (di[r] != 0.0 || dj[r] != 0.0) S[r] += xi.w * di[r] + xj[r].w * dj[r];
+                const bool on = p0 + r * kEamG < p1 && S[r] != 0.0;
+                if (on) F.add(S[r], e[r].y >= 0 ? 1.0 : 0.5, xi.x - xj[r].x, xi.y - xj[r].y, xi.z - xj[r].z);
             }
+#pragma unroll
+            for (int r = 0; r < kEamR; ++r)
+                if (p0 + r * kEamG < p1 && e[r].y >= 0) O.S[e[r].y] = S[r];
         }
-        fx = group_sum<kEamG>(fx);
-        fy = group_sum<kEamG>(fy);
-        fz = group_sum<kEamG>(fz);
-        if (g.l == 0) {
-            fown[(size_t)i * 3 + 0] += fx;
-            fown[(size_t)i * 3 + 1] += fy;
-            fown[(size_t)i * 3 + 2] += fz;
-        }
+        F.store(g.l, fown + (size_t)i * 3);
     }
-    block_sum_store<6>(acc, part);
+    block_sum_store<6>(F.v, part);
 }
 
-__global__ __launch_bounds__(kBlock) void k_eam_gather(int natms, PairBufs L, const double* __restrict__ fown,
-                                                       const double* __restrict__ pairF,
-                                                       const double* __restrict__ pairF2, double* __restrict__ f) {
+// f = own sum + the shares of the pairs that list the site
+__global__ __launch_bounds__(kBlock) void k_eam_gather(int natms, PairBufs L, const int* __restrict__ rowner,
+                                                       const double4* __restrict__ rec, const double* __restrict__ S,
+                                                       const double* __restrict__ fown, double* __restrict__ f) {
     const SiteGroup<kEamG> g;
     const int i = g.site;
     if (i >= natms) return;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+    const double4 xi = rec[i];
+    double a[3] = {0.0, 0.0, 0.0};
     const int q1 = L.roff[i + 1];
-    for (int q = L.roff[i] + g.l; q < q1; q += kEamG) {
-        if (pairF2) {
-            a0 += pairF[(size_t)q * 3] + pairF2[(size_t)q * 3];
-            a1 += pairF[(size_t)q * 3 + 1] + pairF2[(size_t)q * 3 + 1];
-            a2 += pairF[(size_t)q * 3 + 2] + pairF2[(size_t)q * 3 + 2];
-        } else {
-            a0 += pairF[(size_t)q * 3];
-            a1 += pairF[(size_t)q * 3 + 1];
-            a2 += pairF[(size_t)q * 3 + 2];
+    for (int q0 = L.roff[i] + g.l; q0 < q1; q0 += kEamG * kEamR) {
+        int o[kEamR];
+        double s[kEamR];
+        double4 xo[kEamR];
+#pragma unroll
+        for (int r = 0; r < kEamR; ++r) {
+            const int q = q0 + r * kEamG < q1 ? q0 + r * kEamG : q1 - 1;
+            o[r] = rowner[q];
+            s[r] = S[q];
+        }
+#pragma unroll
+        for (int r = 0; r < kEamR; ++r) xo[r] = rec[o[r]];
+#pragma unroll
+        for (int r = 0; r < kEamR; ++r) {
+            if (q0 + r * kEamG >= q1 || s[r] == 0.0) continue;
+            a[0] += s[r] * (xi.x - xo[r].x);
+            a[1] += s[r] * (xi.y - xo[r].y);
+            a[2] += s[r] * (xi.z - xo[r].z);
         }
     }
-    a0 = group_sum<kEamG>(a0);
-    a1 = group_sum<kEamG>(a1);
-    a2 = group_sum<kEamG>(a2);
-    if (g.l == 0) {
-        f[(size_t)i * 3] = fown[(size_t)i * 3] + a0;
-        f[(size_t)i * 3 + 1] = fown[(size_t)i * 3 + 1] + a1;
-        f[(size_t)i * 3 + 2] = fown[(size_t)i * 3 + 2] + a2;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double v = group_sum<kEamG>(a[k]);
+        if (g.l == 0) f[(size_t)i * 3 + k] = fown[(size_t)i * 3 + k] + v;
     }
 }
 
