@@ -563,42 +563,54 @@ void finish_meam(mapp_dmd* ctx) {
 double run_meam(mapp_dmd* ctx, bool energy_only, int st_clc, double* en_st) {
     hipStream_t st = ctx->stream;
     const int natms = ctx->natms;
-    const int nb = (natms + kMeamWaves - 1) / kMeamWaves;
+    const int nb = (natms + kMeamWaves - 1) / kMeamWaves, nbc = nblk(natms);
+    const int sites = meam_pair_sites(natms), nbp = (natms + kMeamWaves * sites - 1) / (kMeamWaves * sites);
     const MeamDev M = ctx->meam.device(ctx->meam_fix);
-    ctx->d_part.reserve((size_t)nb * 14 + 16);
-    double* part1 = ctx->d_part.p;
-    double* part2 = part1 + nb;
-    double* part3 = part2 + (size_t)nb * 7;
-    if (energy_only)
-        hipLaunchKernelGGL((k_meam_density<true>), dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p,
-                           ctx->d_off.p, ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p, ctx->d_mrec.p, part1);
-    else
-        hipLaunchKernelGGL((k_meam_density<false>), dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p,
-                           ctx->d_off.p, ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p, ctx->d_mrec.p, part1);
+    ctx->d_part.reserve((size_t)nbc + (size_t)nbp * 7 + (size_t)nb * 13 + 16);
+    double* part_c = ctx->d_part.p;  // embedding
+    double* part_e = part_c + nbc;   // pair energy (energy_calc)
+    double* part_p = part_e + nb;
+    double* part_t = part_p + (size_t)nbp * 7;
+    double* part_k = part_t + (size_t)nb * 6;
+    hipLaunchKernelGGL((energy_only ? k_meam_density<true> : k_meam_density<false>), dim3(nb), dim3(kBlock), 0, st, M,
+                       ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p, ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p,
+                       ctx->d_mrec.p, ctx->d_mactive.p, ctx->d_mact.p, part_e);
     launch_check("k_meam_density");
+    hipLaunchKernelGGL(k_meam_close, dim3(nbc), dim3(kBlock), 0, st, M, ctx->d_conc.p, natms, ctx->d_mrec.p, part_c);
+    launch_check("k_meam_close");
     if (!energy_only) {
         ghost_copy(ctx, ctx->d_mrec.p, kMeamRec);
-        hipLaunchKernelGGL(k_meam_force, dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p,
-                           ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p, ctx->d_mrec.p, ctx->d_f.p,
-                           ctx->d_mactive.p, ctx->d_mact.p, part2);
-        launch_check("k_meam_force");
+        ctx->d_mforce.reserve((size_t)ctx->npairs + 1);
+        hipLaunchKernelGGL(k_meam_pair, dim3(nbp), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p,
+                           ctx->d_nl.p, ctx->d_mtab.p, natms, ctx->d_mpairs.p, ctx->d_mrec.p, ctx->d_mactive.p,
+                           ctx->d_mact.p, ctx->d_mforce.p, part_p, sites);
+        launch_check("k_meam_pair");
+        hipLaunchKernelGGL(k_meam_three, dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p,
+                           ctx->d_nl.p, natms, ctx->d_mpairs.p, ctx->d_mforce.p, ctx->d_f.p, ctx->d_mactive.p,
+                           ctx->d_mact.p, part_t);
+        launch_check("k_meam_three");
         hipLaunchKernelGGL(k_meam_kforce, dim3(nb), dim3(kBlock), 0, st, M, ctx->d_pos.p, ctx->d_conc.p, ctx->d_off.p,
-                           ctx->d_nl.p, natms, ctx->d_mpairs.p, ctx->d_mactive.p, ctx->d_mact.p, ctx->d_f.p, part3);
+                           ctx->d_nl.p, natms, ctx->d_mpairs.p, ctx->d_mactive.p, ctx->d_mact.p, ctx->d_f.p, part_k);
         launch_check("k_meam_kforce");
     }
     const double* h = ctx->h_box;
-    {
-        const double* parts[3] = {part1, part2, part3};
-        const long nparts[3] = {nb, nb, nb};
-        const int nv[3] = {1, 7, 6}, off[3] = {0, 1, 8};
-        reduce_partials_segs(ctx, energy_only ? 1 : 3, parts, nparts, nv, nv, off, ctx->h_box);
+    if (energy_only) {
+        const double* parts[2] = {part_c, part_e};
+        const long nparts[2] = {nbc, nb};
+        const int nv[2] = {1, 1}, off[2] = {0, 1};
+        reduce_partials_segs(ctx, 2, parts, nparts, nv, nv, off, ctx->h_box);
+    } else {
+        const double* parts[4] = {part_c, part_p, part_t, part_k};
+        const long nparts[4] = {nbc, nbp, nb, nb};
+        const int nv[4] = {1, 7, 6, 6}, off[4] = {0, 1, 8, 14};
+        reduce_partials_segs(ctx, 4, parts, nparts, nv, nv, off, ctx->h_box);
     }
     wait_box(ctx);
-    const double energy = energy_only ? h[0] : h[0] + h[1];
+    const double energy = h[0] + h[1];
     if (en_st) {
         en_st[0] = energy;
         if (st_clc)
-            for (int k = 0; k < 6; ++k) en_st[1 + k] = h[2 + k] + h[8 + k];
+            for (int k = 0; k < 6; ++k) en_st[1 + k] = h[2 + k] + h[8 + k] + h[14 + k];
     }
     return energy;
 }

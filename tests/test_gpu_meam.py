@@ -147,3 +147,25 @@ def test_reader_setup_matches_coef(tmp_path):
     assert np.array_equal(a.get("f"), b.get("f"))
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("keep", [1, 2, 5, 17, 66])
+def test_few_sites(keep):
+    """a cluster in a wide box: sites without an entry, wavefronts of the pair kernel with a few entries or
+    none, block counts off a multiple; bar: a few hundred double roundings"""
+    from mapp_amd import workload as W
+    state = W.meam_state(["Aa", "Bb"], local=W.meam_local(2))
+    H, s, t = W.md_lattice(6, 3.58, "fcc", seed=7)
+    x = s[:, :3] * np.diag(H)
+    x -= x.mean(axis=0)
+    order = np.argsort(np.linalg.norm(x, axis=1), kind="stable")[:keep]
+    L = 40.0
+    _compare(*_pair(state, np.diag([L] * 3), np.ascontiguousarray(0.5 + 0.97 * x[order] / L), t[order]), f"few {keep}")
+
+
+@pytest.mark.parametrize("n", [9, 13])
+def test_sites_per_wavefront(n):
+    """the pair kernel's wavefronts with 2 and 8 sites each"""
+    from mapp_amd import workload as W
+    state = W.meam_state(["Aa", "Bb"], local=W.meam_local(2))
+    _compare(*_pair(state, *W.md_lattice(n, 3.58, "fcc", seed=n)), f"sites {n}")
