@@ -988,6 +988,7 @@ void run_c_d(mapp_dmd* ctx) {
     ensure_pair_cache(ctx);
     const int nbt = nblk((long)ctx->natms * kTableG), nb2 = nblk((long)ctx->natms * kList2G);
     const SiteTable T = site_table(ctx);
+    const Owner at{ctx->d_ghost_owner.p, ctx->natms};
     hipLaunchKernelGGL((k_density_table<NT>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, ctx->d_conc.p, T, ctx->d_F9.p,
                        ctx->d_E.p, ctx->d_n.p, ctx->d_dE.p, (double*)nullptr);
     launch_check("k_density_table");
@@ -996,8 +997,7 @@ void run_c_d(mapp_dmd* ctx) {
     hipLaunchKernelGGL((k_chem_pot<NT, CLOSE>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, ctx->d_alpha.p, ctx->d_conc.p,
                        T, ctx->d_dE.p, ctx->d_qidx.p, ctx->d_n.p);
     launch_check("k_chem_pot");
-    ghost_copy(ctx, ctx->d_n.p, NT);
-    hipLaunchKernelGGL((k_c_d<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, ctx->d_conc.p, ctx->d_foff2.p,
+    hipLaunchKernelGGL((k_c_d<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, at, ctx->d_conc.p, ctx->d_foff2.p,
                        ctx->d_fidx2.p, ctx->d_n.p, ctx->d_cd.p);
     launch_check("k_c_d");
     HIP_OK(hipStreamSynchronize(st));
@@ -1022,6 +1022,7 @@ double run_calc_g(mapp_dmd* ctx, int chk, double alpha_t, const double* a, doubl
     if (!fixed) ensure_pair_cache(ctx);
     const int nbt = nblk((long)ctx->natms * kTableG), nb2 = (int)calc_g_blocks(ctx);
     const SiteTable T = site_table(ctx);
+    const Owner at{ctx->d_ghost_owner.p, ctx->natms};
     hipLaunchKernelGGL((k_density_table<NT>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, ctx->d_conc.p, T, ctx->d_F9.p,
                        ctx->d_E.p, ctx->d_n.p, ctx->d_dE.p, ctx->d_ddE.p);
     launch_check("k_density_table g");
@@ -1030,7 +1031,6 @@ double run_calc_g(mapp_dmd* ctx, int chk, double alpha_t, const double* a, doubl
     hipLaunchKernelGGL((k_chem_pot<NT, CLOSE>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, ctx->d_alpha.p, ctx->d_conc.p,
                        T, ctx->d_dE.p, ctx->d_qidx.p, ctx->d_n.p);
     launch_check("k_chem_pot g");
-    ghost_copy(ctx, ctx->d_n.p, NT);
     GScratch S;
     if (fixed) {
         S = *fixed;
@@ -1039,7 +1039,7 @@ double run_calc_g(mapp_dmd* ctx, int chk, double alpha_t, const double* a, doubl
         ctx->d_stage.reserve((size_t)reduce_stage_doubles(nb2));
         S = GScratch{ctx->d_part.p, ctx->d_stage.p};
     }
-    hipLaunchKernelGGL((k_calc_g_s<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, alpha_t, ctx->d_conc.p, a,
+    hipLaunchKernelGGL((k_calc_g_s<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, at, alpha_t, ctx->d_conc.p, a,
                        ctx->d_foff2.p, ctx->d_fidx2.p, ctx->d_n.p, ctx->d_s.p, ctx->d_cd.p, S.part);
     launch_check("k_calc_g_s");
     {
@@ -1049,17 +1049,13 @@ double run_calc_g(mapp_dmd* ctx, int chk, double alpha_t, const double* a, doubl
         reduce_segs_in(ctx, 1, parts, nparts, &one, &one, &zero, S.stage, ctx->h_box);
     }
     if (!chk) {
-        ghost_copy(ctx, ctx->d_s.p, NT);
-        hipLaunchKernelGGL((k_calc_g_t<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, alpha_t, ctx->d_conc.p,
+        hipLaunchKernelGGL((k_calc_g_t<NT, VAR>), dim3(nb2), dim3(kBlock), 0, st, ctx->P, at, alpha_t, ctx->d_conc.p,
                            ctx->d_foff2.p, ctx->d_fidx2.p, ctx->d_n.p, ctx->d_s.p, ctx->d_t.p, g);
         launch_check("k_calc_g_t");
-        ghost_copy(ctx, ctx->d_t.p, NT);
-        hipLaunchKernelGGL((k_calc_g_v<NT>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, alpha_t, T, ctx->d_dE.p,
+        hipLaunchKernelGGL((k_calc_g_v<NT>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, at, alpha_t, T, ctx->d_dE.p,
                            ctx->d_t.p, ctx->d_v.p, g);
         launch_check("k_calc_g_v");
-        ghost_copy(ctx, ctx->d_v.p, NT);
-        ghost_copy(ctx, ctx->d_ddE.p, NT);
-        hipLaunchKernelGGL((k_calc_g_w<NT>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, alpha_t, ctx->d_conc.p, T,
+        hipLaunchKernelGGL((k_calc_g_w<NT>), dim3(nbt), dim3(kBlock), 0, st, ctx->P, at, alpha_t, ctx->d_conc.p, T,
                            ctx->d_ddE.p, ctx->d_v.p, g);
         launch_check("k_calc_g_w");
     }

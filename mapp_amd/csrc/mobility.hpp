@@ -246,6 +246,17 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
     }
 }
 
+// The vectors that one sweep hands to the next (n, s, t, v, F'') are read where their site
+// is owned, through the ghost's owner, so that no copy to the ghosts stands between two
+// sweeps; c and dE (whose element the quirk picks by the ghost's own index) lie at the
+// ghosts too.  A copy takes the stream about 4 us, six of them stood in a calc_g whose
+// sweeps take 8 to 14 us each on a batch of 12 cells.
+struct Owner {
+    const int* owner;  // owner[g] of ghost natms + g
+    int natms;
+    __device__ __forceinline__ int operator()(int k) const { return k < natms ? k : owner[k - natms]; }
+};
+
 // E = sum c rho_bar; n = E = F(E), dE = F', ddE = F''
 // (first sweep of c_d_calc, src/ff_dmd_I.cpp:2269-2312, and calc_g, :2447-2493).
 // Site i of type m, partner k of type b: E[i][m] += c[k][b] rho[slot(b, m)]
@@ -381,7 +392,7 @@ __device__ __forceinline__ double rate_sij(const FFParams<double>& P, double ni,
 // c_d over the 2nd list; an entry e >= 0 is the own-row partner j (pair (i, j)),
 // e < 0 the owner ~e of the pair (~e, i)
 template <int NT, int VAR>
-__global__ __launch_bounds__(kBlock) void k_c_d(FFParams<double> P, const double* __restrict__ conc,
+__global__ __launch_bounds__(kBlock) void k_c_d(FFParams<double> P, Owner at, const double* __restrict__ conc,
                                                 const int* __restrict__ foff, const int* __restrict__ fidx,
                                                 const double* __restrict__ n, double* __restrict__ c_d) {
     const SiteGroup<kList2G> g;
@@ -397,10 +408,10 @@ __global__ __launch_bounds__(kBlock) void k_c_d(FFParams<double> P, const double
     for (int q = foff[i] + g.l; q < foff[i + 1]; q += kList2G) {
         const int e = fidx[q];
         const bool own = e >= 0;
-        const int k = own ? e : ~e;
+        const int k = own ? e : ~e, ko = at(k);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const double nk = n[(size_t)k * NT + t], ck = conc[(size_t)k * NT + t];
+            const double nk = n[(size_t)ko * NT + t], ck = conc[(size_t)k * NT + t];
             const double sij = own ? rate_sij<VAR>(P, ni[t], nk, ci[t], ck) : rate_sij<VAR>(P, nk, ni[t], ck, ci[t]);
             acc[t] += own ? sij : -sij;
         }
@@ -415,7 +426,7 @@ __global__ __launch_bounds__(kBlock) void k_c_d(FFParams<double> P, const double
 
 // calc_g residual s = 2(c + a) - 2 alpha (rate sums) (and c_d for DMD_II); partial sums of s^2
 template <int NT, int VAR>
-__global__ __launch_bounds__(kBlock) void k_calc_g_s(FFParams<double> P, double alpha_t,
+__global__ __launch_bounds__(kBlock) void k_calc_g_s(FFParams<double> P, Owner at, double alpha_t,
                                                      const double* __restrict__ conc, const double* __restrict__ a,
                                                      const int* __restrict__ foff, const int* __restrict__ fidx,
                                                      const double* __restrict__ n, double* __restrict__ s,
@@ -434,10 +445,10 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_s(FFParams<double> P, double 
         for (int q = foff[i] + g.l; q < foff[i + 1]; q += kList2G) {
             const int e = fidx[q];
             const bool own = e >= 0;
-            const int k = own ? e : ~e;
+            const int k = own ? e : ~e, ko = at(k);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const double nk = n[(size_t)k * NT + t], ck = conc[(size_t)k * NT + t];
+                const double nk = n[(size_t)ko * NT + t], ck = conc[(size_t)k * NT + t];
                 const double sij =
                     own ? rate_sij<VAR>(P, ni[t], nk, ci[t], ck) : rate_sij<VAR>(P, nk, ni[t], ck, ci[t]);
                 acc[t] += own ? sij : -sij;
@@ -506,7 +517,7 @@ __device__ __forceinline__ void tg_pair(const FFParams<double>& P, double alpha_
 
 // t and the first g term over the 2nd list (src/ff_dmd_I.cpp:2576-2606)
 template <int NT, int VAR>
-__global__ __launch_bounds__(kBlock) void k_calc_g_t(FFParams<double> P, double alpha_t,
+__global__ __launch_bounds__(kBlock) void k_calc_g_t(FFParams<double> P, Owner at, double alpha_t,
                                                      const double* __restrict__ conc, const int* __restrict__ foff,
                                                      const int* __restrict__ fidx, const double* __restrict__ n,
                                                      const double* __restrict__ s, double* __restrict__ t,
@@ -527,11 +538,11 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_t(FFParams<double> P, double 
     for (int q = foff[i] + grp.l; q < foff[i + 1]; q += kList2G) {
         const int e = fidx[q];
         const bool own = e >= 0;
-        const int k = own ? e : ~e;
+        const int k = own ? e : ~e, ko = at(k);
 #pragma unroll
         for (int ty = 0; ty < NT; ++ty) {
-            const size_t kk = (size_t)k * NT + ty;
-            const double nk = n[kk], ck = conc[kk], sk = s[kk];
+            const size_t kk = (size_t)ko * NT + ty;
+            const double nk = n[kk], ck = conc[(size_t)k * NT + ty], sk = s[kk];
             double tI, gI, tJ, gJ;
             if (own) {
                 tg_pair<VAR>(P, alpha_t, ni[ty], nk, ci[ty], ck, si[ty], sk, &tI, &gI, &tJ, &gJ);
@@ -564,7 +575,7 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_t(FFParams<double> P, double 
 //   v[i][m] += rho[slot(b, m)] t[k][b]
 //   g[i][m] += alpha beta (phi[(m, b)] + rho[slot(b, m)] dE[i][m] + rho[slot(m, b)] dE[k][b]) t[k][b]
 template <int NT>
-__global__ __launch_bounds__(kBlock) void k_calc_g_v(FFParams<double> P, double alpha_t, SiteTable T,
+__global__ __launch_bounds__(kBlock) void k_calc_g_v(FFParams<double> P, Owner at, double alpha_t, SiteTable T,
                                                      const double* __restrict__ dE, const double* __restrict__ t,
                                                      double* __restrict__ v, double* __restrict__ g) {
     constexpr int NPHI = NT * (NT + 1) / 2;
@@ -580,7 +591,7 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_v(FFParams<double> P, double 
         dEi[ty] = dE[(size_t)i * NT + ty];
     }
     for (int q = T.off[i] + grp.l; q < T.off[i + 1]; q += kTableG) {
-        const int k = T.idx[q];
+        const int k = T.idx[q], ko = at(k);
         double r[NT * NT], f[NPHI], tk[NT], dk[NT];
 #pragma unroll
         for (int x = 0; x < NT * NT; ++x) r[x] = T.rho[(size_t)q * NT * NT + x];
@@ -588,7 +599,7 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_v(FFParams<double> P, double 
         for (int x = 0; x < NPHI; ++x) f[x] = T.phi[(size_t)q * NPHI + x];
 #pragma unroll
         for (int b = 0; b < NT; ++b) {
-            tk[b] = t[(size_t)k * NT + b];
+            tk[b] = t[(size_t)ko * NT + b];
             dk[b] = dE[(size_t)k * NT + b];
         }
 #pragma unroll
@@ -619,7 +630,7 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_v(FFParams<double> P, double 
 // last g term: alpha beta rho ddE c v (src/ff_dmd_I.cpp:2647-2671).
 // Site i of type m, partner k of type b: alpha beta rho[slot(m, b)] ddE[k][b] c[k][b] v[k][b]
 template <int NT>
-__global__ __launch_bounds__(kBlock) void k_calc_g_w(FFParams<double> P, double alpha_t,
+__global__ __launch_bounds__(kBlock) void k_calc_g_w(FFParams<double> P, Owner at, double alpha_t,
                                                      const double* __restrict__ conc, SiteTable T,
                                                      const double* __restrict__ ddE, const double* __restrict__ v,
                                                      double* __restrict__ g) {
@@ -631,14 +642,14 @@ __global__ __launch_bounds__(kBlock) void k_calc_g_w(FFParams<double> P, double 
 #pragma unroll
     for (int ty = 0; ty < NT; ++ty) gg[ty] = 0.0;
     for (int q = T.off[i] + grp.l; q < T.off[i + 1]; q += kTableG) {
-        const int k = T.idx[q];
+        const int k = T.idx[q], ko = at(k);
         double r[NT * NT], w[NT];
 #pragma unroll
         for (int x = 0; x < NT * NT; ++x) r[x] = T.rho[(size_t)q * NT * NT + x];
 #pragma unroll
         for (int b = 0; b < NT; ++b) {
-            const size_t kk = (size_t)k * NT + b;
-            w[b] = ddE[kk] * conc[kk] * v[kk];
+            const size_t kk = (size_t)ko * NT + b;
+            w[b] = ddE[kk] * conc[(size_t)k * NT + b] * v[kk];
         }
 #pragma unroll
         for (int m = 0; m < NT; ++m)
