@@ -209,8 +209,6 @@ void build_ghosts(mapp_dmd* ctx) {
     const int natms = ctx->natms;
     ctx->nghost = 0;
     ctx->swap_off.assign(1, 0);
-    ctx->swap_dim.clear();
-    ctx->swap_dir.clear();
     // One swap per face (init refuses a box that needs more), dimension by dimension over
     // the sites and the ghosts so far.  The flags of both faces are counted by one scan,
     // the low face first, which numbers the ghosts as one swap after the other does.
@@ -238,8 +236,6 @@ void build_ghosts(mapp_dmd* ctx) {
         }
         for (int dir = 0; dir < 2; ++dir) {
             ctx->nghost += dir == 0 ? cnt_lo : cnt - cnt_lo;
-            ctx->swap_dim.push_back(idim);
-            ctx->swap_dir.push_back(dir);
             ctx->swap_off.push_back(ctx->nghost);
         }
     }
@@ -396,15 +392,13 @@ void rebuild_any(mapp_dmd* ctx) {
 
 template <int NT>
 void ghost_update_x(mapp_dmd* ctx) {
-    for (size_t sw = 0; sw + 1 < ctx->swap_off.size(); ++sw) {
-        int g0 = ctx->swap_off[sw], g1 = ctx->swap_off[sw + 1];
-        if (g1 <= g0) continue;
-        int idim = ctx->swap_dim[sw], dir = ctx->swap_dir[sw];
-        hipLaunchKernelGGL((k_ghost_update_x<NT>), dim3(nblk(g1 - g0)), dim3(kBlock), 0, ctx->stream,
-                           ctx->d_pos.p, ctx->d_alpha.p, ctx->natms, g0, g1, ctx->d_ghost_src.p, idim, dir,
-                           ctx->bp.H[idim][0], ctx->bp.H[idim][1], ctx->bp.H[idim][2]);
-        launch_check("k_ghost_update_x");
-    }
+    if (ctx->swap_off.size() != 7 || ctx->nghost <= 0) return;  // a batch has no box-wide swaps
+    GhostSwaps W;
+    for (int k = 0; k < 6; ++k) W.end[k] = ctx->swap_off[k + 1];
+    std::memcpy(W.H, ctx->bp.H, sizeof(W.H));
+    hipLaunchKernelGGL((k_ghost_update_x<NT>), dim3(nblk(ctx->nghost)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p,
+                       ctx->d_alpha.p, ctx->natms, ctx->nghost, ctx->d_ghost_src.p, W);
+    launch_check("k_ghost_update_x");
 }
 
 void ghost_copy(mapp_dmd* ctx, double* v, int d) {
@@ -1543,8 +1537,6 @@ void init_batch(mapp_dmd* ctx, double skin) {
     HIP_OK(hipMemcpyAsync(ctx->d_roff.p + natms, &rlast, sizeof(int), hipMemcpyHostToDevice, st));
     HIP_OK(hipStreamSynchronize(st));
     ctx->swap_off.assign(1, 0);  // no box-wide ghost swaps: positions stay fixed in a batch
-    ctx->swap_dim.clear();
-    ctx->swap_dir.clear();
     finish_lists<NT>(ctx);
     for (int k = 0; k < ncell; ++k) {
         const int n = sub[k]->natms, g = sub[k]->nghost;

@@ -40,7 +40,7 @@ struct mapp_dmd {
     // batch of independent cells (empty: one cell from set_system)
     std::vector<int> cell_natms, cell_nghost;
     std::vector<double> cell_H, cell_x, cell_c;
-    std::vector<int> swap_off, swap_dim, swap_dir;
+    std::vector<int> swap_off;  // ghosts up to each swap (low, high face of each dimension)
 
     // device tables
     mappdmd::DevBuf<double> d_quad64, d_rho7, d_phi7, d_F9, d_F7, d_eam_rows, d_drho;

@@ -155,23 +155,40 @@ __global__ void k_ghost_emit(double4* __restrict__ pos, double* __restrict__ alp
     }
 }
 
-// Atoms::update of x between rebuilds: ghost = source +- H[idim][0..idim]
+// Atoms::update of x between rebuilds: ghost = source +- H[idim][0..idim], its source
+// itself a ghost of an earlier swap or owned.  One thread per ghost walks back to the
+// owned site (at most one swap per dimension) and applies the shifts in the swaps' order,
+// the additions of six launches, one per swap, that took 2.8 us each.
+struct GhostSwaps {
+    int end[6];  // ghosts up to the end of each swap: low and high face of each dimension
+    double H[3][3];
+};
 template <int NT>
-__global__ void k_ghost_update_x(double4* __restrict__ pos, double* __restrict__ alpha, int natms, int gbeg,
-                                 int gend, const int* __restrict__ ghost_src, int idim, int dir, double h0,
-                                 double h1, double h2) {
-    int g = gbeg + blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= gend) return;
-    int src = ghost_src[g];
+__global__ void k_ghost_update_x(double4* __restrict__ pos, double* __restrict__ alpha, int natms, int nghost,
+                                 const int* __restrict__ ghost_src, GhostSwaps W) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= nghost) return;
+    int swap[3], n = 0, src = natms + g;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if (src < natms) break;
+        const int e = src - natms;
+        int w = 0;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) w += e >= W.end[q] ? 1 : 0;
+        swap[k] = w;
+        n = k + 1;
+        src = ghost_src[e];
+    }
     double4 p = pos[src];
-    if (dir == 0) {
-        p.x += h0;
-        if (idim >= 1) p.y += h1;
-        if (idim >= 2) p.z += h2;
-    } else {
-        p.x -= h0;
-        if (idim >= 1) p.y -= h1;
-        if (idim >= 2) p.z -= h2;
+#pragma unroll
+    for (int k = 2; k >= 0; --k) {
+        if (k >= n) continue;
+        const int d = swap[k] >> 1;
+        const double sgn = swap[k] & 1 ? -1.0 : 1.0;
+        p.x += sgn * W.H[d][0];
+        if (d >= 1) p.y += sgn * W.H[d][1];
+        if (d >= 2) p.z += sgn * W.H[d][2];
     }
     pos[natms + g] = p;
 #pragma unroll
