@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
 // is owned, through the ghost's owner, so that no copy to the ghosts stands between two
 // sweeps; c and dE (whose element the quirk picks by the ghost's own index) lie at the
 // ghosts too.  A copy takes the stream about 4 us, six of them stood in a calc_g whose
-// sweeps take 8 to 14 us each on a batch of 12 cells.
+// sweeps take 8 to 14 us each on a batch of six cells of 6^3 to 12^3.
 struct Owner {
     const int* owner;  // owner[g] of ghost natms + g
     int natms;
