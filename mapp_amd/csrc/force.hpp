@@ -420,7 +420,7 @@ __device__ __forceinline__ int pack_in_range(int p, bool in, int* out) {
 //
 // ENERGY_ONLY restates energy_calc's triangle (jtype starts at itype, so phi
 // only for itype == jtype; src/ff_dmd_I.cpp:508).  The partner's density share
-// goes to pairE in reverse-CSR order (rpos), so the embedding reads it
+// goes to pairE in reverse-list order (nlrp[].y), so the embedding reads it
 // contiguously.  Unless ENERGY_ONLY, the rho lane stores {drho/dr, drho/dalpha}
 // and the phi lane {dphi/dr, dphi/dalpha} in the pair's record (PairRec; the
 // reference's per-pair caches, src/ff_dmd_I.cpp:227-242, restricted to what the
