@@ -326,6 +326,12 @@ void rebuild(mapp_dmd* ctx) {
     }
     if (ctx->variant == MAPP_DMD_VARIANT_MEAM) finish_meam(ctx);
     else finish_lists<NT>(ctx);
+    // the positions that the skin test of later moves compares with
+    ctx->d_x0.reserve(natms);
+    HIP_OK(hipMemcpyAsync(ctx->d_x0.p, ctx->d_pos.p, sizeof(double4) * natms, hipMemcpyDeviceToDevice, st));
+    HIP_OK(hipStreamSynchronize(st));
+    ctx->have_list2 = false;
+    ctx->cache_valid = false;
 }
 
 // pair links and per-site / per-pair buffers for the half list in d_off / d_nl and the
@@ -368,11 +374,6 @@ void finish_lists(mapp_dmd* ctx) {
         ctx->d_info.reserve(natms + 1);
     }
     ctx->d_crd.reserve(ntot);
-    ctx->d_x0.reserve(natms);
-    HIP_OK(hipMemcpyAsync(ctx->d_x0.p, ctx->d_pos.p, sizeof(double4) * natms, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipStreamSynchronize(st));
-    ctx->have_list2 = false;
-    ctx->cache_valid = false;
 }
 
 // f(std::integral_constant<int, NT>) for the number of DMD types nt = 1..kMaxTypes
@@ -1545,6 +1546,8 @@ void init_batch(mapp_dmd* ctx, double skin) {
         launch_check("k_quirk_cell");
     }
     HIP_OK(hipStreamSynchronize(st));
+    ctx->have_list2 = false;
+    ctx->cache_valid = false;
     ctx->cell_nghost.assign(ncell, 0);
     for (int k = 0; k < ncell; ++k) ctx->cell_nghost[k] = gh_base[k + 1] - gh_base[k];
 }

@@ -169,3 +169,26 @@ def test_sites_per_wavefront(n):
     from mapp_amd import workload as W
     state = W.meam_state(["Aa", "Bb"], local=W.meam_local(2))
     _compare(*_pair(state, *W.md_lattice(n, 3.58, "fcc", seed=n)), f"sites {n}")
+
+
+def test_moves():
+    """update_0 of a MEAM system: inside the skin (ghosts follow), then past it (the full list and the
+    screening buffers anew), forces after each; then whole minimiser steps from there"""
+    from mapp_amd import workload as W
+    state = W.meam_state(["Aa", "Bb"], local=W.meam_local(2))
+    H, s, t = W.md_lattice(4, 3.58, "fcc", nt=2, seed=41, jitter=0.05)
+    ff, orc = _pair(state, H, s, t)
+    _compare(ff, orc, "start")
+    x = ff.get("x") + np.random.default_rng(1).uniform(-0.05, 0.05, size=(len(s), 3))
+    assert ff.set_x(x) is False and orc.set_x(x) is False
+    _compare(ff, orc, "inside the skin")
+    x[7, 0] += 0.6
+    x[100, 2] -= 0.5
+    assert ff.set_x(x) is True and orc.set_x(x) is True
+    _compare(ff, orc, "past the skin")
+    code, en, nf, ne = ff.min_lbfgs(3, 2, -1.0)
+    code_o, en_o, nf_o, ne_o = orc.min_lbfgs(3, 2, -1.0)
+    print("minimiser", en, en_o, flush=True)
+    assert (code, len(en), nf, ne) == (code_o, len(en_o), nf_o, ne_o)
+    assert np.max(np.abs(en - en_o) / np.abs(en_o)) <= 1e-10  # the bar of the DMD minimiser's energies
+    ff.close()
