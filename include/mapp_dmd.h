@@ -200,7 +200,8 @@ int mapp_dmd_set_system(mapp_dmd_t* ctx, const double* H, int natms,
                         const double* x_reduced, const double* c);
 /* ForceField_DMD_I::init (src/ff_dmd_I.cpp:672-699) + Atoms::ph_setup
    (src/atoms.cpp:317-372) + Neighbor::create_list(0,1)
-   (src/neighbor.cpp:137-292) + Atoms::store_0, on the GPU. */
+   (src/neighbor.cpp:137-292) + Atoms::store_0, on the GPU.  A call that fails
+   leaves the context uninitialised. */
 int mapp_dmd_init(mapp_dmd_t* ctx, double skin);
 /* ForceField_DMD_I::fin (src/ff_dmd_I.cpp:703-725): drops lists and caches. */
 int mapp_dmd_fin(mapp_dmd_t* ctx);
@@ -208,7 +209,9 @@ int mapp_dmd_fin(mapp_dmd_t* ctx);
 /* New owned x (cartesian + alpha; host pointer, or NULL when the device
    vector was written in place), then Atoms::update_0 (src/atoms.cpp:1780-1865):
    rebuild ghosts and lists if a site moved more than skin, else forward-update
-   ghost x.  *rebuilt (may be NULL) reports which. */
+   ghost x.  *rebuilt (may be NULL) reports which.  Where it fails (a list
+   beyond its limits, no memory), here or within min_lbfgs, the context counts
+   as not initialised (MAPP_DMD_E_STATE) until the next mapp_dmd_init. */
 int mapp_dmd_set_x(mapp_dmd_t* ctx, const double* x_host, int* rebuilt);
 /* New owned c (host pointer or NULL for in-place device writes), forwarded to
    ghosts (Atoms::update of c). */

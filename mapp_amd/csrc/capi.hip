@@ -1123,8 +1123,11 @@ void sur_gradient(mapp_dmd* ctx, const SurNorm& N, const float* params, const fl
 // Atoms::update_0 (src/atoms.cpp:1780-1865) for owned x already in d_xaos
 // (cartesian + alpha rows): full-skin test against the positions of the last
 // build, then a rebuild (x2s, ghosts, bins, lists) or a forward ghost update.
+// A build that fails on the way (a list beyond its limits, no memory) leaves lists and
+// buffers of two builds: the context then counts as not initialised until the next init.
 int update_x_device(mapp_dmd* ctx) {
     const int nt = acols(ctx), natms = ctx->natms;
+    ctx->inited = false;
     if (is_md(ctx)) scatter_x<1, 0>(ctx, ctx->d_xaos.p);
     else with_nt(nt, [&](auto c) { scatter_x<decltype(c)::value>(ctx, ctx->d_xaos.p); });
     int* const box = reinterpret_cast<int*>(ctx->h_box);
@@ -1144,6 +1147,7 @@ int update_x_device(mapp_dmd* ctx) {
         HIP_OK(hipStreamSynchronize(ctx->stream));
     }
     ctx->cache_valid = false;
+    ctx->inited = true;
     return flag;
 }
 
@@ -2163,6 +2167,7 @@ int mapp_dmd_init(mapp_dmd_t* ctx, double skin) {
         require(skin >= 0.0, MAPP_DMD_E_ARG, "negative skin");
         HIP_OK(hipSetDevice(ctx->device));
         const int nt = acols(ctx), natms = ctx->natms;
+        ctx->inited = false;  // until all of it is done
         ctx->skin = skin;
         const FFParams<double>& P = ctx->P;
         ctx->bp.full = 0;

@@ -192,3 +192,33 @@ def test_moves():
     assert (code, len(en), nf, ne) == (code_o, len(en_o), nf_o, ne_o)
     assert np.max(np.abs(en - en_o) / np.abs(en_o)) <= 1e-10  # the bar of the DMD minimiser's energies
     ff.close()
+
+
+def test_failed_build_leaves_no_lists():
+    """a move that brings a site more list entries than the kernels stage, and an init whose box is too
+    thin: refused, and so is every later call on the lists they broke off, until an init that succeeds"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import DMDError
+    state = W.meam_state(["Aa", "Bb"], local=W.meam_local(2))
+    Hs, s0, t = W.md_lattice(5, 3.58, "fcc", nt=2, seed=43, jitter=0.05)
+    H = np.diag([40.0] * 3)
+    ff, orc = _pair(state, H, (s0 @ Hs + 10.0) / 40.0, t)
+    want = ff.force_calc(1)
+    x = ff.get("x")
+
+    def refused():
+        for call in (lambda: ff.force_calc(1), ff.energy_calc, lambda: ff.min_lbfgs(1), lambda: ff.set_x(x),
+                     lambda: ff.get("x"), ff.create_2nd_neigh_lst):
+            with pytest.raises(DMDError) as e:
+                call()
+            assert e.value.code == -2, call  # E_STATE
+
+    for fail in (lambda: ff.set_x(20.0 + 0.4 * (x - x.mean(axis=0))), lambda: ff.init(50.0)):
+        with pytest.raises(DMDError) as e:
+            fail()
+        assert e.value.code == -4  # E_RANGE
+        refused()
+        ff.init(0.3)
+        assert np.array_equal(ff.force_calc(1), want)
+    _compare(ff, orc, "after the failures")
+    ff.close()
