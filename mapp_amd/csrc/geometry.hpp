@@ -312,6 +312,12 @@ __global__ void k_bin_place(const int* __restrict__ v, int n, const int* __restr
 constexpr int kBinSites = 4;
 constexpr int kBinWaves = 4;  // wavefronts per bin: they take its groups in turn
 constexpr int kMaskWords = 16;
+// what one lane of a wavefront left in LDS is there for the others (no instruction: LDS
+// accesses of a wavefront are in order, so only the compiler has to keep theirs)
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 // set bits of m below this lane
 __device__ __forceinline__ int lane_rank(unsigned long long m) {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const i
     const unsigned long long occ = __ballot(bsize > 0);
     const int nbin = __popcll(occ);
     if (bsize > 0) bin_lds[wave][lane_rank(occ)] = make_int2(bstart, bsize);
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     bstart = bsize = 0;
     if (lane < nbin) {
         const int2 e = bin_lds[wave][lane];
@@ -399,13 +405,12 @@ __global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const i
         int nb = 0;                   // bins that end before this round
         for (int base = 0, round = 0; base < total; base += 64, ++round) {
             if ((round & 63) == 0) {
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_sync();
                 ends_lds[wave][lane] = 0;
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_sync();
                 const int e = incl - 1 - base;
-                if (lane < nbin && e >= 0 && e < 4096)
-                    atomicOr(reinterpret_cast<unsigned*>(ends_lds[wave]) + (e >> 5), 1u << (e & 31));
-                __builtin_amdgcn_wave_barrier();
+                if (lane < nbin && e >= 0 && e < 4096) atomicOr(&ends_lds[wave][e >> 6], 1ull << (e & 63));
+                wave_lds_sync();
                 ends = ends_lds[wave][lane];
             }
             const unsigned long long last = read_lane_u64(ends, round & 63);
