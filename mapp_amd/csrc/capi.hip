@@ -302,9 +302,27 @@ void rebuild(mapp_dmd* ctx) {
     ctx->d_roff.reserve(natms + 1);
     ctx->d_list_mask.reserve((size_t)natms * kMaskWords);
     HalfLists L{ctx->d_list_mask.p, ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p, ctx->d_roff.p, nullptr, nullptr};
-    const dim3 grid(bp.tot_bin), blk(64 * kBinWaves);
+    int nbin = bp.tot_bin;
+    const int* bins = nullptr;
+    if (nbin > kFewBins && nbin > natms / 4) {
+        ctx->d_flag.reserve(nbin);
+        ctx->d_offs.reserve(nbin);
+        ctx->d_bin_list.reserve(natms);
+        hipLaunchKernelGGL(k_bin_owned, dim3(nblk(nbin)), dim3(kBlock), 0, st, ctx->d_bin_start.p, ctx->d_bin_atoms.p,
+                           nbin, natms, ctx->d_flag.p);
+        scan(ctx, kScanA, ctx->d_flag.p, ctx->d_offs.p, nbin, false);
+        hipLaunchKernelGGL(k_bin_list, dim3(nblk(nbin)), dim3(kBlock), 0, st, ctx->d_flag.p, ctx->d_offs.p, nbin,
+                           ctx->d_bin_list.p);
+        launch_check("k_bin_list");
+        wait_box(ctx);
+        nbin = (int)scan_total(ctx, kScanA);
+        bins = ctx->d_bin_list.p;
+    }
+    // in x at most 2^23 blocks (of 256 threads: a launch holds fewer than 2^32), the rest in z
+    constexpr int kMaxX = 1 << 23;
+    const dim3 grid(std::min(nbin, kMaxX), 1, (nbin + kMaxX - 1) / kMaxX), blk(64 * kBinWaves);
     hipLaunchKernelGGL((bp.pairwise ? k_half_list<false, true> : k_half_list<false, false>), grid, blk, 0, st, natms,
-                       ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
+                       bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
     launch_check("k_half_list count");
     scan(ctx, kScanA, ctx->d_cnt.p, ctx->d_off.p, natms, true);
     scan(ctx, kScanB, ctx->d_rcnt.p, ctx->d_roff.p, natms, true);
@@ -317,7 +335,7 @@ void rebuild(mapp_dmd* ctx) {
     L.nl = ctx->d_nl.p;
     L.rlist = ctx->d_rtmp.p;
     hipLaunchKernelGGL((bp.pairwise ? k_half_list<true, true> : k_half_list<true, false>), grid, blk, 0, st, natms,
-                       ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
+                       bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
     launch_check("k_half_list fill");
     if (ctx->nrev > 0) {
         hipLaunchKernelGGL(k_sort_owners, dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, natms, ctx->d_roff.p,

@@ -50,7 +50,7 @@ struct mapp_dmd {
     mappdmd::DevBuf<double> d_alpha, d_conc;
     mappdmd::DevBuf<int> d_ghost_src, d_ghost_owner;
     // binning and lists
-    mappdmd::DevBuf<int> d_flag, d_offs, d_bin_of, d_bin_cnt, d_bin_slot, d_bin_start, d_bin_atoms, d_arrived;
+    mappdmd::DevBuf<int> d_flag, d_offs, d_bin_of, d_bin_cnt, d_bin_slot, d_bin_start, d_bin_atoms, d_arrived, d_bin_list;
     mappdmd::DevBuf<double4> d_bin_pos;               // positions in bin order
     mappdmd::DevBuf<unsigned long long> d_list_mask;  // accept bits of the list build
     mappdmd::DevBuf<int> d_cnt, d_rcnt, d_off, d_nl, d_roff;

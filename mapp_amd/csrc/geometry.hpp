@@ -309,6 +309,15 @@ __global__ void k_bin_place(const int* __restrict__ v, int n, const int* __restr
 // and the reverse list made from it by atomics, a sort and four passes over the pairs
 // 0.74 where the sort and k_pair_links take 0.24.  Groups of 8 or 16 sites are slower
 // (0.20 and 0.50: fewer wavefronts, more registers).
+//
+// A box that is mostly empty has more bins than sites, and a block for each costs 0.2 us
+// per 1,000 empty bins in either launch, up to the launch limit of 2^24 blocks of this
+// size.  So where there are more than kFewBins bins, and more than a quarter of the sites
+// (a filled box has some 16 sites to a bin), the launch goes over the list of the bins
+// that hold an owned site; three small launches and a wait make it, about 27 us.  864
+// sites in a box of 500 A (730,000 bins), rebuild with the host's part: 478 -> 235 us; in
+// one of 1,000 A (5.6 million bins) 2,534 -> 278 us.
+constexpr long kFewBins = 65536;
 constexpr int kBinSites = 4;
 constexpr int kBinWaves = 4;  // wavefronts per bin: they take its groups in turn
 constexpr int kMaskWords = 16;
@@ -333,16 +342,33 @@ struct HalfLists {
     const int *off, *roff;     // fill: their offsets
     int *nl, *rlist;           // fill: partners in list order; owners in stencil order
 };
+// flag[b] = 1 for a bin with an owned site (owned sites come first in a bin)
+__global__ void k_bin_owned(const int* __restrict__ bin_start, const int* __restrict__ bin_atoms, int tot_bin,
+                            int natms, int* __restrict__ flag) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= tot_bin) return;
+    const int k = bin_start[b];
+    flag[b] = k < bin_start[b + 1] && bin_atoms[k] < natms ? 1 : 0;
+}
+__global__ void k_bin_list(const int* __restrict__ flag, const int* __restrict__ offs, int tot_bin,
+                           int* __restrict__ bins) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < tot_bin && flag[b]) bins[offs[b]] = b;
+}
+// bins: the bins with an owned site, nbin of them; null: every bin.
 // PAIRWISE: a cutoff per type pair (bp.cut_sk_sq_tp), the type in bin_pos[].w
 template <bool FILL, bool PAIRWISE>
-__global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const int* __restrict__ bin_start,
+__global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const int* __restrict__ bins, int nbin,
+                                                              const int* __restrict__ bin_start,
                                                               const int* __restrict__ bin_atoms,
                                                               const double4* __restrict__ bin_pos, BoxParams bp,
                                                               HalfLists L) {
     __shared__ unsigned long long ends_lds[kBinWaves][64];
     __shared__ int2 bin_lds[kBinWaves][32];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int bin = blockIdx.x;
+    const int at = blockIdx.z * gridDim.x + blockIdx.x;
+    if (at >= nbin) return;  // the whole block
+    const int bin = bins ? bins[at] : at;
     const int k1 = bin_start[bin + 1];
     int k0 = bin_start[bin] + wave * kBinSites;
     // owned sites come first in a bin
@@ -364,11 +390,11 @@ __global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const i
     }
     // the occupied bins packed into the low lanes, so that their last candidates are distinct
     const unsigned long long occ = __ballot(bsize > 0);
-    const int nbin = __popcll(occ);
+    const int nocc = __popcll(occ);
     if (bsize > 0) bin_lds[wave][lane_rank(occ)] = make_int2(bstart, bsize);
     wave_lds_sync();
     bstart = bsize = 0;
-    if (lane < nbin) {
+    if (lane < nocc) {
         const int2 e = bin_lds[wave][lane];
         bstart = e.x;
         bsize = e.y;
@@ -409,7 +435,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const i
                 ends_lds[wave][lane] = 0;
                 wave_lds_sync();
                 const int e = incl - 1 - base;
-                if (lane < nbin && e >= 0 && e < 4096) atomicOr(&ends_lds[wave][e >> 6], 1ull << (e & 63));
+                if (lane < nocc && e >= 0 && e < 4096) atomicOr(&ends_lds[wave][e >> 6], 1ull << (e & 63));
                 wave_lds_sync();
                 ends = ends_lds[wave][lane];
             }

@@ -34,3 +34,31 @@ def test_lists_of_sparse_and_dense_boxes(tables, n, a):
     for name in ("E", "dE", "n"):  # the rates of the dense boxes overflow
         assert rel_inf(ff.get(name), orc.get(name)) <= 1e-11, name
     ff.close()
+
+
+@pytest.mark.parametrize("L", [200.0, 300.0, 1500.0])
+def test_lists_of_nearly_empty_boxes(tables, L):
+    """864 sites in two clusters, one across a corner: 5e4 bins (a block each), 1.7e5 (the list of the
+    occupied ones) and 1.8e7 (more than a launch holds blocks)"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    lat = W.fcc_alloy(6, seed=21)
+    s = np.where(np.arange(lat.natms)[:, None] % 2 == 0, lat.cart / L, lat.cart / L + 0.43)
+    s -= 8.0 / L
+    s -= np.floor(s)
+    box = W.Lattice(H=np.diag([L] * 3), x=np.ascontiguousarray(np.concatenate([s, lat.x[:, 3:]], axis=1)), c=lat.c,
+                    cart=s * L)
+    ff, orc = setup(box, tables, no_i=3), O.make(box, tables, no_i=3)
+    x = ff.get("x")
+    x[3, 0] += 0.8  # past the skin
+    for moved in (False, True):
+        if moved:
+            assert ff.set_x(x) and orc.set_x(x)
+        for got, want in ((ff.neighbor_list(), orc.neighbor_list()), (ff.ghosts(), orc.ghosts())):
+            for g, w in zip(got, want):
+                assert np.array_equal(g, w)
+        assert len(orc.neighbor_list()[1]) > 5000 and len(orc.ghosts()[1]) > 100
+        en, eo = ff.force_calc(1), orc.force_calc(1)
+        assert abs(en[0] - eo[0]) <= 1e-12 * abs(eo[0]) and rel_inf(ff.get("f"), orc.get("f")) <= 1e-12
+    ff.close()
