@@ -304,6 +304,7 @@ void rebuild(mapp_dmd* ctx) {
     HalfLists L{ctx->d_list_mask.p, ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p, ctx->d_roff.p, nullptr, nullptr};
     int nbin = bp.tot_bin;
     const int* bins = nullptr;
+    double per_bin = (double)natms * bp.bin_size[0] * bp.bin_size[1] * bp.bin_size[2];  // in a filled box
     if (nbin > kFewBins && nbin > natms / 4) {
         ctx->d_flag.reserve(nbin);
         ctx->d_offs.reserve(nbin);
@@ -317,10 +318,11 @@ void rebuild(mapp_dmd* ctx) {
         wait_box(ctx);
         nbin = (int)scan_total(ctx, kScanA);
         bins = ctx->d_bin_list.p;
+        per_bin = (double)natms / nbin;
     }
     // in x at most 2^23 blocks (of 256 threads: a launch holds fewer than 2^32), the rest in z
     constexpr int kMaxX = 1 << 23;
-    const dim3 grid(std::min(nbin, kMaxX), 1, (nbin + kMaxX - 1) / kMaxX), blk(64 * kBinWaves);
+    const dim3 grid(std::min(nbin, kMaxX), bin_blocks(per_bin), (nbin + kMaxX - 1) / kMaxX), blk(64 * kBinWaves);
     hipLaunchKernelGGL((bp.pairwise ? k_half_list<false, true> : k_half_list<false, false>), grid, blk, 0, st, natms,
                        bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
     launch_check("k_half_list count");

@@ -319,7 +319,18 @@ __global__ void k_bin_place(const int* __restrict__ v, int n, const int* __restr
 // one of 1,000 A (5.6 million bins) 2,534 -> 278 us.
 constexpr long kFewBins = 65536;
 constexpr int kBinSites = 4;
-constexpr int kBinWaves = 4;  // wavefronts per bin: they take its groups in turn
+constexpr int kBinWaves = 4;  // wavefronts per block; those of a bin's blocks take its groups in turn
+// Blocks per bin for a mean of `sites` owned sites to an occupied bin: one for each
+// kBinShare, the sites that a block's wavefronts take in one turn, so that a crowded bin (a
+// long cutoff, a compressed box) is not left to four wavefronts.  Rebuild with the host's
+// part, one block per bin -> this: 4,000 LJ sites with a cutoff of 12 A (150 to a bin) 1.72
+// -> 0.65 ms, 32,000 with 16 A (348) 11.8 -> 4.3, 4,000 sites in a box of 9 A (500) 39.1 ->
+// 4.0; one block per 32 sites 0.77, 4.6 and 5.2.
+constexpr int kBinShare = 16;
+inline int bin_blocks(double sites) {
+    const double b = sites / kBinShare;
+    return b < 1.0 ? 1 : (b > 256.0 ? 256 : (int)b);
+}
 constexpr int kMaskWords = 16;
 // what one lane of a wavefront left in LDS is there for the others (no instruction: LDS
 // accesses of a wavefront are in order, so only the compiler has to keep theirs)
@@ -370,7 +381,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const i
     if (at >= nbin) return;  // the whole block
     const int bin = bins ? bins[at] : at;
     const int k1 = bin_start[bin + 1];
-    int k0 = bin_start[bin] + wave * kBinSites;
+    int k0 = bin_start[bin] + (blockIdx.y * kBinWaves + wave) * kBinSites;
     // owned sites come first in a bin
     if (k0 >= k1 || bin_atoms[k0] >= natms) return;  // the whole wavefront
     int tmp = bin;
@@ -406,7 +417,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void k_half_list(int natms, const i
     }
     const int to_bin = bstart - (incl - bsize);  // candidate number -> place in the bins
     const int total = __builtin_amdgcn_readlane(incl, 31);
-    for (; k0 < k1; k0 += kBinWaves * kBinSites) {
+    for (; k0 < k1; k0 += gridDim.y * kBinWaves * kBinSites) {
         int site[kBinSites], w[kBinSites], wr[kBinSites];
         double4 xi[kBinSites];
         unsigned long long keep[kBinSites];

@@ -36,16 +36,17 @@ def test_lists_of_sparse_and_dense_boxes(tables, n, a):
     ff.close()
 
 
-@pytest.mark.parametrize("L", [200.0, 300.0, 1500.0])
-def test_lists_of_nearly_empty_boxes(tables, L):
-    """864 sites in two clusters, one across a corner: 5e4 bins (a block each), 1.7e5 (the list of the
-    occupied ones) and 1.8e7 (more than a launch holds blocks)"""
+@pytest.mark.parametrize("L,n,squeeze", [(200.0, 6, 1.0), (300.0, 6, 1.0), (300.0, 8, 0.3), (1500.0, 6, 1.0)])
+def test_lists_of_nearly_empty_boxes(tables, L, n, squeeze):
+    """4 n^3 sites in two clusters, one across a corner: 5e4 bins (a block each), 1.7e5 (the list of the
+    occupied ones; squeezed, several blocks to each) and 1.8e7 (more than a launch holds blocks)"""
     from mapp_amd import workload as W
     from mapp_amd.dmd import setup
     from oracle import oracle as O
-    lat = W.fcc_alloy(6, seed=21)
-    s = np.where(np.arange(lat.natms)[:, None] % 2 == 0, lat.cart / L, lat.cart / L + 0.43)
-    s -= 8.0 / L
+    lat = W.fcc_alloy(n, seed=21)
+    s = lat.cart * squeeze / L
+    s[1::2] += 0.43
+    s -= 3.0 / L
     s -= np.floor(s)
     box = W.Lattice(H=np.diag([L] * 3), x=np.ascontiguousarray(np.concatenate([s, lat.x[:, 3:]], axis=1)), c=lat.c,
                     cart=s * L)
@@ -60,5 +61,10 @@ def test_lists_of_nearly_empty_boxes(tables, L):
                 assert np.array_equal(g, w)
         assert len(orc.neighbor_list()[1]) > 5000 and len(orc.ghosts()[1]) > 100
         en, eo = ff.force_calc(1), orc.force_calc(1)
-        assert abs(en[0] - eo[0]) <= 1e-12 * abs(eo[0]) and rel_inf(ff.get("f"), orc.get("f")) <= 1e-12
+        # sites to an occupied bin, and more than the 16 of a block where squeezed
+        xa, cut = ff.get("x")[:, :3], tables.rc + 1.2247448713915890 / 5.0
+        mean = lat.natms / len(np.unique(((xa + cut) / cut).astype(int), axis=0))
+        assert mean > 32.0 if squeeze < 1.0 else mean < 16.0
+        bound = 1e-12 if squeeze == 1.0 else 1e-11  # more pairs to a site
+        assert abs(en[0] - eo[0]) <= bound * abs(eo[0]) and rel_inf(ff.get("f"), orc.get("f")) <= bound
     ff.close()
