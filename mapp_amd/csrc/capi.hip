@@ -912,7 +912,7 @@ void ensure_pair_cache(mapp_dmd* ctx);
 template <int NT, typename Q, int NQ>
 void run_table_values(mapp_dmd* ctx, const Q* quad, const FFParams<Q>& PQ) {
     hipLaunchKernelGGL((k_table_values<NT, Q, NQ>), dim3(nblk((long)ctx->natms * 64)), dim3(kBlock),
-                       (kBlock / 64) * TableStage<NT>::kBytes, ctx->stream, ctx->P, PQ, ctx->d_pos.p, ctx->d_alpha.p,
+                       (kBlock / 64) * TableStage<NT>::kBytes, ctx->stream, ctx->P, PQ, ctx->d_arec.p, ctx->d_alpha.p,
                        ctx->d_off.p, ctx->d_nlrp.p, quad, ctx->d_rho7.p, ctx->d_phi7.p, ctx->d_toff.p, ctx->d_town.p,
                        ctx->d_trank.p, ctx->d_tidx.p, ctx->d_trho.p, ctx->d_tphi.p);
     launch_check("k_table_values");
@@ -933,7 +933,7 @@ void table_values_dispatch(mapp_dmd* ctx) {
     }
 }
 
-// site table of the pair values (both ends of every pair inside the quadrature cut)
+// site table of the pair values (both ends of every pair that can have one)
 template <int NT>
 void build_site_table(mapp_dmd* ctx) {
     hipStream_t st = ctx->stream;
@@ -943,8 +943,13 @@ void build_site_table(mapp_dmd* ctx) {
     ctx->d_cnt.reserve(natms + 1);
     ctx->d_town.reserve(natms + 1);
     ctx->d_trank.reserve(ctx->nrev + 1);
-    hipLaunchKernelGGL(k_table_count, grid, dim3(kBlock), 0, st, L, ctx->d_rowner.p, natms, ctx->d_pos.p,
-                       ctx->P.cut_sq_mod, ctx->d_town.p, ctx->d_cnt.p, ctx->d_trank.p);
+    // the force passes' records are packed anew by every call; until then their buffer holds the table's
+    const int ntot = natms + ctx->nghost;
+    ctx->d_arec.reserve(ntot);
+    hipLaunchKernelGGL((k_table_pack<NT>), dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_pos.p, ctx->d_alpha.p, ntot,
+                       ctx->d_arec.p);
+    hipLaunchKernelGGL(k_table_count, grid, dim3(kBlock), 0, st, ctx->P, L, ctx->d_rowner.p, ctx->d_arec.p,
+                       ctx->d_town.p, ctx->d_cnt.p, ctx->d_trank.p);
     launch_check("k_table_count");
     const long ne = counts_to_offsets(ctx, ctx->d_cnt.p, ctx->d_toff, natms);
     ctx->d_tidx.reserve(ne + 1);

@@ -58,7 +58,8 @@ struct mapp_dmd {
     mappdmd::DevBuf<int> d_rtmp;  // owners of the reverse lists before they are sorted
     mappdmd::DevBuf<double2> d_deriv;  // pass 1's records (PairRec) of the quadrature type
     mappdmd::DevBuf<int2> d_info;      // [natms] {list offset, pairs inside the cut at the last force pass 1}
-    mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}; MD potentials [ntot] {x, y, z, type, then F'}
+    mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}; MD potentials [ntot] {x, y, z, type, then F'};
+                                       // while the site table is built [ntot] {x, y, z, largest 1/alpha}
     long nrev = 0;
     long npairs = 0, npairs2 = 0;
     bool have_list2 = false;
@@ -72,8 +73,8 @@ struct mapp_dmd {
     // pair's owner; the top bit of the first: inside the quadrature cut at the last pass 1
     mappdmd::DevBuf<int2> d_nlrp;
     mappdmd::DevBuf<int> d_rowner;
-    mappdmd::DevBuf<int> d_toff, d_tidx;        // site table: both ends of every pair inside the quadrature cut
-    mappdmd::DevBuf<int> d_town, d_trank;       // own entries per site; a reverse entry's rank among those inside the cut
+    mappdmd::DevBuf<int> d_toff, d_tidx;        // site table: both ends of every pair that can have a value
+    mappdmd::DevBuf<int> d_town, d_trank;       // own entries per site; a reverse entry's rank among those in the table
     mappdmd::DevBuf<double> d_trho, d_tphi;
     long ntable = 0;
     mappdmd::DevBuf<int> d_foff2, d_fidx2;      // 2nd list of both ends (~owner for the partner end)

@@ -10,10 +10,10 @@
 // Pair values.  rho_bar (every ordered type pair) and phi_bar depend on
 // positions and widths only; the reference caches them in force_calc.  Here
 // k_table_values evaluates them with the same quadrature as force_calc into the
-// site table: for each owned site, the entries of its own half-list row inside
-// the quadrature cut, then the entries of the lower-index sites that list it
+// site table: for each owned site, the entries of its own half-list row that can
+// have a value (table_pair), then the entries of the lower-index sites that list it
 // (ascending owner), each holding the partner index and the pair's
-// nt^2 + nt(nt+1)/2 values in the owner's orientation.  Pairs outside the cut add
+// nt^2 + nt(nt+1)/2 values in the owner's orientation.  The other pairs add
 // nothing to any sum and are left out.  Seen from site i with
 // type m and a partner k of type b, each sweep's term is the same expression
 // whichever end owns the pair (slot(b, m) for the density, slot(m, b) for the
@@ -55,6 +55,37 @@ __device__ __forceinline__ double pair_rsq(double4 xi, double4 xj) {
     return rsq;
 }
 
+// {x, y, z, largest 1/alpha} per site, ghosts included, for table_pair (infinite for a
+// width that is no number)
+template <int NT>
+__global__ void k_table_pack(const double4* __restrict__ pos, const double* __restrict__ alpha, int n,
+                             double4* __restrict__ rec) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double4 p = pos[i];
+    p.w = 1.0 / alpha[(size_t)i * NT];
+#pragma unroll
+    for (int t = 1; t < NT; ++t) {
+        const double v = 1.0 / alpha[(size_t)i * NT + t];
+        if (!(v <= p.w)) p.w = v;
+    }
+    if (!(p.w == p.w)) p.w = INFINITY;
+    rec[i] = p;
+}
+// Whether the pair can have a value: inside the quadrature cut, and its rule's nearest
+// point r - xi_max/sqrt(alpha), at the widths of the two sites, not beyond rc (by more than
+// the rounding of FP32 sums).  alpha_min sets the cut and may lie far below the widths in
+// use: with 5 points, alpha_min = 1 and widths of 60 to 120, more than half of the pairs
+// inside the cut have none.  256,000 sites so: c_d_calc after a move 2.82 ms and calc_g 1.59
+// with every pair inside the cut in the table, 1.63 and 0.69 with these; with alpha_min =
+// 25 the records cost 0.01 ms of 1.24.  The same bits from either end and in every kernel.
+__device__ __forceinline__ bool table_pair(const FFParams<double>& P, double4 xi, double4 xj, double* rsq) {
+#pragma clang fp contract(off)
+    *rsq = pair_rsq(xi, xj);
+    const double reach = P.rc + P.xi[P.no_i - 1] * sqrt(xi.w + xj.w);
+    return *rsq < P.cut_sq_mod && !(*rsq > reach * reach * (1.0 + 4e-6));
+}
+
 // rank of this lane's flag among the set flags of lower lanes of its 16-lane group,
 // and the number of set flags in the group
 __device__ __forceinline__ int group_rank16(bool flag, int l, int* total) {
@@ -65,24 +96,24 @@ __device__ __forceinline__ int group_rank16(bool flag, int l, int* total) {
     return __popc(bits & ((1u << l) - 1u));
 }
 
-// Entries per site: the pairs inside the quadrature cut of the own row (own[i]) and of
-// the reverse list, and for each reverse entry its rank among those inside the cut
+// Entries per site: the pairs of the own row (own[i]) and of the reverse list that can have
+// a value (table_pair), and for each reverse entry its rank among those
 // (16 lanes per site, strided over both ranges).
-__global__ __launch_bounds__(kBlock) void k_table_count(PairBufs L, const int* __restrict__ rowner, int natms,
-                                                        const double4* __restrict__ pos, double cut_sq,
-                                                        int* __restrict__ own, int* __restrict__ cnt,
-                                                        int* __restrict__ rrank) {
+__global__ __launch_bounds__(kBlock) void k_table_count(FFParams<double> P, PairBufs L, const int* __restrict__ rowner,
+                                                        const double4* __restrict__ rec, int* __restrict__ own,
+                                                        int* __restrict__ cnt, int* __restrict__ rrank) {
     const SiteGroup<kTableG> g;
     const int i = g.site;
-    if (i >= natms) return;
-    const double4 xi = pos[i];
+    if (i >= P.natms) return;
+    const double4 xi = rec[i];
     int c = 0, r = 0;
+    double rsq;
     for (int p = L.off[i] + g.l; p < L.off[i + 1]; p += kTableG)
-        c += pair_rsq(xi, pos[list_partner(L.nlrp[p])]) < cut_sq ? 1 : 0;
+        c += table_pair(P, xi, rec[list_partner(L.nlrp[p])], &rsq) ? 1 : 0;
     const int q1 = L.roff[i + 1];
     for (int b = L.roff[i]; b < q1; b += kTableG) {
         const int q = b + g.l;
-        const bool in = q < q1 && pair_rsq(xi, pos[rowner[q < q1 ? q : b] & ~kInsideBit]) < cut_sq;
+        const bool in = q < q1 && table_pair(P, xi, rec[rowner[q < q1 ? q : b] & ~kInsideBit], &rsq);
         int tot;
         const int rk = group_rank16(in, g.l, &tot);
         if (in) rrank[q] = r + rk;
@@ -96,8 +127,8 @@ __global__ __launch_bounds__(kBlock) void k_table_count(PairBufs L, const int* _
 }
 
 // The table: rho_bar of every ordered type pair and phi_bar for it >= jt of the pairs
-// inside the quadrature cut, written from the pair's owner to both ends' rows; zeros
-// where the reference computes nothing (alpha out of range, or the whole rule beyond
+// that can have a value, written from the pair's owner to both ends' rows; zeros where the
+// reference computes nothing (alpha out of range, or the whole rule of a type pair beyond
 // rc).  A site's row holds its own pairs in list order, then those of its reverse list
 // in that order (rrank, k_table_count).  One wavefront per site and two lanes per
 // (pair, type pair), the lanes and the arithmetic of pass 1 (k_pass1) without the
@@ -122,7 +153,7 @@ struct TableStage {
 };
 template <int NT, typename Q, int NQ>
 __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFParams<Q> PQ,
-                                                         const double4* __restrict__ pos,
+                                                         const double4* __restrict__ rec,
                                                          const double* __restrict__ alpha,
                                                          const int* __restrict__ off, const int2* __restrict__ nlrp,
                                                          const Q* __restrict__ quad, const double* __restrict__ rho7,
@@ -147,7 +178,7 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
     for (int i0 = sl.first; i0 < sl.end; i0 += sl.stride) {
         const int i = __builtin_amdgcn_readfirstlane(i0);
         const int p0 = off[i], p1 = off[i + 1];
-        const double4 xi = pos[i];
+        const double4 xi = rec[i];
         const double ai = alpha[(size_t)i * NT + it], iai = rcp_nr(ai);
         double ia_min = rcp_nr(alpha[(size_t)i * NT]), ia_max = ia_min;
 #pragma unroll
@@ -169,8 +200,7 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
                     const int2 e = nlrp[pc];
                     jc = e.x & ~kInsideBit;
                     qc = e.y;
-                    r2 = pair_rsq(xi, pos[jc]);
-                    in = r2 < P.cut_sq_mod;
+                    in = table_pair(P, xi, rec[jc], &r2);
                 }
                 const int dest = pack_dest(in, &cnt);
                 if (in) {

@@ -72,3 +72,39 @@ def test_few_and_many_pairs(tables, keep):
     _check(ff, orc, 1e-12)
     _check_rates(ff, orc, 1e-12)
     ff.close()
+
+
+@pytest.mark.parametrize("no_i", [1, 3, 5])
+@pytest.mark.parametrize("alpha_min", [0.25, 1.0, 30.0])
+@pytest.mark.parametrize("nt", [1, 2, 4])
+def test_widths_far_from_alpha_min(nt, alpha_min, no_i):
+    """the site table leaves out the pairs inside the cut (set by alpha_min) whose rules end beyond rc at
+    their own widths: with alpha_min far below the widths most pairs near the cut, with alpha_min among
+    the pair widths few (and rates beyond e^100, not compared); widths from 20 to 300.  In FP64 with tables that do not vanish at the cutoff
+    (with FP32 sums a point within rounding of it would count or not); the bars of the rates above"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    lat = W.fcc_alloy(6, nt=nt, seed=60 + no_i)
+    rng = np.random.default_rng(no_i)
+    lat.x[:, 3:] = np.exp(rng.uniform(np.log(20.0), np.log(300.0), size=lat.c.shape))
+    a = rng.uniform(-0.2, 0.2, size=lat.c.shape)
+    for precision, bound in (("fp64", 1e-12), ("mixed", 1e-5)):
+        tables = W.johnson_tables(elements=("Ni", "Cu", "Pd", "Ag")[:nt], nr=2001, nrho=2001)
+        if precision == "fp64":
+            tables.rho = tables.rho + 1e-3
+            tables.rphi = tables.rphi + 1e-3
+        ff = setup(lat, tables, no_i=no_i, precision=precision, alpha_min=alpha_min)
+        orc = O.make(lat, tables, no_i=no_i, alpha_min=alpha_min)
+        if precision == "mixed":
+            orc.force_calc(1)
+            _check_rates(ff, orc, bound, ("E", "dE"))
+        else:
+            _check(ff, orc, bound)
+            _check_rates(ff, orc, bound, ("E", "dE", "n") if alpha_min == 30.0 else ("E", "dE", "n", "c_d"))
+        if precision == "fp64" and alpha_min < 30.0:
+            cost_o, g_o = orc.calc_g(0, 0.37, a)
+            ff.set_vec("a", a)
+            assert abs(ff.calc_g(0, 0.37) - cost_o) <= bound * abs(cost_o)
+            assert rel_inf(ff.get("g"), g_o) <= bound
+        ff.close()
