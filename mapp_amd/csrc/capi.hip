@@ -2239,6 +2239,9 @@ int mapp_dmd_init(mapp_dmd_t* ctx, double skin) {
             ctx->inited = true;
             return 0;
         }
+        double bins = 1.0;  // set_ph's product in int wraps beyond 2^31
+        for (int d = 0; d < 3; ++d) bins *= (2.0 * ctx->bp.cut_ph_s[d] + 1.0) / ctx->bp.bin_size[d] + 1.0;
+        require(bins < 2147483647.0, MAPP_DMD_E_RANGE, "the box has 2^31 cutoff-sized bins or more");
         ctx->d_pos.reserve(natms);
         ctx->d_alpha.reserve((size_t)natms * nt);
         ctx->d_conc.reserve((size_t)natms * nt);

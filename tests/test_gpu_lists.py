@@ -68,3 +68,15 @@ def test_lists_of_nearly_empty_boxes(tables, L, n, squeeze):
         bound = 1e-12 if squeeze == 1.0 else 1e-11  # more pairs to a site
         assert abs(en[0] - eo[0]) <= bound * abs(eo[0]) and rel_inf(ff.get("f"), orc.get("f")) <= bound
     ff.close()
+
+
+@pytest.mark.parametrize("L", [8000.0, 9325.0])
+def test_box_with_too_many_bins_is_refused(tables, L):
+    """2.7e9 bins (negative as a 32-bit product) and 4.3e9 (a small positive one)"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import DMDError, setup
+    lat = W.fcc_alloy(2, seed=3)
+    box = W.Lattice(H=np.diag([L] * 3), x=lat.x, c=lat.c, cart=lat.x[:, :3] * L)
+    with pytest.raises(DMDError) as e:
+        setup(box, tables, no_i=3)
+    assert e.value.code == -4  # E_RANGE
