@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
     using Q2 = typename Vec2<Q>::T;
     using Map = Pass1Map<NT, 2>;
     constexpr int NPHI = NT * (NT + 1) / 2;
-    constexpr int KP = NQ > 0 ? NQ : kMaxPoints;
+    constexpr int KP = kRowPoints<NQ>;
     const int lane = threadIdx.x & 63;
     const Map map(lane);
     const int k = map.k, prt = map.prt, it = map.it, jt = map.jt;
@@ -228,30 +228,30 @@ __global__ __launch_bounds__(kBlock) void k_table_values(FFParams<double> P, FFP
                 const double r_inv = geo.y, r = geo.x * r_inv;
                 const double ia = iai + st.typ[s * NT + jt], asq = rsqrt_nr(ia);
                 const Q rq = (Q)r, inv = (Q)ia * (Q)asq;
-                const int nq = NQ > 0 ? NQ : PQ.no_i;
-                Q2 lo[KP], hi[KP];
-                Q ppv[KP];
+                Q sum[3] = {0, 0, 0};
+                for_points<NQ>(PQ.no_i, [&](int k0) {
+                    Q2 lo[KP], hi[KP];
+                    Q ppv[KP];
 #pragma unroll
-                for (int kp = 0; kp < KP; ++kp) {
-                    if (NQ == 0 && kp >= nq) break;
-                    const Q u = rq - PQ.xi[kp] * inv;
-                    int m = (int)(fabs(u) * PQ.dr_inv);
-                    m = m < P.nr - 1 ? m : P.nr - 1;  // the zero row beyond the cutoff
-                    ppv[kp] = fabs(u) * PQ.dr_inv - (Q)m;
-                    const int row = tab_off + m * (quad_stride(NT) * (int)sizeof(Q));
-                    lo[kp] = RowLoad<Q2>::get(qrs, row);
-                    hi[kp] = RowLoad<Q2>::get(qrs, row + (int)sizeof(Q2));
-                }
-                if constexpr (KP * 2 * sizeof(Q2) <= 96) __builtin_amdgcn_sched_barrier(0);
-                Q x[KP], s0, s1, s2;
+                    for (int kp = 0; kp < KP; ++kp) {
+                        const Q u = rq - PQ.xi[k0 + kp] * inv;
+                        int m = (int)(fabs(u) * PQ.dr_inv);
+                        m = m < P.nr - 1 ? m : P.nr - 1;  // the zero row beyond the cutoff
+                        ppv[kp] = fabs(u) * PQ.dr_inv - (Q)m;
+                        const int row = tab_off + m * (quad_stride(NT) * (int)sizeof(Q));
+                        lo[kp] = RowLoad<Q2>::get(qrs, row);
+                        hi[kp] = RowLoad<Q2>::get(qrs, row + (int)sizeof(Q2));
+                    }
+                    if constexpr (KP * 2 * sizeof(Q2) <= 96) __builtin_amdgcn_sched_barrier(0);
+                    Q x[KP];
 #pragma unroll
-                for (int kp = 0; kp < KP; ++kp) {
-                    if (NQ == 0 && kp >= nq) break;
-                    const Q u = rq - PQ.xi[kp] * inv, pp = ppv[kp], p2 = pp * pp;
-                    x[kp] = ((lo[kp].x + lo[kp].y * pp) + p2 * (hi[kp].x + hi[kp].y * pp)) * odd(u);
-                }
-                gh_sums<Q, NQ, false>(PQ, nq, x, &s0, &s1, &s2);
-                double v = (double)(s0 * (Q(kPiInSq) * (Q)r_inv));
+                    for (int kp = 0; kp < KP; ++kp) {
+                        const Q u = rq - PQ.xi[k0 + kp] * inv, pp = ppv[kp], p2 = pp * pp;
+                        x[kp] = ((lo[kp].x + lo[kp].y * pp) + p2 * (hi[kp].x + hi[kp].y * pp)) * odd(u);
+                    }
+                    gh_sums<Q, NQ, false>(PQ, k0, x, sum);
+                });
+                double v = (double)(sum[0] * (Q(kPiInSq) * (Q)r_inv));
                 if (!regular && keeps) {
                     const int br = alpha_branch(P, ia, ai, alpha[(size_t)st.idx[s].x * NT + jt]);
                     if (br != 1) {

@@ -52,6 +52,21 @@ def test_rules_and_schedules(nt, parts, no_i):
         ff.close()
 
 
+@pytest.mark.parametrize("no_i", [13, 14])
+def test_longest_rules(tables, no_i):
+    """the general loop at its end, with and without a point of zero weight"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    lat = W.fcc_alloy(6, seed=no_i)
+    for parts in (1, 2, 4):
+        ff, orc = setup(lat, tables, no_i=no_i), O.make(lat, tables, no_i=no_i)
+        ff.set_schedule([parts, 4, 0, 2, 0])
+        _check(ff, orc, 1e-12)
+        _check_rates(ff, orc, 1e-12)
+        ff.close()
+
+
 @pytest.mark.parametrize("keep", [1, 2, 5, 33, 200])
 def test_few_and_many_pairs(tables, keep):
     """a cluster in a large box: from no pair at all to a whole half wavefront and more"""
