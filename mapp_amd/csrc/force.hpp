@@ -478,14 +478,19 @@ struct Pass1Map {
 // src/ff_dmd_I.cpp:244-248, :376), then {partner, reverse position or -1 for a
 // ghost partner} as two ints.  The k-th inside pair of site i is pair k % kG of
 // the site's group k / kG; a group holds its kG pairs component by component, so
-// a component of a group is one 64-byte run: pass 1's lanes (pair, type pair)
-// write whole cache lines, and pass 2's lanes (one pair each) read 16-byte
-// quarters of the same 64-byte runs instead of 16-byte pieces 112 bytes apart.
+// a component of a group is one run: pass 1's lanes (pair, type pair) write it
+// whole, and pass 2's lanes (one pair each) read 16-byte pieces of the same runs
+// instead of 16-byte pieces 112 bytes apart.  A run is 64 bytes, or what one round
+// of pass 1 fills (two lanes per type pair) where that is less: runs of 64 bytes
+// that two or four rounds wrote in parts, past L2, cost four types more than the
+// rest gained -- 131,072 sites, 3 points, FP64 2.15 ms (1.89 with a record in one
+// piece) and FP32 2.01 (1.64); runs of 32 and 16 bytes, two pairs, 1.69 and 1.22.
 // Site i's groups start at off[i] / kG + i, which leaves room for every listed
 // pair in whole groups.
 template <int NT, typename Q>
 struct PairRec {
-    static constexpr int kG = 64 / (2 * (int)sizeof(Q));
+    static constexpr int kRun = 64 / (2 * (int)sizeof(Q)), kRound = Pass1Map<NT, 2>::kPPW;
+    static constexpr int kG = kRun < kRound ? kRun : kRound;
     static constexpr int kComps = NT * NT + NT * (NT + 1) / 2 + 1;
     __host__ __device__ static constexpr int rho(int q) { return q; }
     __host__ __device__ static constexpr int phi(int it, int jt) { return NT * NT + type2phi(it, jt); }

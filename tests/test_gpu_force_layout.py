@@ -52,6 +52,22 @@ def test_rules_and_schedules(nt, parts, no_i):
         ff.close()
 
 
+@pytest.mark.parametrize("nt,parts", [(1, 4), (2, 4), (3, 4), (4, 1), (4, 4)])
+def test_record_runs(nt, parts):
+    """rounds of pass 1 that write less than a run of the records, or several"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    tables = W.johnson_tables(elements=("Ni", "Cu", "Pd", "Ag")[:nt], nr=2001, nrho=2001)
+    lat = W.fcc_alloy(6, nt=nt, seed=30 + nt)
+    orc = O.make(lat, tables, no_i=3)
+    for precision, bound in (("fp64", 1e-12), ("mixed", 1e-5)):
+        ff = setup(lat, tables, no_i=3, precision=precision)
+        ff.set_schedule([parts, 4, 0, 2, 0])
+        _check(ff, orc, bound)
+        ff.close()
+
+
 @pytest.mark.parametrize("no_i", [13, 14])
 def test_longest_rules(tables, no_i):
     """the general loop at its end, with and without a point of zero weight"""
