@@ -579,6 +579,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p, int nb
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, nbytes, 0x00020000);
 }
 
+constexpr int kNoRow = 0x60000000;  // a row offset beyond any table (its reads give 0)
+
 // 1/x by the hardware estimate and two Newton steps (x normal and positive here)
 __device__ __forceinline__ double rcp_nr(double x) {
     double y = __builtin_amdgcn_rcp(x);
@@ -677,8 +679,8 @@ __device__ __forceinline__ void for_points(int no_i, F&& f) {
 // beyond the cutoff reads the table's zero row nr - 1 (u < rc exactly when
 // u/dr < nr - 1, so this is the reference's window test, src/ff_dmd_I.cpp:196-204),
 // 1/r is formed once per list entry when it is staged, and the pair widths
-// outside the quadrature regime, if a chunk has any, are put right behind one
-// uniform branch: 2.90 -> 2.68 ms at 1,048,576 sites of two types, 3-point rule,
+// outside the quadrature regime, if a chunk has any, are told before and put
+// right behind uniform branches: 2.90 -> 2.68 ms at 1,048,576 sites of two types, 3-point rule,
 // FP64, with 14% more bytes of records.  Of the 2.68 ms, 0.5 go with the record
 // stores, 0.24 with the scattered density shares and 0.2 with the rows' L1 misses.
 // Loads of the next round ahead of a round's stores (128 registers) took 2.73 ms,
@@ -706,7 +708,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const bool live = on && (PARTS == 1 || prt < PARTS / 2 || want_phi);
     // a phi lane whose phi is not kept reads its type pair's rho row instead (the same cache line)
     const int half = PARTS == 1 ? 0 : (prt >= PARTS / 2 && !want_phi ? prt - PARTS / 2 : prt) * (8 / PARTS);
-    const int tab_off = (q * kQuadRow + half) * (int)sizeof(Q);
+    // energy_calc: the lanes without a part in it (three of eight with two types) read beyond
+    // the buffer, which fetches nothing; 131,072 sites, 5 points, FP32 sums: 0.33 -> 0.29 ms
+    const int tab_off = ENERGY_ONLY && !live ? kNoRow : (q * kQuadRow + half) * (int)sizeof(Q);
     const __amdgpu_buffer_rsrc_t qrs = raw_rsrc(quad, P.nr * quad_stride(NT) * (int)sizeof(Q));
     const OddFactor<Q> odd(prt < (PARTS + 1) / 2);
     // the lane's record component; the partner goes out on a lane whose phi is not kept
@@ -796,8 +800,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                 // v1: the lane's function (rho on the rho lane, phi on the phi lane) or,
                 // with one lane per pair, rho; v2: phi with one lane per pair.
                 // Each holds value, d/dr, d/dalpha.
-                double v1[3], v2[3];
-                {
+                double v1[3] = {0.0, 0.0, 0.0}, v2[3] = {0.0, 0.0, 0.0};
+                // pair widths outside the quadrature regime, or within rounding of its bounds; a
+                // round without a lane that needs the quadrature goes past it (131,072 sites of
+                // two types, every pair classical: force_calc 0.80 -> 0.69 ms, energy_calc 0.37
+                // -> 0.28, for 0.3% of force_calc where every pair has its rule)
+                int br = 1;
+                bool some = true;
+                if (!regular) {
+                    if (live) br = alpha_branch(P, ia, ai, arec[(size_t)e.x * NT + jt].x);
+                    some = __builtin_amdgcn_ballot_w64(live && br == 1) != 0;
+                }
+                if (some) {
                     const Q rq = (Q)r, iq = (Q)ia, aq = (Q)asq, inv = iq * aq;
                     // the rows of a set of points are requested before any is used, so their
                     // latencies overlap
@@ -856,9 +870,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
                     close(sx, v1);
                     if constexpr (PARTS == 1) close(sy, v2);
                 }
-                // pair widths outside the quadrature regime, or within rounding of its bounds
                 if (!regular) {
-                    const int br = live ? alpha_branch(P, ia, ai, arec[(size_t)e.x * NT + jt].x) : 1;
                     if (br != 1) {
                         double g[3] = {0.0, 0.0, 0.0}, f[3] = {0.0, 0.0, 0.0};
                         if (br == 2 && geo.x < P.cut_sq)

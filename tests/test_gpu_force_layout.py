@@ -68,6 +68,33 @@ def test_record_runs(nt, parts):
         ff.close()
 
 
+@pytest.mark.parametrize("nt,parts", [(1, 2), (2, 1), (2, 2), (2, 4), (3, 2), (4, 2)])
+@pytest.mark.parametrize("lo,hi,odd", [(3000.0, 4000.0, 0), (10.0, 20.0, 0), (3000.0, 4000.0, 3), (10.0, 20.0, 3)])
+def test_rounds_without_quadrature(nt, parts, lo, hi, odd):
+    """every pair classical, or every pair skipped (rounds that evaluate no rule), and all but those of
+    neighbouring cells; energy_calc over the triangle and over every ordered pair (lanes that fetch no row)"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    from oracle import oracle as O
+    tables = W.johnson_tables(elements=("Ni", "Cu", "Pd", "Ag")[:nt], nr=2001, nrho=2001)
+    lat = W.fcc_alloy(6, nt=nt, seed=70 + nt, alpha_lo=lo, alpha_hi=hi)
+    if odd:
+        lat.x[: 4 * odd, 3:] = 60.0 if lo < 100.0 else 500.0
+    orc = O.make(lat, tables, no_i=3)
+    for precision, bound in (("fp64", 1e-12), ("mixed", 1e-5)):
+        ff = setup(lat, tables, no_i=3, precision=precision)
+        ff.set_schedule([parts, 4, 0, 2, 0])
+        _check(ff, orc, bound)
+        for full in (False, True):
+            ff.set_energy_mode(full)
+            orc.set_energy_full(full)
+            e, eo = ff.energy_calc(), orc.energy_calc()
+            assert abs(e - eo) <= bound * abs(eo)
+        ff.set_energy_mode(False)
+        orc.set_energy_full(False)
+        ff.close()
+
+
 @pytest.mark.parametrize("no_i", [13, 14])
 def test_longest_rules(tables, no_i):
     """the general loop at its end, with and without a point of zero weight"""
