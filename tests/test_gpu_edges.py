@@ -142,6 +142,46 @@ def test_tilted_box(tables):
     assert len(nl) > 30 * lat.natms
 
 
+@pytest.mark.parametrize("md", [False, True])
+def test_moves_in_a_tilted_box(tables, md):
+    """positions moved inside the skin: ghosts follow by H[d][0..d] of each face they crossed, over edges
+    and corners; then past it.  Ghosts bit for bit, forces as above"""
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup, setup_eam
+    from oracle import oracle as O
+    n, a = 6, 3.6
+    cube = W.fcc_alloy(n, a=a, seed=55)
+    L = a * n
+    H = np.array([[L, 0.0, 0.0], [2 * a, L, 0.0], [a, -a, L]])
+    lat = _lattice_from_cart(H, cube.cart, cube.x[:, 3:], cube.c)
+    if md:
+        t = (np.arange(lat.natms) % 3 == 0).astype(np.float64)
+        ff = setup_eam(H, lat.x[:, :3].copy(), t, tables)
+        orc = O.Oracle(nt=2, variant="EAM")
+        orc.set_fs(tables)
+        orc.set_params(masses=tables.masses)
+        orc.set_system(H, lat.x[:, :3].copy(), t.reshape(-1, 1))
+        orc.init(0.5)
+    else:
+        ff, orc = setup(lat, tables), O.make(lat, tables)
+    rng = np.random.default_rng(5)
+    x = ff.get("x")
+    for far in (False, True):
+        x[:, :3] += rng.uniform(-0.04, 0.04, size=(lat.natms, 3))
+        x[:, 3:] *= rng.uniform(0.98, 1.02, size=(lat.natms, x.shape[1] - 3))
+        if far:
+            x[11, 1] += 0.7
+        assert ff.set_x(x) is far and orc.set_x(x) is far
+        (gx, gsrc), (ox, osrc) = ff.ghosts(), orc.ghosts()
+        assert np.array_equal(gsrc, osrc) and np.array_equal(gx.view(np.uint64), ox.view(np.uint64))
+        for g, o in zip(ff.neighbor_list(), orc.neighbor_list()):
+            assert np.array_equal(g, o)
+        eg, eo = ff.force_calc(1), orc.force_calc(1)
+        assert abs(eg[0] - eo[0]) <= 1e-12 * abs(eo[0]) and rel_inf(eg[1:], eo[1:]) <= 1e-12
+        assert rel_inf(ff.get("f"), orc.get("f")) <= 1e-12
+    ff.close()
+
+
 def test_cluster_in_vacuum(tables):
     """a 3^3-cell FCC cluster (108 sites) in a 40 A box plus four isolated
     sites farther than the list cut from every other site and image"""

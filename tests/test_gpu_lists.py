@@ -1,14 +1,27 @@
 """The neighbour lists where the build can go wrong: boxes hardly wider than the
-ghost shell (a site is a ghost at both faces), a few candidates per site, more than the kept accept bits cover (1024) and more than one group of 64
-rounds (4096); rows and reverse lists of more than 64 entries.  Lists, ghosts
-and the 2nd list are the oracle's, entry for entry; the reverse list is what the
-densities of partners come from (a few thousand double roundings)."""
+ghost shell (a site is a ghost at both faces), a few candidates per site, more
+than the kept accept bits cover (1024) and more than one group of 64 rounds
+(4096); rows and reverse lists of more than 64 entries; boxes with far more bins
+than sites, and crowded bins.  Lists, ghosts and the 2nd list are the oracle's,
+entry for entry; the reverse list is what the densities of partners come from
+(a few thousand double roundings)."""
 import numpy as np
 import pytest
 
 from tests.conftest import rel_inf
 
 pytestmark = pytest.mark.gpu
+
+
+def _most_candidates(orc, L, cut):
+    """sites and ghosts in the 27 bins (of the shell's width) around an owned site, the largest number"""
+    w = cut / L
+    b = ((orc.x_all()[:, :3] / L + w) / w).astype(int) + 1
+    cnt = np.zeros(b.max(axis=0) + 2, dtype=int)
+    np.add.at(cnt, tuple(b.T), 1)
+    g = (-1, 0, 1)
+    around = sum(np.roll(cnt, (i, j, k), (0, 1, 2)) for i in g for j in g for k in g)
+    return around[tuple(b[: orc.natms].T)].max()
 
 
 @pytest.mark.parametrize("n,a", [(2, 3.6), (4, 1.8), (5, 2.4), (6, 1.45), (7, 3.6), (3, 5.0)])
@@ -28,7 +41,16 @@ def test_lists_of_sparse_and_dense_boxes(tables, n, a):
             assert np.array_equal(g, w)
     off, nl = pairs[0][0]
     owned = np.bincount(nl[nl < len(off) - 1], minlength=1)
-    print(n, a, "row", np.diff(off).max(), "reverse", owned.max(initial=0), flush=True)
+    # the branch each box stands for
+    most = _most_candidates(orc, n * a, tables.rc + 1.2247448713915890 / 5.0 + 0.5)  # alpha_min = 25, skin 0.5
+    if a == 1.45:
+        assert most > 4096
+    elif a in (1.8, 2.4):
+        assert 1024 < most <= 4096
+    else:
+        assert most <= 1024
+    if a < 3.0:
+        assert np.diff(off).max() > 64 and owned.max() > 64
     ff.c_d_calc()
     orc.c_d_calc()
     for name in ("E", "dE", "n"):  # the rates of the dense boxes overflow
