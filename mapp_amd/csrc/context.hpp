@@ -26,8 +26,10 @@ struct mapp_dmd {
     mappdmd::DevBuf<double> d_mtab, d_mrec;  // MEAM pair table, per-site records [ntot][38]
     mappdmd::DevBuf<double4> d_mpairs;       // MEAM per list entry {fc, S, dS, dU/dS}
     mappdmd::DevBuf<double4> d_mforce;       // MEAM force of each entry that screening leaves
-    mappdmd::DevBuf<int> d_mactive, d_mact;  // MEAM: per site the count and list positions of its own
-                                             // entries (j > i) with dU/dS != 0 and 0 < S fc < 1
+    // MEAM: per site the count and list positions of some of its entries, in list order: from
+    // k_meam_density to k_meam_three those that screening leaves (S != 0, either direction),
+    // from then on its own (j > i) whose screening moves other atoms (dU/dS != 0)
+    mappdmd::DevBuf<int> d_mactive, d_mact;
     mappdmd::FFParams<float> Pf{};
     double rsq_crd = 0, mod_rc = 0;
     double wi1_ref[mappdmd::kMaxPoints]{}, wi2_ref[mappdmd::kMaxPoints]{};
@@ -82,7 +84,7 @@ struct mapp_dmd {
     mappdmd::DevBuf<double> d_part, d_xaos, d_stage;
     double* h_box = nullptr;  // pinned host memory for the scalars a call's last kernel writes (64 doubles)
     mappdmd::DevBuf<int> d_iflag;
-    mappdmd::DevBuf<unsigned long long> d_scan;  // tile sums of exclusive_scan
+    mappdmd::DevBuf<unsigned long long> d_scan;  // tile sums of scan(), then their total
     long n_inrange = 0;
 
     // learned surrogate

@@ -384,12 +384,6 @@ __device__ __forceinline__ int pack_dest(bool in, int* count) {
     return in ? rank : cnt + (lane - rank);
 }
 __device__ __forceinline__ int packed(int dest, int v) { return __builtin_amdgcn_ds_permute(dest << 2, v); }
-__device__ __forceinline__ double packed(int dest, double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_ds_permute(dest << 2, (int)(b & 0xffffffffLL));
-    const int hi = __builtin_amdgcn_ds_permute(dest << 2, (int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 __device__ __forceinline__ int pack_in_range(int p, bool in, int* out) {
     int cnt;
     *out = packed(pack_dest(in, &cnt), p);
@@ -425,8 +419,9 @@ __device__ __forceinline__ int pack_in_range(int p, bool in, int* out) {
 // and the phi lane {dphi/dr, dphi/dalpha} in the pair's record (PairRec; the
 // reference's per-pair caches, src/ff_dmd_I.cpp:227-242, restricted to what the
 // back-pass reads), for the site's pairs inside the quadrature cut, whose number
-// goes to info with the site's list offset.  The phi lanes of the type pairs it < jt do not evaluate: the
-// back-pass takes their phi from the transposed pair.
+// goes to info with the site's list offset.  The phi lanes of the type pairs it < jt
+// have no value of their own: the back-pass takes their phi from the transposed pair.
+//
 // Lanes of pass 1.  In general lane l works on pair slot k = l / kLPP and, within it,
 // on part prt of type pair q: lane k*kLPP + q*PARTS + prt.
 // Three types with two lanes per type pair have their own map: of the 18 lanes of
@@ -1164,9 +1159,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT <= 2 
             vir[3] -= wf * (h1 * dx2);
             vir[4] -= wf * (h2 * dx0);
             vir[5] -= wf * (h0 * dx1);
-            // partner shares: the two lanes of a pair of lanes write the 16-byte halves
-            // {fx, fy}, {fz, alpha force 0} of one share together, first the even lane's
-            // pair, then the odd lane's (32 contiguous bytes each)
+            // the partner's share (ForceShare)
             double out[ForceShare<NT>::kLen] = {S};
 #pragma unroll
             for (int t = 0; t < NT; ++t) out[1 + t] = aJ[t];
