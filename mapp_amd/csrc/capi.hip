@@ -268,6 +268,12 @@ __global__ void k_quirk_cell(int n, int g, int own_base, int gh_dst, int nt, int
     }
 }
 
+// doubles of the force shares of the reverse list
+template <int NT>
+size_t share_doubles(const mapp_dmd* ctx) {
+    return (size_t)(ctx->nrev + 1) * (is_md(ctx) ? 1 : ForceShare<NT>::kLen);
+}
+
 // ghosts + bins + s->x + half list + reverse list; positions hold s on entry
 template <int NT>
 void rebuild(mapp_dmd* ctx) {
@@ -276,6 +282,14 @@ void rebuild(mapp_dmd* ctx) {
     build_ghosts<NT>(ctx);
     const int ntot = natms + ctx->nghost;
     hipStream_t st = ctx->stream;
+    // What the build alone needs lies in buffers that it or the next evaluation writes anew:
+    // positions in bin order in d_arec, unsorted owners in d_pairF, and in d_rowner, until the
+    // owners are sorted, the accept bits (room for 48 owners a site, or no more than the bits
+    // where the list is full and has none, so that the first build allocates it once).
+    ctx->d_arec.reserve((size_t)ntot * (is_md(ctx) ? 1 : NT));
+    constexpr size_t kMaskInts = kMaskWords * sizeof(unsigned long long) / sizeof(int);
+    static_assert(kMaskInts <= 48, "the accept bits fit");
+    double4* const bin_pos = ctx->d_arec.p;
     // bins
     ctx->d_bin_of.reserve(ntot);
     ctx->d_bin_slot.reserve(ntot);
@@ -283,7 +297,6 @@ void rebuild(mapp_dmd* ctx) {
     ctx->d_bin_start.reserve((size_t)bp.tot_bin + 1);
     ctx->d_arrived.reserve(ntot);
     ctx->d_bin_atoms.reserve(ntot);
-    ctx->d_bin_pos.reserve(ntot);
     HIP_OK(hipMemsetAsync(ctx->d_bin_cnt.p, 0, sizeof(int) * (bp.tot_bin + 1), st));
     hipLaunchKernelGGL(k_s2bin, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_pos.p, ntot, bp, ctx->d_bin_of.p,
                        ctx->d_bin_cnt.p, ctx->d_bin_slot.p);
@@ -293,15 +306,15 @@ void rebuild(mapp_dmd* ctx) {
                        ctx->d_bin_start.p, ctx->d_bin_slot.p, ctx->d_arrived.p);
     launch_check("k_bin_fill");
     hipLaunchKernelGGL(k_bin_place, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_arrived.p, ntot, ctx->d_bin_of.p,
-                       ctx->d_bin_start.p, bp, ctx->d_conc.p, ctx->d_pos.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p);
+                       ctx->d_bin_start.p, bp, ctx->d_conc.p, ctx->d_pos.p, ctx->d_bin_atoms.p, bin_pos);
     launch_check("k_bin_place");
     // half list and reverse list
     ctx->d_cnt.reserve(natms + 1);
     ctx->d_rcnt.reserve(natms + 1);
     ctx->d_off.reserve(natms + 1);
     ctx->d_roff.reserve(natms + 1);
-    ctx->d_list_mask.reserve((size_t)natms * kMaskWords);
-    HalfLists L{ctx->d_list_mask.p, ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p, ctx->d_roff.p, nullptr, nullptr};
+    ctx->d_rowner.reserve((size_t)natms * (bp.full ? kMaskInts : 48));
+    HalfLists L{reinterpret_cast<unsigned long long*>(ctx->d_rowner.p), ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p, ctx->d_roff.p, nullptr, nullptr};
     int nbin = bp.tot_bin;
     const int* bins = nullptr;
     double per_bin = (double)natms * bp.bin_size[0] * bp.bin_size[1] * bp.bin_size[2];  // in a filled box
@@ -324,7 +337,7 @@ void rebuild(mapp_dmd* ctx) {
     constexpr int kMaxX = 1 << 23;
     const dim3 grid(std::min(nbin, kMaxX), bin_blocks(per_bin), (nbin + kMaxX - 1) / kMaxX), blk(64 * kBinWaves);
     hipLaunchKernelGGL((bp.pairwise ? k_half_list<false, true> : k_half_list<false, false>), grid, blk, 0, st, natms,
-                       bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
+                       bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, bin_pos, bp, L);
     launch_check("k_half_list count");
     scan(ctx, kScanA, ctx->d_cnt.p, ctx->d_off.p, natms, true);
     scan(ctx, kScanB, ctx->d_rcnt.p, ctx->d_roff.p, natms, true);
@@ -332,16 +345,20 @@ void rebuild(mapp_dmd* ctx) {
     ctx->npairs = scan_total(ctx, kScanA);
     ctx->nrev = scan_total(ctx, kScanB);
     ctx->d_nl.reserve(ctx->npairs + 1);
-    ctx->d_rowner.reserve(ctx->nrev + 1);
-    ctx->d_rtmp.reserve(ctx->nrev + 1);
+    ctx->d_pairF.reserve(share_doubles<NT>(ctx));
+    int* const owners = reinterpret_cast<int*>(ctx->d_pairF.p);
     L.nl = ctx->d_nl.p;
-    L.rlist = ctx->d_rtmp.p;
+    L.rlist = owners;
     hipLaunchKernelGGL((bp.pairwise ? k_half_list<true, true> : k_half_list<true, false>), grid, blk, 0, st, natms,
-                       bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, ctx->d_bin_pos.p, bp, L);
+                       bins, nbin, ctx->d_bin_start.p, ctx->d_bin_atoms.p, bin_pos, bp, L);
     launch_check("k_half_list fill");
+    if ((size_t)ctx->nrev + 1 > ctx->d_rowner.cap) {
+        wait_box(ctx);  // the fill reads the bits there
+        ctx->d_rowner.reserve(ctx->nrev + 1);
+    }
     if (ctx->nrev > 0) {
         hipLaunchKernelGGL(k_sort_owners, dim3(nblk((long)natms * 64)), dim3(kBlock), 0, st, natms, ctx->d_roff.p,
-                           ctx->d_rtmp.p, ctx->d_rowner.p);
+                           owners, ctx->d_rowner.p);
         launch_check("k_sort_owners");
     }
     if (ctx->variant == MAPP_DMD_VARIANT_MEAM) finish_meam(ctx);
@@ -382,12 +399,10 @@ void finish_lists(mapp_dmd* ctx) {
     ctx->d_f.reserve((size_t)natms * (3 + NT));
     ctx->d_fown.reserve((size_t)natms * (3 + NT));
     ctx->d_pairE.reserve((size_t)(nrev + 1) * NT);
-    if (is_md(ctx)) {
-        ctx->d_pairF.reserve(nrev + 1);
-    } else {
+    ctx->d_pairF.reserve(share_doubles<NT>(ctx));
+    if (!is_md(ctx)) {
         // pass 1's records in either quadrature type
         using R = PairRec<NT, double>;
-        ctx->d_pairF.reserve((size_t)(nrev + 1) * ForceShare<NT>::kLen);
         // every pair starts outside the quadrature cut with a zero density share
         HIP_OK(hipMemsetAsync(ctx->d_pairE.p, 0, sizeof(double) * (size_t)(nrev + 1) * NT, st));
         ctx->d_deriv.reserve(R::groups(ctx->npairs, natms) * R::kG * R::kComps);

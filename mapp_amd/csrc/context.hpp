@@ -53,11 +53,8 @@ struct mapp_dmd {
     mappdmd::DevBuf<int> d_ghost_src, d_ghost_owner;
     // binning and lists
     mappdmd::DevBuf<int> d_flag, d_offs, d_bin_of, d_bin_cnt, d_bin_slot, d_bin_start, d_bin_atoms, d_arrived, d_bin_list;
-    mappdmd::DevBuf<double4> d_bin_pos;               // positions in bin order
-    mappdmd::DevBuf<unsigned long long> d_list_mask;  // accept bits of the list build
     mappdmd::DevBuf<int> d_cnt, d_rcnt, d_off, d_nl, d_roff;
     mappdmd::DevBuf<int> d_off2, d_nl2, d_crd;
-    mappdmd::DevBuf<int> d_rtmp;  // owners of the reverse lists before they are sorted
     mappdmd::DevBuf<double2> d_deriv;  // pass 1's records (PairRec) of the quadrature type
     mappdmd::DevBuf<int2> d_info;      // [natms] {list offset, pairs inside the cut at the last force pass 1}
     mappdmd::DevBuf<double4> d_arec;   // [ntot][nt] {alpha, c, 1/alpha, dE}; MD potentials [ntot] {x, y, z, type, then F'};

@@ -79,7 +79,8 @@ struct ApiError {
     ApiError(int c, std::string m) : code(c), msg(std::move(m)) {}
 };
 
-// Minimal owning device buffer (capacity grows, contents not preserved unless asked).
+// Minimal owning device buffer (capacity grows, contents not preserved unless asked).  A
+// sixteenth is kept in hand: list lengths of a moving system vary by less.
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
@@ -95,7 +96,7 @@ struct DevBuf {
     }
     void reserve(size_t n, bool keep = false, hipStream_t s = nullptr) {
         if (n <= cap) return;
-        size_t nc = n + n / 8 + 64;
+        size_t nc = n + n / 16 + 64;
         T* q = nullptr;
         HIP_OK(hipMalloc(&q, nc * sizeof(T)));
         if (keep && p && cap) HIP_OK(hipMemcpyAsync(q, p, cap * sizeof(T), hipMemcpyDeviceToDevice, s));

@@ -153,3 +153,28 @@ def test_one_type_everything_tiled(one_type):
     assert abs(cost_b - NREP * cost_s) <= 1e-12 * abs(NREP * cost_s)
     assert rel_inf(fs.get("g"), g_o) <= 1e-12
     assert _per_site(fs.get("g"), fb.get("g")) <= 1e-12
+
+
+def test_memory_of_a_large_box(tables):
+    """device memory that a two-type DMD context takes for its lists and force_calc: 9.1 kB a site, so
+    that 31 million sites fit the 288 GB of one GPU (the list build's own arrays share the force passes')"""
+    import ctypes as C
+
+    from mapp_amd import workload as W
+    from mapp_amd.dmd import setup
+    lat = W.fcc_alloy(64, seed=1)
+    setup(W.fcc_alloy(2, seed=1), tables, no_i=3).close()  # the device is in use
+    hip = C.CDLL("libamdhip64.so.7")  # the library's own runtime, loaded already
+
+    def free():
+        n, total = C.c_size_t(0), C.c_size_t(0)
+        assert hip.hipMemGetInfo(C.byref(n), C.byref(total)) == 0
+        return n.value
+
+    before = free()
+    ff = setup(lat, tables, no_i=3)
+    ff.force_calc(1)
+    used = (before - free()) / lat.natms
+    print("bytes per site", used, flush=True)
+    ff.close()
+    assert used < 9250.0
