@@ -184,7 +184,7 @@ struct ForceSums {
     }
 };
 
-// Pass 1 is bound by the gathers of positions and table rows (L2).  At 1,048,576 sites
+// Pass 1 is bound by the gathers of positions and table rows (L2; TA 86% busy).  At 1,048,576 sites
 // of two EAM types (41 million list entries): 0.74 ms, pass 2 0.41 and the gather 0.18;
 // with rows of 7 coefficients, one entry at a time and both shares as vectors they took
 // 1.27, 0.65 and 0.28.  kEamR = 2 gives 0.76, 0.45, 0.21; 4 gives 0.77, 0.46, 0.20.

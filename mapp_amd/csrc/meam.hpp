@@ -263,8 +263,8 @@ __device__ __forceinline__ double wave_sums32(const double* v, int lane) {
 }
 
 // pass 1: screening, the entries it leaves and the density sums; ENERGY adds the pair
-// energy at half weight per direction (energy_calc, :2148-2589).  Bound by the screening
-// walk.  At 131,072 sites 0.82 ms; 1.03 when each of the 30 sums was summed by itself and
+// energy at half weight per direction (energy_calc, :2148-2589).  Bound by the divergent
+// screening walk (vector ALU 61% busy, 0.4 TB/s).  At 131,072 sites 0.82 ms; 1.03 when each of the 30 sums was summed by itself and
 // one lane of the wavefront closed the site (k_meam_close: 0.015 ms).
 template <bool ENERGY>
 __global__ __launch_bounds__(kBlock) void k_meam_density(MeamDev M, const double4* __restrict__ pos,
@@ -425,8 +425,9 @@ __global__ __launch_bounds__(kBlock) void k_meam_close(MeamDev M, const double* 
 // = energy, virial.  fm: the force of each entry that screening leaves, pairs[].w its
 // dU/dS where that moves other atoms.
 //
-// Bound by its FP64 work (some 1300 instructions per entry and 300 registers, one
-// wavefront per SIMD).  Screening leaves few of a list's entries, so a wavefront takes
+// Bound by the latency of its loads (247 per wavefront, the two 38-double records of an
+// entry above all) at one wavefront per SIMD: some 1300 instructions per entry keep 312
+// registers, and the vector ALU is 25% busy.  Screening leaves few of a list's entries, so a wavefront takes
 // those of `sites` sites one after the other, as many as leave every SIMD a wavefront,
 // up to kMeamPairSites.  At 131,072 sites: 0.23 ms with 16 (0.29 with 8; 0.37 held to
 // half the registers), and 0.47 for k_meam_three; both in one kernel with a wavefront
