@@ -100,7 +100,10 @@ enum ScanSlot { kScanA = 0, kScanB = 1, kScanFree = 2 };  // kScanFree: the tota
 unsigned long long* scan_box(mapp_dmd* ctx, ScanSlot slot) {
     return reinterpret_cast<unsigned long long*>(ctx->h_box) + 2 * slot;
 }
-void scan(mapp_dmd* ctx, ScanSlot slot, const int* in, int* out, long n, bool end, long mid = -1) {
+// *aux (optional, device) goes to scan_aux.
+int* scan_aux(mapp_dmd* ctx) { return reinterpret_cast<int*>(ctx->h_box + 6); }
+void scan(mapp_dmd* ctx, ScanSlot slot, const int* in, int* out, long n, bool end, long mid = -1,
+          const int* aux = nullptr) {
     unsigned long long* box = scan_box(ctx, slot);
     if (n <= 0) {
         if (end) HIP_OK(hipMemsetAsync(out, 0, sizeof(int), ctx->stream));
@@ -113,7 +116,7 @@ void scan(mapp_dmd* ctx, ScanSlot slot, const int* in, int* out, long n, bool en
     hipLaunchKernelGGL(k_scan_tile, dim3(nb), dim3(kScanThreads), 0, ctx->stream, in, out, sums, n);
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanSumThreads), 0, ctx->stream, sums, nb, sums + nb);
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kScanThreads), 0, ctx->stream, out, sums, n, sums + nb,
-                       end ? out + n : (int*)nullptr, mid, box);
+                       end ? out + n : (int*)nullptr, mid, box, aux, scan_aux(ctx));
     launch_check("k_scan");
 }
 // Refused when the total does not fit the int offsets.
@@ -219,7 +222,7 @@ void build_ghosts(mapp_dmd* ctx) {
         hipLaunchKernelGGL(k_ghost_flag, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, ctx->d_pos.p, n, idim,
                            bp.s_ph_lo[idim], bp.s_ph_hi[idim], ctx->d_flag.p);
         launch_check("k_ghost_flag");
-        scan(ctx, kScanA, ctx->d_flag.p, ctx->d_offs.p, 2 * (long)n, false, n);
+        scan(ctx, kScanA, ctx->d_flag.p, ctx->d_offs.p, 2 * (long)n, false, n, ctx->d_bin_cnt.p + bp.tot_bin);
         wait_box(ctx);
         const int cnt = (int)scan_total(ctx, kScanA), cnt_lo = (int)scan_mid(ctx, kScanA);
         const int need = n + cnt;
@@ -279,9 +282,21 @@ template <int NT>
 void rebuild(mapp_dmd* ctx) {
     BoxParams& bp = ctx->bp;
     const int natms = ctx->natms;
-    build_ghosts<NT>(ctx);
-    const int ntot = natms + ctx->nghost;
     hipStream_t st = ctx->stream;
+    // the owned sites' bins, counted while the ghosts are built
+    ctx->d_bin_of.reserve(natms);
+    ctx->d_bin_slot.reserve(natms);
+    ctx->d_bin_cnt.reserve((size_t)bp.tot_bin + 1);
+    HIP_OK(hipMemsetAsync(ctx->d_bin_cnt.p, 0, sizeof(int) * ((size_t)bp.tot_bin + 1), st));
+    auto bin = [&](int first, int n) {
+        if (n <= first) return;
+        hipLaunchKernelGGL(k_s2bin, dim3(nblk(n - first)), dim3(kBlock), 0, st, ctx->d_pos.p, first, n, bp,
+                           ctx->d_bin_of.p, ctx->d_bin_cnt.p, ctx->d_bin_slot.p);
+        launch_check("k_s2bin");
+    };
+    bin(0, natms);
+    build_ghosts<NT>(ctx);
+    const int ntot = natms + ctx->nghost, nocc = *scan_aux(ctx);  // bins with an owned site
     // What the build alone needs lies in buffers that it or the next evaluation writes anew:
     // positions in bin order in d_arec, unsorted owners in d_pairF, and in d_rowner, until the
     // owners are sorted, the accept bits (room for 48 owners a site, or no more than the bits
@@ -291,16 +306,12 @@ void rebuild(mapp_dmd* ctx) {
     static_assert(kMaskInts <= 48, "the accept bits fit");
     double4* const bin_pos = ctx->d_arec.p;
     // bins
-    ctx->d_bin_of.reserve(ntot);
-    ctx->d_bin_slot.reserve(ntot);
-    ctx->d_bin_cnt.reserve(bp.tot_bin + 1);
+    ctx->d_bin_of.reserve(ntot, true, st);
+    ctx->d_bin_slot.reserve(ntot, true, st);
     ctx->d_bin_start.reserve((size_t)bp.tot_bin + 1);
     ctx->d_arrived.reserve(ntot);
     ctx->d_bin_atoms.reserve(ntot);
-    HIP_OK(hipMemsetAsync(ctx->d_bin_cnt.p, 0, sizeof(int) * (bp.tot_bin + 1), st));
-    hipLaunchKernelGGL(k_s2bin, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_pos.p, ntot, bp, ctx->d_bin_of.p,
-                       ctx->d_bin_cnt.p, ctx->d_bin_slot.p);
-    launch_check("k_s2bin");
+    bin(natms, ntot);
     scan(ctx, kScanFree, ctx->d_bin_cnt.p, ctx->d_bin_start.p, bp.tot_bin, true);  // the total is ntot
     hipLaunchKernelGGL(k_bin_fill, dim3(nblk(ntot)), dim3(kBlock), 0, st, ctx->d_bin_of.p, ntot,
                        ctx->d_bin_start.p, ctx->d_bin_slot.p, ctx->d_arrived.p);
@@ -314,25 +325,27 @@ void rebuild(mapp_dmd* ctx) {
     ctx->d_off.reserve(natms + 1);
     ctx->d_roff.reserve(natms + 1);
     ctx->d_rowner.reserve((size_t)natms * (bp.full ? kMaskInts : 48));
-    HalfLists L{reinterpret_cast<unsigned long long*>(ctx->d_rowner.p), ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p, ctx->d_roff.p, nullptr, nullptr};
+    HalfLists L{reinterpret_cast<unsigned long long*>(ctx->d_rowner.p), ctx->d_cnt.p, ctx->d_rcnt.p, ctx->d_off.p,
+                ctx->d_roff.p, nullptr, nullptr};
     int nbin = bp.tot_bin;
     const int* bins = nullptr;
-    double per_bin = (double)natms * bp.bin_size[0] * bp.bin_size[1] * bp.bin_size[2];  // in a filled box
     if (nbin > kFewBins && nbin > natms / 4) {
         ctx->d_flag.reserve(nbin);
         ctx->d_offs.reserve(nbin);
         ctx->d_bin_list.reserve(natms);
         hipLaunchKernelGGL(k_bin_owned, dim3(nblk(nbin)), dim3(kBlock), 0, st, ctx->d_bin_start.p, ctx->d_bin_atoms.p,
                            nbin, natms, ctx->d_flag.p);
-        scan(ctx, kScanA, ctx->d_flag.p, ctx->d_offs.p, nbin, false);
+        scan(ctx, kScanFree, ctx->d_flag.p, ctx->d_offs.p, nbin, false);
         hipLaunchKernelGGL(k_bin_list, dim3(nblk(nbin)), dim3(kBlock), 0, st, ctx->d_flag.p, ctx->d_offs.p, nbin,
                            ctx->d_bin_list.p);
         launch_check("k_bin_list");
-        wait_box(ctx);
-        nbin = (int)scan_total(ctx, kScanA);
+        nbin = nocc;
         bins = ctx->d_bin_list.p;
-        per_bin = (double)natms / nbin;
     }
+    // owned sites to a full bin: the mean over the occupied ones, or that of a filled box,
+    // whose outermost bins hold less
+    const double per_bin =
+        std::max((double)natms / nocc, (double)natms * bp.bin_size[0] * bp.bin_size[1] * bp.bin_size[2]);
     // in x at most 2^23 blocks (of 256 threads: a launch holds fewer than 2^32), the rest in z
     constexpr int kMaxX = 1 << 23;
     const dim3 grid(std::min(nbin, kMaxX), bin_blocks(per_bin), (nbin + kMaxX - 1) / kMaxX), blk(64 * kBinWaves);

@@ -95,11 +95,12 @@ __global__ __launch_bounds__(kScanSumThreads) void k_scan_sums(unsigned long lon
 }
 
 // adds the tile sums; *end (optional) = the total; host[0] = the total and, with
-// mid >= 0, host[1] = out[mid]
+// mid >= 0, host[1] = out[mid]; *aux (optional) to *host_aux
 __global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ out,
                                                            const unsigned long long* __restrict__ add, long n,
                                                            const unsigned long long* __restrict__ total,
-                                                           int* __restrict__ end, long mid, unsigned long long* host) {
+                                                           int* __restrict__ end, long mid, unsigned long long* host,
+                                                           const int* __restrict__ aux, int* host_aux) {
     const long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
     const int a = (int)add[blockIdx.x];
 #pragma unroll
@@ -114,6 +115,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_add(int* __restrict__ out
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (end) *end = (int)*total;
         host[0] = *total;
+        if (aux) *host_aux = *aux;
     }
 }
 
@@ -238,21 +240,30 @@ __global__ void k_x2s(double4* __restrict__ pos, int n, BoxParams bp) {
 }
 
 // ---- cell binning (reduced coordinates) -----------------------------------
-// slot[i] = the arrival number of atom i in its bin (arbitrary: atomics)
-__global__ void k_s2bin(const double4* __restrict__ pos, int n, BoxParams bp, int* __restrict__ bin_of,
-                        int* __restrict__ bin_cnt, int* __restrict__ slot) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double4 s = pos[i];
-    int no = 0;
+// slot[i] = the arrival number of atom i in its bin (arbitrary: atomics); the atoms are
+// [first, n).  bin_cnt[bp.tot_bin] += the bins that were empty (the owned sites come first,
+// so after their launch it is the number of bins with an owned site).
+__global__ __launch_bounds__(256) void k_s2bin(const double4* __restrict__ pos, int first, int n, BoxParams bp,
+                                               int* __restrict__ bin_of, int* __restrict__ bin_cnt,
+                                               int* __restrict__ slot) {
+    const int i = first + blockIdx.x * blockDim.x + threadIdx.x;
+    int opened = 0;
+    if (i < n) {
+        double4 s = pos[i];
+        int no = 0;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        int t = (int)((comp3c(s, d) + bp.cut_ph_s[d] - 0.0) / bp.bin_size[d]);
-        t = t < 0 ? 0 : (t > bp.grid[d] - 1 ? bp.grid[d] - 1 : t);  // in range for valid input
-        no += t * bp.denom[d];
+        for (int d = 0; d < 3; ++d) {
+            int t = (int)((comp3c(s, d) + bp.cut_ph_s[d] - 0.0) / bp.bin_size[d]);
+            t = t < 0 ? 0 : (t > bp.grid[d] - 1 ? bp.grid[d] - 1 : t);  // in range for valid input
+            no += t * bp.denom[d];
+        }
+        bin_of[i] = no;
+        const int at = atomicAdd(&bin_cnt[no], 1);
+        slot[i] = at;
+        opened = at == 0 ? 1 : 0;
     }
-    bin_of[i] = no;
-    slot[i] = atomicAdd(&bin_cnt[no], 1);
+    const int total = __syncthreads_count(opened);
+    if (threadIdx.x == 0 && total) atomicAdd(&bin_cnt[bp.tot_bin], total);
 }
 
 __global__ void k_bin_fill(const int* __restrict__ bin_of, int n, const int* __restrict__ bin_start,
@@ -314,9 +325,9 @@ __global__ void k_bin_place(const int* __restrict__ v, int n, const int* __restr
 // per 1,000 empty bins in either launch, up to the launch limit of 2^24 blocks of this
 // size.  So where there are more than kFewBins bins, and more than a quarter of the sites
 // (a filled box has some 16 sites to a bin), the launch goes over the list of the bins
-// that hold an owned site; three small launches and a wait make it, about 27 us.  864
-// sites in a box of 500 A (730,000 bins), rebuild with the host's part: 478 -> 235 us; in
-// one of 1,000 A (5.6 million bins) 2,534 -> 278 us.
+// that hold an owned site, which five small launches make.  864 sites in a box of 500 A
+// (730,000 bins), rebuild with the host's part: 478 -> 212 us; in one of 1,000 A (5.6
+// million bins) 2,534 -> 264 us.
 constexpr long kFewBins = 65536;
 constexpr int kBinSites = 4;
 constexpr int kBinWaves = 4;  // wavefronts per block; those of a bin's blocks take its groups in turn
@@ -324,8 +335,9 @@ constexpr int kBinWaves = 4;  // wavefronts per block; those of a bin's blocks t
 // kBinShare, the sites that a block's wavefronts take in one turn, so that a crowded bin (a
 // long cutoff, a compressed box) is not left to four wavefronts.  Rebuild with the host's
 // part, one block per bin -> this: 4,000 LJ sites with a cutoff of 12 A (150 to a bin) 1.72
-// -> 0.65 ms, 32,000 with 16 A (348) 11.8 -> 4.3, 4,000 sites in a box of 9 A (500) 39.1 ->
-// 4.0; one block per 32 sites 0.77, 4.6 and 5.2.
+// -> 0.62 ms, 32,000 with 16 A (348) 11.8 -> 4.3, 4,000 sites in a box of 9 A (500) 39.1 ->
+// 4.0; a cluster of 4,000 with 16 A in a box of 20 cutoffs 3.21 -> 0.99 (the mean over the
+// occupied bins, not over the box, counts).
 constexpr int kBinShare = 16;
 inline int bin_blocks(double sites) {
     const double b = sites / kBinShare;

@@ -58,10 +58,12 @@ def test_lists_of_sparse_and_dense_boxes(tables, n, a):
     ff.close()
 
 
-@pytest.mark.parametrize("L,n,squeeze", [(200.0, 6, 1.0), (300.0, 6, 1.0), (300.0, 8, 0.3), (1500.0, 6, 1.0)])
+@pytest.mark.parametrize("L,n,squeeze", [(100.0, 8, 0.3), (200.0, 6, 1.0), (300.0, 6, 1.0), (300.0, 8, 0.3),
+                                         (1500.0, 6, 1.0)])
 def test_lists_of_nearly_empty_boxes(tables, L, n, squeeze):
-    """4 n^3 sites in two clusters, one across a corner: 5e4 bins (a block each), 1.7e5 (the list of the
-    occupied ones; squeezed, several blocks to each) and 1.8e7 (more than a launch holds blocks)"""
+    """4 n^3 sites in two clusters, one across a corner: 8e3 bins (squeezed, several blocks to each by the
+    mean of the occupied ones), 5e4 (a block each), 1.7e5 (the list of the occupied ones; squeezed, several
+    blocks to each) and 1.8e7 (more than a launch holds blocks)"""
     from mapp_amd import workload as W
     from mapp_amd.dmd import setup
     from oracle import oracle as O
