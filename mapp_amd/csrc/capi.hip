@@ -284,8 +284,9 @@ void rebuild(mapp_dmd* ctx) {
     const int natms = ctx->natms;
     hipStream_t st = ctx->stream;
     // the owned sites' bins, counted while the ghosts are built
-    ctx->d_bin_of.reserve(natms);
-    ctx->d_bin_slot.reserve(natms);
+    const size_t guess = (size_t)natms + natms / 4 + 8192;  // with ghosts, so that they rarely grow
+    ctx->d_bin_of.reserve(guess);
+    ctx->d_bin_slot.reserve(guess);
     ctx->d_bin_cnt.reserve((size_t)bp.tot_bin + 1);
     HIP_OK(hipMemsetAsync(ctx->d_bin_cnt.p, 0, sizeof(int) * ((size_t)bp.tot_bin + 1), st));
     auto bin = [&](int first, int n) {
